@@ -121,6 +121,19 @@ struct SymSet {
   int key = -1;
 };
 
+// Work units of the F(Q) spreading kernel, cached against the structure.
+struct SpreadSet {
+  Buf units, items;
+  Buf perm;    // int32 [n]: atom per position (weighted tables: element order)
+  Buf sorted;  // AtomRec [n]: positions in that order (weighted tables)
+  Buf grids;   // uint64 [chain][element pair][fq_grid_stride]: zero between calls
+  Buf done;    // int32 [chain]: zero between calls
+  bool dirty = false;  // a launch failed between spreading and transform
+  int n_units = 0, shift = 0;
+  uint64_t stamp = ~0ull;
+  int key = -1;
+};
+
 // One captured proposal and the parameters it was captured with.
 struct GraphSlot {
   hipGraph_t graph = nullptr;
@@ -180,6 +193,11 @@ struct pyiid_ctx {
   int max_elem = 0;
   Buf counts_d, natoms_d;
   uint64_t struct_stamp = 1;  // bumps when sizes / offsets / elements change
+  // Largest distance within a chain (a bound from its bounding sphere) of the
+  // positions seen last by ensure_extent or, for at most kExtentAtoms atoms,
+  // passed in host memory: sets scales and table lengths, never what is right.
+  double r_max = 0.0;
+  std::vector<int64_t> extent_off;  // the layout it was taken for
 
   Table tab[2];
   uint64_t tab_stamp[2] = {1, 1};
@@ -190,6 +208,7 @@ struct pyiid_ctx {
   bool t_set = false;
 
   ItemSet fq_items;     // unordered pairs, ranges per chain
+  SpreadSet spread;     // unordered pairs of the F(Q) spreading kernel
   ItemSet fused_items;  // ordered pairs with j splits, ranges per i tile
   ItemSet pair_items;   // tile pairs (I, J <= I) of the contracted-force kernel
   SymSet sym;           // unordered tile pairs of the symmetric F + gradient kernel
@@ -280,6 +299,53 @@ __global__ void unpack_kernel(const AtomRec* __restrict__ a, int64_t n, float* _
   p[3 * i + 0] = static_cast<float>(a[i].x);
   p[3 * i + 1] = static_cast<float>(a[i].y);
   p[3 * i + 2] = static_cast<float>(a[i].z);
+}
+
+// Positions up to this count have their extent taken on every host upload
+// (about 10 us at the limit); larger ones once per layout.
+constexpr int64_t kExtentAtoms = 4096;
+
+template <typename T>
+double chain_extent(const T* p, int stride, const std::vector<int64_t>& off) {
+  double r_max = 0.0;
+  for (size_t b = 0; b + 1 < off.size(); ++b) {
+    if (off[b + 1] - off[b] < 2) continue;
+    double lo[3], hi[3], mid[3];
+    for (int k = 0; k < 3; ++k) lo[k] = hi[k] = p[off[b] * stride + k];
+    for (int64_t a = off[b]; a < off[b + 1]; ++a)
+      for (int k = 0; k < 3; ++k) {
+        lo[k] = std::min<double>(lo[k], p[a * stride + k]);
+        hi[k] = std::max<double>(hi[k], p[a * stride + k]);
+      }
+    double diag = 0.0, rad = 0.0;
+    for (int k = 0; k < 3; ++k) {
+      mid[k] = 0.5 * (lo[k] + hi[k]);
+      diag += (hi[k] - lo[k]) * (hi[k] - lo[k]);
+    }
+    for (int64_t a = off[b]; a < off[b + 1]; ++a) {
+      double d = 0.0;
+      for (int k = 0; k < 3; ++k) d += (p[a * stride + k] - mid[k]) * (p[a * stride + k] - mid[k]);
+      rad = std::max(rad, d);
+    }
+    r_max = std::max(r_max, std::min(std::sqrt(diag), 2.0 * std::sqrt(rad)));
+  }
+  return r_max;
+}
+
+// r_max of the current layout, from the device positions when no host upload
+// gave it (once per layout; waits for the stream).
+int ensure_extent(pyiid_ctx* c) {
+  if (c->extent_off == c->off) return PYIID_OK;
+  if (c->capturing) return fail(PYIID_E_STATE, "structure changed during graph capture");
+  std::vector<double> h(static_cast<size_t>(c->n) * 4);
+  if (c->n > 0) {
+    HIPCHK(hipMemcpyAsync(h.data(), c->pos.p, sizeof(AtomRec) * c->n, hipMemcpyDeviceToHost,
+                          c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+  }
+  c->r_max = chain_extent(h.data(), 4, c->off);
+  c->extent_off = c->off;
+  return PYIID_OK;
 }
 
 int ensure_packed(pyiid_ctx* c) {
@@ -742,6 +808,158 @@ struct Timed {
   }
 };
 
+// ---- F(Q) by spreading ----
+
+// Largest grid buffer of the spreading path (grids of every chain and element
+// pair); beyond it the recurrence kernel runs.
+constexpr size_t kSpreadGridBudget = static_cast<size_t>(512) << 20;
+
+size_t spread_grid_bytes(pyiid_ctx* c, const Table& t) {
+  const size_t pairs =
+      weighted_table(t) ? static_cast<size_t>(t.n_elem) * (t.n_elem + 1) / 2 : 1;
+  return sizeof(uint64_t) * static_cast<size_t>(fq_grid_stride(t.nq)) * pairs * c->n_chain;
+}
+
+// Whether F(Q) runs on the spreading kernel: its grid fits LDS, the grids fit
+// their budget, and neither compensated sums nor a fixed shape of the
+// recurrence kernel is asked for.
+bool use_spread_fq(pyiid_ctx* c, const Table& t) {
+  return !c->compensated && c->fq_m_fixed == 0 &&
+         sizeof(uint64_t) * static_cast<size_t>(fq_grid_stride(t.nq)) <= kSpreadLds &&
+         spread_grid_bytes(c, t) <= kSpreadGridBudget;
+}
+
+// Atoms as positions in element order per chain (stable), and each chain's
+// element runs.
+struct ElemRun {
+  int64_t begin, end;
+  int elem;
+};
+void element_runs(pyiid_ctx* c, bool weighted, std::vector<int32_t>& perm,
+                  std::vector<std::vector<ElemRun>>& runs) {
+  perm.resize(static_cast<size_t>(c->n));
+  for (int64_t a = 0; a < c->n; ++a) perm[a] = static_cast<int32_t>(a);
+  runs.assign(static_cast<size_t>(c->n_chain), {});
+  for (int b = 0; b < c->n_chain; ++b) {
+    const int64_t o = c->off[b], e = c->off[b + 1];
+    if (o == e) continue;
+    if (!weighted || c->elem_h.empty()) {
+      runs[b].push_back(ElemRun{o, e, 0});
+      continue;
+    }
+    // counting sort by element
+    std::vector<int64_t> at(static_cast<size_t>(c->max_elem) + 2, 0);
+    for (int64_t a = o; a < e; ++a) at[c->elem_h[a] + 1]++;
+    for (size_t k = 1; k < at.size(); ++k) at[k] += at[k - 1];
+    for (size_t k = 0; k + 1 < at.size(); ++k)
+      if (at[k + 1] > at[k])
+        runs[b].push_back(ElemRun{o + at[k], o + at[k + 1], static_cast<int>(k)});
+    for (int64_t a = o; a < e; ++a) perm[o + at[c->elem_h[a]]++] = static_cast<int32_t>(a);
+  }
+}
+
+// Work units: per chain and element pair the (i tile, j range) items of its
+// pairs, cut so that the units of a pair have equal numbers of j steps.  A
+// single grid gets 512 units, one for each of the two blocks that a CU holds;
+// several grids about 1,536 (their sizes differ, so the last blocks to run
+// should be short), longest first.
+int ensure_spread(pyiid_ctx* c, const Table& t) {
+  SpreadSet& s = c->spread;
+  const bool weighted = weighted_table(t);
+  const int key = weighted ? t.n_elem : 0;
+  const size_t bytes = spread_grid_bytes(c, t);
+  CHK(ensure_extent(c));
+  if (s.stamp != c->struct_stamp || s.key != key) {
+    if (c->capturing) return fail(PYIID_E_STATE, "structure changed during graph capture");
+    std::vector<int32_t> perm;
+    std::vector<std::vector<ElemRun>> runs;
+    element_runs(c, weighted, perm, runs);
+    struct Group {
+      int64_t i0, i1, j0, j1;
+      int grid;
+      int64_t steps;
+    };
+    std::vector<Group> groups;
+    const int n_pair = weighted ? t.n_elem * (t.n_elem + 1) / 2 : 1;
+    int64_t total = 0, max_pairs = 0;
+    for (int b = 0; b < c->n_chain; ++b) {
+      const int64_t nb = c->off[b + 1] - c->off[b];
+      max_pairs = std::max(max_pairs, nb * (nb - 1) / 2);
+      for (size_t x = 0; x < runs[b].size(); ++x)
+        for (size_t y = 0; y <= x; ++y) {
+          const ElemRun &ri = runs[b][x], &rj = runs[b][y];
+          Group g{ri.begin, ri.end, rj.begin, rj.end,
+                  b * n_pair + ri.elem * (ri.elem + 1) / 2 + rj.elem, 0};
+          for (int64_t i = g.i0; i < g.i1; i += 64)
+            g.steps += std::min(g.j1, std::min(g.i1, i + 64)) - g.j0;
+          if (nb < 2) continue;
+          total += g.steps;
+          groups.push_back(g);
+        }
+    }
+    const int64_t target = groups.size() <= 1 ? 512 : 1536;
+    std::vector<SpreadItem> items;
+    std::vector<SpreadUnit> units;
+    std::vector<int64_t> cost;
+    for (const Group& g : groups) {
+      // at least 64 j steps a unit (4 for each of its 16 waves)
+      int64_t n_unit = (g.steps * target + total / 2) / std::max<int64_t>(1, total);
+      n_unit = std::max<int64_t>(1, std::min(n_unit, (g.steps + 63) / 64));
+      int64_t done = 0, u = 0;
+      int begin = static_cast<int>(items.size());
+      for (int64_t i = g.i0; i < g.i1; i += 64) {
+        const int64_t ie = std::min(g.i1, i + 64), je = std::min(g.j1, ie);
+        for (int64_t j = g.j0; j < je;) {
+          const int64_t limit = g.steps * (u + 1) / n_unit;
+          const int64_t take = std::min(je - j, limit - done);
+          if (take > 0) {
+            items.push_back(SpreadItem{static_cast<int>(i), static_cast<int>(ie),
+                                       static_cast<int>(j), static_cast<int>(j + take)});
+            j += take;
+            done += take;
+          }
+          if (done == limit) {
+            units.push_back(SpreadUnit{begin, static_cast<int>(items.size()), g.grid, 0});
+            cost.push_back(limit - g.steps * u / n_unit);
+            begin = static_cast<int>(items.size());
+            ++u;
+          }
+        }
+      }
+    }
+    if (groups.size() > 1) {
+      std::vector<size_t> ord(units.size());
+      for (size_t k = 0; k < ord.size(); ++k) ord[k] = k;
+      std::stable_sort(ord.begin(), ord.end(), [&](size_t x, size_t y) { return cost[x] > cost[y]; });
+      std::vector<SpreadUnit> v(units.size());
+      for (size_t k = 0; k < ord.size(); ++k) v[k] = units[ord[k]];
+      units.swap(v);
+    }
+    CHK(upload_vec(s.items, items));
+    CHK(upload_vec(s.units, units));
+    if (weighted) {
+      CHK(upload_vec(s.perm, perm));
+      CHK(s.sorted.reserve(sizeof(AtomRec) * std::max<int64_t>(1, c->n)));
+    }
+    s.n_units = static_cast<int>(units.size());
+    s.shift = 0;
+    while ((max_pairs >> 31) >> s.shift) ++s.shift;
+    s.stamp = c->struct_stamp;
+    s.key = key;
+  }
+  const size_t done_bytes = sizeof(int) * static_cast<size_t>(c->n_chain);
+  const bool grow = s.grids.bytes < bytes || s.done.bytes < done_bytes;
+  if (grow && c->capturing) return fail(PYIID_E_STATE, "structure changed during graph capture");
+  CHK(s.grids.reserve(bytes));
+  CHK(s.done.reserve(done_bytes));
+  if (grow || s.dirty) {
+    HIPCHK(hipMemsetAsync(s.grids.p, 0, s.grids.bytes, c->stream));
+    HIPCHK(hipMemsetAsync(s.done.p, 0, s.done.bytes, c->stream));
+    s.dirty = false;
+  }
+  return PYIID_OK;
+}
+
 int64_t min_chain_atoms(pyiid_ctx* c) {
   int64_t m = INT64_MAX;
   for (int b = 0; b < c->n_chain; ++b) m = std::min(m, c->off[b + 1] - c->off[b]);
@@ -770,6 +988,29 @@ int compute_fq(pyiid_ctx* c, int slot, double qbin) {
   CHK(c->fq32.reserve(sizeof(float) * (size_t)std::max(1, nq) * B));
   CHK(ensure_packed(c));
   CHK(ensure_norm(c, slot));
+  if (use_spread_fq(c, t)) {
+    CHK(ensure_spread(c, t));
+    SpreadSet& s = c->spread;
+    const bool weighted = weighted_table(t);
+    const double dq = static_cast<double>(static_cast<float>(qbin));
+    const AtomRec* sp = c->pos.as<AtomRec>();
+    if (weighted) {
+      HIPCHK(launch_gather(c->stream, sp, s.perm.as<int32_t>(), c->n, s.sorted.as<AtomRec>()));
+      sp = s.sorted.as<AtomRec>();
+    }
+    const int bits = fq_scale_bits(nq, dq, c->r_max);
+    s.dirty = true;
+    Timed tm(c, 1);
+    HIPCHK(launch_spread_fq(c->stream, sp, s.units.as<SpreadUnit>(), s.n_units,
+                            s.items.as<SpreadItem>(), nq, dq, s.shift, bits,
+                            s.grids.as<unsigned long long>()));
+    CHK(tm.done());
+    HIPCHK(launch_transform_fq(c->stream, s.grids.as<unsigned long long>(), B, t.n_elem, weighted,
+                               t.tab.as<float>(), nq, dq, s.shift, bits, t.fsu.as<double>(),
+                               c->fq64.as<double>(), c->fq32.as<float>(), s.done.as<int>()));
+    s.dirty = false;
+    return PYIID_OK;
+  }
   CHK(ensure_fq_items(c, weighted_table(t)));
   CHK(c->fpart.reserve(sizeof(double) * (size_t)std::max(1, c->fq_items.n_items) * nq));
   CHK(tune_fq(c, slot, qbin));
@@ -1267,6 +1508,10 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
   c->pos_set = true;
   c->pos_dirty = true;
   CHK(ensure_packed(c));
+  if (!(flags & PYIID_DEVICE) && n <= kExtentAtoms) {
+    c->r_max = chain_extent(pos, 3, c->off);
+    c->extent_off = c->off;
+  }
   return finish(c, flags);
 }
 
@@ -1738,7 +1983,9 @@ int pyiid_destroy(pyiid_ctx* c) {
   for (Buf* b : {&c->posf, &c->elem, &c->pos, &c->counts_d, &c->natoms_d, &c->tmat, &c->gpart,
                  &c->fpart, &c->fq64, &c->fq32, &c->g64, &c->io_a, &c->io_b,
                  &c->io_c, &c->w, &c->out5, &c->u, &c->gobs, &c->fq_items.items,
-                 &c->fq_items.ranges, &c->fq_items.perm, &c->fused_items.items, &c->fused_items.ranges,
+                 &c->fq_items.ranges, &c->fq_items.perm, &c->spread.units, &c->spread.items,
+                 &c->spread.perm, &c->spread.sorted, &c->spread.grids, &c->spread.done,
+                 &c->fused_items.items, &c->fused_items.ranges,
                  &c->fused_items.perm, &c->hmc.mass,
                  &c->hmc.mom, &c->hmc.fcur, &c->hmc.fnew, &c->hmc.pos_save, &c->hmc.kin0,
                  &c->hmc.ecur, &c->hmc.ehist, &c->hmc.acchist, &c->hmc.counter, &c->hmc.chains,

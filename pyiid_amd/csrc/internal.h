@@ -106,6 +106,38 @@ hipError_t launch_norm(hipStream_t st, const float* ftab, const int64_t* counts,
 hipError_t launch_pair_geometry(hipStream_t st, const AtomRec* pos, int64_t k_offset,
                                 int64_t k_count, float* d, float* r);
 
+// ---- F(Q) by spreading (spread.hip) ----
+// Item: positions [i0, i1) (at most 64) against positions [j0, j1), pairs
+// j < i.  Unit: items [begin, end) of one chain and element pair, added to
+// grid `grid`.
+struct SpreadItem {
+  int i0, i1, j0, j1;
+};
+struct SpreadUnit {
+  int begin, end, grid, pad;
+};
+constexpr size_t kSpreadLds = 160 * 1024;  // a block's grid lives in LDS
+int fq_grid_points(int nq);
+int fq_grid_stride(int nq);  // 64-bit words per grid (points, close-contact nodes, flag)
+// Bits of the grid's fixed point for distances up to about r_max.
+int fq_scale_bits(int nq, double dq, double r_max);
+// Spreads every unit's pairs and adds them to grids[unit.grid] (zero before
+// the first call; launch_transform_fq clears them again).  shift: right shift
+// of a unit's sums (0 up to 2^32 pairs).
+hipError_t launch_spread_fq(hipStream_t st, const AtomRec* pos, const SpreadUnit* units,
+                            int n_units, const SpreadItem* items, int nq, double dq, int shift,
+                            int scale_bits, unsigned long long* grids);
+// out[b][q] = scale[b][q] * sum over the chain's element pairs (grid index
+// b * n_pair + e_i (e_i + 1) / 2 + e_j, e_j <= e_i) of f_i f_j times the pair's
+// sum of sin(Q r) / r.  done: n_chain counters, zero before and after.
+hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_chain, int n_elem,
+                               bool weighted, const float* ftab, int nq, double dq, int shift,
+                               int scale_bits, const double* scale, double* out_f64,
+                               float* out_f32, int* done);
+// out[p] = pos[perm[p]]
+hipError_t launch_gather(hipStream_t st, const AtomRec* pos, const int32_t* perm, int64_t n,
+                         AtomRec* out);
+
 // ---- transform / potential (transform.hip) ----
 // C[m][ldc] = A[m][K] . B[n][K]^T in FP32 MFMA; A float or double.
 hipError_t launch_gemm_nt(hipStream_t st, const void* a, bool a_f64, int64_t m, int k,

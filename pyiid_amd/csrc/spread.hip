@@ -1,0 +1,350 @@
+// F(Q) by spreading the pair distances onto a fine grid (gfx950, wave64).
+//
+// F needs sum_{pairs} sin(Q_m r) / r on the bins Q_m = m dq: the transform of
+// a sum of point weights 1/r at the distances r onto equidistant bins.  A
+// recurrence per pair and bin costs pairs x bins; here every pair is handled
+// once, whatever the number of bins:
+//
+//  1. spread_fq_kernel adds the pair's weight to kFqW = 6 points of a grid of
+//     spacing h = 2 pi / (dq n_f), n_f = 12 n_q (six times finer than the
+//     bins need), with window values phi_j(y) that are polynomials of the
+//     pair's place y between the grid points;
+//  2. transform_fq_kernel sums grid[g] sin(2 pi g m / n_f) in FP64 and divides
+//     by the window's transform phihat(q), q = Q h.
+//
+// Window: phihat(q) = sinh(a) / a, a = sqrt(beta^2 - (3 q)^2), scaled to 1 at
+// q = 0 (the Kaiser-Bessel window's transform), and the phi_j(y) are the least
+// squares solution of sum_j phi_j(y) exp(i q (g_j - y)) = phihat(q) over the
+// band |q| <= pi / 6, fitted by polynomials of degree 5 in y.  The result is
+// exp(i Q r) to 2.3e-8 at worst and 3.6e-9 r.m.s. over the band and y
+// (coefficients rounded to float: 2.5e-8 r.m.s.; single-precision sin and cos
+// of the phase have 3e-8).
+//
+// The grid is folded: sin(2 pi g m / n_f) is odd about g = 0 and g = n_f / 2
+// and has period n_f, so a distance of any size is brought into [0, n_f / 2]
+// with a sign, and the grid has n_f / 2 + 7 points (3 beyond each end).
+//
+// Grid sums are 64-bit integers (fixed point): ds_add_u64 adds 64 lanes in
+// 4.8 ns per CU (ds_add_f64: 9.1 ns, ds_add_f32: 80 ns, ds_add_u32: 2.7 ns, at
+// random addresses), the sums are exact, and they do not depend on the order
+// in which waves and blocks add, so results repeat bit for bit.
+//
+// Reference semantics (pyIID): cpu_flat.py:77-114,
+// flat_multi_cpu_wrap.py:22-60.
+#include <algorithm>
+#include <cmath>
+
+#include "internal.h"
+
+namespace pyiid {
+namespace {
+
+// ---- window of the F grid ----
+constexpr int kFqW = 6;             // grid points per pair
+constexpr double kFqBeta = 15.160;  // window shape (smallest r.m.s. error at 6 points)
+// phi_j(y), j < 3, y in [-1/2, 1/2] about the middle of the window;
+// phi_{5-j}(y) = phi_j(-y)
+constexpr float kFqVal[3][6] = {
+    {0.000792858506f, -0.00591184293f, 0.0172319146f, -0.0255775783f, 0.0208579919f,
+     -0.00803987611f},
+    {0.0737481676f, -0.206023853f, 0.19830423f, -0.0388040482f, -0.062571443f, 0.0402357172f},
+    {0.425458973f, -0.352369105f, -0.215536146f, 0.244299265f, 0.041713486f, -0.0805066679f},
+};
+// Fixed point of the grid: phi_j 2^s / t, t = r / h.  s is chosen from the
+// structure's extent so that a pair at its largest distance still has 2^24
+// units (at most 2^25), and s >= 36.  From t = 2^(s - 31) on (0.7 A for a
+// particle of 85 A at 25 1/A) the value is below 2^31 and one int32 conversion
+// serves; closer pairs take spread_rare.
+constexpr int kFqBits = 24;
+constexpr int kFqMinScale = 36, kFqMaxScale = 48;
+// Below t = kFqClose the window's error over 1/r would show: there sin(Qr)/r,
+// an even function of r, is interpolated in r^2 from kFqNodes Chebyshev nodes
+// on (0, kFqClose h) (error below 1e-9 for Q h <= pi / 6).  Their weights
+// follow the grid, scaled by 2^30.
+constexpr double kFqClose = 2.0;
+constexpr int kFqNodes = 5;
+constexpr double kNodeScale = 1073741824.0;
+
+__host__ __device__ inline double fq_node(int k) {  // t of node k
+  constexpr double c[kFqNodes] = {0.98768834059513773, 0.89100652418836787, 0.70710678118654752,
+                                  0.45399049973954675, 0.15643446504023087};  // cos((2k+1) pi/20)
+  return kFqClose * c[k];
+}
+
+// ---- spreading ----
+
+// Brings t = r / h into [0, n_f / 2]; neg: the reflected half (sin changes sign).
+__device__ __forceinline__ double fold(double t, double nf, bool& neg) {
+  const double u = t - nf * floor(t / nf);
+  neg = u > 0.5 * nf;
+  return neg ? nf - u : u;
+}
+
+// A pair closer than the fixed point's fast range, or at an infinite
+// distance: 64-bit conversions.  Few pairs of a physical structure come here.
+__device__ __noinline__ void spread_rare(unsigned long long* hist, int n_grid, double t, double nf,
+                                         double scale) {
+  unsigned long long* nodes = hist + n_grid;
+  if (!(t < 1e300)) {  // infinite: F is not a number
+    atomicAdd(&nodes[kFqNodes], 1ull);
+    return;
+  }
+  if (t < kFqClose) {
+    const double s = t * t;
+    for (int k = 0; k < kFqNodes; ++k) {
+      double l = 1.0;
+      for (int j = 0; j < kFqNodes; ++j)
+        if (j != k) l *= (s - fq_node(j) * fq_node(j)) / (fq_node(k) * fq_node(k) - fq_node(j) * fq_node(j));
+      atomicAdd(&nodes[k], static_cast<unsigned long long>(static_cast<long long>(rint(l * kNodeScale))));
+    }
+    return;
+  }
+  bool neg;
+  const double tf = fold(t, nf, neg);
+  const double fl = floor(tf);
+  const double y = tf - fl - 0.5, w = (neg ? -scale : scale) / t;
+  unsigned long long* h = hist + (static_cast<int>(fl) + 1);
+  for (int j = 0; j < kFqW; ++j) {
+    const float* c = kFqVal[j < 3 ? j : kFqW - 1 - j];
+    const double z = j < 3 ? y : -y;
+    double p = c[5];
+    for (int k = 4; k >= 0; --k) p = p * z + static_cast<double>(c[k]);
+    atomicAdd(&h[j], static_cast<unsigned long long>(static_cast<long long>(rint(p * w))));
+  }
+}
+
+// One block (16 waves) per work unit: a run of items of one chain and element
+// pair, whose pairs are spread into the block's grid in LDS, then added to the
+// chain's grid in global memory.  An item is an i tile of at most 64 positions
+// (one lane each) against a j range; the 16 waves take consecutive slices of
+// the range, and a j atom's position is wave-uniform (scalar loads, so the
+// FP64 differences take it from SGPRs).
+//
+// Per 64 pairs about 16 FP64 or conversion instructions (distance to 1e-14:
+// a phase of 1,500 rad to 1e-11), 18 FMAs for the window, 6 conversions to
+// integer and 6 ds_add_u64.  The LDS adds (29 ns per CU) and the VALU (about
+// as long, 4 SIMDs) run side by side, and 2 blocks (32 waves) per CU hide
+// each other's latency.
+__global__ __launch_bounds__(1024, 2) void spread_fq_kernel(
+    const AtomRec* __restrict__ pos, const SpreadUnit* __restrict__ units,
+    const SpreadItem* __restrict__ items, double inv_h, int nf, int n_grid, int stride, int shift,
+    float scale, double near, unsigned long long* __restrict__ grids) {
+  extern __shared__ unsigned long long hist[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n_wave = blockDim.x >> 6;
+  for (int g = threadIdx.x; g < stride; g += blockDim.x) hist[g] = 0ull;
+  __syncthreads();
+  const SpreadUnit un = units[blockIdx.x];
+  const double half_nf = 0.5 * nf;
+  for (int it = un.begin; it < un.end; ++it) {
+    const SpreadItem item = items[it];
+    const int len = item.j1 - item.j0;
+    const int jb = item.j0 + static_cast<int>(static_cast<int64_t>(len) * wave / n_wave);
+    const int je = item.j0 + static_cast<int>(static_cast<int64_t>(len) * (wave + 1) / n_wave);
+    const int i = item.i0 + lane;
+    const bool have = i < item.i1;
+    const AtomRec pi = pos[have ? i : item.i0];
+    for (int j = jb; j < je; ++j) {
+      const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
+      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+      // j < i; a pair at distance 0 (and one with a NaN) contributes nothing
+      if (!(have && j < i && r2 > 0.0)) continue;
+      // FP32 root refined by one Newton step in FP64
+      const float r2f = static_cast<float>(r2);
+      const float y0 = __builtin_amdgcn_rsqf(r2f);
+      const float rf = r2f * y0;
+      const double rd = static_cast<double>(rf);
+      const double r = fma(fma(-rd, rd, r2), static_cast<double>(0.5f * y0), rd);
+      double t = r * inv_h;
+      if (!(t >= near && t <= half_nf)) {
+        // (r2 outside float's range reaches this branch with any r: take the
+        // FP64 root)
+        const double ta = sqrt(r2) * inv_h;
+        if (!(ta >= near && ta < 1e300)) {
+          spread_rare(hist, n_grid, ta, static_cast<double>(nf), static_cast<double>(scale));
+          continue;
+        }
+        t = ta;
+      }
+      float w = scale * __builtin_amdgcn_rcpf(static_cast<float>(t));
+      if (t > half_nf) {
+        bool neg;
+        t = fold(t, static_cast<double>(nf), neg);
+        if (neg) w = -w;
+      }
+      const double fl = floor(t);
+      const float y = static_cast<float>(t - fl) - 0.5f;
+      const float half = __builtin_copysignf(0.5f, w);
+      const float y2 = y * y;
+      unsigned long long* h = hist + (static_cast<int>(fl) + 1);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const float e = fmaf(fmaf(kFqVal[k][4], y2, kFqVal[k][2]), y2, kFqVal[k][0]);
+        const float o = y * fmaf(fmaf(kFqVal[k][5], y2, kFqVal[k][3]), y2, kFqVal[k][1]);
+        // truncation after + 1/2 rounds to nearest
+        const int a = static_cast<int>(fmaf(e + o, w, half));
+        const int b = static_cast<int>(fmaf(e - o, w, half));
+        atomicAdd(&h[k], static_cast<unsigned long long>(static_cast<long long>(a)));
+        atomicAdd(&h[kFqW - 1 - k], static_cast<unsigned long long>(static_cast<long long>(b)));
+      }
+    }
+  }
+  __syncthreads();
+  unsigned long long* out = grids + static_cast<size_t>(un.grid) * stride;
+  for (int g = threadIdx.x; g < stride; g += blockDim.x) {
+    const long long v = static_cast<long long>(hist[g]);
+    if (v == 0) continue;
+    const long long s = (shift == 0 || g == n_grid + kFqNodes) ? v : (v + (1ll << (shift - 1))) >> shift;
+    atomicAdd(&out[g], static_cast<unsigned long long>(s));
+  }
+}
+
+// ---- grid -> F(Q) ----
+
+constexpr int kTrChunk = 4096;  // grid points in LDS at a time (32 KiB)
+
+// One block: 64 bins (lanes) of one chain; its 16 waves take consecutive
+// slices of every chunk of grid points.  sin(2 pi g m / n_f) starts from an
+// exact phase and follows the FP64 three-term recurrence along g.  The last
+// block of a chain to finish clears the chain's grids for the next call, so
+// no launch is spent on it.
+__global__ __launch_bounds__(1024) void transform_fq_kernel(
+    unsigned long long* __restrict__ grids, int n_pair, int n_elem, int nf, int n_grid, int stride,
+    int shift, int scale_bits, const float* __restrict__ ftab, int nq, double inv_h, int weighted,
+    const double* __restrict__ scale, double* __restrict__ out64, float* __restrict__ out32,
+    int* __restrict__ done) {
+  __shared__ double buf[kTrChunk];
+  __shared__ double part[16][65];
+  __shared__ int last;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m = blockIdx.x * 64 + lane;
+  const int b = blockIdx.y;
+  unsigned long long* chain = grids + static_cast<size_t>(b) * n_pair * stride;
+  const double unit = ldexp(inv_h, shift - scale_bits);
+  const double node_unit = ldexp(inv_h, shift) / kNodeScale;
+  const double two_over = 2.0 / static_cast<double>(nf);
+  const double c2 = 2.0 * cospi(two_over * m);
+  const double q = M_PI * two_over * m;  // Q h
+  const double a2 = kFqBeta * kFqBeta - 0.25 * kFqW * kFqW * q * q;
+  const double a = sqrt(a2 > 1.0 ? a2 : 1.0);
+  const double inv_phihat = (sinh(kFqBeta) / kFqBeta) / (sinh(a) / a);
+  double total = 0.0;
+  int ei = 0, ej = 0;
+  for (int p = 0; p < n_pair; ++p) {
+    const unsigned long long* h = chain + static_cast<size_t>(p) * stride;
+    double acc = 0.0;
+    for (int g0 = 0; g0 < n_grid; g0 += kTrChunk) {
+      const int cnt = min(kTrChunk, n_grid - g0);
+      __syncthreads();
+      for (int g = threadIdx.x; g < cnt; g += blockDim.x)
+        buf[g] = static_cast<double>(static_cast<long long>(h[g0 + g]));
+      __syncthreads();
+      const int lo = cnt * wave / 16, hi = cnt * (wave + 1) / 16;
+      // phases of grid points g0 + lo - 3 and one before, reduced as integers
+      const long long s0 = static_cast<long long>(g0 + lo - 3) * m % nf;
+      const long long s1 = static_cast<long long>(g0 + lo - 4) * m % nf;
+      double y = sinpi(two_over * static_cast<double>(s0));
+      double yp = sinpi(two_over * static_cast<double>(s1));
+      for (int g = lo; g < hi; ++g) {
+        acc = fma(buf[g], y, acc);
+        const double yn = fma(c2, y, -yp);
+        yp = y;
+        y = yn;
+      }
+    }
+    acc *= unit * inv_phihat;
+    if (wave == 0) {  // close contacts (almost always none)
+      for (int k = 0; k < kFqNodes; ++k) {
+        const long long v = static_cast<long long>(h[n_grid + k]);
+        if (v != 0) acc += static_cast<double>(v) * node_unit * sin(q * fq_node(k)) / fq_node(k);
+      }
+      if (h[n_grid + kFqNodes] != 0ull) acc = __builtin_nan("");
+    }
+    if (m < nq) {
+      const double f = weighted ? static_cast<double>(ftab[static_cast<size_t>(ei) * nq + m]) *
+                                      static_cast<double>(ftab[static_cast<size_t>(ej) * nq + m])
+                                : 1.0;
+      total = fma(f, acc, total);
+    }
+    if (++ej > ei) {
+      ++ei;
+      ej = 0;
+    }
+  }
+  part[wave][lane] = total;
+  __syncthreads();
+  if (wave == 0 && m < nq) {
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) t += part[k][lane];
+    const size_t o = static_cast<size_t>(b) * nq + m;
+    const double v = t * scale[o];
+    if (out64) out64[o] = v;
+    if (out32) out32[o] = static_cast<float>(v);
+  }
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(&done[b], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+           static_cast<int>(gridDim.x) - 1;
+  __syncthreads();
+  if (!last) return;
+  const size_t all = static_cast<size_t>(n_pair) * stride;
+  for (size_t g = threadIdx.x; g < all; g += blockDim.x) chain[g] = 0ull;
+  if (threadIdx.x == 0) done[b] = 0;
+}
+
+__global__ void gather_kernel(const AtomRec* __restrict__ pos, const int32_t* __restrict__ perm,
+                              int n, AtomRec* __restrict__ out) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < n) out[p] = pos[perm[p]];
+}
+
+}  // namespace
+
+int fq_grid_points(int nq) { return 6 * nq + 7; }
+int fq_grid_stride(int nq) { return (fq_grid_points(nq) + kFqNodes + 2) & ~1; }
+int fq_scale_bits(int nq, double dq, double r_max) {
+  const double t = r_max * dq * 12.0 * nq / (2.0 * M_PI);
+  if (!(t < 1e30)) return kFqMinScale;
+  int e = kFqMinScale;
+  while (e < kFqMaxScale && std::ldexp(1.0, e - kFqBits) < t) ++e;
+  return e;
+}
+
+hipError_t launch_spread_fq(hipStream_t st, const AtomRec* pos, const SpreadUnit* units,
+                            int n_units, const SpreadItem* items, int nq, double dq, int shift,
+                            int scale_bits, unsigned long long* grids) {
+  if (n_units == 0) return hipSuccess;
+  const int nf = 12 * nq, stride = fq_grid_stride(nq);
+  const size_t lds = sizeof(unsigned long long) * static_cast<size_t>(stride);
+  if (lds > kSpreadLds) return hipErrorInvalidValue;
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(spread_fq_kernel),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kSpreadLds));
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL(spread_fq_kernel, dim3(n_units), dim3(1024), lds, st, pos, units, items,
+                     dq * nf / (2.0 * M_PI), nf, fq_grid_points(nq), stride, shift,
+                     std::ldexp(1.0f, scale_bits), std::ldexp(1.0, scale_bits - 31), grids);
+  return hipGetLastError();
+}
+
+hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_chain, int n_elem,
+                               bool weighted, const float* ftab, int nq, double dq, int shift,
+                               int scale_bits, const double* scale, double* out_f64, float* out_f32, int* done) {
+  const int nf = 12 * nq;
+  const int n_pair = weighted ? n_elem * (n_elem + 1) / 2 : 1;
+  hipLaunchKernelGGL(transform_fq_kernel, dim3((nq + 63) / 64, n_chain), dim3(1024), 0, st, grids,
+                     n_pair, n_elem, nf, fq_grid_points(nq), fq_grid_stride(nq), shift, scale_bits,
+                     ftab, nq, dq * nf / (2.0 * M_PI), weighted ? 1 : 0, scale, out_f64, out_f32, done);
+  return hipGetLastError();
+}
+
+hipError_t launch_gather(hipStream_t st, const AtomRec* pos, const int32_t* perm, int64_t n,
+                         AtomRec* out) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(gather_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st,
+                     pos, perm, static_cast<int>(n), out);
+  return hipGetLastError();
+}
+
+}  // namespace pyiid

@@ -1,0 +1,126 @@
+"""The spreading kernels (F(Q) from pair distances put onto a fine grid)
+against the FP64 oracle where they can go wrong: tile and bin remainders,
+distances folded at the grid's period, close contacts, duplicated atoms,
+several elements, batches.
+
+Tolerance, derived from the kernel's arithmetic: a pair's term sin(Qr)/r is
+off by at most 6.6e-8 / r (window 2.3e-8 and its single-precision values), so
+F by 6.6e-8 of the sum of its pair weights 1/r, plus the rounding of the
+float32 result; twice that is allowed."""
+import numpy as np
+import pytest
+
+from oracle import scatter as oracle
+from pyiid_amd import _lib, structures
+from pyiid_amd.formfactors import element_table
+
+pytestmark = pytest.mark.gpu
+
+
+def load(ctx, pos, numbers, qbin, nq):
+    table, index, _ = element_table(numbers, qbin, nq)
+    ctx.set_positions(pos)
+    ctx.set_elements(index)
+    ctx.set_scatter(_lib.SLOT_FQ, table)
+    return table[index]
+
+
+def bound(pos, per_atom, want):
+    """Twice the error the arithmetic allows, per bin."""
+    p = pos.astype(np.float64)
+    i, j = np.tril_indices(len(pos), -1)
+    r = np.linalg.norm(p[i] - p[j], axis=1)
+    inv = np.divide(1.0, r, out=np.zeros_like(r), where=r > 0)
+    f = per_atom.astype(np.float64)
+    w = np.einsum("k,kq,kq->q", inv, np.abs(f[i]), np.abs(f[j]))
+    na = np.abs(oracle.normalization(per_atom))
+    return 2 * (6.6e-8 * 2 * w / na + 6e-8 * np.abs(want)) + 1e-30
+
+
+def debye(pos, per_atom, qbin):
+    """The oracle's F(Q); with duplicated atoms (for which the oracle zeroes
+    every bin, as the reference's NaN does) the FP64 sum over the other pairs."""
+    i, j = np.tril_indices(len(pos), -1)
+    p, f = pos.astype(np.float64), per_atom.astype(np.float64)
+    r = np.linalg.norm(p[i] - p[j], axis=1)
+    if np.all(r > 0):
+        return oracle.fq(pos, per_atom, qbin)
+    i, j, r = i[r > 0], j[r > 0], r[r > 0]
+    q = oracle.q_values(qbin, per_atom.shape[1])
+    return 2.0 / oracle.normalization(per_atom) * np.sum(
+        f[i] * f[j] * np.sin(np.outer(r, q)) / r[:, None], axis=0)
+
+
+def check(ctx, pos, numbers, qbin, nq):
+    per_atom = load(ctx, pos, numbers, qbin, nq)
+    got = ctx.fq(_lib.SLOT_FQ, qbin, nq)
+    want = debye(pos, per_atom, qbin)
+    off = np.abs(got - want) / bound(pos, per_atom, want)
+    assert np.all(np.isfinite(got)) and off.max() < 1.0, (off.argmax(), off.max())
+
+
+@pytest.mark.parametrize("n", [2, 3, 63, 64, 65, 129, 300])
+@pytest.mark.parametrize("nq", [1, 2, 7, 32, 65, 330])
+def test_tiles_and_bins(ctx, n, nq):
+    pos = structures.jitter(structures.fcc_nearest(n), 0.05, seed=n).astype(np.float32)
+    check(ctx, pos, np.full(n, 79), 25.0 / nq, nq)
+
+
+def test_largest_grid(ctx):
+    pos = structures.jitter(structures.fcc_nearest(40), 0.05, seed=1).astype(np.float32)
+    for nq in (3400, 3420):  # the last with a grid in LDS, and past it (recurrence kernel)
+        check(ctx, pos, np.full(len(pos), 79), 0.008, nq)
+
+
+@pytest.mark.parametrize("length", [30.0, 314.0, 4e3, 3e5])
+def test_distances_beyond_the_period(ctx, length):
+    """Periods of the 0.1 bins: 62.8 A; the distances span many of them, and
+    one is an exact multiple."""
+    rs = np.random.RandomState(3)
+    pos = rs.uniform(-length, length, (90, 3)).astype(np.float32)
+    pos[0], pos[1] = 0.0, (np.float32(4 * np.pi / np.float32(0.1)), 0, 0)
+    check(ctx, pos, np.full(90, 79), 0.1, 250)
+
+
+@pytest.mark.parametrize("r", [1e-6, 1e-3, 0.02, 0.0418, 0.042, 0.2, 0.355, 0.36, 1.0])
+def test_close_contacts(ctx, r):
+    """A pair at each of the kernel's short ranges (grid spacing 0.0209 A:
+    interpolation below 2, 64-bit conversion below 17 of them), beside a
+    duplicated atom, which contributes nothing."""
+    pos = structures.jitter(structures.fcc_nearest(50), 0.05, seed=5).astype(np.float32)
+    pos[7] = 0.0
+    pos[20] = (r, 0, 0)
+    pos[31] = pos[30]
+    check(ctx, pos, np.full(50, 79), 0.1, 250)
+
+
+def test_elements_and_batch(ctx):
+    """Three elements in one particle, and a batch whose chains hold one
+    atom, one element, and all three; a second call sees cleared grids."""
+    rs = np.random.RandomState(8)
+    zs = np.array([28, 78, 79])
+    pos = structures.jitter(structures.fcc_nearest(210), 0.05, seed=9).astype(np.float32)
+    check(ctx, pos, zs[rs.randint(0, 3, 210)], 0.05, 500)
+    qbin, nq = 0.0756865, 330
+    numbers = [np.array([79]), np.full(70, 28), zs[rs.randint(0, 3, 131)], np.array([78, 79])]
+    chains = [structures.jitter(structures.fcc_nearest(len(z)), 0.05, seed=len(z)).astype(np.float32)
+              for z in numbers]
+    table, index, elems = element_table(np.concatenate(numbers), qbin, nq)
+    ctx.set_batch(chains)
+    ctx.set_elements(index)
+    ctx.set_scatter(_lib.SLOT_FQ, table)
+    first = ctx.fq(_lib.SLOT_FQ, qbin, nq, n_chain=4)
+    again = ctx.fq(_lib.SLOT_FQ, qbin, nq, n_chain=4)
+    np.testing.assert_array_equal(first, again)
+    assert not np.any(first[0])
+    for b in (1, 2, 3):
+        per_atom = table[np.searchsorted(elems, numbers[b])]
+        want = oracle.fq(chains[b], per_atom, qbin)
+        assert np.all(np.abs(first[b] - want) < bound(chains[b], per_atom, want))
+
+
+def test_infinite_position_is_not_a_number(ctx):
+    pos = structures.fcc_nearest(20).astype(np.float32)
+    pos[3, 0] = np.inf
+    load(ctx, pos, np.full(20, 79), 0.1, 100)
+    assert np.all(np.isnan(ctx.fq(_lib.SLOT_FQ, 0.1, 100)[1:]))
