@@ -134,6 +134,16 @@ struct SpreadSet {
   int key = -1;
 };
 
+// Work units and tables of the contracted-force kernel, cached against the
+// structure (the table length follows the structure's extent).
+struct ForceSet {
+  Buf units, planes, perm, sorted;  // sorted: positions in perm order (weighted tables)
+  Buf t4, t2, part;
+  int n_units = 0, n_planes = 0;
+  uint64_t stamp = ~0ull;
+  int key = -1;
+};
+
 // One captured proposal and the parameters it was captured with.
 struct GraphSlot {
   hipGraph_t graph = nullptr;
@@ -209,6 +219,7 @@ struct pyiid_ctx {
 
   ItemSet fq_items;     // unordered pairs, ranges per chain
   SpreadSet spread;     // unordered pairs of the F(Q) spreading kernel
+  ForceSet force;       // ordered pairs of the contracted-force kernel
   ItemSet fused_items;  // ordered pairs with j splits, ranges per i tile
   ItemSet pair_items;   // tile pairs (I, J <= I) of the contracted-force kernel
   SymSet sym;           // unordered tile pairs of the symmetric F + gradient kernel
@@ -1407,13 +1418,151 @@ int tune_grad(pyiid_ctx* c, int slot, double qbin) {
   return best_k ? PYIID_OK : tune_fused(c, slot, qbin);
 }
 
-// forces (n x 3 doubles) = scale * sum_q u[chain][q] grad(i, c, q), by the
-// unordered-pair contracted-force kernel.
+// ---- contracted forces from a pair-force table ----
+
+void destroy_graph(Hmc& h);
+
+constexpr size_t kForceTableBudget = static_cast<size_t>(512) << 20;
+
+// Cells of the force table: the structure's extent and a tenth more (atoms
+// that move farther still get their force, from the sums themselves).
+int64_t force_cells(pyiid_ctx* c, const Table& t, double dq) {
+  const double cells = 1.1 * c->r_max / force_cell(t.nq, dq) + 8.0;
+  return cells < 1e9 ? static_cast<int64_t>(cells) : static_cast<int64_t>(1e9);
+}
+
+// Whether the tables fit LDS and their budget (else the recurrence kernel runs).
+bool use_force_table(pyiid_ctx* c, const Table& t, double dq) {
+  const int64_t cells = force_cells(c, t, dq);
+  const int64_t pairs =
+      weighted_table(t) ? static_cast<int64_t>(t.n_elem) * (t.n_elem + 1) / 2 : 1;
+  return force_lds_bytes(cells) <= kForceLds && pairs * c->n_chain <= 65535 &&
+         24.0 * static_cast<double>(cells) * pairs * c->n_chain <=
+             static_cast<double>(kForceTableBudget);
+}
+
+// Units: per chain the i tiles of each element against each element's j run.
+// A wave should have about `steps` j steps: total work over the 8,192 waves
+// that the chip holds, at least 16 and at most 1,024 (a block loads its table,
+// so it should not be shorter than needed).  The slices of a tile's range are
+// the waves of a block as far as they go, and planes beyond that.
+int ensure_force(pyiid_ctx* c, const Table& t) {
+  ForceSet& s = c->force;
+  const bool weighted = weighted_table(t);
+  const int key = weighted ? t.n_elem : 0;
+  if (s.stamp == c->struct_stamp && s.key == key) return PYIID_OK;
+  if (c->capturing) return fail(PYIID_E_STATE, "structure changed during graph capture");
+  std::vector<int32_t> perm;
+  std::vector<std::vector<ElemRun>> runs;
+  element_runs(c, weighted, perm, runs);
+  int64_t total = 0;
+  for (int b = 0; b < c->n_chain; ++b)
+    for (const ElemRun& r : runs[b])
+      total += (r.end - r.begin + 63) / 64 * (c->off[b + 1] - c->off[b]);
+  const int64_t steps = std::min<int64_t>(1024, std::max<int64_t>(16, total / 8192));
+  const int n_pair = weighted ? t.n_elem * (t.n_elem + 1) / 2 : 1;
+  std::vector<ForceUnit> units;
+  std::vector<int32_t> planes(static_cast<size_t>(std::max<int64_t>(1, c->n)), 0);
+  int n_planes = 1;
+  for (int b = 0; b < c->n_chain; ++b) {
+    if (c->off[b + 1] - c->off[b] < 2) continue;
+    for (const ElemRun& ri : runs[b]) {
+      int plane = 0;
+      for (const ElemRun& rj : runs[b]) {
+        const int64_t len = rj.end - rj.begin, slices = (len + steps - 1) / steps;
+        int in_block = 1;
+        while (in_block < 16 && in_block < slices) in_block *= 2;
+        const int tiles = 16 / in_block;
+        const int64_t n_split = (slices + in_block - 1) / in_block;
+        const int hi = std::max(ri.elem, rj.elem), lo = std::min(ri.elem, rj.elem);
+        const int table = b * n_pair + hi * (hi + 1) / 2 + lo;
+        for (int64_t sp = 0; sp < n_split; ++sp, ++plane)
+          for (int64_t i = ri.begin; i < ri.end; i += 64 * tiles)
+            units.push_back(ForceUnit{static_cast<int>(i),
+                                      static_cast<int>(std::min(ri.end, i + 64 * tiles)),
+                                      static_cast<int>(rj.begin + len * sp / n_split),
+                                      static_cast<int>(rj.begin + len * (sp + 1) / n_split), tiles,
+                                      plane, table, b, weighted ? ri.elem : -1,
+                                      weighted ? rj.elem : -1, 0, 0});
+      }
+      for (int64_t p = ri.begin; p < ri.end; ++p) planes[p] = plane;
+      n_planes = std::max(n_planes, plane);
+    }
+  }
+  // longest first
+  std::stable_sort(units.begin(), units.end(), [](const ForceUnit& x, const ForceUnit& y) {
+    return static_cast<int64_t>(x.j1 - x.j0) * x.tiles > static_cast<int64_t>(y.j1 - y.j0) * y.tiles;
+  });
+  CHK(upload_vec(s.units, units));
+  CHK(upload_vec(s.planes, planes));
+  if (weighted) {
+    CHK(upload_vec(s.perm, perm));
+    CHK(s.sorted.reserve(sizeof(AtomRec) * std::max<int64_t>(1, c->n)));
+  }
+  s.n_units = static_cast<int>(units.size());
+  s.n_planes = n_planes;
+  s.stamp = c->struct_stamp;
+  s.key = key;
+  return PYIID_OK;
+}
+
+// out5 (5 values per chain) and, behind them, the flag of a pair past the
+// force table.
+int reserve_out5(pyiid_ctx* c, int n_chain) {
+  const size_t want = sizeof(double) * (5 * static_cast<size_t>(n_chain) + 1);
+  if (want > c->out5.bytes) {
+    CHK(c->out5.reserve(want));
+    HIPCHK(hipMemsetAsync(c->out5.p, 0, c->out5.bytes, c->stream));
+  }
+  return PYIID_OK;
+}
+
+// A pair lay past the force table: take the extent anew for the next call.
+int note_far(pyiid_ctx* c, double flag) {
+  if (flag == 0.0) return PYIID_OK;
+  c->extent_off.clear();
+  destroy_graph(c->hmc);
+  HIPCHK(hipMemsetAsync(c->out5.as<double>() + 5 * static_cast<size_t>(c->n_chain), 0,
+                        sizeof(double), c->stream));
+  return PYIID_OK;
+}
+
+// forces (n x 3 doubles) = scale * sum_q u[chain][q] grad(i, c, q).
 int contract_forces(pyiid_ctx* c, int slot, double qbin, double scale, double* out) {
   Table& t = c->tab[slot];
   const int nq = t.nq, B = c->n_chain;
   CHK(ensure_packed(c));
   CHK(ensure_norm(c, slot));
+  CHK(ensure_extent(c));
+  const double dq = static_cast<double>(static_cast<float>(qbin));
+  if (use_force_table(c, t, dq)) {
+    CHK(ensure_force(c, t));
+    ForceSet& s = c->force;
+    const bool weighted = weighted_table(t);
+    const int n_cell = static_cast<int>(force_cells(c, t, dq));
+    const size_t cells = static_cast<size_t>(n_cell) * B *
+                         (weighted ? t.n_elem * (t.n_elem + 1) / 2 : 1);
+    CHK(s.t4.reserve(sizeof(float4) * cells));
+    CHK(s.t2.reserve(sizeof(float2) * cells));
+    CHK(s.part.reserve(sizeof(double) * 3 * static_cast<size_t>(std::max<int64_t>(1, c->n)) *
+                       s.n_planes));
+    const AtomRec* sp = c->pos.as<AtomRec>();
+    if (weighted) {
+      HIPCHK(launch_gather(c->stream, sp, s.perm.as<int32_t>(), c->n, s.sorted.as<AtomRec>()));
+      sp = s.sorted.as<AtomRec>();
+    }
+    Timed tm(c, 4);
+    HIPCHK(launch_force_table(c->stream, c->u.as<float>(), t.tab.as<float>(), nq, dq, weighted,
+                              t.n_elem, B, n_cell, s.t4.as<float4>(), s.t2.as<float2>()));
+    HIPCHK(launch_table_force(c->stream, sp, s.units.as<ForceUnit>(), s.n_units, n_cell,
+                              s.t4.as<float4>(), s.t2.as<float2>(), c->u.as<float>(),
+                              t.tab.as<float>(), nq, dq, c->n, s.part.as<double>(),
+                              c->out5.as<double>() + 5 * static_cast<size_t>(B)));
+    CHK(tm.done());
+    HIPCHK(launch_reduce_force(c->stream, s.part.as<double>(), c->n, s.planes.as<int32_t>(),
+                               weighted ? s.perm.as<int32_t>() : nullptr, scale, out));
+    return PYIID_OK;
+  }
   CHK(c->uq.reserve(sizeof(float) * static_cast<size_t>(std::max(1, nq)) * B));
   HIPCHK(launch_uq(c->stream, c->u.as<float>(), B, nq,
                    static_cast<double>(static_cast<float>(qbin)), c->uq.as<float>()));
@@ -1444,7 +1593,7 @@ int energy_forces_device(pyiid_ctx* c, int slot, double qbin, int potential,
   CHK(compute_fq(c, slot, qbin));
   CHK(c->g64.reserve(sizeof(double) * (size_t)nr * B));
   CHK(gemm_t(c, c->fq32.p, false, B, c->g64.as<double>()));
-  CHK(c->out5.reserve(sizeof(double) * 5 * B));
+  CHK(reserve_out5(c, B));
   CHK(c->w.reserve(sizeof(double) * (size_t)nr * B));
   HIPCHK(launch_potential(c->stream, potential, gobs_dev, c->g64.as<double>(), nr, B,
                           c->out5.as<double>(), c->w.as<double>()));
@@ -1985,6 +2134,8 @@ int pyiid_destroy(pyiid_ctx* c) {
                  &c->io_c, &c->w, &c->out5, &c->u, &c->gobs, &c->fq_items.items,
                  &c->fq_items.ranges, &c->fq_items.perm, &c->spread.units, &c->spread.items,
                  &c->spread.perm, &c->spread.sorted, &c->spread.grids, &c->spread.done,
+                 &c->force.units, &c->force.planes, &c->force.perm, &c->force.sorted,
+                 &c->force.t4, &c->force.t2, &c->force.part,
                  &c->fused_items.items, &c->fused_items.ranges,
                  &c->fused_items.perm, &c->hmc.mass,
                  &c->hmc.mom, &c->hmc.fcur, &c->hmc.fnew, &c->hmc.pos_save, &c->hmc.kin0,
@@ -2428,7 +2579,7 @@ int pyiid_potential(pyiid_ctx* c, int potential, const double* gobs, const doubl
   CHK(c->io_a.reserve(sizeof(double) * n));
   CHK(c->io_b.reserve(sizeof(double) * n));
   CHK(c->w.reserve(sizeof(double) * n));
-  CHK(c->out5.reserve(sizeof(double) * 5));
+  CHK(reserve_out5(c, c->n_chain));
   CHK(upload(c, c->io_a.p, gcalc, sizeof(double) * n, flags));
   CHK(upload(c, c->io_b.p, gobs, sizeof(double) * n, flags));
   HIPCHK(launch_potential(c->stream, potential, c->io_b.as<double>(), c->io_a.as<double>(), n, 1,
@@ -2482,10 +2633,11 @@ int pyiid_pdf_energy_forces(pyiid_ctx* c, int slot, double qbin, const double* g
   }
   CHK(energy_forces_device(c, slot, qbin, potential, c->gobs.as<double>(), conv, fdst));
   if (energy) {
-    std::vector<double> o5(5 * (size_t)B);
-    HIPCHK(hipMemcpyAsync(o5.data(), c->out5.p, sizeof(double) * 5 * B, hipMemcpyDeviceToHost,
+    std::vector<double> o5(5 * (size_t)B + 1);
+    HIPCHK(hipMemcpyAsync(o5.data(), c->out5.p, sizeof(double) * o5.size(), hipMemcpyDeviceToHost,
                           c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    CHK(note_far(c, o5[5 * (size_t)B]));
     for (int b = 0; b < B; ++b) energy[b] = o5[5 * (size_t)b] * conv;
   }
   if (forces && !(flags & PYIID_DEVICE))
@@ -2509,14 +2661,15 @@ int pyiid_fq_energy_forces(pyiid_ctx* c, int slot, double qbin, int32_t q_first,
   CHK(compute_fq(c, slot, qbin));
   CHK(c->gobs.reserve(sizeof(double) * ng));
   CHK(upload(c, c->gobs.p, gobs, sizeof(double) * ng, flags));
-  CHK(c->out5.reserve(sizeof(double) * 5));
+  CHK(reserve_out5(c, c->n_chain));
   CHK(c->w.reserve(sizeof(double) * ng));
   HIPCHK(launch_potential(c->stream, potential, c->gobs.as<double>(),
                           c->fq64.as<double>() + q_first, ng, 1, c->out5.as<double>(),
                           c->w.as<double>()));
-  double out5[5];
+  double out5[6];
   HIPCHK(hipMemcpyAsync(out5, c->out5.p, sizeof(out5), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  CHK(note_far(c, out5[5]));  // of the call before
   if (energy) *energy = out5[0] * conv;
   if (!forces) return PYIID_OK;
   if (c->n < 2) {
@@ -2599,6 +2752,13 @@ int pyiid_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step, do
     CHK(download(c, energies, h.ehist.p, sizeof(double) * (size_t)n_proposals * B, flags));
   if (accepted)
     CHK(download(c, accepted, h.acchist.p, sizeof(int32_t) * (size_t)n_proposals * B, flags));
+  if (!(flags & PYIID_DEVICE)) {
+    double far = 0.0;
+    HIPCHK(hipMemcpyAsync(&far, c->out5.as<double>() + 5 * static_cast<size_t>(B), sizeof(far),
+                          hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    CHK(note_far(c, far));
+  }
   return finish(c, flags);
 }
 

@@ -1,0 +1,300 @@
+// Contracted forces from a table of the pair force (gfx950, wave64).
+//
+// Forces need sum_q u_q grad F(q) only, so a pair of elements (I, J) at
+// distance r acts on its atoms with P(r) (q_i - q_j),
+//   P(r) = sum_q u_q f_I f_J (Q cos(Q r) - sin(Q r) / r) / r^2,
+// one function of r for all pairs of a chain and element pair.
+//
+//  1. force_table_kernel tabulates P on cells of width h = pi / (5 n_q dq) as
+//     polynomials of degree 5 through the cell's Chebyshev nodes, where the Q
+//     sums run in FP64.  The highest frequency turns by pi / 5 in a cell, so
+//     the interpolation error is 2 (pi / 20)^6 / 6! = 4.2e-8 of its amplitude.
+//  2. table_force_kernel forms every ordered pair's distance in FP64, reads
+//     its cell's six coefficients from LDS and adds P (q_i - q_j) to atom i.
+//
+// A recurrence per pair and bin took 5.8 VALU instructions for each; the table
+// takes about 30 instructions per ordered pair, whatever the number of bins.
+//
+// Reference semantics (pyIID): calc_1d.py:78-95 through cpu_flat.py:117-153.
+#include <cmath>
+
+#include "internal.h"
+
+namespace pyiid {
+namespace {
+
+constexpr int kNodes = 6;
+
+struct NodeFit {
+  double y[kNodes];           // Chebyshev nodes on [-1/2, 1/2]
+  double c[kNodes][kNodes];   // monomial coefficient k of the interpolant: sum_n c[k][n] P(y_n)
+};
+
+NodeFit node_fit() {
+  NodeFit f;
+  for (int n = 0; n < kNodes; ++n) f.y[n] = 0.5 * std::cos(M_PI * (2 * n + 1) / (2 * kNodes));
+  for (int n = 0; n < kNodes; ++n) {
+    // Lagrange basis polynomial of node n, expanded
+    double p[kNodes] = {1.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    int deg = 0;
+    for (int m = 0; m < kNodes; ++m) {
+      if (m == n) continue;
+      const double s = 1.0 / (f.y[n] - f.y[m]);
+      ++deg;
+      for (int k = deg; k >= 0; --k) p[k] = s * ((k > 0 ? p[k - 1] : 0.0) - f.y[m] * (k < deg ? p[k] : 0.0));
+    }
+    for (int k = 0; k < kNodes; ++k) f.c[k][n] = p[k];
+  }
+  return f;
+}
+
+constexpr int kTabChunk = 1024;  // Q bins staged in LDS at a time
+
+// Block: 64 cells (lanes) x 6 nodes (waves) of one table (chain, element
+// pair).  sin and cos of Q r follow the FP64 three-term recurrence along Q.
+__global__ __launch_bounds__(64 * kNodes) void force_table_kernel(
+    const float* __restrict__ u, const float* __restrict__ ftab, int nq, double dq, int weighted,
+    int n_elem, int n_pair, int n_cell, double h, NodeFit fit, float4* __restrict__ t4,
+    float2* __restrict__ t2) {
+  __shared__ double ca[kTabChunk], cb[kTabChunk];
+  __shared__ double val[kNodes][64];
+  const int lane = threadIdx.x & 63, node = threadIdx.x >> 6;
+  const int cell = blockIdx.x * 64 + lane;
+  const int table = blockIdx.y;
+  const int chain = table / n_pair;
+  int ei = 0, ej = table % n_pair;
+  while (ej > ei) ej -= ++ei;
+  const float* uc = u + static_cast<size_t>(chain) * nq;
+  const double r = (cell + 0.5 + fit.y[node]) * h;
+  double s1, c1;
+  sincos(dq * r, &s1, &c1);
+  const double k2 = 2.0 * c1;
+  double s = 0.0, sp = -s1, c = 1.0, cp = c1, a = 0.0, b = 0.0;
+  for (int m0 = 0; m0 < nq; m0 += kTabChunk) {
+    const int cnt = min(kTabChunk, nq - m0);
+    __syncthreads();
+    for (int m = threadIdx.x; m < cnt; m += blockDim.x) {
+      double w = uc[m0 + m];
+      if (weighted)
+        w *= static_cast<double>(ftab[static_cast<size_t>(ei) * nq + m0 + m]) *
+             static_cast<double>(ftab[static_cast<size_t>(ej) * nq + m0 + m]);
+      cb[m] = w;
+      ca[m] = w * (dq * (m0 + m));
+    }
+    __syncthreads();
+    for (int m = 0; m < cnt; ++m) {
+      a = fma(ca[m], c, a);
+      b = fma(cb[m], s, b);
+      const double sn = fma(k2, s, -sp), cn = fma(k2, c, -cp);
+      sp = s;
+      cp = c;
+      s = sn;
+      c = cn;
+    }
+  }
+  val[node][lane] = (a - b / r) / (r * r);
+  __syncthreads();
+  if (cell >= n_cell) return;
+  double p = 0.0;
+#pragma unroll
+  for (int n = 0; n < kNodes; ++n) p = fma(fit.c[node][n], val[n][lane], p);
+  const size_t at = static_cast<size_t>(table) * n_cell + cell;
+  // wave k holds coefficient k: 0..3 in t4, 4 and 5 in t2
+  if (node < 4)
+    reinterpret_cast<float*>(t4 + at)[node] = static_cast<float>(p);
+  else
+    reinterpret_cast<float*>(t2 + at)[node - 4] = static_cast<float>(p);
+}
+
+// P(r) beyond the table (an atom that has left the extent the table was made
+// for): the sums themselves.
+__device__ __noinline__ float pair_force_far(double r, const float* u, const float* fi,
+                                             const float* fj, int nq, double dq, double* far_seen) {
+  *far_seen = 1.0;
+  double s1, c1;
+  sincos(dq * r, &s1, &c1);
+  const double k2 = 2.0 * c1;
+  double s = 0.0, sp = -s1, c = 1.0, cp = c1, a = 0.0, b = 0.0;
+  for (int m = 0; m < nq; ++m) {
+    const double w = fi ? static_cast<double>(u[m]) * fi[m] * fj[m] : static_cast<double>(u[m]);
+    a = fma(w * (dq * m), c, a);
+    b = fma(w, s, b);
+    const double sn = fma(k2, s, -sp), cn = fma(k2, c, -cp);
+    sp = s;
+    cp = c;
+    s = sn;
+    c = cn;
+  }
+  return static_cast<float>((a - b / r) / (r * r));
+}
+
+// Block (16 waves): the unit's 64-position i tiles against its j range, its
+// table in LDS.  Wave w takes tile w mod tiles and slice w / tiles of the
+// range; a j atom's position is wave-uniform (scalar loads).  Each lane owns
+// its atom: FP32 sums over 64 j atoms, FP64 across them, then across slices
+// through LDS and across planes in reduce_force_kernel, in a fixed order.
+//
+// Per 64 ordered pairs: 11 FP64 and 8 conversion or transcendental
+// instructions, 8 FMAs, and one ds_read_b128 + ds_read_b64 gather.  Forming
+// every pair from both sides keeps the accumulators in registers: the
+// exchange of unordered pairs between lanes would cost about as much as the
+// distance saved.
+__global__ __launch_bounds__(1024, 8) void table_force_kernel(
+    const AtomRec* __restrict__ pos, const ForceUnit* __restrict__ units, int n_cell, double inv_h,
+    const float4* __restrict__ t4, const float2* __restrict__ t2, const float* __restrict__ u,
+    const float* __restrict__ ftab, int nq, double dq, int64_t n, double* __restrict__ part,
+    double* __restrict__ far_seen) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  float4* l4 = reinterpret_cast<float4*>(lds);
+  float2* l2 = reinterpret_cast<float2*>(lds + sizeof(float4) * static_cast<size_t>(n_cell));
+  const ForceUnit un = units[blockIdx.x];
+  {
+    const float4* g4 = t4 + static_cast<size_t>(un.table) * n_cell;
+    const float2* g2 = t2 + static_cast<size_t>(un.table) * n_cell;
+    for (int e = threadIdx.x; e < n_cell; e += blockDim.x) {
+      l4[e] = g4[e];
+      l2[e] = g2[e];
+    }
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n_slice = (blockDim.x >> 6) / un.tiles;
+  const int tile = wave % un.tiles, slice = wave / un.tiles;
+  const int i = un.i0 + tile * 64 + lane;
+  const bool have = i < un.i1;
+  const int len = un.j1 - un.j0;
+  const int jb = un.j0 + static_cast<int>(static_cast<int64_t>(len) * slice / n_slice);
+  const int je = un.j0 + static_cast<int>(static_cast<int64_t>(len) * (slice + 1) / n_slice);
+  const AtomRec pi = pos[have ? i : un.i0];
+  const double limit = static_cast<double>(n_cell);
+  double gx = 0.0, gy = 0.0, gz = 0.0;
+  for (int j0 = jb; j0 < je; j0 += 64) {
+    const int j1 = min(je, j0 + 64);
+    float fx = 0.f, fy = 0.f, fz = 0.f;
+    for (int j = j0; j < j1; ++j) {
+      const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
+      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+      if (!(r2 > 0.0)) continue;  // the atom itself, a duplicate, a NaN
+      const float r2f = static_cast<float>(r2);
+      const float y0 = __builtin_amdgcn_rsqf(r2f);
+      const float rf = r2f * y0;
+      const double rd = static_cast<double>(rf);
+      double t = fma(fma(-rd, rd, r2), static_cast<double>(0.5f * y0), rd) * inv_h;
+      float p;
+      if (t < limit) {
+        const double fl = floor(t);
+        const float y = static_cast<float>(t - fl) - 0.5f;
+        const int cell = static_cast<int>(fl);
+        const float4 a = l4[cell];
+        const float2 b = l2[cell];
+        p = fmaf(fmaf(fmaf(fmaf(fmaf(b.y, y, b.x), y, a.w), y, a.z), y, a.y), y, a.x);
+      } else {
+        // past the table, or r2 outside float's range
+        const double r = sqrt(r2);
+        t = r * inv_h;
+        if (t < limit) {
+          const float y = static_cast<float>(t - floor(t)) - 0.5f;
+          const float4 a = l4[static_cast<int>(t)];
+          const float2 b = l2[static_cast<int>(t)];
+          p = fmaf(fmaf(fmaf(fmaf(fmaf(b.y, y, b.x), y, a.w), y, a.z), y, a.y), y, a.x);
+        } else {
+          p = pair_force_far(r, u + static_cast<size_t>(un.chain) * nq,
+                             un.ei < 0 ? nullptr : ftab + static_cast<size_t>(un.ei) * nq,
+                             un.ei < 0 ? nullptr : ftab + static_cast<size_t>(un.ej) * nq, nq, dq,
+                             far_seen);
+        }
+      }
+      fx = fmaf(p, static_cast<float>(dx), fx);
+      fy = fmaf(p, static_cast<float>(dy), fy);
+      fz = fmaf(p, static_cast<float>(dz), fz);
+    }
+    gx += static_cast<double>(fx);
+    gy += static_cast<double>(fy);
+    gz += static_cast<double>(fz);
+  }
+  if (n_slice > 1) {
+    __syncthreads();  // the table is no longer read
+    double* red = reinterpret_cast<double*>(lds);
+    double* mine = red + (static_cast<size_t>(wave) * 64 + lane) * 3;
+    mine[0] = gx;
+    mine[1] = gy;
+    mine[2] = gz;
+    __syncthreads();
+    if (slice != 0) return;
+    for (int k = 1; k < n_slice; ++k) {
+      const double* o = red + (static_cast<size_t>(k * un.tiles + tile) * 64 + lane) * 3;
+      gx += o[0];
+      gy += o[1];
+      gz += o[2];
+    }
+  }
+  if (have) {
+    double* o = part + (static_cast<size_t>(un.plane) * n + i) * 3;
+    o[0] = gx;
+    o[1] = gy;
+    o[2] = gz;
+  }
+}
+
+// out[perm[p]][c] = conv * sum over the position's planes
+__global__ void reduce_force_kernel(const double* __restrict__ part, int64_t n,
+                                    const int32_t* __restrict__ planes,
+                                    const int32_t* __restrict__ perm, double conv,
+                                    double* __restrict__ out) {
+  const int64_t e = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (e >= 3 * n) return;
+  const int64_t p = e / 3;
+  double s = 0.0;
+  const int np = planes[p];
+  for (int k = 0; k < np; ++k) s += part[static_cast<size_t>(k) * n * 3 + e];
+  out[static_cast<size_t>(perm ? perm[p] : p) * 3 + (e - 3 * p)] = conv * s;
+}
+
+}  // namespace
+
+double force_cell(int nq, double dq) { return M_PI / (5.0 * std::max(1, nq) * dq); }
+
+size_t force_lds_bytes(int64_t n_cell) {
+  const size_t table = (sizeof(float4) + sizeof(float2)) * static_cast<size_t>(n_cell);
+  const size_t red = sizeof(double) * 16 * 64 * 3;
+  return table > red ? table : red;
+}
+
+hipError_t launch_force_table(hipStream_t st, const float* u, const float* ftab, int nq, double dq,
+                              bool weighted, int n_elem, int n_chain, int n_cell, float4* t4,
+                              float2* t2) {
+  static const NodeFit fit = node_fit();
+  const int n_pair = weighted ? n_elem * (n_elem + 1) / 2 : 1;
+  hipLaunchKernelGGL(force_table_kernel, dim3((n_cell + 63) / 64, n_chain * n_pair),
+                     dim3(64 * kNodes), 0, st, u, ftab, nq, dq, weighted ? 1 : 0, n_elem, n_pair,
+                     n_cell, force_cell(nq, dq), fit, t4, t2);
+  return hipGetLastError();
+}
+
+hipError_t launch_table_force(hipStream_t st, const AtomRec* pos, const ForceUnit* units,
+                              int n_units, int n_cell, const float4* t4, const float2* t2,
+                              const float* u, const float* ftab, int nq, double dq, int64_t n,
+                              double* part, double* far_seen) {
+  if (n_units == 0) return hipSuccess;
+  const size_t lds = force_lds_bytes(n_cell);
+  if (lds > kForceLds) return hipErrorInvalidValue;
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(table_force_kernel),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kForceLds));
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL(table_force_kernel, dim3(n_units), dim3(1024), lds, st, pos, units, n_cell,
+                     1.0 / force_cell(nq, dq), t4, t2, u, ftab, nq, dq, n, part, far_seen);
+  return hipGetLastError();
+}
+
+hipError_t launch_reduce_force(hipStream_t st, const double* part, int64_t n,
+                               const int32_t* planes, const int32_t* perm, double conv,
+                               double* out) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(reduce_force_kernel, dim3(static_cast<unsigned>((3 * n + 255) / 256)),
+                     dim3(256), 0, st, part, n, planes, perm, conv, out);
+  return hipGetLastError();
+}
+
+}  // namespace pyiid

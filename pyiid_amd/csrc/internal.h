@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 namespace pyiid {
@@ -137,6 +138,32 @@ hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_
 // out[p] = pos[perm[p]]
 hipError_t launch_gather(hipStream_t st, const AtomRec* pos, const int32_t* perm, int64_t n,
                          AtomRec* out);
+
+// ---- contracted forces from a pair-force table (forcetab.hip) ----
+// Unit: positions [i0, i1) in `tiles` (1, 2, 4, 8 or 16) tiles of 64 against
+// positions [j0, j1), all of elements ei, ej (-1: single element) of one
+// chain, with table `table`; its sums go to plane `plane`.
+struct ForceUnit {
+  int i0, i1, j0, j1;
+  int tiles, plane, table, chain;
+  int ei, ej, pad0, pad1;
+};
+constexpr size_t kForceLds = 160 * 1024;
+double force_cell(int nq, double dq);       // cell width of the table
+size_t force_lds_bytes(int64_t n_cell);     // LDS of a block
+// t4 / t2 [chain * n_pair + pair][n_cell]: coefficients 0..3 / 4, 5
+hipError_t launch_force_table(hipStream_t st, const float* u, const float* ftab, int nq, double dq,
+                              bool weighted, int n_elem, int n_chain, int n_cell, float4* t4,
+                              float2* t2);
+// part[plane][position][3]; *far_seen becomes 1 when a pair lies past the table
+hipError_t launch_table_force(hipStream_t st, const AtomRec* pos, const ForceUnit* units,
+                              int n_units, int n_cell, const float4* t4, const float2* t2,
+                              const float* u, const float* ftab, int nq, double dq, int64_t n,
+                              double* part, double* far_seen);
+// out[perm[p]][c] = conv * sum_{k < planes[p]} part[k][p][c] (perm null: identity)
+hipError_t launch_reduce_force(hipStream_t st, const double* part, int64_t n,
+                               const int32_t* planes, const int32_t* perm, double conv,
+                               double* out);
 
 // ---- transform / potential (transform.hip) ----
 // C[m][ldc] = A[m][K] . B[n][K]^T in FP32 MFMA; A float or double.

@@ -125,7 +125,7 @@ __device__ __noinline__ void spread_rare(unsigned long long* hist, int n_grid, d
 // integer and 6 ds_add_u64.  The LDS adds (29 ns per CU) and the VALU (about
 // as long, 4 SIMDs) run side by side, and 2 blocks (32 waves) per CU hide
 // each other's latency.
-__global__ __launch_bounds__(1024, 2) void spread_fq_kernel(
+__global__ __launch_bounds__(1024, 8) void spread_fq_kernel(
     const AtomRec* __restrict__ pos, const SpreadUnit* __restrict__ units,
     const SpreadItem* __restrict__ items, double inv_h, int nf, int n_grid, int stride, int shift,
     float scale, double near, unsigned long long* __restrict__ grids) {

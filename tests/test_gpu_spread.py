@@ -124,3 +124,65 @@ def test_infinite_position_is_not_a_number(ctx):
     pos[3, 0] = np.inf
     load(ctx, pos, np.full(20, 79), 0.1, 100)
     assert np.all(np.isnan(ctx.fq(_lib.SLOT_FQ, 0.1, 100)[1:]))
+
+
+def force_check(ctx, pos, base, numbers, qbin, nq, upload=None):
+    """F(Q)-Rw energy and forces against the oracle.  Allowed: 4e-7 of the sum
+    of the amplitudes of an atom's pair forces (table polynomial 4.2e-8, its
+    single-precision coefficients and evaluation about 3e-7), and 2e-6 of the
+    largest force for the error of F in the residual."""
+    n, first = len(pos), 5
+    per_atom = load(ctx, base if upload else pos, numbers, qbin, nq)
+    target = oracle.fq((pos * np.float32(0.98)).astype(np.float32), per_atom, qbin)[first:]
+    if upload:
+        ctx.fq_energy_forces(_lib.SLOT_FQ, qbin, first, target, _lib.POT_RW, 10.0, n)
+        upload(pos)
+    e, f = ctx.fq_energy_forces(_lib.SLOT_FQ, qbin, first, target, _lib.POT_RW, 10.0, n)
+    fq = oracle.fq(pos, per_atom, qbin)[first:]
+    g = oracle.grad_fq(pos, per_atom, qbin)[:, :, first:]
+    want = 10.0 * oracle.wrap_grad_rw(g, fq, target)
+    rw, a = oracle.get_rw(target, fq)
+    w = 10.0 * np.abs(rw / np.sum((target - a * fq) ** 2) * a * (target - a * fq))
+    q = oracle.q_values(qbin, nq)[first:]
+    x, ff = pos.astype(np.float64), per_atom.astype(np.float64)[:, first:]
+    r = np.linalg.norm(x[:, None] - x[None], axis=-1)
+    inv = np.divide(1.0, r, out=np.zeros_like(r), where=r > 0)
+    na = np.abs(oracle.normalization(per_atom))[first:]
+    amp = np.einsum("q,iq,jq,ij->i", w * q / na, ff, ff, inv) + \
+        np.einsum("q,iq,jq,ij->i", w / na, ff, ff, inv * inv)
+    allowed = 4e-7 * amp[:, None] + 2e-6 * np.abs(want).max()
+    assert abs(e - 10.0 * rw) < 1e-5
+    off = (np.abs(f - want) / allowed).max()
+    assert off < 1.0, off
+
+
+@pytest.mark.parametrize("n", [2, 3, 64, 65, 150, 400])
+def test_force_table_tiles(ctx, n):
+    base = structures.fcc_nearest(n)
+    pos = structures.jitter(base, 0.05, seed=n).astype(np.float32)
+    force_check(ctx, pos, base, np.full(n, 79), 0.1, 250)
+    zs = np.random.RandomState(n).permutation(np.array([28, 78, 79])[np.arange(n) % 3])
+    force_check(ctx, pos, base, zs, 0.05, 330)
+
+
+def test_force_past_the_table(ctx):
+    """Positions moved on the device after the table's length was taken: the
+    pairs past its end are summed directly, and the next call has a longer
+    table."""
+    import torch
+    base = structures.fcc_nearest(90).astype(np.float32)
+    pos = structures.jitter(base, 0.05, seed=2).astype(np.float32)
+    pos[40:] += np.float32(17.3)
+
+    def upload(p):
+        ctx.set_positions(torch.from_numpy(p).cuda(), flags=_lib.PYIID_DEVICE)
+    for _ in range(2):
+        force_check(ctx, pos, base, np.full(90, 79), 0.1, 250, upload)
+
+
+def test_long_force_table(ctx):
+    """A structure whose table fills most of LDS, and one past it (which runs
+    the recurrence kernel)."""
+    for length in (140.0, 400.0):
+        pos = np.random.RandomState(4).uniform(0, length, (70, 3)).astype(np.float32)
+        force_check(ctx, pos, pos, np.full(70, 79), 0.05, 600)
