@@ -115,7 +115,9 @@ int pyiid_set_grad_kernel(pyiid_ctx *ctx, int kernel);
 /* Launch shape of the last pyiid_grad_fq call: *symmetric = 1 for the
  * symmetric (unordered-pair) kernel, with its Q bins per wave and tiles per
  * item in *group; 0 for the ordered kernel, with its Q bins per wave and its
- * number of j ranges per tile in *group.  No counterpart in the reference. */
+ * number of j ranges per tile in *group; 0 with 0 bins per wave and group 0
+ * for the spreading kernel (whose pair work does not depend on the bins).  No
+ * counterpart in the reference. */
 int pyiid_grad_shape(pyiid_ctx *ctx, int *symmetric, int *bins_per_wave, int *group);
 /* Autotuning of the Debye kernels' launch shapes (F + gradient kernel and its
  * grouping, F-only bins per wave, contracted-force Q groups), on by

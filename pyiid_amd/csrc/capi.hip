@@ -144,6 +144,19 @@ struct ForceSet {
   int key = -1;
 };
 
+// Element runs, rows and sine matrices of the gradient by spreading.
+struct GradSet {
+  Buf perm, sorted;     // weighted tables: atoms in element order
+  Buf runs, run_elem;   // int32: run boundaries (n_run + 1), their elements
+  Buf rows, row_scale;  // split rows of one chunk of atoms, their scales
+  Buf w[2], inv_phihat[2];  // per table slot
+  int w_nq[2] = {0, 0};
+  Buf k_used;           // int32: points of a row in use
+  int n_run = 0;
+  uint64_t stamp = ~0ull;
+  int key = -1;
+};
+
 // One captured proposal and the parameters it was captured with.
 struct GraphSlot {
   hipGraph_t graph = nullptr;
@@ -208,6 +221,7 @@ struct pyiid_ctx {
   // passed in host memory: sets scales and table lengths, never what is right.
   double r_max = 0.0;
   std::vector<int64_t> extent_off;  // the layout it was taken for
+  bool extent_exact = false;        // r_max bounds the current positions' distances
 
   Table tab[2];
   uint64_t tab_stamp[2] = {1, 1};
@@ -220,6 +234,8 @@ struct pyiid_ctx {
   ItemSet fq_items;     // unordered pairs, ranges per chain
   SpreadSet spread;     // unordered pairs of the F(Q) spreading kernel
   ForceSet force;       // ordered pairs of the contracted-force kernel
+  GradSet grad;         // gradient by spreading
+  bool grad_spread = false;  // the last gradient ran on it
   ItemSet fused_items;  // ordered pairs with j splits, ranges per i tile
   ItemSet pair_items;   // tile pairs (I, J <= I) of the contracted-force kernel
   SymSet sym;           // unordered tile pairs of the symmetric F + gradient kernel
@@ -1418,6 +1434,92 @@ int tune_grad(pyiid_ctx* c, int slot, double qbin) {
   return best_k ? PYIID_OK : tune_fused(c, slot, qbin);
 }
 
+// ---- gradient by spreading ----
+
+// Bytes of the rows of one chunk of atoms; a large structure runs in several.
+constexpr size_t kGradRowBudget = static_cast<size_t>(1) << 30;
+
+// Whether the gradient runs on the spreading kernel: its grids fit LDS, and
+// neither compensated sums nor a recurrence kernel or its shape is asked for.
+bool use_spread_grad(pyiid_ctx* c, const Table& t) {
+  return !c->compensated && c->grad_kernel == PYIID_GRAD_AUTO && c->grad_m_fixed == 0 &&
+         c->sym_k_fixed == 0 && grad_lds_bytes(t.nq) <= kGradLds;
+}
+
+int run_spread_grad(pyiid_ctx* c, int slot, double qbin, void* out, bool out_f64) {
+  Table& t = c->tab[slot];
+  GradSet& s = c->grad;
+  const int nq = t.nq;
+  const bool weighted = weighted_table(t);
+  const double dq = static_cast<double>(static_cast<float>(qbin));
+  CHK(ensure_extent(c));
+  const int key = weighted ? 1 : 0;
+  if (s.stamp != c->struct_stamp || s.key != key) {
+    if (c->capturing) return fail(PYIID_E_STATE, "structure changed during graph capture");
+    std::vector<int32_t> perm;
+    std::vector<std::vector<ElemRun>> runs;
+    element_runs(c, weighted, perm, runs);
+    std::vector<int32_t> begin, elem;
+    for (const ElemRun& r : runs[0]) {
+      begin.push_back(static_cast<int32_t>(r.begin));
+      elem.push_back(r.elem);
+    }
+    s.n_run = static_cast<int>(elem.size());
+    begin.push_back(static_cast<int32_t>(c->n));
+    CHK(upload_vec(s.runs, begin));
+    CHK(upload_vec(s.run_elem, elem));
+    if (weighted) {
+      CHK(upload_vec(s.perm, perm));
+      CHK(s.sorted.reserve(sizeof(AtomRec) * std::max<int64_t>(1, c->n)));
+    }
+    CHK(s.k_used.reserve(sizeof(int)));
+    s.stamp = c->struct_stamp;
+    s.key = key;
+  }
+  const int len = grad_row_len(nq);
+  if (s.w_nq[slot] != nq) {
+    CHK(s.w[slot].reserve(sizeof(uint16_t) * 2 * static_cast<size_t>(len) * nq));
+    CHK(s.inv_phihat[slot].reserve(sizeof(float) * nq));
+    HIPCHK(launch_sine_matrix(c->stream, nq, s.w[slot].p, s.inv_phihat[slot].as<float>()));
+    s.w_nq[slot] = nq;
+  }
+  const size_t per_atom = sizeof(uint16_t) * 6 * static_cast<size_t>(len) * s.n_run;
+  const int64_t chunk = std::min<int64_t>(
+      c->n, std::max<int64_t>(128, static_cast<int64_t>(kGradRowBudget / per_atom) / 128 * 128));
+  CHK(s.rows.reserve(per_atom * chunk));
+  CHK(s.row_scale.reserve(sizeof(float) * 3 * static_cast<size_t>(chunk) * s.n_run));
+  const AtomRec* sp = c->pos.as<AtomRec>();
+  if (weighted) {
+    HIPCHK(launch_gather(c->stream, sp, s.perm.as<int32_t>(), c->n, s.sorted.as<AtomRec>()));
+    sp = s.sorted.as<AtomRec>();
+  }
+  // points of a row in use: from the host's extent when it bounds the current
+  // positions, else from the positions on the device (no wait either way)
+  int k_fixed = 0;
+  const int* k_dev = nullptr;
+  if (c->extent_exact) {
+    const double reach = grad_reach(nq, dq, c->r_max * 1.000001);
+    k_fixed = reach < len ? (static_cast<int>(reach) + 31) & ~31 : len;
+    k_fixed = std::min(k_fixed, len);
+  } else {
+    HIPCHK(launch_grad_extent(c->stream, sp, c->n, nq, dq, s.k_used.as<int>()));
+    k_dev = s.k_used.as<int>();
+  }
+  Timed tm(c, 0);
+  for (int64_t p0 = 0; p0 < c->n; p0 += chunk) {
+    const int m = static_cast<int>(std::min<int64_t>(chunk, c->n - p0));
+    HIPCHK(launch_spread_grad(c->stream, sp, static_cast<int>(p0), m, c->n, s.runs.as<int>(),
+                              s.n_run, nq, dq, c->r_max, k_fixed, k_dev, s.rows.p,
+                              s.row_scale.as<float>()));
+    HIPCHK(launch_gemm_split(c->stream, s.rows.p, s.row_scale.as<float>(), m, s.n_run,
+                             s.w[slot].p, s.inv_phihat[slot].as<float>(), nq, dq, k_fixed, k_dev,
+                             t.gs.as<double>(), t.tab.as<float>(), s.run_elem.as<int>(), weighted,
+                             sp, weighted ? s.perm.as<int32_t>() : nullptr, static_cast<int>(p0),
+                             out, out_f64));
+  }
+  return tm.done();
+}
+
 // ---- contracted forces from a pair-force table ----
 
 void destroy_graph(Hmc& h);
@@ -1657,9 +1759,11 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
   c->pos_set = true;
   c->pos_dirty = true;
   CHK(ensure_packed(c));
+  c->extent_exact = false;
   if (!(flags & PYIID_DEVICE) && n <= kExtentAtoms) {
     c->r_max = chain_extent(pos, 3, c->off);
     c->extent_off = c->off;
+    c->extent_exact = true;
   }
   return finish(c, flags);
 }
@@ -2136,6 +2240,9 @@ int pyiid_destroy(pyiid_ctx* c) {
                  &c->spread.perm, &c->spread.sorted, &c->spread.grids, &c->spread.done,
                  &c->force.units, &c->force.planes, &c->force.perm, &c->force.sorted,
                  &c->force.t4, &c->force.t2, &c->force.part,
+                 &c->grad.perm, &c->grad.sorted, &c->grad.runs, &c->grad.run_elem, &c->grad.rows,
+                 &c->grad.row_scale, &c->grad.w[0], &c->grad.w[1], &c->grad.inv_phihat[0],
+                 &c->grad.inv_phihat[1], &c->grad.k_used,
                  &c->fused_items.items, &c->fused_items.ranges,
                  &c->fused_items.perm, &c->hmc.mass,
                  &c->hmc.mom, &c->hmc.fcur, &c->hmc.fnew, &c->hmc.pos_save, &c->hmc.kin0,
@@ -2261,6 +2368,12 @@ int pyiid_set_grad_kernel(pyiid_ctx* c, int kernel) {
 int pyiid_grad_shape(pyiid_ctx* c, int* symmetric, int* bins_per_wave, int* group) {
   CHK(check_ctx(c));
   if (!symmetric || !bins_per_wave || !group) return fail(PYIID_E_INVALID, "null output");
+  if (c->grad_spread) {
+    *symmetric = 0;
+    *bins_per_wave = 0;
+    *group = 0;
+    return PYIID_OK;
+  }
   *symmetric = c->sym_k ? 1 : 0;
   *bins_per_wave = c->sym_k ? c->sym_m : c->grad_m;
   *group = c->sym_k ? c->sym_k : c->fused_items.split;
@@ -2415,18 +2528,26 @@ int pyiid_grad_fq(pyiid_ctx* c, int slot, double qbin, void* grad, float* fq, in
   }
   CHK(ensure_packed(c));
   CHK(ensure_norm(c, slot));
-  CHK(tune_grad(c, slot, qbin));
-  const bool sym = c->sym_k != 0;
-  if (sym)
-    CHK(run_sym(c, slot, qbin));
-  else
-    CHK(run_fused(c, slot, qbin, false));
   Table& t = c->tab[slot];
   void* gdst = grad;
   if (!(flags & PYIID_DEVICE)) {
     CHK(c->io_c.reserve(gbytes));
     gdst = c->io_c.p;
   }
+  c->grad_spread = use_spread_grad(c, t);
+  if (c->grad_spread) {
+    CHK(run_spread_grad(c, slot, qbin, gdst, (flags & PYIID_F64) != 0));
+    if (fq) CHK(compute_fq(c, slot, qbin));
+    if (!(flags & PYIID_DEVICE)) CHK(download(c, grad, gdst, gbytes, flags));
+    if (fq) CHK(download(c, fq, c->fq32.p, sizeof(float) * nq, flags));
+    return finish(c, flags);
+  }
+  CHK(tune_grad(c, slot, qbin));
+  const bool sym = c->sym_k != 0;
+  if (sym)
+    CHK(run_sym(c, slot, qbin));
+  else
+    CHK(run_fused(c, slot, qbin, false));
   if (sym)
     HIPCHK(reduce_sym(c, t, gdst, (flags & PYIID_F64) != 0));
   else
@@ -2740,6 +2861,7 @@ int pyiid_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step, do
     return fail(PYIID_E_INVALID, "need n_proposals >= 0, n_leapfrog >= 1, beta > 0");
   const int B = c->n_chain;
   if (n_proposals == 0) return PYIID_OK;
+  c->extent_exact = false;
   CHK(prepare_history(c, n_proposals));
   CHK(refresh_exact(c));
   RunClock clock(c, times_ms != nullptr);
@@ -2930,6 +3052,7 @@ int pyiid_sur_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step
   if (min_chain_atoms(c) < 2) return fail(PYIID_E_INVALID, "every chain needs at least two atoms");
   const int B = c->n_chain;
   if (n_proposals == 0) return PYIID_OK;
+  c->extent_exact = false;
   CHK(prepare_history(c, n_proposals));
   RunClock clock(c, times_ms != nullptr);
   bool exact_block = false;

@@ -18,7 +18,7 @@
 // Reference semantics (pyIID): calc_1d.py:78-95 through cpu_flat.py:117-153.
 #include <cmath>
 
-#include "internal.h"
+#include "pair_math.h"
 
 namespace pyiid {
 namespace {
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(64 * kNodes) void force_table_kernel(
 
 // P(r) beyond the table (an atom that has left the extent the table was made
 // for): the sums themselves.
-__device__ __noinline__ float pair_force_far(double r, const float* u, const float* fi,
+__device__ double pair_force_far(double r, const float* u, const float* fi,
                                              const float* fj, int nq, double dq, double* far_seen) {
   *far_seen = 1.0;
   double s1, c1;
@@ -125,7 +125,7 @@ __device__ __noinline__ float pair_force_far(double r, const float* u, const flo
     s = sn;
     c = cn;
   }
-  return static_cast<float>((a - b / r) / (r * r));
+  return (a - b / r) / (r * r);
 }
 
 // Block (16 waves): the unit's 64-position i tiles against its j range, its
@@ -169,6 +169,7 @@ __global__ __launch_bounds__(1024, 8) void table_force_kernel(
   const AtomRec pi = pos[have ? i : un.i0];
   const double limit = static_cast<double>(n_cell);
   double gx = 0.0, gy = 0.0, gz = 0.0;
+  bool far = false;
   for (int j0 = jb; j0 < je; j0 += 64) {
     const int j1 = min(je, j0 + 64);
     float fx = 0.f, fy = 0.f, fz = 0.f;
@@ -176,35 +177,16 @@ __global__ __launch_bounds__(1024, 8) void table_force_kernel(
       const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
       const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
       if (!(r2 > 0.0)) continue;  // the atom itself, a duplicate, a NaN
-      const float r2f = static_cast<float>(r2);
-      const float y0 = __builtin_amdgcn_rsqf(r2f);
-      const float rf = r2f * y0;
-      const double rd = static_cast<double>(rf);
-      double t = fma(fma(-rd, rd, r2), static_cast<double>(0.5f * y0), rd) * inv_h;
-      float p;
-      if (t < limit) {
-        const double fl = floor(t);
-        const float y = static_cast<float>(t - fl) - 0.5f;
-        const int cell = static_cast<int>(fl);
-        const float4 a = l4[cell];
-        const float2 b = l2[cell];
-        p = fmaf(fmaf(fmaf(fmaf(fmaf(b.y, y, b.x), y, a.w), y, a.z), y, a.y), y, a.x);
-      } else {
-        // past the table, or r2 outside float's range
-        const double r = sqrt(r2);
-        t = r * inv_h;
-        if (t < limit) {
-          const float y = static_cast<float>(t - floor(t)) - 0.5f;
-          const float4 a = l4[static_cast<int>(t)];
-          const float2 b = l2[static_cast<int>(t)];
-          p = fmaf(fmaf(fmaf(fmaf(fmaf(b.y, y, b.x), y, a.w), y, a.z), y, a.y), y, a.x);
-        } else {
-          p = pair_force_far(r, u + static_cast<size_t>(un.chain) * nq,
-                             un.ei < 0 ? nullptr : ftab + static_cast<size_t>(un.ei) * nq,
-                             un.ei < 0 ? nullptr : ftab + static_cast<size_t>(un.ej) * nq, nq, dq,
-                             far_seen);
-        }
+      const double t = scaled_root(r2, inv_h);
+      if (!(t < limit)) {  // past the table, or r2 outside float's range
+        far = true;
+        continue;
       }
+      const double fl = floor(t);
+      const float y = static_cast<float>(t - fl) - 0.5f;
+      const float4 a = l4[static_cast<int>(fl)];
+      const float2 b = l2[static_cast<int>(fl)];
+      const float p = fmaf(fmaf(fmaf(fmaf(fmaf(b.y, y, b.x), y, a.w), y, a.z), y, a.y), y, a.x);
       fx = fmaf(p, static_cast<float>(dx), fx);
       fy = fmaf(p, static_cast<float>(dy), fy);
       fz = fmaf(p, static_cast<float>(dz), fz);
@@ -212,6 +194,20 @@ __global__ __launch_bounds__(1024, 8) void table_force_kernel(
     gx += static_cast<double>(fx);
     gy += static_cast<double>(fy);
     gz += static_cast<double>(fz);
+  }
+  if (far) {  // atoms that have left the extent the table was made for
+    const float* uc = u + static_cast<size_t>(un.chain) * nq;
+    const float* fi = un.ei < 0 ? nullptr : ftab + static_cast<size_t>(un.ei) * nq;
+    const float* fj = un.ei < 0 ? nullptr : ftab + static_cast<size_t>(un.ej) * nq;
+    for (int j = jb; j < je; ++j) {
+      const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
+      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+      if (!(r2 > 0.0) || scaled_root(r2, inv_h) < limit) continue;
+      const double p = pair_force_far(sqrt(r2), uc, fi, fj, nq, dq, far_seen);
+      gx = fma(p, dx, gx);
+      gy = fma(p, dy, gy);
+      gz = fma(p, dz, gz);
+    }
   }
   if (n_slice > 1) {
     __syncthreads();  // the table is no longer read

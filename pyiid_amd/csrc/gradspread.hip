@@ -1,0 +1,555 @@
+// Position gradient of F(Q) by spreading (gfx950, wave64).
+//
+// grad F of atom i is sum_j f_i f_j d_ij K(Q, r_ij), with d_ij = q_i - q_j and
+// K(Q, r) = (Q cos(Q r) - sin(Q r) / r) / r^2.  As for F alone, a pair is
+// handled once whatever the number of bins:
+//
+//  1. spread_grad_kernel keeps three grids (x, y, z) of spacing h = 2 pi / (dq
+//     n_f), n_f = 4.5 n_q, for its atom and adds every j to 8 points of each:
+//     with phi_j(y) the window values and chi_j(y) those of its derivative,
+//     sum_g (chi_g / h / r^2 - phi_g / r^3) sin(Q g h) = phihat(Q h) K(Q, r),
+//     so one sine transform serves both terms.
+//  2. gemm_split_kernel is that transform for all atoms at once: grids (3 N
+//     rows) times the n_q x grid sine matrix on the matrix cores, with the
+//     weights -1 / na, f_i, f_j and 1 / phihat in its epilogue.
+//
+// Window: phihat as in the F grid, beta = 19.062 and 8 points; phi and chi are
+// least squares over |q| <= pi / 2.25, polynomials of degree 6 and 7.  With
+// single-precision values the result is off by 5.8e-8 (phi) and 5.7e-8 (chi,
+// of Q_max) r.m.s. over the band.  A grid of n_f = 4 n_q has 1.3e-7 for chi
+// and left the gradient 3.8e-7 off at 6,699 atoms.
+//
+// The product's operands are split into two halves, x = hi + lo, each 11
+// bits, rows scaled by a power of two of their own: hi hi + hi lo + lo hi in
+// FP32 leaves 2^-22 of an entry, at three FP16 products for one in FP32, whose
+// matrix rate is 16 times lower.
+//
+// Reference semantics (pyIID): cpu_flat.py:117-153, cpu_experimental.py:8-15,
+// flat_multi_cpu_wrap.py:63-102.
+#include <cmath>
+
+#include "pair_math.h"
+
+namespace pyiid {
+namespace {
+
+constexpr int kGw = 8;
+constexpr double kGBeta = 19.062;
+// phi_j(y) and chi_j(y), j < 4, y in [-1/2, 1/2] about the window's middle;
+// phi_{7-j}(y) = phi_j(-y), chi_{7-j}(y) = -chi_j(-y)
+constexpr float kPhi[4][7] = {
+    {3.40901582e-05f, -0.00027549045f, 0.000964908494f, -0.0018895139f, 0.00225111831f,
+     -0.00166305554f, 0.000637135338f},
+    {0.00759243827f, -0.0279834767f, 0.0424969158f, -0.0322129548f, 0.00961409082f,
+     0.00329632756f, -0.0032371457f},
+    {0.11335156f, -0.212225827f, 0.116716452f, 0.0208575311f, -0.0423386611f, 0.006792028f,
+     0.00587311726f},
+    {0.379021922f, -0.221476835f, -0.160178429f, 0.111719934f, 0.0304739315f, -0.0252178211f,
+     -0.0032738704f},
+};
+constexpr float kChi[4][8] = {
+    {-0.000275315306f, 0.00193018817f, -0.0056853555f, 0.00898962606f, -0.00809109359f,
+     0.00396534477f, -0.000717389118f, -0.000380087321f},
+    {-0.0279849156f, 0.0849923757f, -0.0965007299f, 0.0385146002f, 0.0146398433f, -0.0199819486f,
+     0.00589374241f, 0.00149086504f},
+    {-0.212221186f, 0.23343518f, 0.0621270564f, -0.169445683f, 0.0399006315f, 0.0361126777f,
+     -0.0190095727f, -0.00233059775f},
+    {-0.221484802f, -0.320358043f, 0.33592471f, 0.121943086f, -0.136287886f, -0.0200978749f,
+     0.032636098f, 0.00121240683f},
+};
+// Below t = r / h = kGClose K(Q, r), an even function of r, is interpolated in
+// r^2 from kGNodes Chebyshev nodes on (0, kGClose h): below 1e-9 for Q h <= pi / 2.25.
+constexpr double kGClose = 2.0;
+constexpr int kGNodes = 8;
+// Fixed point: (chi_j - phi_j / t) (d / h) / t^2 2^s, at most 1.2 2^s / t; s as in
+// the F grid (2^24 units at the largest distance), at least 35; from t = 1.2
+// 2^(s - 31) on one int32 conversion serves (1.2 A at 25 1/A).
+constexpr int kGBits = 24, kGMinScale = 35, kGMaxScale = 48;
+constexpr double kGFar = 1e15;  // beyond: the second look
+
+__host__ __device__ inline double g_node(int k) {
+  constexpr double c[kGNodes] = {  // cos((2 k + 1) pi / 32)
+      0.99518472667219693, 0.95694033573220882, 0.88192126434835505, 0.77301045336273699,
+      0.63439328416364549, 0.47139673682599764, 0.29028467725446233, 0.098017140329560604};
+  return kGClose * c[k];
+}
+
+// n_f / 2 of the folded grid.
+__host__ __device__ inline int half_grid(int nq) { return (9 * nq + 3) / 4; }
+// Row length of the grids: nodes, then grid points -4 .. n_f / 2 + 4.
+__host__ __device__ inline int row_points(int nq) { return kGNodes + half_grid(nq) + 9; }
+
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+
+// Element k of a split row: 32 hi, then 32 lo, for every 32 points.
+__device__ __forceinline__ size_t split_at(int k) {
+  return static_cast<size_t>(k >> 5) * 64 + (k & 31);
+}
+
+// ---- extent ----
+
+// Points of a row that the structure's distances reach (a multiple of 32),
+// from its bounding sphere.
+__global__ __launch_bounds__(1024) void extent_kernel(const AtomRec* __restrict__ pos, int n,
+                                                      double inv_h, int full,
+                                                      int* __restrict__ out) {
+  __shared__ double sh[16][6];
+  __shared__ double rad[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double v[6];  // max of x, y, z and of -x, -y, -z
+  for (int k = 0; k < 6; ++k) v[k] = -1e308;
+  bool bad = false;
+  for (int a = threadIdx.x; a < n; a += 1024) {
+    const AtomRec p = pos[a];
+    const double x[3] = {p.x, p.y, p.z};
+    for (int k = 0; k < 3; ++k) {
+      bad = bad || !(fabs(x[k]) < 1e300);
+      v[k] = fmax(v[k], x[k]);
+      v[k + 3] = fmax(v[k + 3], -x[k]);
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1)
+    for (int k = 0; k < 6; ++k) v[k] = fmax(v[k], __shfl_xor(v[k], off, 64));
+  if (lane == 0)
+    for (int k = 0; k < 6; ++k) sh[wave][k] = v[k];
+  const int any_bad = __syncthreads_or(bad ? 1 : 0);
+  for (int w = 0; w < 16; ++w)
+    for (int k = 0; k < 6; ++k) v[k] = fmax(v[k], sh[w][k]);
+  double r2 = 0.0;
+  for (int a = threadIdx.x; a < n; a += 1024) {
+    const AtomRec p = pos[a];
+    const double x = p.x - 0.5 * (v[0] - v[3]), y = p.y - 0.5 * (v[1] - v[4]),
+                 z = p.z - 0.5 * (v[2] - v[5]);
+    r2 = fmax(r2, x * x + y * y + z * z);
+  }
+  for (int off = 32; off > 0; off >>= 1) r2 = fmax(r2, __shfl_xor(r2, off, 64));
+  if (lane == 0) rad[wave] = r2;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 0; w < 16; ++w) r2 = fmax(r2, rad[w]);
+  const double t = 2.0 * sqrt(r2) * 1.000001 * inv_h;
+  const double want = any_bad || !(t < full) ? full : fmin(static_cast<double>(full), t + kGNodes + 10.0);
+  *out = (static_cast<int>(want) + 31) & ~31;
+}
+
+// ---- spreading ----
+
+// A pair closer than the fixed point's fast range, or at an infinite
+// distance: FP64 and 64-bit conversions.
+__device__ void spread_grad_rare(unsigned long long* grid, int plane, int* bad, const double* d,
+                                 double t, double nf, double scale) {
+  if (!(t < 1e300)) {
+    *bad = 1;
+    return;
+  }
+  auto add = [&](int at, double v) {
+    for (int c = 0; c < 3; ++c)
+      atomicAdd(&grid[c * plane + at],
+                static_cast<unsigned long long>(static_cast<long long>(rint(v * d[c]))));
+  };
+  if (t < kGClose) {
+    const double s = t * t;
+    for (int k = 0; k < kGNodes; ++k) {
+      double l = scale;
+      for (int j = 0; j < kGNodes; ++j)
+        if (j != k)
+          l *= (s - g_node(j) * g_node(j)) / (g_node(k) * g_node(k) - g_node(j) * g_node(j));
+      add(k, l);
+    }
+    return;
+  }
+  double u = t - nf * floor(t / nf);
+  const bool neg = u > 0.5 * nf;
+  if (neg) u = nf - u;
+  const double fl = floor(u);
+  const double y = u - fl - 0.5;
+  const int g = kGNodes + static_cast<int>(fl) + 1;
+  for (int j = 0; j < kGw; ++j) {
+    const int jj = j < 4 ? j : kGw - 1 - j;
+    const double z = j < 4 ? y : -y;
+    double phi = kPhi[jj][6], chi = kChi[jj][7];
+    for (int k = 5; k >= 0; --k) phi = phi * z + static_cast<double>(kPhi[jj][k]);
+    for (int k = 6; k >= 0; --k) chi = chi * z + static_cast<double>(kChi[jj][k]);
+    if (j >= 4) chi = -chi;
+    // past half the period sin changes sign and cos does not
+    add(g + j, (neg ? chi + phi / t : chi - phi / t) * scale / (t * t));
+  }
+}
+
+// One block per atom and element run: the lanes of its waves take the run's
+// atoms in turn and add their 8 points to the block's three grids in LDS.
+// ds_add_u64 bounds it: 24 per 64 pairs, 115 ns per CU at random addresses,
+// against about 90 ns of VALU work on the 4 SIMDs beside it.  64-bit sums are
+// needed: entries reach far above the noise level where distant atoms add up
+// coherently, and 32 bits scaled to a safe bound would leave 1e-6 of the
+// gradient.
+//
+// Afterwards the grids leave as split rows (hi and lo halves), each scaled so
+// that its largest entry lies in [2^14, 2^15).
+__global__ __launch_bounds__(1024, 8) void spread_grad_kernel(
+    const AtomRec* __restrict__ pos, int p0, int n_rows, const int* __restrict__ runs, double inv_h, int nf, int plane, int row_len, int k_fixed,
+    const int* __restrict__ k_dev, float scale, double near,
+    _Float16* __restrict__ rows, float* __restrict__ row_scale) {
+  extern __shared__ unsigned long long grid[];
+  __shared__ int bad;
+  __shared__ unsigned int top[3];
+  const int p = p0 + blockIdx.x;
+  const int n_thread = blockDim.x;
+  const int k_used = k_dev ? *k_dev : k_fixed;
+  const int k_end = min(k_used, plane);  // no distance reaches past k_used
+  const int run = blockIdx.y;
+  const int jb = runs[run], je = runs[run + 1];
+  for (int c = 0; c < 3; ++c)
+    for (int g = threadIdx.x; g < k_end; g += n_thread) grid[c * plane + g] = 0ull;
+  if (threadIdx.x == 0) bad = 0;
+  if (threadIdx.x < 3) top[threadIdx.x] = 0u;
+  __syncthreads();
+  const AtomRec pi = pos[p];
+  const double half_nf = 0.5 * nf;
+  const float fh = static_cast<float>(inv_h);
+  bool rare = false;
+  for (int j = jb + static_cast<int>(threadIdx.x); j < je; j += n_thread) {
+    const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
+    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    if (!(r2 > 0.0)) continue;  // the atom itself, a duplicate, a NaN
+    double t = scaled_root(r2, inv_h);
+    if (!(t >= near && t < kGFar)) {
+      rare = true;
+      continue;
+    }
+    float it = __builtin_amdgcn_rcpf(static_cast<float>(t));
+    const float w = scale * it * it * fh;
+    const float wx = w * static_cast<float>(dx), wy = w * static_cast<float>(dy),
+                wz = w * static_cast<float>(dz);
+    if (t > half_nf) {
+      t -= nf * floor(t / nf);
+      if (t > half_nf) {
+        t = nf - t;
+        it = -it;
+      }
+    }
+    const double fl = floor(t);
+    const float y = static_cast<float>(t - fl) - 0.5f;
+    const float y2 = y * y;
+    unsigned long long* gx = grid + kGNodes + static_cast<int>(fl) + 1;
+    unsigned long long *gy = gx + plane, *gz = gy + plane;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float ec = fmaf(fmaf(fmaf(kChi[k][6], y2, kChi[k][4]), y2, kChi[k][2]), y2, kChi[k][0]);
+      const float oc = fmaf(fmaf(fmaf(kChi[k][7], y2, kChi[k][5]), y2, kChi[k][3]), y2, kChi[k][1]);
+      const float ep = fmaf(fmaf(fmaf(kPhi[k][6], y2, kPhi[k][4]), y2, kPhi[k][2]), y2, kPhi[k][0]);
+      const float op = fmaf(fmaf(kPhi[k][5], y2, kPhi[k][3]), y2, kPhi[k][1]);
+      // point k: chi - phi / t at y; point 7 - k: -chi - phi / t at -y
+      const float a = fmaf(y, fmaf(-it, op, oc), fmaf(-it, ep, ec));
+      const float b = fmaf(y, fmaf(it, op, oc), -fmaf(it, ep, ec));
+      auto add = [](unsigned long long* at, float v) {
+        atomicAdd(at, static_cast<unsigned long long>(static_cast<long long>(nearest(v))));
+      };
+      add(&gx[k], a * wx);
+      add(&gy[k], a * wy);
+      add(&gz[k], a * wz);
+      add(&gx[kGw - 1 - k], b * wx);
+      add(&gy[kGw - 1 - k], b * wy);
+      add(&gz[kGw - 1 - k], b * wz);
+    }
+  }
+  // few pairs of a physical structure, if any, are left for a second look
+  if (__syncthreads_or(rare ? 1 : 0)) {
+    for (int j = jb + static_cast<int>(threadIdx.x); j < je; j += n_thread) {
+      const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
+      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+      if (!(r2 > 0.0)) continue;
+      const double t = scaled_root(r2, inv_h);
+      if (t >= near && t < kGFar) continue;
+      const double d[3] = {dx * inv_h, dy * inv_h, dz * inv_h};
+      spread_grad_rare(grid, plane, &bad, d, sqrt(r2) * inv_h, static_cast<double>(nf),
+                       static_cast<double>(scale));
+    }
+    __syncthreads();
+  }
+  // the largest entry of each row, as a non-negative float's bits
+  for (int c = 0; c < 3; ++c) {
+    float m = 0.f;
+    for (int k = threadIdx.x; k < k_end; k += n_thread)
+      m = fmaxf(m, fabsf(static_cast<float>(static_cast<long long>(grid[c * plane + k]))));
+    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+    if ((threadIdx.x & 63) == 0) atomicMax(&top[c], __float_as_uint(m));
+  }
+  __syncthreads();
+  for (int c = 0; c < 3; ++c) {
+    const size_t row = static_cast<size_t>(run) * n_rows + 3 * static_cast<size_t>(blockIdx.x) + c;
+    const float m = __uint_as_float(top[c]);
+    int e = 0;
+    if (m > 0.f) (void)frexpf(m, &e);  // m in [2^(e-1), 2^e)
+    _Float16* out = rows + row * 2 * row_len;
+    for (int k = threadIdx.x; k < k_used; k += n_thread) {
+      const double v = k < k_end ? static_cast<double>(static_cast<long long>(grid[c * plane + k])) : 0.0;
+      const float x = static_cast<float>(ldexp(v, 15 - e));
+      const _Float16 hi = static_cast<_Float16>(x);
+      out[split_at(k)] = hi;
+      out[split_at(k) + 32] = static_cast<_Float16>(x - static_cast<float>(hi));
+    }
+    if (threadIdx.x == 0) row_scale[row] = bad ? __builtin_nanf("") : ldexpf(1.0f / scale, e - 15);
+  }
+}
+
+// ---- the sine matrix ----
+
+// w[m][k], split like the rows, scaled by 2^14: node columns
+// phihat (q cos(q t) / t^2 - sin(q t) / t^3), grid columns sin(2 pi g m / n_f).
+__global__ void sine_matrix_kernel(int nq, int nf, int row_len, _Float16* __restrict__ w,
+                                   float* __restrict__ inv_phihat) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  const int m = blockIdx.y;
+  if (k >= row_len) return;
+  const double q = 2.0 * M_PI * m / nf;
+  const double a = sqrt(fmax(kGBeta * kGBeta - 0.25 * kGw * kGw * q * q, 1.0));
+  const double phihat = (sinh(a) / a) / (sinh(kGBeta) / kGBeta);
+  double v = 0.0;
+  if (k < kGNodes) {
+    const double t = g_node(k);
+    v = phihat * (q * cos(q * t) - sin(q * t) / t) / (t * t);
+  } else if (k < row_points(nq)) {
+    const long long g = k - kGNodes - 4;
+    v = sinpi(2.0 * static_cast<double>(g * m % nf) / nf);
+  }
+  const float x = static_cast<float>(v * 16384.0);
+  const _Float16 hi = static_cast<_Float16>(x);
+  _Float16* out = w + static_cast<size_t>(m) * 2 * row_len;
+  out[split_at(k)] = hi;
+  out[split_at(k) + 32] = static_cast<_Float16>(static_cast<float>(v * 16384.0 - static_cast<double>(hi)));
+  if (k == 0) inv_phihat[m] = static_cast<float>(1.0 / phihat / 16384.0);
+}
+
+// ---- rows times sine matrix ----
+
+// out[atom][c][m] = gs[m] f_i(m) / phihat(m) sum_run f_run(m) sum_k rows w.
+// Block tile 128 rows x 128 bins, 4 waves of 64 x 64 (2 x 2 MFMA 32x32x16 in
+// FP16, three products each), K in steps of 32 through double-buffered LDS.  A
+// row's 32 hi and 32 lo values of a step are one 128-byte line in memory and in
+// LDS, where its eight 16-byte chunks are permuted by the row (chunk ^ row mod
+// 8), so the eight rows read together meet different banks.  Consecutive
+// blocks of an XCD (block id mod 8) share a row tile, which stays in its L2.
+// Sums leave the MFMA accumulators every 128 points: a single FP32 chain over
+// the row rounds at the size of its running sum, and left the gradient 3.9e-7
+// off at 6,699 atoms.
+// Operand layout (lane l): A[l % 32][8 (l / 32) + i], B likewise; result
+// register v: row v % 4 + 8 (v / 4) + 4 (l / 32), column l % 32.
+constexpr int kFold = 4;  // steps of 32 points
+
+template <typename OUT, bool MULTI>
+__global__ __launch_bounds__(256, 2) void gemm_split_kernel(
+    const _Float16* __restrict__ rows, const float* __restrict__ row_scale, int n_rows, int n_run,
+    const _Float16* __restrict__ w, const float* __restrict__ inv_phihat, int row_len, int k_fixed,
+    const int* __restrict__ k_dev, int nq, int n_ct, int n_rt, float unit,
+    const double* __restrict__ gs, const float* __restrict__ ftab,
+    const int* __restrict__ run_elem, const AtomRec* __restrict__ pos,
+    const int32_t* __restrict__ perm, int p0, OUT* __restrict__ out) {
+  __shared__ __align__(16) unsigned char tile[2][2][128 * 128];
+  __shared__ float rsc[2][128];  // the row scales of this and the next run
+  const int bid = blockIdx.x;
+  const int rt = (bid / 8) / n_ct * 8 + bid % 8;
+  const int ct = (bid / 8) % n_ct;
+  if (rt >= n_rt) return;  // padding block (uniform, before any barrier)
+  const int bm = rt * 128, bn = ct * 128;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int k_used = k_dev ? *k_dev : k_fixed;
+  const int nk = k_used >> 5;
+  const int steps = MULTI ? nk * n_run : nk;
+
+  // a thread moves chunk c = threadIdx.x % 8 of rows threadIdx.x / 8 + 32 s
+  const int chunk = threadIdx.x & 7, trow = threadIdx.x >> 3;
+  v4u ra[4], rb[4];
+  auto load = [&](int step) {
+    const int run = MULTI ? step / nk : 0, kk = MULTI ? step % nk : step;
+    const size_t at = static_cast<size_t>(kk) * 64 + chunk * 8;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int r = min(bm + trow + 32 * s, n_rows - 1), q = min(bn + trow + 32 * s, nq - 1);
+      ra[s] = *reinterpret_cast<const v4u*>(
+          rows + (static_cast<size_t>(run) * n_rows + r) * 2 * row_len + at);
+      rb[s] = *reinterpret_cast<const v4u*>(w + static_cast<size_t>(q) * 2 * row_len + at);
+    }
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int r = trow + 32 * s;
+      const int at = r * 128 + ((chunk ^ (r & 7)) * 16);
+      *reinterpret_cast<v4u*>(&tile[buf][0][at]) = ra[s];
+      *reinterpret_cast<v4u*>(&tile[buf][1][at]) = rb[s];
+    }
+  };
+  v16f acc[2][2], tot[2][2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[x][y][v] = 0.f, tot[x][y][v] = 0.f;
+  auto fragment = [&](const unsigned char* base, int r, int c) {
+    return *reinterpret_cast<const v8h*>(base + r * 128 + ((c ^ (r & 7)) * 16));
+  };
+  auto stage = [&](int run) {
+    if (threadIdx.x < 128)
+      rsc[run & 1][threadIdx.x] = row_scale[static_cast<size_t>(run) * n_rows +
+                                            min(bm + static_cast<int>(threadIdx.x), n_rows - 1)];
+  };
+  auto fold = [&](int run) {  // with several elements weighted by f_run and the row scale
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+      const int m = min(bn + wn * 64 + y * 32 + (lane & 31), nq - 1);
+      const float f = MULTI ? ftab[static_cast<size_t>(run_elem[run]) * nq + m] : 1.f;
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int r = wm * 64 + x * 32 + (v & 3) + 8 * (v >> 2) + 4 * (lane >> 5);
+          tot[x][y][v] = MULTI ? fmaf(acc[x][y][v] * f, rsc[run & 1][r], tot[x][y][v])
+                               : tot[x][y][v] + acc[x][y][v];
+          acc[x][y][v] = 0.f;
+        }
+    }
+  };
+  load(0);
+  store(0);
+  stage(0);
+  __syncthreads();
+  for (int step = 0; step < steps; ++step) {
+    const int cur = step & 1;
+    if (step + 1 < steps) load(step + 1);
+    const unsigned char* a_s = tile[cur][0];
+    const unsigned char* b_s = tile[cur][1];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {  // 16 of the step's 32 points
+      const int c = h * 2 + (lane >> 5);
+      v8h ah[2], al[2], bh[2], bl[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int r = wm * 64 + x * 32 + (lane & 31);
+        ah[x] = fragment(a_s, r, c);
+        al[x] = fragment(a_s, r, c + 4);
+        const int q = wn * 64 + x * 32 + (lane & 31);
+        bh[x] = fragment(b_s, q, c);
+        bl[x] = fragment(b_s, q, c + 4);
+      }
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+          acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[x], bh[y], acc[x][y], 0, 0, 0);
+          acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[x], bl[y], acc[x][y], 0, 0, 0);
+          acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[x], bh[y], acc[x][y], 0, 0, 0);
+        }
+    }
+    if (step + 1 < steps) store(cur ^ 1);
+    const int kk = MULTI ? step % nk : step;
+    if (kk + 1 == nk || kk % kFold == kFold - 1) {
+      const int run = MULTI ? step / nk : 0;
+      fold(run);
+      if (MULTI && kk + 1 == nk && run + 1 < n_run) stage(run + 1);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int y = 0; y < 2; ++y) {
+    const int m = bn + wn * 64 + y * 32 + (lane & 31);
+    if (m >= nq) continue;
+    const float col = static_cast<float>(gs[m] * static_cast<double>(unit)) * inv_phihat[m];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int r = bm + wm * 64 + x * 32 + (v & 3) + 8 * (v >> 2) + 4 * (lane >> 5);
+        if (r >= n_rows) continue;
+        const int p = p0 + r / 3;
+        float g;
+        if constexpr (MULTI)
+          g = tot[x][y][v] * ftab[static_cast<size_t>(static_cast<int>(pos[p].w)) * nq + m];
+        else
+          g = tot[x][y][v] * rsc[0][r - bm];
+        const size_t o = (3 * static_cast<size_t>(perm ? perm[p] : p) + r % 3) * nq + m;
+        out[o] = static_cast<OUT>(g * col);
+      }
+  }
+}
+
+}  // namespace
+
+double grad_reach(int nq, double dq, double r_max) { return r_max * dq * half_grid(nq) / M_PI + kGNodes + 10.0; }
+int grad_row_len(int nq) { return (row_points(nq) + 31) & ~31; }
+size_t grad_lds_bytes(int nq) {
+  return sizeof(unsigned long long) * 3 * static_cast<size_t>(row_points(nq) | 1);
+}
+
+hipError_t launch_grad_extent(hipStream_t st, const AtomRec* pos, int64_t n, int nq, double dq,
+                              int* out) {
+  hipLaunchKernelGGL(extent_kernel, dim3(1), dim3(1024), 0, st, pos, static_cast<int>(n),
+                     dq * half_grid(nq) / M_PI, row_points(nq), out);
+  return hipGetLastError();
+}
+
+hipError_t launch_sine_matrix(hipStream_t st, int nq, void* w, float* inv_phihat) {
+  const int len = grad_row_len(nq);
+  if (nq > 65535) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(sine_matrix_kernel, dim3((len + 255) / 256, nq), dim3(256), 0, st, nq, 2 * half_grid(nq),
+                     len, static_cast<_Float16*>(w), inv_phihat);
+  return hipGetLastError();
+}
+
+hipError_t launch_spread_grad(hipStream_t st, const AtomRec* pos, int p0, int n_atoms, int64_t n,
+                              const int* runs, int n_run, int nq, double dq, double r_max,
+                              int k_fixed, const int* k_dev, void* rows, float* row_scale) {
+  const int nf = 2 * half_grid(nq);
+  const double inv_h = dq * half_grid(nq) / M_PI;
+  const size_t lds = grad_lds_bytes(nq);
+  if (lds > kGradLds || n_run > 65535) return hipErrorInvalidValue;
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(spread_grad_kernel),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kGradLds));
+  if (attr != hipSuccess) return attr;
+  int s = kGMinScale;
+  while (s < kGMaxScale && std::ldexp(1.0, s - kGBits) < r_max * inv_h && r_max < 1e30) ++s;
+  const unsigned threads = n <= 256 ? 256 : n <= 2048 ? 512 : 1024;
+  hipLaunchKernelGGL(spread_grad_kernel, dim3(n_atoms, n_run), dim3(threads), lds, st, pos, p0,
+                     3 * n_atoms, runs, inv_h, nf, row_points(nq) | 1, grad_row_len(nq), k_fixed,
+                     k_dev, std::ldexp(1.0f, s), 1.2 * std::ldexp(1.0, s - 31),
+                     static_cast<_Float16*>(rows), row_scale);
+  return hipGetLastError();
+}
+
+hipError_t launch_gemm_split(hipStream_t st, const void* rows, const float* row_scale, int n_atoms,
+                             int n_run, const void* w, const float* inv_phihat, int nq, double dq,
+                             int k_fixed, const int* k_dev, const double* gs, const float* ftab,
+                             const int* run_elem, bool weighted, const AtomRec* pos,
+                             const int32_t* perm, int p0, void* out, bool out_f64) {
+  const int n_rows = 3 * n_atoms;
+  const int n_ct = (nq + 127) / 128, n_rt = (n_rows + 127) / 128;
+  const double inv_h = dq * half_grid(nq) / M_PI;
+  const float unit = static_cast<float>(inv_h * inv_h);
+  const dim3 grid(8u * static_cast<unsigned>((n_rt + 7) / 8) * n_ct);
+  const int len = grad_row_len(nq);
+#define PYIID_GEMM(T, M)                                                                        \
+  hipLaunchKernelGGL((gemm_split_kernel<T, M>), grid, dim3(256), 0, st,                         \
+                     static_cast<const _Float16*>(rows), row_scale, n_rows, n_run,              \
+                     static_cast<const _Float16*>(w), inv_phihat, len, k_fixed, k_dev, nq, n_ct, \
+                     n_rt, unit, gs, ftab, run_elem, pos, perm, p0, static_cast<T*>(out))
+  if (weighted) {
+    if (out_f64)
+      PYIID_GEMM(double, true);
+    else
+      PYIID_GEMM(float, true);
+  } else {
+    if (out_f64)
+      PYIID_GEMM(double, false);
+    else
+      PYIID_GEMM(float, false);
+  }
+#undef PYIID_GEMM
+  return hipGetLastError();
+}
+
+}  // namespace pyiid

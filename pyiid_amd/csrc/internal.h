@@ -117,7 +117,7 @@ struct SpreadItem {
 struct SpreadUnit {
   int begin, end, grid, pad;
 };
-constexpr size_t kSpreadLds = 160 * 1024;  // a block's grid lives in LDS
+constexpr size_t kSpreadLds = 160 * 1024 - 256;  // a block's grid lives in LDS
 int fq_grid_points(int nq);
 int fq_grid_stride(int nq);  // 64-bit words per grid (points, close-contact nodes, flag)
 // Bits of the grid's fixed point for distances up to about r_max.
@@ -138,6 +138,30 @@ hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_
 // out[p] = pos[perm[p]]
 hipError_t launch_gather(hipStream_t st, const AtomRec* pos, const int32_t* perm, int64_t n,
                          AtomRec* out);
+
+// ---- gradient by spreading (gradspread.hip) ----
+constexpr size_t kGradLds = 160 * 1024 - 512;   // a block's three grids live in LDS
+int grad_row_len(int nq);                     // points per row (a multiple of 32)
+size_t grad_lds_bytes(int nq);
+double grad_reach(int nq, double dq, double r_max);  // points of a row that r_max reaches
+// *out: points of a row (a multiple of 32) that distances within pos reach
+hipError_t launch_grad_extent(hipStream_t st, const AtomRec* pos, int64_t n, int nq, double dq,
+                              int* out);
+// w: 2 * nq * grad_row_len(nq) halves; inv_phihat: nq floats
+hipError_t launch_sine_matrix(hipStream_t st, int nq, void* w, float* inv_phihat);
+// Grids of positions [p0, p0 + n_atoms) against each of the n_run element
+// runs [runs[e], runs[e + 1]): rows (e * 3 n_atoms + 3 (p - p0) + c), 2 *
+// grad_row_len halves each, and row_scale.  Points used: k_fixed, or *k_dev.
+hipError_t launch_spread_grad(hipStream_t st, const AtomRec* pos, int p0, int n_atoms, int64_t n,
+                              const int* runs, int n_run, int nq, double dq, double r_max,
+                              int k_fixed, const int* k_dev, void* rows, float* row_scale);
+// out[perm[p]][c][m] = gs[m] f_p(m) sum_e f_e(m) sum_k rows w / phihat
+// (single element: without f).  perm null: identity.
+hipError_t launch_gemm_split(hipStream_t st, const void* rows, const float* row_scale, int n_atoms,
+                             int n_run, const void* w, const float* inv_phihat, int nq, double dq,
+                             int k_fixed, const int* k_dev, const double* gs, const float* ftab,
+                             const int* run_elem, bool weighted, const AtomRec* pos,
+                             const int32_t* perm, int p0, void* out, bool out_f64);
 
 // ---- contracted forces from a pair-force table (forcetab.hip) ----
 // Unit: positions [i0, i1) in `tiles` (1, 2, 4, 8 or 16) tiles of 64 against

@@ -34,7 +34,7 @@
 #include <algorithm>
 #include <cmath>
 
-#include "internal.h"
+#include "pair_math.h"
 
 namespace pyiid {
 namespace {
@@ -80,9 +80,11 @@ __device__ __forceinline__ double fold(double t, double nf, bool& neg) {
   return neg ? nf - u : u;
 }
 
+constexpr double kFqFar = 1e15;  // beyond: spread_rare
+
 // A pair closer than the fixed point's fast range, or at an infinite
 // distance: 64-bit conversions.  Few pairs of a physical structure come here.
-__device__ __noinline__ void spread_rare(unsigned long long* hist, int n_grid, double t, double nf,
+__device__ void spread_rare(unsigned long long* hist, int n_grid, double t, double nf,
                                          double scale) {
   unsigned long long* nodes = hist + n_grid;
   if (!(t < 1e300)) {  // infinite: F is not a number
@@ -137,6 +139,7 @@ __global__ __launch_bounds__(1024, 8) void spread_fq_kernel(
   __syncthreads();
   const SpreadUnit un = units[blockIdx.x];
   const double half_nf = 0.5 * nf;
+  bool rare = false;
   for (int it = un.begin; it < un.end; ++it) {
     const SpreadItem item = items[it];
     const int len = item.j1 - item.j0;
@@ -150,22 +153,10 @@ __global__ __launch_bounds__(1024, 8) void spread_fq_kernel(
       const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
       // j < i; a pair at distance 0 (and one with a NaN) contributes nothing
       if (!(have && j < i && r2 > 0.0)) continue;
-      // FP32 root refined by one Newton step in FP64
-      const float r2f = static_cast<float>(r2);
-      const float y0 = __builtin_amdgcn_rsqf(r2f);
-      const float rf = r2f * y0;
-      const double rd = static_cast<double>(rf);
-      const double r = fma(fma(-rd, rd, r2), static_cast<double>(0.5f * y0), rd);
-      double t = r * inv_h;
-      if (!(t >= near && t <= half_nf)) {
-        // (r2 outside float's range reaches this branch with any r: take the
-        // FP64 root)
-        const double ta = sqrt(r2) * inv_h;
-        if (!(ta >= near && ta < 1e300)) {
-          spread_rare(hist, n_grid, ta, static_cast<double>(nf), static_cast<double>(scale));
-          continue;
-        }
-        t = ta;
+      double t = scaled_root(r2, inv_h);
+      if (!(t >= near && t < kFqFar)) {
+        rare = true;
+        continue;
       }
       float w = scale * __builtin_amdgcn_rcpf(static_cast<float>(t));
       if (t > half_nf) {
@@ -175,22 +166,37 @@ __global__ __launch_bounds__(1024, 8) void spread_fq_kernel(
       }
       const double fl = floor(t);
       const float y = static_cast<float>(t - fl) - 0.5f;
-      const float half = __builtin_copysignf(0.5f, w);
       const float y2 = y * y;
       unsigned long long* h = hist + (static_cast<int>(fl) + 1);
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         const float e = fmaf(fmaf(kFqVal[k][4], y2, kFqVal[k][2]), y2, kFqVal[k][0]);
         const float o = y * fmaf(fmaf(kFqVal[k][5], y2, kFqVal[k][3]), y2, kFqVal[k][1]);
-        // truncation after + 1/2 rounds to nearest
-        const int a = static_cast<int>(fmaf(e + o, w, half));
-        const int b = static_cast<int>(fmaf(e - o, w, half));
+        const int a = nearest((e + o) * w), b = nearest((e - o) * w);
         atomicAdd(&h[k], static_cast<unsigned long long>(static_cast<long long>(a)));
         atomicAdd(&h[kFqW - 1 - k], static_cast<unsigned long long>(static_cast<long long>(b)));
       }
     }
   }
-  __syncthreads();
+  // few pairs of a physical structure, if any, are left for a second look
+  if (__syncthreads_or(rare ? 1 : 0)) {
+    for (int it = un.begin; it < un.end; ++it) {
+      const SpreadItem item = items[it];
+      const int i = item.i0 + lane;
+      if (i >= item.i1) continue;
+      const AtomRec pi = pos[i];
+      for (int j = item.j0 + wave; j < item.j1; j += n_wave) {
+        const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
+        const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+        if (!(j < i && r2 > 0.0)) continue;
+        const double t = scaled_root(r2, inv_h);
+        if (t >= near && t < kFqFar) continue;
+        spread_rare(hist, n_grid, sqrt(r2) * inv_h, static_cast<double>(nf),
+                    static_cast<double>(scale));
+      }
+    }
+    __syncthreads();
+  }
   unsigned long long* out = grids + static_cast<size_t>(un.grid) * stride;
   for (int g = threadIdx.x; g < stride; g += blockDim.x) {
     const long long v = static_cast<long long>(hist[g]);

@@ -186,3 +186,68 @@ def test_long_force_table(ctx):
     for length in (140.0, 400.0):
         pos = np.random.RandomState(4).uniform(0, length, (70, 3)).astype(np.float32)
         force_check(ctx, pos, pos, np.full(70, 79), 0.05, 600)
+
+
+def grad_check(ctx, pos, numbers, qbin, nq, f64=False, per_atom=None):
+    """The gradient against the oracle.  Allowed per entry: the window's worst
+    errors (3.2e-7 of the largest Q for the cosine term, 3.5e-7 for the sine
+    term, single-precision values included) for every pair, and 2^-20 of the
+    largest entry for the two-half products."""
+    if per_atom is None:
+        per_atom = load(ctx, pos, numbers, qbin, nq)
+    got = ctx.grad_fq(_lib.SLOT_FQ, qbin, len(pos), nq, f64=f64)
+    assert ctx.grad_shape() == (False, 0, 0)
+    want = oracle.grad_fq(pos, per_atom, qbin)
+    x, f = pos.astype(np.float64), np.abs(per_atom.astype(np.float64))
+    r = np.linalg.norm(x[:, None] - x[None], axis=-1)
+    inv = np.divide(1.0, r, out=np.zeros_like(r), where=r > 0)
+    na = np.abs(oracle.normalization(per_atom))
+    pair = 3.2e-7 * qbin * nq * inv + 3.5e-7 * inv * inv
+    allowed = np.einsum("iq,jq,ij->iq", f, f, pair) / na + 2.0 ** -20 * np.abs(want).max() + 1e-30
+    assert np.all(np.isfinite(got))
+    off = (np.abs(got - want) / allowed[:, None, :]).max()
+    assert off < 1.0, off
+
+
+@pytest.mark.parametrize("n", [2, 3, 42, 43, 65, 300])
+@pytest.mark.parametrize("nq", [1, 2, 31, 127, 128, 129, 330])
+def test_gradient_tiles(ctx, n, nq):
+    pos = structures.jitter(structures.fcc_nearest(n), 0.05, seed=n).astype(np.float32)
+    numbers = np.full(n, 79) if nq != 129 else np.array([28, 78, 79])[np.arange(n) % 3]
+    grad_check(ctx, pos, numbers, 25.0 / nq, nq, f64=nq % 2 == 1)
+
+
+def test_gradient_largest_grid(ctx):
+    pos = structures.jitter(structures.fcc_nearest(25), 0.05, seed=1).astype(np.float32)
+    grad_check(ctx, pos, np.full(25, 79), 0.009, 3010)
+
+
+@pytest.mark.parametrize("r", [1e-3, 0.02, 0.1116, 0.1118, 0.5, 1.07, 1.08])
+def test_gradient_close_contacts(ctx, r):
+    """A pair at the kernel's short ranges (grid spacing 0.0558 A)."""
+    pos = structures.jitter(structures.fcc_nearest(50), 0.05, seed=5).astype(np.float32)
+    pos[7], pos[20] = 0.0, (r, 0, 0)
+    grad_check(ctx, pos, np.full(50, 79), 0.1, 250)
+
+
+@pytest.mark.parametrize("length", [30.0, 314.0, 4e3])
+def test_gradient_beyond_the_period(ctx, length):
+    rs = np.random.RandomState(3)
+    pos = rs.uniform(-length, length, (90, 3)).astype(np.float32)
+    pos[0], pos[1] = 0.0, (np.float32(4 * np.pi / np.float32(0.1)), 0, 0)
+    grad_check(ctx, pos, np.full(90, 79), 0.1, 250)
+
+
+def test_gradient_of_positions_moved_on_the_device(ctx):
+    """The reach of the grid comes from the device after an upload there: a
+    larger structure of the same size, then a smaller one, equal to host mode."""
+    import torch
+    base = structures.jitter(structures.fcc_nearest(150), 0.05, seed=6).astype(np.float32)
+    per_atom = load(ctx, base, np.full(150, 79), 0.05, 400)
+    for scale in (1.0, 2.5, 0.8):
+        pos = (base * np.float32(scale)).astype(np.float32)
+        ctx.set_positions(torch.from_numpy(pos).cuda(), flags=_lib.PYIID_DEVICE)
+        got = ctx.grad_fq(_lib.SLOT_FQ, 0.05, 150, 400)
+        grad_check(ctx, pos, None, 0.05, 400, per_atom=per_atom)
+        ctx.set_positions(pos)
+        np.testing.assert_array_equal(got, ctx.grad_fq(_lib.SLOT_FQ, 0.05, 150, 400))
