@@ -127,7 +127,7 @@ struct SpreadSet {
   Buf perm;    // int32 [n]: atom per position (weighted tables: element order)
   Buf sorted;  // AtomRec [n]: positions in that order (weighted tables)
   Buf grids;   // uint64 [chain][element pair][fq_grid_stride]: zero between calls
-  Buf done;    // int32 [chain]: zero between calls
+  Buf part;    // FP64 partial transforms
   bool dirty = false;  // a launch failed between spreading and transform
   int n_units = 0, shift = 0;
   uint64_t stamp = ~0ull;
@@ -841,10 +841,13 @@ struct Timed {
 // pair); beyond it the recurrence kernel runs.
 constexpr size_t kSpreadGridBudget = static_cast<size_t>(512) << 20;
 
+int64_t element_pairs(const Table& t) {
+  return weighted_table(t) ? static_cast<int64_t>(t.n_elem) * (t.n_elem + 1) / 2 : 1;
+}
+
 size_t spread_grid_bytes(pyiid_ctx* c, const Table& t) {
-  const size_t pairs =
-      weighted_table(t) ? static_cast<size_t>(t.n_elem) * (t.n_elem + 1) / 2 : 1;
-  return sizeof(uint64_t) * static_cast<size_t>(fq_grid_stride(t.nq)) * pairs * c->n_chain;
+  return sizeof(uint64_t) * static_cast<size_t>(fq_grid_stride(t.nq)) *
+         static_cast<size_t>(element_pairs(t)) * c->n_chain;
 }
 
 // Whether F(Q) runs on the spreading kernel: its grid fits LDS, the grids fit
@@ -853,7 +856,7 @@ size_t spread_grid_bytes(pyiid_ctx* c, const Table& t) {
 bool use_spread_fq(pyiid_ctx* c, const Table& t) {
   return !c->compensated && c->fq_m_fixed == 0 &&
          sizeof(uint64_t) * static_cast<size_t>(fq_grid_stride(t.nq)) <= kSpreadLds &&
-         spread_grid_bytes(c, t) <= kSpreadGridBudget;
+         spread_grid_bytes(c, t) <= kSpreadGridBudget && c->n_chain <= 65535;
 }
 
 // Atoms as positions in element order per chain (stable), and each chain's
@@ -907,7 +910,7 @@ int ensure_spread(pyiid_ctx* c, const Table& t) {
       int64_t steps;
     };
     std::vector<Group> groups;
-    const int n_pair = weighted ? t.n_elem * (t.n_elem + 1) / 2 : 1;
+    const int n_pair = static_cast<int>(element_pairs(t));
     int64_t total = 0, max_pairs = 0;
     for (int b = 0; b < c->n_chain; ++b) {
       const int64_t nb = c->off[b + 1] - c->off[b];
@@ -974,14 +977,14 @@ int ensure_spread(pyiid_ctx* c, const Table& t) {
     s.stamp = c->struct_stamp;
     s.key = key;
   }
-  const size_t done_bytes = sizeof(int) * static_cast<size_t>(c->n_chain);
-  const bool grow = s.grids.bytes < bytes || s.done.bytes < done_bytes;
+  const int64_t parts =
+      element_pairs(t) * fq_transform_parts(t.nq, c->n_chain, static_cast<int>(element_pairs(t)));
+  CHK(s.part.reserve(sizeof(double) * static_cast<size_t>(parts) * t.nq * c->n_chain));
+  const bool grow = s.grids.bytes < bytes;
   if (grow && c->capturing) return fail(PYIID_E_STATE, "structure changed during graph capture");
   CHK(s.grids.reserve(bytes));
-  CHK(s.done.reserve(done_bytes));
   if (grow || s.dirty) {
     HIPCHK(hipMemsetAsync(s.grids.p, 0, s.grids.bytes, c->stream));
-    HIPCHK(hipMemsetAsync(s.done.p, 0, s.done.bytes, c->stream));
     s.dirty = false;
   }
   return PYIID_OK;
@@ -1032,9 +1035,9 @@ int compute_fq(pyiid_ctx* c, int slot, double qbin) {
                             s.items.as<SpreadItem>(), nq, dq, s.shift, bits,
                             s.grids.as<unsigned long long>()));
     CHK(tm.done());
-    HIPCHK(launch_transform_fq(c->stream, s.grids.as<unsigned long long>(), B, t.n_elem, weighted,
-                               t.tab.as<float>(), nq, dq, s.shift, bits, t.fsu.as<double>(),
-                               c->fq64.as<double>(), c->fq32.as<float>(), s.done.as<int>()));
+    HIPCHK(launch_transform_fq(c->stream, s.grids.as<unsigned long long>(), B,
+                               static_cast<int>(element_pairs(t)), weighted, t.tab.as<float>(), nq,
+                               dq, s.shift, bits, t.fsu.as<double>(), s.part.as<double>(), c->fq64.as<double>(), c->fq32.as<float>()));
     s.dirty = false;
     return PYIID_OK;
   }
@@ -1536,8 +1539,7 @@ int64_t force_cells(pyiid_ctx* c, const Table& t, double dq) {
 // Whether the tables fit LDS and their budget (else the recurrence kernel runs).
 bool use_force_table(pyiid_ctx* c, const Table& t, double dq) {
   const int64_t cells = force_cells(c, t, dq);
-  const int64_t pairs =
-      weighted_table(t) ? static_cast<int64_t>(t.n_elem) * (t.n_elem + 1) / 2 : 1;
+  const int64_t pairs = element_pairs(t);
   return force_lds_bytes(cells) <= kForceLds && pairs * c->n_chain <= 65535 &&
          24.0 * static_cast<double>(cells) * pairs * c->n_chain <=
              static_cast<double>(kForceTableBudget);
@@ -1562,7 +1564,7 @@ int ensure_force(pyiid_ctx* c, const Table& t) {
     for (const ElemRun& r : runs[b])
       total += (r.end - r.begin + 63) / 64 * (c->off[b + 1] - c->off[b]);
   const int64_t steps = std::min<int64_t>(1024, std::max<int64_t>(16, total / 8192));
-  const int n_pair = weighted ? t.n_elem * (t.n_elem + 1) / 2 : 1;
+  const int n_pair = static_cast<int>(element_pairs(t));
   std::vector<ForceUnit> units;
   std::vector<int32_t> planes(static_cast<size_t>(std::max<int64_t>(1, c->n)), 0);
   int n_planes = 1;
@@ -1642,8 +1644,7 @@ int contract_forces(pyiid_ctx* c, int slot, double qbin, double scale, double* o
     ForceSet& s = c->force;
     const bool weighted = weighted_table(t);
     const int n_cell = static_cast<int>(force_cells(c, t, dq));
-    const size_t cells = static_cast<size_t>(n_cell) * B *
-                         (weighted ? t.n_elem * (t.n_elem + 1) / 2 : 1);
+    const size_t cells = static_cast<size_t>(n_cell) * B * element_pairs(t);
     CHK(s.t4.reserve(sizeof(float4) * cells));
     CHK(s.t2.reserve(sizeof(float2) * cells));
     CHK(s.part.reserve(sizeof(double) * 3 * static_cast<size_t>(std::max<int64_t>(1, c->n)) *
@@ -2237,7 +2238,7 @@ int pyiid_destroy(pyiid_ctx* c) {
                  &c->fpart, &c->fq64, &c->fq32, &c->g64, &c->io_a, &c->io_b,
                  &c->io_c, &c->w, &c->out5, &c->u, &c->gobs, &c->fq_items.items,
                  &c->fq_items.ranges, &c->fq_items.perm, &c->spread.units, &c->spread.items,
-                 &c->spread.perm, &c->spread.sorted, &c->spread.grids, &c->spread.done,
+                 &c->spread.perm, &c->spread.sorted, &c->spread.grids, &c->spread.part,
                  &c->force.units, &c->force.planes, &c->force.perm, &c->force.sorted,
                  &c->force.t4, &c->force.t2, &c->force.part,
                  &c->grad.perm, &c->grad.sorted, &c->grad.runs, &c->grad.run_elem, &c->grad.rows,

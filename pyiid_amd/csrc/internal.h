@@ -130,11 +130,13 @@ hipError_t launch_spread_fq(hipStream_t st, const AtomRec* pos, const SpreadUnit
                             int scale_bits, unsigned long long* grids);
 // out[b][q] = scale[b][q] * sum over the chain's element pairs (grid index
 // b * n_pair + e_i (e_i + 1) / 2 + e_j, e_j <= e_i) of f_i f_j times the pair's
-// sum of sin(Q r) / r.  done: n_chain counters, zero before and after.
-hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_chain, int n_elem,
+// sum of sin(Q r) / r; clears the grids.  part: n_chain * n_pair *
+// fq_transform_parts * nq doubles.
+int fq_transform_parts(int nq, int n_chain, int n_pair);
+hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_chain, int n_pair,
                                bool weighted, const float* ftab, int nq, double dq, int shift,
-                               int scale_bits, const double* scale, double* out_f64,
-                               float* out_f32, int* done);
+                               int scale_bits, const double* scale, double* part, double* out_f64,
+                               float* out_f32);
 // out[p] = pos[perm[p]]
 hipError_t launch_gather(hipStream_t st, const AtomRec* pos, const int32_t* perm, int64_t n,
                          AtomRec* out);

@@ -208,95 +208,102 @@ __global__ __launch_bounds__(1024, 8) void spread_fq_kernel(
 
 // ---- grid -> F(Q) ----
 
-constexpr int kTrChunk = 4096;  // grid points in LDS at a time (32 KiB)
+constexpr int kTrChunk = 2048;  // grid points in LDS at a time (16 KiB)
 
-// One block: 64 bins (lanes) of one chain; its 16 waves take consecutive
-// slices of every chunk of grid points.  sin(2 pi g m / n_f) starts from an
-// exact phase and follows the FP64 three-term recurrence along g.  The last
-// block of a chain to finish clears the chain's grids for the next call, so
-// no launch is spent on it.
+// part[b][z][m]: one block takes 64 bins (lanes) of one chain against one of
+// the n_split parts of one element pair's grid; its 16 waves take consecutive
+// slices of every chunk of points.  sin(2 pi g m / n_f) starts from an exact
+// phase and follows the FP64 three-term recurrence along g.  The parts are
+// there to fill the chip: one block per 64 bins took 47 us for 1,250 bins and
+// 155 us for three element pairs at 1,500.
 __global__ __launch_bounds__(1024) void transform_fq_kernel(
-    unsigned long long* __restrict__ grids, int n_pair, int n_elem, int nf, int n_grid, int stride,
-    int shift, int scale_bits, const float* __restrict__ ftab, int nq, double inv_h, int weighted,
-    const double* __restrict__ scale, double* __restrict__ out64, float* __restrict__ out32,
-    int* __restrict__ done) {
-  __shared__ double buf[kTrChunk];
-  __shared__ double part[16][65];
-  __shared__ int last;
+    const unsigned long long* __restrict__ grids, int n_pair, int n_split, int nf, int n_grid,
+    int stride, int shift, int scale_bits, const float* __restrict__ ftab, int nq, double inv_h,
+    int weighted, double* __restrict__ part) {
+  __shared__ __align__(16) double buf[kTrChunk];
+  __shared__ double sums[16][65];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = blockIdx.x * 64 + lane;
-  const int b = blockIdx.y;
-  unsigned long long* chain = grids + static_cast<size_t>(b) * n_pair * stride;
-  const double unit = ldexp(inv_h, shift - scale_bits);
-  const double node_unit = ldexp(inv_h, shift) / kNodeScale;
+  const int b = blockIdx.y, z = blockIdx.z;
+  const int pair = z / n_split, split = z % n_split;
+  const unsigned long long* h = grids + (static_cast<size_t>(b) * n_pair + pair) * stride;
+  const int g_lo = static_cast<int>(static_cast<int64_t>(n_grid) * split / n_split);
+  const int g_hi = static_cast<int>(static_cast<int64_t>(n_grid) * (split + 1) / n_split);
   const double two_over = 2.0 / static_cast<double>(nf);
   const double c2 = 2.0 * cospi(two_over * m);
-  const double q = M_PI * two_over * m;  // Q h
-  const double a2 = kFqBeta * kFqBeta - 0.25 * kFqW * kFqW * q * q;
-  const double a = sqrt(a2 > 1.0 ? a2 : 1.0);
-  const double inv_phihat = (sinh(kFqBeta) / kFqBeta) / (sinh(a) / a);
+  double acc = 0.0;
+  for (int g0 = g_lo; g0 < g_hi; g0 += kTrChunk) {
+    const int cnt = min(kTrChunk, g_hi - g0);
+    __syncthreads();
+    for (int g = threadIdx.x; g < cnt; g += blockDim.x)
+      buf[g] = static_cast<double>(static_cast<long long>(h[g0 + g]));
+    __syncthreads();
+    const int lo = cnt * wave / 16, hi = cnt * (wave + 1) / 16;
+    // phases of grid points g0 + lo - 3 and one before, reduced as integers
+    // (below 2^31: n_f <= 12 * 3,400, g + n_f < 1.6 n_f)
+    const unsigned g = static_cast<unsigned>(g0 + lo - 3 + nf);
+    const unsigned s0 = g * static_cast<unsigned>(m) % static_cast<unsigned>(nf);
+    const unsigned s1 = (g - 1u) * static_cast<unsigned>(m) % static_cast<unsigned>(nf);
+    double y = sinpi(two_over * static_cast<double>(s0));
+    double yp = sinpi(two_over * static_cast<double>(s1));
+#pragma unroll 4
+    for (int k = lo; k < hi; ++k) {
+      acc = fma(buf[k], y, acc);
+      const double yn = fma(c2, y, -yp);
+      yp = y;
+      y = yn;
+    }
+  }
+  sums[wave][lane] = acc;
+  __syncthreads();
+  if (wave != 0 || m >= nq) return;
   double total = 0.0;
-  int ei = 0, ej = 0;
-  for (int p = 0; p < n_pair; ++p) {
-    const unsigned long long* h = chain + static_cast<size_t>(p) * stride;
-    double acc = 0.0;
-    for (int g0 = 0; g0 < n_grid; g0 += kTrChunk) {
-      const int cnt = min(kTrChunk, n_grid - g0);
-      __syncthreads();
-      for (int g = threadIdx.x; g < cnt; g += blockDim.x)
-        buf[g] = static_cast<double>(static_cast<long long>(h[g0 + g]));
-      __syncthreads();
-      const int lo = cnt * wave / 16, hi = cnt * (wave + 1) / 16;
-      // phases of grid points g0 + lo - 3 and one before, reduced as integers
-      const long long s0 = static_cast<long long>(g0 + lo - 3) * m % nf;
-      const long long s1 = static_cast<long long>(g0 + lo - 4) * m % nf;
-      double y = sinpi(two_over * static_cast<double>(s0));
-      double yp = sinpi(two_over * static_cast<double>(s1));
-      for (int g = lo; g < hi; ++g) {
-        acc = fma(buf[g], y, acc);
-        const double yn = fma(c2, y, -yp);
-        yp = y;
-        y = yn;
-      }
-    }
-    acc *= unit * inv_phihat;
-    if (wave == 0) {  // close contacts (almost always none)
-      for (int k = 0; k < kFqNodes; ++k) {
-        const long long v = static_cast<long long>(h[n_grid + k]);
-        if (v != 0) acc += static_cast<double>(v) * node_unit * sin(q * fq_node(k)) / fq_node(k);
-      }
-      if (h[n_grid + kFqNodes] != 0ull) acc = __builtin_nan("");
-    }
-    if (m < nq) {
-      const double f = weighted ? static_cast<double>(ftab[static_cast<size_t>(ei) * nq + m]) *
-                                      static_cast<double>(ftab[static_cast<size_t>(ej) * nq + m])
-                                : 1.0;
-      total = fma(f, acc, total);
-    }
-    if (++ej > ei) {
-      ++ei;
-      ej = 0;
-    }
-  }
-  part[wave][lane] = total;
-  __syncthreads();
-  if (wave == 0 && m < nq) {
-    double t = 0.0;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) t += part[k][lane];
-    const size_t o = static_cast<size_t>(b) * nq + m;
-    const double v = t * scale[o];
-    if (out64) out64[o] = v;
-    if (out32) out32[o] = static_cast<float>(v);
+  for (int k = 0; k < 16; ++k) total += sums[k][lane];
+  const double q = M_PI * two_over * m;  // Q h
+  const double a = sqrt(fmax(kFqBeta * kFqBeta - 0.25 * kFqW * kFqW * q * q, 1.0));
+  total *= ldexp(inv_h, shift - scale_bits) * (sinh(kFqBeta) / kFqBeta) * a / sinh(a);
+  if (split == 0) {  // close contacts (almost always none)
+    for (int k = 0; k < kFqNodes; ++k) {
+      const long long v = static_cast<long long>(h[n_grid + k]);
+      if (v != 0)
+        total += static_cast<double>(v) * (ldexp(inv_h, shift) / kNodeScale) *
+                 sin(q * fq_node(k)) / fq_node(k);
+    }
+    if (h[n_grid + kFqNodes] != 0ull) total = __builtin_nan("");
   }
-  if (threadIdx.x == 0)
-    last = __hip_atomic_fetch_add(&done[b], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
-           static_cast<int>(gridDim.x) - 1;
-  __syncthreads();
-  if (!last) return;
-  const size_t all = static_cast<size_t>(n_pair) * stride;
-  for (size_t g = threadIdx.x; g < all; g += blockDim.x) chain[g] = 0ull;
-  if (threadIdx.x == 0) done[b] = 0;
+  if (weighted) {
+    int ei = 0, ej = pair;
+    while (ej > ei) ej -= ++ei;
+    total *= static_cast<double>(ftab[static_cast<size_t>(ei) * nq + m]) *
+             static_cast<double>(ftab[static_cast<size_t>(ej) * nq + m]);
+  }
+  part[(static_cast<size_t>(b) * n_pair * n_split + z) * nq + m] = total;
+}
+
+// F from the parts (blocks below n_out, one thread per chain and bin), and the
+// grids cleared for the next call (the blocks from n_out).  A launch of its
+// own: with the same work in the transform's last blocks, the agent-scope
+// fences between 288 blocks took 20 us.
+__global__ __launch_bounds__(256) void finish_fq_kernel(
+    const double* __restrict__ part, int n_part, int nq, int64_t total, int n_out,
+    const double* __restrict__ scale, double* __restrict__ out64, float* __restrict__ out32,
+    ulonglong2* __restrict__ grids, int64_t words2) {
+  if (static_cast<int>(blockIdx.x) < n_out) {
+    const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (e >= total) return;
+    const double* p = part + (e / nq) * n_part * nq + e % nq;
+    double t = 0.0;
+#pragma unroll 8
+    for (int z = 0; z < n_part; ++z) t += p[static_cast<size_t>(z) * nq];
+    const double v = t * scale[e];
+    if (out64) out64[e] = v;
+    if (out32) out32[e] = static_cast<float>(v);
+    return;
+  }
+  for (int64_t w = static_cast<int64_t>(blockIdx.x - n_out) * 256 + threadIdx.x; w < words2;
+       w += static_cast<int64_t>(gridDim.x - n_out) * 256)
+    grids[w] = ulonglong2{0ull, 0ull};
 }
 
 __global__ void gather_kernel(const AtomRec* __restrict__ pos, const int32_t* __restrict__ perm,
@@ -334,14 +341,30 @@ hipError_t launch_spread_fq(hipStream_t st, const AtomRec* pos, const SpreadUnit
   return hipGetLastError();
 }
 
-hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_chain, int n_elem,
+// About 512 blocks, and at least 32 grid points for each of a block's waves.
+int fq_transform_parts(int nq, int n_chain, int n_pair) {
+  const int64_t blocks = static_cast<int64_t>((nq + 63) / 64) * n_chain * n_pair;
+  return static_cast<int>(
+      std::max<int64_t>(1, std::min<int64_t>((512 + blocks - 1) / blocks, fq_grid_points(nq) / 512)));
+}
+
+hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_chain, int n_pair,
                                bool weighted, const float* ftab, int nq, double dq, int shift,
-                               int scale_bits, const double* scale, double* out_f64, float* out_f32, int* done) {
-  const int nf = 12 * nq;
-  const int n_pair = weighted ? n_elem * (n_elem + 1) / 2 : 1;
-  hipLaunchKernelGGL(transform_fq_kernel, dim3((nq + 63) / 64, n_chain), dim3(1024), 0, st, grids,
-                     n_pair, n_elem, nf, fq_grid_points(nq), fq_grid_stride(nq), shift, scale_bits,
-                     ftab, nq, dq * nf / (2.0 * M_PI), weighted ? 1 : 0, scale, out_f64, out_f32, done);
+                               int scale_bits, const double* scale, double* part, double* out_f64,
+                               float* out_f32) {
+  const int nf = 12 * nq, stride = fq_grid_stride(nq);
+  const int n_split = fq_transform_parts(nq, n_chain, n_pair);
+  if (n_chain > 65535 || n_pair * n_split > 65535) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(transform_fq_kernel, dim3((nq + 63) / 64, n_chain, n_pair * n_split),
+                     dim3(1024), 0, st, grids, n_pair, n_split, nf, fq_grid_points(nq), stride,
+                     shift, scale_bits, ftab, nq, dq * nf / (2.0 * M_PI), weighted ? 1 : 0, part);
+  const int64_t total = static_cast<int64_t>(n_chain) * nq;
+  const int64_t words2 = static_cast<int64_t>(n_chain) * n_pair * stride / 2;  // stride is even
+  const int64_t n_out = (total + 255) / 256;
+  const int64_t n_clear = std::min<int64_t>((words2 + 511) / 512, 1024);
+  hipLaunchKernelGGL(finish_fq_kernel, dim3(static_cast<unsigned>(n_out + n_clear)), dim3(256), 0,
+                     st, part, n_pair * n_split, nq, total, static_cast<int>(n_out), scale, out_f64,
+                     out_f32, reinterpret_cast<ulonglong2*>(grids), words2);
   return hipGetLastError();
 }
 
