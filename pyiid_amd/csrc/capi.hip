@@ -140,6 +140,7 @@ struct ForceSet {
   Buf units, planes, perm, sorted;  // sorted: positions in perm order (weighted tables)
   Buf t4, t2, part;
   int n_units = 0, n_planes = 0;
+  bool direct = false;  // every atom is in one plane: the kernel writes the forces
   uint64_t stamp = ~0ull;
   int key = -1;
 };
@@ -259,6 +260,8 @@ struct pyiid_ctx {
   std::map<std::vector<int64_t>, std::vector<int64_t>> tuned;
 
   // workspaces
+  Buf upart;  // slices of the adjoint
+  Buf ucoef;  // double2 [chain][element pair][nq]: the force table's coefficients
   Buf gpart, fpart, fq64, fq32, g64, io_a, io_b, io_c, w, out5, u, uq, gobs, pfpart;
   Buf formcnt;  // uint64 [2]: F-only steps in the three-term / Reinsch form (while timing)
 
@@ -1547,8 +1550,9 @@ bool use_force_table(pyiid_ctx* c, const Table& t, double dq) {
 
 // Units: per chain the i tiles of each element against each element's j run.
 // A wave should have about `steps` j steps: total work over the 8,192 waves
-// that the chip holds, at least 16 and at most 1,024 (a block loads its table,
-// so it should not be shorter than needed).  The slices of a tile's range are
+// that the chip holds, at most 1,024 (a block loads its table, so it should not
+// be shorter than needed) and at least 32 (then a chain of up to 512 atoms of
+// one element is in one plane, and the kernel writes its forces itself).  The slices of a tile's range are
 // the waves of a block as far as they go, and planes beyond that.
 int ensure_force(pyiid_ctx* c, const Table& t) {
   ForceSet& s = c->force;
@@ -1563,7 +1567,7 @@ int ensure_force(pyiid_ctx* c, const Table& t) {
   for (int b = 0; b < c->n_chain; ++b)
     for (const ElemRun& r : runs[b])
       total += (r.end - r.begin + 63) / 64 * (c->off[b + 1] - c->off[b]);
-  const int64_t steps = std::min<int64_t>(1024, std::max<int64_t>(16, total / 8192));
+  const int64_t steps = std::min<int64_t>(1024, std::max<int64_t>(32, total / 8192));
   const int n_pair = static_cast<int>(element_pairs(t));
   std::vector<ForceUnit> units;
   std::vector<int32_t> planes(static_cast<size_t>(std::max<int64_t>(1, c->n)), 0);
@@ -1605,8 +1609,20 @@ int ensure_force(pyiid_ctx* c, const Table& t) {
   }
   s.n_units = static_cast<int>(units.size());
   s.n_planes = n_planes;
+  s.direct = std::all_of(planes.begin(), planes.begin() + c->n, [](int32_t k) { return k == 1; });
   s.stamp = c->struct_stamp;
   s.key = key;
+  return PYIID_OK;
+}
+
+// The force table's coefficients; null where the forces run without a table.
+int reserve_coef(pyiid_ctx* c, int slot, double qbin, double2** coef) {
+  Table& t = c->tab[slot];
+  CHK(ensure_extent(c));
+  *coef = nullptr;
+  if (!use_force_table(c, t, static_cast<double>(static_cast<float>(qbin)))) return PYIID_OK;
+  CHK(c->ucoef.reserve(sizeof(double2) * static_cast<size_t>(element_pairs(t)) * t.nq * c->n_chain));
+  *coef = c->ucoef.as<double2>();
   return PYIID_OK;
 }
 
@@ -1655,15 +1671,19 @@ int contract_forces(pyiid_ctx* c, int slot, double qbin, double scale, double* o
       sp = s.sorted.as<AtomRec>();
     }
     Timed tm(c, 4);
-    HIPCHK(launch_force_table(c->stream, c->u.as<float>(), t.tab.as<float>(), nq, dq, weighted,
-                              t.n_elem, B, n_cell, s.t4.as<float4>(), s.t2.as<float2>()));
+    HIPCHK(launch_force_table(c->stream, c->ucoef.as<double2>(), nq, dq,
+                              static_cast<int>(element_pairs(t)) * B, n_cell, s.t4.as<float4>(),
+                              s.t2.as<float2>()));
+    const int32_t* perm = weighted ? s.perm.as<int32_t>() : nullptr;
     HIPCHK(launch_table_force(c->stream, sp, s.units.as<ForceUnit>(), s.n_units, n_cell,
                               s.t4.as<float4>(), s.t2.as<float2>(), c->u.as<float>(),
-                              t.tab.as<float>(), nq, dq, c->n, s.part.as<double>(),
+                              t.tab.as<float>(), nq, dq, c->n, s.part.as<double>(), perm, scale,
+                              s.direct ? out : nullptr,
                               c->out5.as<double>() + 5 * static_cast<size_t>(B)));
     CHK(tm.done());
-    HIPCHK(launch_reduce_force(c->stream, s.part.as<double>(), c->n, s.planes.as<int32_t>(),
-                               weighted ? s.perm.as<int32_t>() : nullptr, scale, out));
+    if (!s.direct)
+      HIPCHK(launch_reduce_force(c->stream, s.part.as<double>(), c->n, s.planes.as<int32_t>(), perm,
+                                 scale, out));
     return PYIID_OK;
   }
   CHK(c->uq.reserve(sizeof(float) * static_cast<size_t>(std::max(1, nq)) * B));
@@ -1702,8 +1722,14 @@ int energy_forces_device(pyiid_ctx* c, int slot, double qbin, int potential,
                           c->out5.as<double>(), c->w.as<double>()));
   if (!forces_dev) return PYIID_OK;
   CHK(c->u.reserve(sizeof(float) * (size_t)nq * B));
+  double2* coef = nullptr;
+  CHK(reserve_coef(c, slot, qbin, &coef));
+  CHK(c->upart.reserve(sizeof(double) * kAdjointSlices * (size_t)nq * B));
   HIPCHK(launch_adjoint(c->stream, c->tmat.as<float>(), nr, nq, c->w.as<double>(),
-                        c->tab[slot].gs.as<double>(), B, c->u.as<float>()));
+                        c->tab[slot].gs.as<double>(), B,
+                        static_cast<double>(static_cast<float>(qbin)), c->tab[slot].tab.as<float>(),
+                        weighted_table(c->tab[slot]), static_cast<int>(element_pairs(c->tab[slot])),
+                        c->upart.as<double>(), c->u.as<float>(), coef));
   return contract_forces(c, slot, qbin, force_scale, forces_dev);
 }
 
@@ -1778,13 +1804,16 @@ int hmc_proposal(pyiid_ctx* c, int n_leapfrog, double eps, double beta, uint64_t
                           h.mom.as<double>(), h.fcur.as<double>(), h.mass.as<double>(),
                           h.chains.as<HmcChain>(), B, beta, eps, seed, h.counter.as<int64_t>(),
                           h.kin0.as<double>()));
+  HIPCHK(launch_hmc_drift(c->stream, c->pos.as<AtomRec>(), h.mom.as<double>(), h.mass.as<double>(),
+                          c->n, eps));
   for (int l = 1; l <= n_leapfrog; ++l) {
-    HIPCHK(launch_hmc_drift(c->stream, c->pos.as<AtomRec>(), h.mom.as<double>(),
-                            h.mass.as<double>(), c->n, eps));
     CHK(energy_forces_device(c, h.slot, h.qbin, h.potential, h.gobs.as<double>(), fscale,
                              h.fnew.as<double>()));
-    HIPCHK(launch_hmc_kick(c->stream, h.mom.as<double>(), h.fnew.as<double>(), c->n,
-                           l < n_leapfrog ? eps : 0.5 * eps));
+    if (l < n_leapfrog)
+      HIPCHK(launch_hmc_kick_drift(c->stream, c->pos.as<AtomRec>(), h.mom.as<double>(),
+                                   h.fnew.as<double>(), h.mass.as<double>(), c->n, eps, eps));
+    else
+      HIPCHK(launch_hmc_kick(c->stream, h.mom.as<double>(), h.fnew.as<double>(), c->n, 0.5 * eps));
   }
   HIPCHK(launch_hmc_end(c->stream, c->pos.as<AtomRec>(), h.pos_save.as<double>(),
                         h.mom.as<double>(), h.mass.as<double>(), h.fcur.as<double>(),
@@ -2236,7 +2265,7 @@ int pyiid_destroy(pyiid_ctx* c) {
   destroy_graph(c->hmc);
   for (Buf* b : {&c->posf, &c->elem, &c->pos, &c->counts_d, &c->natoms_d, &c->tmat, &c->gpart,
                  &c->fpart, &c->fq64, &c->fq32, &c->g64, &c->io_a, &c->io_b,
-                 &c->io_c, &c->w, &c->out5, &c->u, &c->gobs, &c->fq_items.items,
+                 &c->io_c, &c->w, &c->out5, &c->u, &c->ucoef, &c->upart, &c->gobs, &c->fq_items.items,
                  &c->fq_items.ranges, &c->fq_items.perm, &c->spread.units, &c->spread.items,
                  &c->spread.perm, &c->spread.sorted, &c->spread.grids, &c->spread.part,
                  &c->force.units, &c->force.planes, &c->force.perm, &c->force.sorted,
@@ -2800,8 +2829,12 @@ int pyiid_fq_energy_forces(pyiid_ctx* c, int slot, double qbin, int32_t q_first,
     return finish(c, flags);
   }
   CHK(c->u.reserve(sizeof(float) * nq));
+  double2* coef = nullptr;
+  CHK(reserve_coef(c, slot, qbin, &coef));
   HIPCHK(launch_adjoint_fq(c->stream, nq, q_first, c->w.as<double>(), c->tab[slot].gs.as<double>(),
-                           c->u.as<float>()));
+                           static_cast<double>(static_cast<float>(qbin)),
+                           c->tab[slot].tab.as<float>(), weighted_table(c->tab[slot]),
+                           static_cast<int>(element_pairs(c->tab[slot])), c->u.as<float>(), coef));
   CHK(c->io_c.reserve(sizeof(double) * 3 * c->n));
   double* fdst = (flags & PYIID_DEVICE) ? forces : c->io_c.as<double>();
   CHK(contract_forces(c, slot, qbin, conv, fdst));

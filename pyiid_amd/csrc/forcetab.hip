@@ -48,43 +48,46 @@ NodeFit node_fit() {
   return f;
 }
 
-constexpr int kTabChunk = 1024;  // Q bins staged in LDS at a time
+constexpr int kTabSplit = 2;     // halves of a chunk of bins, side by side in a block
+constexpr int kTabChunk = 1024;  // bins staged in LDS at a time
 
-// Block: 64 cells (lanes) x 6 nodes (waves) of one table (chain, element
-// pair).  sin and cos of Q r follow the FP64 three-term recurrence along Q.
-__global__ __launch_bounds__(64 * kNodes) void force_table_kernel(
-    const float* __restrict__ u, const float* __restrict__ ftab, int nq, double dq, int weighted,
-    int n_elem, int n_pair, int n_cell, double h, NodeFit fit, float4* __restrict__ t4,
-    float2* __restrict__ t2) {
-  __shared__ double ca[kTabChunk], cb[kTabChunk];
-  __shared__ double val[kNodes][64];
-  const int lane = threadIdx.x & 63, node = threadIdx.x >> 6;
-  const int cell = blockIdx.x * 64 + lane;
-  const int table = blockIdx.y;
-  const int chain = table / n_pair;
-  int ei = 0, ej = table % n_pair;
-  while (ej > ei) ej -= ++ei;
-  const float* uc = u + static_cast<size_t>(chain) * nq;
-  const double r = (cell + 0.5 + fit.y[node]) * h;
+// Block: 64 / PARTS cells x 6 nodes x 2 halves of every chunk of bins of one
+// table (chain, element pair); a wave holds PARTS parts of its half side by
+// side.  sin and cos of Q r follow the FP64 three-term recurrence along Q from
+// the part's first bin.  Tables of 64 chains are bound by their FP64 operations
+// (PARTS = 1: the two starting phases of a chain of 165 bins are a few percent);
+// a single table of 400 cells by the chain's length (PARTS = 4).
+template <int PARTS>
+__global__ __launch_bounds__(64 * kNodes * kTabSplit) void force_table_kernel(
+    const double2* __restrict__ coef, int nq, double dq, int n_cell, double h, NodeFit fit,
+    float4* __restrict__ t4, float2* __restrict__ t2) {
+  constexpr int kCells = 64 / PARTS;
+  __shared__ double2 cf[kTabChunk];
+  __shared__ double val[kTabSplit][2][kNodes][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int node = wave % kNodes, half = wave / kNodes;
+  const int cell = blockIdx.x * kCells + lane % kCells;
+  const int sub = half * PARTS + lane / kCells;
+  const size_t table = blockIdx.y;
+  const double x = dq * ((cell + 0.5 + fit.y[node]) * h) / M_PI;  // phase per bin / pi
   double s1, c1;
-  sincos(dq * r, &s1, &c1);
+  sincospi(x, &s1, &c1);
   const double k2 = 2.0 * c1;
-  double s = 0.0, sp = -s1, c = 1.0, cp = c1, a = 0.0, b = 0.0;
+  double a = 0.0, b = 0.0;
   for (int m0 = 0; m0 < nq; m0 += kTabChunk) {
     const int cnt = min(kTabChunk, nq - m0);
+    if (m0 > 0) __syncthreads();
+    for (int m = threadIdx.x; m < cnt; m += blockDim.x) cf[m] = coef[table * nq + m0 + m];
+    const int lo = cnt * sub / (kTabSplit * PARTS), hi = cnt * (sub + 1) / (kTabSplit * PARTS);
+    double s, c;
+    sincospi(x * (m0 + lo), &s, &c);
+    double sp = s * c1 - c * s1, cp = c * c1 + s * s1;  // one bin before
     __syncthreads();
-    for (int m = threadIdx.x; m < cnt; m += blockDim.x) {
-      double w = uc[m0 + m];
-      if (weighted)
-        w *= static_cast<double>(ftab[static_cast<size_t>(ei) * nq + m0 + m]) *
-             static_cast<double>(ftab[static_cast<size_t>(ej) * nq + m0 + m]);
-      cb[m] = w;
-      ca[m] = w * (dq * (m0 + m));
-    }
-    __syncthreads();
-    for (int m = 0; m < cnt; ++m) {
-      a = fma(ca[m], c, a);
-      b = fma(cb[m], s, b);
+#pragma unroll 8
+    for (int m = lo; m < hi; ++m) {
+      const double2 w = cf[m];
+      a = fma(w.x, c, a);
+      b = fma(w.y, s, b);
       const double sn = fma(k2, s, -sp), cn = fma(k2, c, -cp);
       sp = s;
       cp = c;
@@ -92,13 +95,23 @@ __global__ __launch_bounds__(64 * kNodes) void force_table_kernel(
       c = cn;
     }
   }
-  val[node][lane] = (a - b / r) / (r * r);
+  val[half][0][node][lane] = a;
+  val[half][1][node][lane] = b;
   __syncthreads();
-  if (cell >= n_cell) return;
+  if (cell >= n_cell || half != 0 || lane >= kCells) return;
   double p = 0.0;
 #pragma unroll
-  for (int n = 0; n < kNodes; ++n) p = fma(fit.c[node][n], val[n][lane], p);
-  const size_t at = static_cast<size_t>(table) * n_cell + cell;
+  for (int n = 0; n < kNodes; ++n) {
+    const double inv = 1.0 / ((cell + 0.5 + fit.y[n]) * h);
+    double an = 0.0, bn = 0.0;
+#pragma unroll
+    for (int k = 0; k < PARTS; ++k) {
+      an += val[0][0][n][k * kCells + lane] + val[1][0][n][k * kCells + lane];
+      bn += val[0][1][n][k * kCells + lane] + val[1][1][n][k * kCells + lane];
+    }
+    p = fma(fit.c[node][n], (an - bn * inv) * (inv * inv), p);
+  }
+  const size_t at = table * n_cell + cell;
   // wave k holds coefficient k: 0..3 in t4, 4 and 5 in t2
   if (node < 4)
     reinterpret_cast<float*>(t4 + at)[node] = static_cast<float>(p);
@@ -128,6 +141,8 @@ __device__ double pair_force_far(double r, const float* u, const float* fi,
   return (a - b / r) / (r * r);
 }
 
+constexpr int kAhead = 2;
+
 // Block (16 waves): the unit's 64-position i tiles against its j range, its
 // table in LDS.  Wave w takes tile w mod tiles and slice w / tiles of the
 // range; a j atom's position is wave-uniform (scalar loads).  Each lane owns
@@ -143,6 +158,7 @@ __global__ __launch_bounds__(1024, 8) void table_force_kernel(
     const AtomRec* __restrict__ pos, const ForceUnit* __restrict__ units, int n_cell, double inv_h,
     const float4* __restrict__ t4, const float2* __restrict__ t2, const float* __restrict__ u,
     const float* __restrict__ ftab, int nq, double dq, int64_t n, double* __restrict__ part,
+    const int32_t* __restrict__ perm, double conv, double* __restrict__ out,
     double* __restrict__ far_seen) {
   extern __shared__ __align__(16) unsigned char lds[];
   float4* l4 = reinterpret_cast<float4*>(lds);
@@ -164,8 +180,9 @@ __global__ __launch_bounds__(1024, 8) void table_force_kernel(
   const int i = un.i0 + tile * 64 + lane;
   const bool have = i < un.i1;
   const int len = un.j1 - un.j0;
-  const int jb = un.j0 + static_cast<int>(static_cast<int64_t>(len) * slice / n_slice);
-  const int je = un.j0 + static_cast<int>(static_cast<int64_t>(len) * (slice + 1) / n_slice);
+  // (wave-uniform, so that the j atoms come by scalar loads)
+  const int jb = __builtin_amdgcn_readfirstlane(un.j0 + static_cast<int>(static_cast<int64_t>(len) * slice / n_slice));
+  const int je = __builtin_amdgcn_readfirstlane(un.j0 + static_cast<int>(static_cast<int64_t>(len) * (slice + 1) / n_slice));
   const AtomRec pi = pos[have ? i : un.i0];
   const double limit = static_cast<double>(n_cell);
   double gx = 0.0, gy = 0.0, gz = 0.0;
@@ -173,23 +190,45 @@ __global__ __launch_bounds__(1024, 8) void table_force_kernel(
   for (int j0 = jb; j0 < je; j0 += 64) {
     const int j1 = min(je, j0 + 64);
     float fx = 0.f, fy = 0.f, fz = 0.f;
-    for (int j = j0; j < j1; ++j) {
-      const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
-      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-      if (!(r2 > 0.0)) continue;  // the atom itself, a duplicate, a NaN
-      const double t = scaled_root(r2, inv_h);
-      if (!(t < limit)) {  // past the table, or r2 outside float's range
-        far = true;
-        continue;
+    for (int j = j0; j < j1; j += kAhead) {
+      // kAhead pairs side by side, so that their loads and chains overlap
+      double dx[kAhead], dy[kAhead], dz[kAhead], t[kAhead];
+      bool keep[kAhead], in[kAhead];
+      float y[kAhead], p[kAhead];
+      float4 a[kAhead];
+      float2 b[kAhead];
+#pragma unroll
+      for (int e = 0; e < kAhead; ++e) {
+        const AtomRec* pj = pos + min(j + e, j1 - 1);
+        dx[e] = pi.x - pj->x;
+        dy[e] = pi.y - pj->y;
+        dz[e] = pi.z - pj->z;
       }
-      const double fl = floor(t);
-      const float y = static_cast<float>(t - fl) - 0.5f;
-      const float4 a = l4[static_cast<int>(fl)];
-      const float2 b = l2[static_cast<int>(fl)];
-      const float p = fmaf(fmaf(fmaf(fmaf(fmaf(b.y, y, b.x), y, a.w), y, a.z), y, a.y), y, a.x);
-      fx = fmaf(p, static_cast<float>(dx), fx);
-      fy = fmaf(p, static_cast<float>(dy), fy);
-      fz = fmaf(p, static_cast<float>(dz), fz);
+#pragma unroll
+      for (int e = 0; e < kAhead; ++e) {
+        const double r2 = fma(dx[e], dx[e], fma(dy[e], dy[e], dz[e] * dz[e]));
+        keep[e] = r2 > 0.0 && j + e < j1;  // not the atom itself, a duplicate, a NaN
+        t[e] = scaled_root(r2, inv_h);
+      }
+#pragma unroll
+      for (int e = 0; e < kAhead; ++e) {
+        in[e] = t[e] < limit;  // else past the table, or r2 outside float's range
+        const double fl = floor(t[e]);
+        y[e] = static_cast<float>(t[e] - fl) - 0.5f;
+        const int cell = in[e] ? static_cast<int>(fl) : 0;
+        a[e] = l4[cell];
+        b[e] = l2[cell];
+      }
+#pragma unroll
+      for (int e = 0; e < kAhead; ++e) {
+        far = far || (keep[e] && !in[e]);
+        p[e] = fmaf(fmaf(fmaf(fmaf(fmaf(b[e].y, y[e], b[e].x), y[e], a[e].w), y[e], a[e].z), y[e],
+                         a[e].y), y[e], a[e].x);
+        p[e] = keep[e] && in[e] ? p[e] : 0.f;
+        fx = fmaf(p[e], static_cast<float>(dx[e]), fx);
+        fy = fmaf(p[e], static_cast<float>(dy[e]), fy);
+        fz = fmaf(p[e], static_cast<float>(dz[e]), fz);
+      }
     }
     gx += static_cast<double>(fx);
     gy += static_cast<double>(fy);
@@ -226,10 +265,12 @@ __global__ __launch_bounds__(1024, 8) void table_force_kernel(
     }
   }
   if (have) {
-    double* o = part + (static_cast<size_t>(un.plane) * n + i) * 3;
-    o[0] = gx;
-    o[1] = gy;
-    o[2] = gz;
+    double* o = out ? out + static_cast<size_t>(perm ? perm[i] : i) * 3
+                    : part + (static_cast<size_t>(un.plane) * n + i) * 3;
+    const double f = out ? conv : 1.0;
+    o[0] = f * gx;
+    o[1] = f * gy;
+    o[2] = f * gz;
   }
 }
 
@@ -257,21 +298,29 @@ size_t force_lds_bytes(int64_t n_cell) {
   return table > red ? table : red;
 }
 
-hipError_t launch_force_table(hipStream_t st, const float* u, const float* ftab, int nq, double dq,
-                              bool weighted, int n_elem, int n_chain, int n_cell, float4* t4,
-                              float2* t2) {
+hipError_t launch_force_table(hipStream_t st, const double2* coef, int nq, double dq, int n_table,
+                              int n_cell, float4* t4, float2* t2) {
   static const NodeFit fit = node_fit();
-  const int n_pair = weighted ? n_elem * (n_elem + 1) / 2 : 1;
-  hipLaunchKernelGGL(force_table_kernel, dim3((n_cell + 63) / 64, n_chain * n_pair),
-                     dim3(64 * kNodes), 0, st, u, ftab, nq, dq, weighted ? 1 : 0, n_elem, n_pair,
-                     n_cell, force_cell(nq, dq), fit, t4, t2);
+  // four parts while their blocks fit the chip at once (two per CU): 10 us
+  // instead of 16 for one table of 1,600 cells; beyond, the starting phases of
+  // the parts cost more than the shorter chains save (16 tables of 1,080 cells:
+  // 20 us against 15)
+  if (static_cast<int64_t>((n_cell + 15) / 16) * n_table <= 512)
+    hipLaunchKernelGGL(force_table_kernel<4>, dim3((n_cell + 15) / 16, n_table),
+                       dim3(64 * kNodes * kTabSplit), 0, st, coef, nq, dq, n_cell,
+                       force_cell(nq, dq), fit, t4, t2);
+  else
+    hipLaunchKernelGGL(force_table_kernel<1>, dim3((n_cell + 63) / 64, n_table),
+                       dim3(64 * kNodes * kTabSplit), 0, st, coef, nq, dq, n_cell,
+                       force_cell(nq, dq), fit, t4, t2);
   return hipGetLastError();
 }
 
 hipError_t launch_table_force(hipStream_t st, const AtomRec* pos, const ForceUnit* units,
                               int n_units, int n_cell, const float4* t4, const float2* t2,
                               const float* u, const float* ftab, int nq, double dq, int64_t n,
-                              double* part, double* far_seen) {
+                              double* part, const int32_t* perm, double conv, double* out,
+                              double* far_seen) {
   if (n_units == 0) return hipSuccess;
   const size_t lds = force_lds_bytes(n_cell);
   if (lds > kForceLds) return hipErrorInvalidValue;
@@ -280,7 +329,8 @@ hipError_t launch_table_force(hipStream_t st, const AtomRec* pos, const ForceUni
                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kForceLds));
   if (attr != hipSuccess) return attr;
   hipLaunchKernelGGL(table_force_kernel, dim3(n_units), dim3(1024), lds, st, pos, units, n_cell,
-                     1.0 / force_cell(nq, dq), t4, t2, u, ftab, nq, dq, n, part, far_seen);
+                     1.0 / force_cell(nq, dq), t4, t2, u, ftab, nq, dq, n, part, perm, conv, out,
+                     far_seen);
   return hipGetLastError();
 }
 

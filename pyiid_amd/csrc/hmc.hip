@@ -84,6 +84,23 @@ __global__ void hmc_drift_kernel(AtomRec* __restrict__ pos, const double* __rest
   pos[i].z += s * mom[3 * i + 2];
 }
 
+__global__ void hmc_kick_drift_kernel(AtomRec* __restrict__ pos, double* __restrict__ mom,
+                                      const double* __restrict__ force,
+                                      const double* __restrict__ mass, int64_t n, double h,
+                                      double eps) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double s = eps / mass[i];
+  double p[3];
+  for (int c = 0; c < 3; ++c) {
+    p[c] = mom[3 * i + c] + h * force[3 * i + c];
+    mom[3 * i + c] = p[c];
+  }
+  pos[i].x += s * p[0];
+  pos[i].y += s * p[1];
+  pos[i].z += s * p[2];
+}
+
 __global__ void hmc_kick_kernel(double* __restrict__ mom, const double* __restrict__ force,
                                 int64_t n3, double h) {
   const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -166,6 +183,13 @@ hipError_t launch_hmc_drift(hipStream_t st, AtomRec* pos, const double* mom, con
                             int64_t n, double eps) {
   hipLaunchKernelGGL(hmc_drift_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
                      st, pos, mom, mass, n, eps);
+  return hipGetLastError();
+}
+
+hipError_t launch_hmc_kick_drift(hipStream_t st, AtomRec* pos, double* mom, const double* force,
+                                 const double* mass, int64_t n, double h, double eps) {
+  hipLaunchKernelGGL(hmc_kick_drift_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256),
+                     0, st, pos, mom, force, mass, n, h, eps);
   return hipGetLastError();
 }
 

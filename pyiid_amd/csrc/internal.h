@@ -177,15 +177,17 @@ struct ForceUnit {
 constexpr size_t kForceLds = 160 * 1024;
 double force_cell(int nq, double dq);       // cell width of the table
 size_t force_lds_bytes(int64_t n_cell);     // LDS of a block
-// t4 / t2 [chain * n_pair + pair][n_cell]: coefficients 0..3 / 4, 5
-hipError_t launch_force_table(hipStream_t st, const float* u, const float* ftab, int nq, double dq,
-                              bool weighted, int n_elem, int n_chain, int n_cell, float4* t4,
-                              float2* t2);
-// part[plane][position][3]; *far_seen becomes 1 when a pair lies past the table
+// t4 / t2 [table][n_cell]: coefficients 0..3 / 4, 5; coef[table][q] (table =
+// chain * n_pair + pair) as launch_adjoint writes it
+hipError_t launch_force_table(hipStream_t st, const double2* coef, int nq, double dq, int n_table,
+                              int n_cell, float4* t4, float2* t2);
+// part[plane][position][3], or with out the forces themselves (a single plane):
+// out[perm[p]][c] = conv * sum; *far_seen becomes 1 when a pair lies past the table
 hipError_t launch_table_force(hipStream_t st, const AtomRec* pos, const ForceUnit* units,
                               int n_units, int n_cell, const float4* t4, const float2* t2,
                               const float* u, const float* ftab, int nq, double dq, int64_t n,
-                              double* part, double* far_seen);
+                              double* part, const int32_t* perm, double conv, double* out,
+                              double* far_seen);
 // out[perm[p]][c] = conv * sum_{k < planes[p]} part[k][p][c] (perm null: identity)
 hipError_t launch_reduce_force(hipStream_t st, const double* part, int64_t n,
                                const int32_t* planes, const int32_t* perm, double conv,
@@ -202,12 +204,17 @@ hipError_t launch_potential(hipStream_t st, int potential, const double* gobs,
 // y[row] = sum_t X[row][t] * w[t]  (FP64), one wave per row
 hipError_t launch_gemv_rows(hipStream_t st, const double* x, int64_t rows, int n,
                             const double* w, double* y);
-// u[b][q] = gscale[b][q] * sum_t T[t][q] w[b][t]   (FP64 accumulation)
+// u[b][q] = gscale[b][q] * sum_t T[t][q] w[b][t]   (FP64 accumulation) and,
+// unless null, coef[b][pair][q] = (u f_I f_J q dq, u f_I f_J) for the force table;
+// part: kAdjointSlices * n_chain * nq doubles
+constexpr int kAdjointSlices = 4;
 hipError_t launch_adjoint(hipStream_t st, const float* t, int n_r, int nq, const double* w,
-                          const double* gscale, int n_chain, float* u);
-// u[q] = gscale[q] * w[q - q_first] (0 below q_first)
+                          const double* gscale, int n_chain, double dq, const float* ftab,
+                          bool weighted, int n_pair, double* part, float* u, double2* coef);
+// the same from u[q] = gscale[q] * w[q - q_first] (0 below q_first), one chain
 hipError_t launch_adjoint_fq(hipStream_t st, int nq, int q_first, const double* w,
-                             const double* gscale, float* u);
+                             const double* gscale, double dq, const float* ftab, bool weighted,
+                             int n_pair, float* u, double2* coef);
 hipError_t launch_f64_to_f32(hipStream_t st, const double* x, int64_t n, float* y);
 hipError_t launch_f32_to_f64(hipStream_t st, const float* x, int64_t n, double* y);
 
@@ -225,6 +232,9 @@ hipError_t launch_hmc_begin(hipStream_t st, AtomRec* pos, double* pos_save, doub
 // x += eps p / m
 hipError_t launch_hmc_drift(hipStream_t st, AtomRec* pos, const double* mom, const double* mass,
                             int64_t n, double eps);
+// p += h F, then x += eps p / m: the end of one step and the start of the next
+hipError_t launch_hmc_kick_drift(hipStream_t st, AtomRec* pos, double* mom, const double* force,
+                                 const double* mass, int64_t n, double h, double eps);
 // p += h F
 hipError_t launch_hmc_kick(hipStream_t st, double* mom, const double* force, int64_t n, double h);
 // End of a proposal: K1, Metropolis with exp(beta (H0 - H1)), restore or

@@ -13,75 +13,62 @@ namespace {
 
 using v4f = float __attribute__((ext_vector_type(4)));
 
-// C[m][n] = sum_k A[m][k] * B[n][k]; block tile 64 x 64, 4 waves of 32 x 32,
-// each wave 2 x 2 MFMA 16x16x4 tiles; K staged through LDS 16 at a time.
-// MFMA f32 16x16x4 operand layout (lane l): A[l%16][l/16], B[l/16][l%16];
-// result register v holds C[4*(l/16)+v][l%16].
+// C[m][n] = sum_k A[m][k] * B[n][k] for few rows (F -> G of a batch of chains).
+// Block: one 16 x 16 tile, its 4 waves a quarter of k each, added through LDS.
+// The product is far too small for the chip (64 chains: 0.17 GFLOP), so what
+// counts is the length of a block's chain: with 64 x 64 tiles staged through
+// LDS it took 23 to 50 us, in 63 blocks of 21 barriers each; here a wave loads
+// its operands straight from L2, 16 of k at a time, and runs 6 steps at 330
+// bins.  Lane l holds k0 + 4 (l / 16) .. + 3 of row l % 16 of both operands and
+// MFMA step s takes element s: any order of k gives the same sum.
 template <bool A64>
-__global__ __launch_bounds__(256) void gemm_nt_kernel(const void* __restrict__ a_raw, int64_t m,
-                                                      int k, const float* __restrict__ b, int n,
-                                                      double* __restrict__ c64,
-                                                      float* __restrict__ c32) {
-  constexpr int KS = 16;
-  __shared__ float as[64][KS + 1];
-  __shared__ float bs[64][KS + 1];
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int64_t bm = static_cast<int64_t>(blockIdx.y) * 64;
-  const int bn = blockIdx.x * 64;
-  v4f acc[2][2];
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y) acc[x][y] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  for (int k0 = 0; k0 < k; k0 += KS) {
-    __syncthreads();
+__global__ __launch_bounds__(256) void gemm_rows_kernel(const void* __restrict__ a_raw, int64_t m,
+                                                        int k, const float* __restrict__ b, int n,
+                                                        double* __restrict__ c64,
+                                                        float* __restrict__ c32) {
+  __shared__ float red[3][4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t bm = static_cast<int64_t>(blockIdx.y) * 16;
+  const int bn = blockIdx.x * 16;
+  const int64_t ar = min(bm + (lane & 15), m - 1);
+  const int br = min(bn + (lane & 15), n - 1);
+  const int steps = (k + 15) / 16;
+  const int s0 = steps * wave / 4, s1 = steps * (wave + 1) / 4;
+  v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+  for (int s = s0; s < s1; ++s) {
+    const int kk = s * 16 + 4 * (lane >> 4);
+    float av[4], bv[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int idx = threadIdx.x + e * 256;
-      const int row = idx / KS, kk = idx % KS;
-      const int64_t ar = bm + row;
-      float av = 0.0f;
-      if (ar < m && k0 + kk < k) {
-        if constexpr (A64)
-          av = static_cast<float>(static_cast<const double*>(a_raw)[ar * k + k0 + kk]);
-        else
-          av = static_cast<const float*>(a_raw)[ar * k + k0 + kk];
-      }
-      as[row][kk] = av;
-      const int br = bn + row;
-      bs[row][kk] = (br < n && k0 + kk < k) ? b[(int64_t)br * k + k0 + kk] : 0.0f;
+      const bool in = kk + e < k;
+      const int at = in ? kk + e : 0;
+      if constexpr (A64)
+        av[e] = static_cast<float>(static_cast<const double*>(a_raw)[ar * k + at]);
+      else
+        av[e] = static_cast<const float*>(a_raw)[ar * k + at];
+      bv[e] = b[static_cast<int64_t>(br) * k + at];
+      av[e] = in ? av[e] : 0.f;
+      bv[e] = in ? bv[e] : 0.f;
     }
-    __syncthreads();
 #pragma unroll
-    for (int kk = 0; kk < KS; kk += 4) {
-      float af[2], bf[2];
+    for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], bv[e], acc, 0, 0, 0);
+  }
+  if (wave != 0)
 #pragma unroll
-      for (int x = 0; x < 2; ++x) af[x] = as[wm * 32 + x * 16 + (lane & 15)][kk + (lane >> 4)];
+    for (int v = 0; v < 4; ++v) red[wave - 1][v][lane] = acc[v];
+  __syncthreads();
+  if (wave != 0) return;
 #pragma unroll
-      for (int y = 0; y < 2; ++y) bf[y] = bs[wn * 32 + y * 16 + (lane & 15)][kk + (lane >> 4)];
-#pragma unroll
-      for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y)
-          acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[x], bf[y], acc[x][y], 0, 0, 0);
+  for (int v = 0; v < 4; ++v) {
+    const float t = ((acc[v] + red[0][v][lane]) + red[1][v][lane]) + red[2][v][lane];
+    const int64_t row = bm + 4 * (lane >> 4) + v;
+    const int col = bn + (lane & 15);
+    if (row < m && col < n) {
+      if (c64) c64[row * n + col] = static_cast<double>(t);
+      if (c32) c32[row * n + col] = t;
     }
   }
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int64_t row = bm + wm * 32 + x * 16 + 4 * (lane >> 4) + v;
-        const int col = bn + wn * 32 + y * 16 + (lane & 15);
-        if (row < m && col < n) {
-          if (c64) c64[row * n + col] = static_cast<double>(acc[x][y][v]);
-          if (c32) c32[row * n + col] = acc[x][y][v];
-        }
-      }
 }
 
 // The same product for tall A (the gradient rows): block tile 128 x 128,
@@ -190,17 +177,29 @@ __global__ __launch_bounds__(256) void gemm_nt128_kernel(const void* __restrict_
       }
 }
 
-__device__ double block_sum(double v, double* sh) {
+// The block's sums of three values, in every thread (one pass through LDS).
+__device__ void block_sum3(double& x, double& y, double& z, double (*sh)[16]) {
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  for (int off = 32; off > 0; off >>= 1) {
+    x += __shfl_xor(x, off, 64);
+    y += __shfl_xor(y, off, 64);
+    z += __shfl_xor(z, off, 64);
+  }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   __syncthreads();
-  if (lane == 0) sh[wave] = v;
+  if (lane == 0) {
+    sh[0][wave] = x;
+    sh[1][wave] = y;
+    sh[2][wave] = z;
+  }
   __syncthreads();
-  double t = 0.0;
+  x = y = z = 0.0;
   const int nw = blockDim.x >> 6;
-  for (int w = 0; w < nw; ++w) t += sh[w];
-  return t;
+  for (int w = 0; w < nw; ++w) {
+    x += sh[0][w];
+    y += sh[1][w];
+    z += sh[2][w];
+  }
 }
 
 // One block per chain.  Rw: master_kernel.py:206-236; chi^2: :239-266; the adjoint
@@ -208,36 +207,50 @@ __device__ double block_sum(double v, double* sh) {
 // (:293-375): grad = gradG . w with
 //   w = c * (s * res + (g.res)/(g.g) * (o - 2 a g)),
 //   c = -value/|res|^2 (Rw) or -2 (chi^2), res = o - s g, a = optimal scale.
+constexpr int kPotKeep = 6;
 __global__ __launch_bounds__(1024) void potential_kernel(int potential,
                                                          const double* __restrict__ o_all,
                                                          const double* __restrict__ g_all, int n,
                                                          double* __restrict__ out5_all,
                                                          double* __restrict__ w_all) {
-  __shared__ double sh[16];
+  __shared__ double sh[3][16];
   // one block per chain
   const double* o = o_all + (size_t)blockIdx.x * n;
   const double* g = g_all + (size_t)blockIdx.x * n;
   double* out5 = out5_all + (size_t)blockIdx.x * 5;
   double* w = w_all ? w_all + (size_t)blockIdx.x * n : nullptr;
-  double go = 0.0, gg = 0.0, oo = 0.0;
-  for (int t = threadIdx.x; t < n; t += blockDim.x) {
-    go += g[t] * o[t];
-    gg += g[t] * g[t];
-    oo += o[t] * o[t];
+  // the thread's points stay in registers between the passes (kPotKeep of them;
+  // longer arrays are read again)
+  double ok[kPotKeep], gk[kPotKeep];
+#pragma unroll
+  for (int e = 0; e < kPotKeep; ++e) {
+    const int t = threadIdx.x + e * 1024;
+    ok[e] = t < n ? o[t] : 0.0;
+    gk[e] = t < n ? g[t] : 0.0;
   }
-  go = block_sum(go, sh);
-  gg = block_sum(gg, sh);
-  oo = block_sum(oo, sh);
+  double go = 0.0, gg = 0.0, oo = 0.0;
+  auto first = [&](double ot, double gt) {
+    go += gt * ot;
+    gg += gt * gt;
+    oo += ot * ot;
+  };
+#pragma unroll
+  for (int e = 0; e < kPotKeep; ++e) first(ok[e], gk[e]);
+  for (int t = threadIdx.x + kPotKeep * 1024; t < n; t += 1024) first(o[t], g[t]);
+  block_sum3(go, gg, oo, sh);
   const double a = go / gg;
   const double s = (a <= 0.0) ? 1.0 : a;
-  double rr = 0.0, gr = 0.0;
-  for (int t = threadIdx.x; t < n; t += blockDim.x) {
-    const double res = o[t] - s * g[t];
+  double rr = 0.0, gr = 0.0, none = 0.0;
+  auto second = [&](double ot, double gt) {
+    const double res = ot - s * gt;
     rr += res * res;
-    gr += g[t] * res;
-  }
-  rr = block_sum(rr, sh);
-  gr = block_sum(gr, sh);
+    gr += gt * res;
+  };
+#pragma unroll
+  for (int e = 0; e < kPotKeep; ++e)
+    if (threadIdx.x + e * 1024 < n) second(ok[e], gk[e]);
+  for (int t = threadIdx.x + kPotKeep * 1024; t < n; t += 1024) second(o[t], g[t]);
+  block_sum3(rr, gr, none, sh);
   double value, coef;
   if (potential == 0) {
     value = (a <= 0.0) ? 1.0 : sqrt(rr / oo);
@@ -248,10 +261,14 @@ __global__ __launch_bounds__(1024) void potential_kernel(int potential,
   }
   if (w) {
     const double gfac = gr / gg;
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
-      const double res = o[t] - s * g[t];
-      w[t] = coef * (s * res + gfac * (o[t] - 2.0 * a * g[t]));
-    }
+    auto third = [&](int t, double ot, double gt) {
+      const double res = ot - s * gt;
+      w[t] = coef * (s * res + gfac * (ot - 2.0 * a * gt));
+    };
+#pragma unroll
+    for (int e = 0; e < kPotKeep; ++e)
+      if (threadIdx.x + e * 1024 < n) third(threadIdx.x + e * 1024, ok[e], gk[e]);
+    for (int t = threadIdx.x + kPotKeep * 1024; t < n; t += 1024) third(t, o[t], g[t]);
   }
   if (threadIdx.x == 0) {
     out5[0] = value;
@@ -274,47 +291,103 @@ __global__ void gemv_rows_kernel(const double* __restrict__ x, int64_t rows, int
   if (lane == 0) y[row] = acc;
 }
 
-// u[b][q] = gscale[b][q] * sum_t T[t][q] w[b][t]  (FP64 accumulation; T float).
-// A block takes 64 bins of one chain (lane = bin, coalesced rows of T) with
-// kAdjWaves waves, each summing a contiguous slice of the rows into four
-// independent accumulators so that its loads overlap; the waves' partials
-// are added in wave order through LDS (deterministic).
-constexpr int kAdjWaves = 16;
-__global__ __launch_bounds__(64 * kAdjWaves) void adjoint_kernel(
-    const float* __restrict__ t, int n_r, int nq, const double* __restrict__ w,
-    const double* __restrict__ gscale, float* __restrict__ u) {
-  __shared__ double part[kAdjWaves][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int q = blockIdx.x * 64 + lane;
-  const int b = blockIdx.y;
-  const double* wb = w + (size_t)b * n_r;
-  const int per = (n_r + kAdjWaves - 1) / kAdjWaves;
-  const int r0 = wave * per, r1 = min(n_r, r0 + per);
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-  if (q < nq) {
-    int r = r0;
-    for (; r + 4 <= r1; r += 4) {
-      a0 += static_cast<double>(t[(size_t)r * nq + q]) * wb[r];
-      a1 += static_cast<double>(t[(size_t)(r + 1) * nq + q]) * wb[r + 1];
-      a2 += static_cast<double>(t[(size_t)(r + 2) * nq + q]) * wb[r + 2];
-      a3 += static_cast<double>(t[(size_t)(r + 3) * nq + q]) * wb[r + 3];
+// What the force table reads for bin q of chain b: u and, per element pair,
+// (u f_I f_J Q, u f_I f_J).
+__device__ __forceinline__ void put_u(double v, int b, int q, int nq, double dq,
+                                      const float* __restrict__ ftab, int weighted, int n_pair,
+                                      float* __restrict__ u, double2* __restrict__ coef) {
+  const float uf = static_cast<float>(v);
+  u[static_cast<size_t>(b) * nq + q] = uf;
+  if (!coef) return;
+  int ei = 0, ej = 0;
+  for (int p = 0; p < n_pair; ++p) {
+    double w = uf;
+    if (weighted)
+      w *= static_cast<double>(ftab[static_cast<size_t>(ei) * nq + q]) *
+           static_cast<double>(ftab[static_cast<size_t>(ej) * nq + q]);
+    coef[(static_cast<size_t>(b) * n_pair + p) * nq + q] = double2{w * (dq * q), w};
+    if (++ej > ei) {
+      ++ei;
+      ej = 0;
     }
-    for (; r < r1; ++r) a0 += static_cast<double>(t[(size_t)r * nq + q]) * wb[r];
   }
-  part[wave][lane] = (a0 + a1) + (a2 + a3);
-  __syncthreads();
-  if (wave != 0 || q >= nq) return;
-  double acc = 0.0;
+}
+
+// part[z][b][q] = sum over slice z of t of w[b][t] T[t][q] in FP64 (T float), on
+// the FP64 matrix cores: a block takes 16 chains x 16 bins, its 16 waves
+// consecutive parts of its slice, 4 of t per MFMA, added in wave order through
+// LDS.  All chains of a tile share the read of T.  It is latency and the reach
+// of a few CUs' loads that count (one block per 64 bins and chain, reading T for
+// each, took 25 us for one chain and 52 us for 64; the tiles in one slice 31 us):
+// four slices give 84 blocks at 330 bins, and a wave has 8 steps' loads in flight.
+// Layout of v_mfma_f64_16x16x4 (lane l): A[l % 16][l / 16], B[l / 16][l % 16];
+// result v: row 4 v + l / 16, column l % 16.
+using v4d = double __attribute__((ext_vector_type(4)));
+constexpr int kAdjWaves = 16, kAdjAhead = 8;
+
+__global__ __launch_bounds__(64 * kAdjWaves) void adjoint_kernel(const float* __restrict__ t,
+                                                                 int n_r, int nq,
+                                                                 const double* __restrict__ w,
+                                                                 int n_chain,
+                                                                 double* __restrict__ part) {
+  __shared__ double red[kAdjWaves][4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int q = min(static_cast<int>(blockIdx.x) * 16 + (lane & 15), nq - 1);
+  const int b = min(static_cast<int>(blockIdx.y) * 16 + (lane & 15), n_chain - 1);
+  const int steps = (n_r + 3) / 4;
+  const int64_t sub = blockIdx.z * kAdjWaves + wave, n_sub = gridDim.z * kAdjWaves;
+  const int s0 = static_cast<int>(steps * sub / n_sub), s1 = static_cast<int>(steps * (sub + 1) / n_sub);
+  const double* wb = w + static_cast<size_t>(b) * n_r;
+  v4d acc = v4d{0.0, 0.0, 0.0, 0.0};
+  for (int s = s0; s < s1; s += kAdjAhead) {
+    double x[kAdjAhead];
+    float y[kAdjAhead];
 #pragma unroll
-  for (int k = 0; k < kAdjWaves; ++k) acc += part[k][lane];
-  u[(size_t)b * nq + q] = static_cast<float>(acc * gscale[(size_t)b * nq + q]);
+    for (int e = 0; e < kAdjAhead; ++e) {
+      const int at = min((s + e) * 4 + (lane >> 4), n_r - 1);
+      x[e] = wb[at];
+      y[e] = t[static_cast<size_t>(at) * nq + q];
+    }
+#pragma unroll
+    for (int e = 0; e < kAdjAhead; ++e) {
+      const bool in = s + e < s1 && (s + e) * 4 + (lane >> 4) < n_r;
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(in ? x[e] : 0.0,
+                                                 in ? static_cast<double>(y[e]) : 0.0, acc, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) red[wave][v][lane] = acc[v];
+  __syncthreads();
+  if (wave >= 4) return;
+  double v = 0.0;  // wave v adds result v
+#pragma unroll
+  for (int k = 0; k < kAdjWaves; ++k) v += red[k][wave][lane];
+  const int row = blockIdx.y * 16 + 4 * wave + (lane >> 4), col = blockIdx.x * 16 + (lane & 15);
+  if (row < n_chain && col < nq)
+    part[(static_cast<size_t>(blockIdx.z) * n_chain + row) * nq + col] = v;
+}
+
+__global__ void adjoint_sum_kernel(const double* __restrict__ part, int n_slice, int n_chain, int nq,
+                                   const double* __restrict__ gscale, double dq,
+                                   const float* __restrict__ ftab, int weighted, int n_pair,
+                                   float* __restrict__ u, double2* __restrict__ coef) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
+  if (q >= nq) return;
+  const size_t e = static_cast<size_t>(b) * nq + q, total = static_cast<size_t>(n_chain) * nq;
+  double v = 0.0;
+#pragma unroll 4
+  for (int s = 0; s < n_slice; ++s) v += part[s * total + e];
+  put_u(v * gscale[e], b, q, nq, dq, ftab, weighted, n_pair, u, coef);
 }
 
 __global__ void adjoint_fq_kernel(int nq, int q_first, const double* __restrict__ w,
-                                  const double* __restrict__ gscale, float* __restrict__ u) {
+                                  const double* __restrict__ gscale, double dq,
+                                  const float* __restrict__ ftab, int weighted, int n_pair,
+                                  float* __restrict__ u, double2* __restrict__ coef) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= nq) return;
-  u[q] = (q >= q_first) ? static_cast<float>(w[q - q_first] * gscale[q]) : 0.0f;
+  put_u(q >= q_first ? w[q - q_first] * gscale[q] : 0.0, 0, q, nq, dq, ftab, weighted, n_pair, u,
+        coef);
 }
 
 __global__ void f64_to_f32_kernel(const double* __restrict__ x, int64_t n, float* __restrict__ y) {
@@ -354,13 +427,12 @@ hipError_t launch_gemm_nt(hipStream_t st, const void* a, bool a_f64, int64_t m, 
                          n_rt, c_f64, c_f32);
     return hipGetLastError();
   }
-  const int64_t gy = (m + 63) / 64;
-  if (gy > 2147483647LL) return hipErrorInvalidValue;
-  dim3 grid((n + 63) / 64, static_cast<unsigned>(gy));
+  if (m < 1) return hipSuccess;
+  dim3 grid((n + 15) / 16, static_cast<unsigned>((m + 15) / 16));
   if (a_f64)
-    hipLaunchKernelGGL(gemm_nt_kernel<true>, grid, dim3(256), 0, st, a, m, k, b, n, c_f64, c_f32);
+    hipLaunchKernelGGL(gemm_rows_kernel<true>, grid, dim3(256), 0, st, a, m, k, b, n, c_f64, c_f32);
   else
-    hipLaunchKernelGGL(gemm_nt_kernel<false>, grid, dim3(256), 0, st, a, m, k, b, n, c_f64, c_f32);
+    hipLaunchKernelGGL(gemm_rows_kernel<false>, grid, dim3(256), 0, st, a, m, k, b, n, c_f64, c_f32);
   return hipGetLastError();
 }
 
@@ -380,16 +452,22 @@ hipError_t launch_gemv_rows(hipStream_t st, const double* x, int64_t rows, int n
 }
 
 hipError_t launch_adjoint(hipStream_t st, const float* t, int n_r, int nq, const double* w,
-                          const double* gscale, int n_chain, float* u) {
-  hipLaunchKernelGGL(adjoint_kernel, dim3((nq + 63) / 64, n_chain), dim3(64 * kAdjWaves), 0, st, t,
-                     n_r, nq, w, gscale, u);
+                          const double* gscale, int n_chain, double dq, const float* ftab,
+                          bool weighted, int n_pair, double* part, float* u, double2* coef) {
+  const dim3 tiles((nq + 15) / 16, (n_chain + 15) / 16, kAdjointSlices);
+  hipLaunchKernelGGL(adjoint_kernel, tiles, dim3(64 * kAdjWaves), 0, st, t, n_r, nq, w, n_chain,
+                     part);
+  hipLaunchKernelGGL(adjoint_sum_kernel, dim3((nq + 63) / 64, n_chain), dim3(64), 0, st, part,
+                     kAdjointSlices, n_chain, nq, gscale, dq, ftab, weighted ? 1 : 0, n_pair, u,
+                     coef);
   return hipGetLastError();
 }
 
 hipError_t launch_adjoint_fq(hipStream_t st, int nq, int q_first, const double* w,
-                             const double* gscale, float* u) {
+                             const double* gscale, double dq, const float* ftab, bool weighted,
+                             int n_pair, float* u, double2* coef) {
   hipLaunchKernelGGL(adjoint_fq_kernel, dim3((nq + 255) / 256), dim3(256), 0, st, nq, q_first, w,
-                     gscale, u);
+                     gscale, dq, ftab, weighted ? 1 : 0, n_pair, u, coef);
   return hipGetLastError();
 }
 
