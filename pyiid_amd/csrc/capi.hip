@@ -152,7 +152,6 @@ struct GradSet {
   Buf rows, row_scale;  // split rows of one chunk of atoms, their scales
   Buf w[2], inv_phihat[2];  // per table slot
   int w_nq[2] = {0, 0};
-  Buf k_used;           // int32: points of a row in use
   int n_run = 0;
   uint64_t stamp = ~0ull;
   int key = -1;
@@ -216,6 +215,8 @@ struct pyiid_ctx {
   std::vector<int32_t> elem_h;
   int max_elem = 0;
   Buf counts_d, natoms_d;
+  Buf off_d;  // int32 chain offsets
+  std::vector<int64_t> off_d_of;  // the layout in off_d
   uint64_t struct_stamp = 1;  // bumps when sizes / offsets / elements change
   // Largest distance within a chain (a bound from its bounding sphere) of the
   // positions seen last by ensure_extent or, for at most kExtentAtoms atoms,
@@ -223,6 +224,8 @@ struct pyiid_ctx {
   double r_max = 0.0;
   std::vector<int64_t> extent_off;  // the layout it was taken for
   bool extent_exact = false;        // r_max bounds the current positions' distances
+  Buf reach;                        // double: such a bound on the device
+  bool reach_set = false;           // of the current positions
 
   Table tab[2];
   uint64_t tab_stamp[2] = {1, 1};
@@ -269,6 +272,20 @@ struct pyiid_ctx {
   Sur sur;
   bool capturing = false;
 
+  // Page-locked memory that host arrays pass through (kArenaBytes, from the
+  // first use on): inputs are copied in by the CPU and read from there by
+  // copies or kernels in stream order, results land there and reach the
+  // caller's arrays once the call has waited for the stream.
+  unsigned char* arena = nullptr;
+  bool arena_failed = false;
+  size_t arena_used = 0;
+  struct HostCopy {
+    void* dst;
+    const void* src;
+    size_t bytes;
+  };
+  std::vector<HostCopy> arena_out;
+
   // timing: event pairs recorded around launches, resolved when queried
   bool timing = false;
   std::vector<hipEvent_t> ev_pool;
@@ -284,22 +301,85 @@ int ensure_device(pyiid_ctx* c) {
   return PYIID_OK;
 }
 
+constexpr size_t kArenaBytes = static_cast<size_t>(4) << 20;
+constexpr size_t kArenaMost = static_cast<size_t>(1) << 20;  // of one array
+
 int check_ctx(pyiid_ctx* c) {
   if (!c) return fail(PYIID_E_INVALID, "null context");
-  return ensure_device(c);
+  CHK(ensure_device(c));
+  if (!c->arena_out.empty()) {  // left by a call that failed half way
+    c->arena_out.clear();
+    HIPCHK(hipStreamSynchronize(c->stream));
+    c->arena_used = 0;
+  }
+  return PYIID_OK;
+}
+
+// Waits for the stream, hands pending results over and empties the arena.
+int arena_flush(pyiid_ctx* c) {
+  HIPCHK(hipStreamSynchronize(c->stream));
+  for (const auto& o : c->arena_out) std::memcpy(o.dst, o.src, o.bytes);
+  c->arena_out.clear();
+  c->arena_used = 0;
+  return PYIID_OK;
+}
+
+// Arena memory for one array, or null (too large, or none to be had).
+int arena_take(pyiid_ctx* c, size_t bytes, void** p) {
+  *p = nullptr;
+  if (bytes == 0 || bytes > kArenaMost || c->arena_failed) return PYIID_OK;
+  if (!c->arena) {
+    void* m = nullptr;
+    if (hipHostMalloc(&m, kArenaBytes, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      c->arena_failed = true;
+      return PYIID_OK;
+    }
+    c->arena = static_cast<unsigned char*>(m);
+  }
+  if (c->arena_used + bytes > kArenaBytes) {
+    if (!c->arena_out.empty()) return PYIID_OK;
+    CHK(arena_flush(c));
+  }
+  *p = c->arena + c->arena_used;
+  c->arena_used += (bytes + 255) & ~static_cast<size_t>(255);
+  return PYIID_OK;
+}
+
+// Where a kernel may write a result of `bytes` for a host array: arena memory
+// handed over by finish(), or null.
+int arena_result(pyiid_ctx* c, void* dst, size_t bytes, void** p) {
+  CHK(arena_take(c, bytes, p));
+  if (*p) c->arena_out.push_back({dst, *p, bytes});
+  return PYIID_OK;
 }
 
 // Copy `bytes` from a user pointer (host or device per flags) into dst (device).
 int upload(pyiid_ctx* c, void* dst, const void* src, size_t bytes, int flags) {
   if (bytes == 0) return PYIID_OK;
+  if (!(flags & PYIID_DEVICE)) {
+    void* p = nullptr;
+    CHK(arena_take(c, bytes, &p));
+    if (p) {
+      std::memcpy(p, src, bytes);
+      src = p;
+    }
+  }
   HIPCHK(hipMemcpyAsync(dst, src, bytes,
                         (flags & PYIID_DEVICE) ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
                         c->stream));
   return PYIID_OK;
 }
 
+// Copy `bytes` of device memory to a user pointer; a host array has them after
+// finish().
 int download(pyiid_ctx* c, void* dst, const void* src, size_t bytes, int flags) {
   if (bytes == 0) return PYIID_OK;
+  if (!(flags & PYIID_DEVICE)) {
+    void* p = nullptr;
+    CHK(arena_result(c, dst, bytes, &p));
+    if (p) dst = p;
+  }
   HIPCHK(hipMemcpyAsync(dst, src, bytes,
                         (flags & PYIID_DEVICE) ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost,
                         c->stream));
@@ -307,20 +387,8 @@ int download(pyiid_ctx* c, void* dst, const void* src, size_t bytes, int flags) 
 }
 
 int finish(pyiid_ctx* c, int flags) {
-  if (!(flags & PYIID_DEVICE)) HIPCHK(hipStreamSynchronize(c->stream));
+  if (!(flags & PYIID_DEVICE)) return arena_flush(c);
   return PYIID_OK;
-}
-
-__global__ void pack_kernel(const float* __restrict__ p, const int32_t* __restrict__ e, int64_t n,
-                            AtomRec* __restrict__ out) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  AtomRec a;
-  a.x = p[3 * i + 0];
-  a.y = p[3 * i + 1];
-  a.z = p[3 * i + 2];
-  a.w = static_cast<double>(e[i]);
-  out[i] = a;
 }
 
 __global__ void unpack_kernel(const AtomRec* __restrict__ a, int64_t n, float* __restrict__ p) {
@@ -381,11 +449,8 @@ int ensure_extent(pyiid_ctx* c) {
 int ensure_packed(pyiid_ctx* c) {
   if (!c->pos_set) return fail(PYIID_E_STATE, "positions not set");
   if (!c->pos_dirty || c->n == 0) return PYIID_OK;
-  const int64_t n = c->n;
-  hipLaunchKernelGGL(pack_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
-                     c->stream, c->posf.as<float>(), c->elem.as<int32_t>(), n,
-                     c->pos.as<AtomRec>());
-  HIPCHK(hipGetLastError());
+  HIPCHK(launch_pack(c->stream, c->posf.as<float>(), c->elem.as<int32_t>(), c->n,
+                     c->pos.as<AtomRec>(), nullptr, nullptr));
   c->pos_dirty = false;
   return PYIID_OK;
 }
@@ -862,6 +927,32 @@ bool use_spread_fq(pyiid_ctx* c, const Table& t) {
          spread_grid_bytes(c, t) <= kSpreadGridBudget && c->n_chain <= 65535;
 }
 
+// Whether F(Q) runs in one launch: small chains, whose pairs each block of 64
+// bins spreads for itself.  A block takes 0.6 us for 1,024 pairs (11 us at 192
+// atoms) and the chip about 5 us for two million; past these sizes the repeated
+// spreading takes longer than two more launches (5 us of the host each), and
+// past 512 bins the transform by one block per 64 bins does (60 atoms at 1,400
+// bins: 60 us against 31).
+bool use_small_fq(pyiid_ctx* c, const Table& t) {
+  if (t.nq > 512 || element_pairs(t) > 3) return false;
+  int64_t pairs = 0;
+  for (int b = 0; b < c->n_chain; ++b) {
+    const int64_t n = c->off[b + 1] - c->off[b];
+    if (n > kSmallAtoms) return false;
+    pairs += n * (n - 1) / 2;
+  }
+  return pairs * ((t.nq + 63) / 64) * element_pairs(t) <= 2000000;
+}
+
+int ensure_offsets(pyiid_ctx* c) {
+  if (c->off_d_of == c->off) return PYIID_OK;
+  if (c->capturing) return fail(PYIID_E_STATE, "structure changed during graph capture");
+  std::vector<int> o(c->off.begin(), c->off.end());
+  CHK(upload_vec(c->off_d, o));
+  c->off_d_of = c->off;
+  return PYIID_OK;
+}
+
 // Atoms as positions in element order per chain (stable), and each chain's
 // element runs.
 struct ElemRun {
@@ -1013,19 +1104,31 @@ hipError_t launch_fq_items(pyiid_ctx* c, const Table& t, double qbin, bool count
                    c->fpart.as<double>(), forms);
 }
 
-// F(Q) of every chain (full grid) into c->fq64 [B][nq] (double) and c->fq32.
-int compute_fq(pyiid_ctx* c, int slot, double qbin) {
+// F(Q) of every chain (full grid) into c->fq64 [B][nq] (double) and c->fq32, or
+// into `direct` only (device floats).
+int compute_fq(pyiid_ctx* c, int slot, double qbin, float* direct = nullptr) {
   Table& t = c->tab[slot];
   const int nq = t.nq, B = c->n_chain;
   CHK(c->fq64.reserve(sizeof(double) * (size_t)std::max(1, nq) * B));
   CHK(c->fq32.reserve(sizeof(float) * (size_t)std::max(1, nq) * B));
   CHK(ensure_packed(c));
   CHK(ensure_norm(c, slot));
+  double* out64 = direct ? nullptr : c->fq64.as<double>();
+  float* out32 = direct ? direct : c->fq32.as<float>();
   if (use_spread_fq(c, t)) {
-    CHK(ensure_spread(c, t));
     SpreadSet& s = c->spread;
     const bool weighted = weighted_table(t);
     const double dq = static_cast<double>(static_cast<float>(qbin));
+    if (use_small_fq(c, t)) {
+      CHK(ensure_extent(c));
+      CHK(ensure_offsets(c));
+      Timed tm(c, 1);
+      HIPCHK(launch_small_fq(c->stream, c->pos.as<AtomRec>(), c->off_d.as<int>(), B,
+                             static_cast<int>(element_pairs(t)), weighted, t.tab.as<float>(), nq, dq,
+                             fq_scale_bits(nq, dq, c->r_max), t.fsu.as<double>(), out64, out32));
+      return tm.done();
+    }
+    CHK(ensure_spread(c, t));
     const AtomRec* sp = c->pos.as<AtomRec>();
     if (weighted) {
       HIPCHK(launch_gather(c->stream, sp, s.perm.as<int32_t>(), c->n, s.sorted.as<AtomRec>()));
@@ -1040,7 +1143,7 @@ int compute_fq(pyiid_ctx* c, int slot, double qbin) {
     CHK(tm.done());
     HIPCHK(launch_transform_fq(c->stream, s.grids.as<unsigned long long>(), B,
                                static_cast<int>(element_pairs(t)), weighted, t.tab.as<float>(), nq,
-                               dq, s.shift, bits, t.fsu.as<double>(), s.part.as<double>(), c->fq64.as<double>(), c->fq32.as<float>()));
+                               dq, s.shift, bits, t.fsu.as<double>(), s.part.as<double>(), out64, out32));
     s.dirty = false;
     return PYIID_OK;
   }
@@ -1052,7 +1155,7 @@ int compute_fq(pyiid_ctx* c, int slot, double qbin) {
   CHK(tm.done());
   // chains without pairs have empty ranges: their F is 0
   HIPCHK(launch_reduce_ranges(c->stream, c->fpart.as<double>(), c->fq_items.ranges.as<Range>(), B,
-                              nq, t.fsu.as<double>(), c->fq64.as<double>(), c->fq32.as<float>()));
+                              nq, t.fsu.as<double>(), out64, out32));
   return PYIID_OK;
 }
 
@@ -1478,7 +1581,6 @@ int run_spread_grad(pyiid_ctx* c, int slot, double qbin, void* out, bool out_f64
       CHK(upload_vec(s.perm, perm));
       CHK(s.sorted.reserve(sizeof(AtomRec) * std::max<int64_t>(1, c->n)));
     }
-    CHK(s.k_used.reserve(sizeof(int)));
     s.stamp = c->struct_stamp;
     s.key = key;
   }
@@ -1502,23 +1604,27 @@ int run_spread_grad(pyiid_ctx* c, int slot, double qbin, void* out, bool out_f64
   // points of a row in use: from the host's extent when it bounds the current
   // positions, else from the positions on the device (no wait either way)
   int k_fixed = 0;
-  const int* k_dev = nullptr;
+  const double* reach = nullptr;
   if (c->extent_exact) {
-    const double reach = grad_reach(nq, dq, c->r_max * 1.000001);
-    k_fixed = reach < len ? (static_cast<int>(reach) + 31) & ~31 : len;
+    const double points = grad_reach(nq, dq, c->r_max * 1.000001);
+    k_fixed = points < len ? (static_cast<int>(points) + 31) & ~31 : len;
     k_fixed = std::min(k_fixed, len);
   } else {
-    HIPCHK(launch_grad_extent(c->stream, sp, c->n, nq, dq, s.k_used.as<int>()));
-    k_dev = s.k_used.as<int>();
+    if (!c->reach_set) {
+      CHK(c->reach.reserve(sizeof(double)));
+      HIPCHK(launch_reach(c->stream, sp, c->n, c->reach.as<double>()));
+      c->reach_set = true;
+    }
+    reach = c->reach.as<double>();
   }
   Timed tm(c, 0);
   for (int64_t p0 = 0; p0 < c->n; p0 += chunk) {
     const int m = static_cast<int>(std::min<int64_t>(chunk, c->n - p0));
     HIPCHK(launch_spread_grad(c->stream, sp, static_cast<int>(p0), m, c->n, s.runs.as<int>(),
-                              s.n_run, nq, dq, c->r_max, k_fixed, k_dev, s.rows.p,
+                              s.n_run, nq, dq, c->r_max, k_fixed, reach, s.rows.p,
                               s.row_scale.as<float>()));
     HIPCHK(launch_gemm_split(c->stream, s.rows.p, s.row_scale.as<float>(), m, s.n_run,
-                             s.w[slot].p, s.inv_phihat[slot].as<float>(), nq, dq, k_fixed, k_dev,
+                             s.w[slot].p, s.inv_phihat[slot].as<float>(), nq, dq, k_fixed, reach,
                              t.gs.as<double>(), t.tab.as<float>(), s.run_elem.as<int>(), weighted,
                              sp, weighted ? s.perm.as<int32_t>() : nullptr, static_cast<int>(p0),
                              out, out_f64));
@@ -1782,17 +1888,39 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
   }
   CHK(c->posf.reserve(sizeof(float) * 3 * std::max<int64_t>(1, n)));
   CHK(c->pos.reserve(sizeof(AtomRec) * std::max<int64_t>(1, n)));
-  CHK(upload(c, c->posf.p, pos, sizeof(float) * 3 * n, flags));
+  // one kernel reads the caller's device positions, or the arena's copy of host
+  // ones, and writes the records and the float copy; nothing waits
+  const float* src = pos;
+  if (!(flags & PYIID_DEVICE) && n > 0) {
+    void* p = nullptr;
+    CHK(arena_take(c, sizeof(float) * 3 * n, &p));
+    if (p) std::memcpy(p, pos, sizeof(float) * 3 * n);
+    src = static_cast<const float*>(p);
+  }
+  if (src && n > 0) {
+    // (the gradient of a single structure asks how far its distances reach)
+    CHK(c->reach.reserve(sizeof(double)));
+    const bool reach = (flags & PYIID_DEVICE) && c->n_chain == 1 && n <= kReachAtoms;
+    HIPCHK(launch_pack(c->stream, src, c->elem.as<int32_t>(), n, c->pos.as<AtomRec>(),
+                       c->posf.as<float>(), reach ? c->reach.as<double>() : nullptr));
+    c->reach_set = reach;
+    c->pos_dirty = false;
+  } else {
+    CHK(upload(c, c->posf.p, pos, sizeof(float) * 3 * n, flags));
+    c->reach_set = false;
+    c->pos_set = true;
+    c->pos_dirty = true;
+    CHK(ensure_packed(c));
+    HIPCHK(hipStreamSynchronize(c->stream));
+  }
   c->pos_set = true;
-  c->pos_dirty = true;
-  CHK(ensure_packed(c));
   c->extent_exact = false;
   if (!(flags & PYIID_DEVICE) && n <= kExtentAtoms) {
     c->r_max = chain_extent(pos, 3, c->off);
     c->extent_off = c->off;
     c->extent_exact = true;
   }
-  return finish(c, flags);
+  return PYIID_OK;
 }
 
 // One proposal of the batched sampler (fixed launch sequence).
@@ -2263,7 +2391,7 @@ int pyiid_destroy(pyiid_ctx* c) {
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
   destroy_graph(c->hmc);
-  for (Buf* b : {&c->posf, &c->elem, &c->pos, &c->counts_d, &c->natoms_d, &c->tmat, &c->gpart,
+  for (Buf* b : {&c->posf, &c->elem, &c->pos, &c->counts_d, &c->natoms_d, &c->off_d, &c->tmat, &c->gpart,
                  &c->fpart, &c->fq64, &c->fq32, &c->g64, &c->io_a, &c->io_b,
                  &c->io_c, &c->w, &c->out5, &c->u, &c->ucoef, &c->upart, &c->gobs, &c->fq_items.items,
                  &c->fq_items.ranges, &c->fq_items.perm, &c->spread.units, &c->spread.items,
@@ -2272,7 +2400,7 @@ int pyiid_destroy(pyiid_ctx* c) {
                  &c->force.t4, &c->force.t2, &c->force.part,
                  &c->grad.perm, &c->grad.sorted, &c->grad.runs, &c->grad.run_elem, &c->grad.rows,
                  &c->grad.row_scale, &c->grad.w[0], &c->grad.w[1], &c->grad.inv_phihat[0],
-                 &c->grad.inv_phihat[1], &c->grad.k_used,
+                 &c->grad.inv_phihat[1], &c->reach,
                  &c->fused_items.items, &c->fused_items.ranges,
                  &c->fused_items.perm, &c->hmc.mass,
                  &c->hmc.mom, &c->hmc.fcur, &c->hmc.fnew, &c->hmc.pos_save, &c->hmc.kin0,
@@ -2296,6 +2424,7 @@ int pyiid_destroy(pyiid_ctx* c) {
     (void)hipEventDestroy(pe.second.second);
   }
   for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
+  if (c->arena) (void)hipHostFree(c->arena);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
   delete c;
   return PYIID_OK;
@@ -2303,6 +2432,7 @@ int pyiid_destroy(pyiid_ctx* c) {
 
 int pyiid_set_stream(pyiid_ctx* c, void* stream) {
   CHK(check_ctx(c));
+  if (c->arena_used > 0) CHK(arena_flush(c));  // inputs the old stream may still read
   c->stream = stream ? static_cast<hipStream_t>(stream) : c->own_stream;
   destroy_graph(c->hmc);
   return PYIID_OK;
@@ -2526,12 +2656,11 @@ int pyiid_fq(pyiid_ctx* c, int slot, double qbin, float* fq, int flags) {
   if (!fq) return fail(PYIID_E_INVALID, "null output");
   const int nq = c->tab[slot].nq;
   const size_t cnt = (size_t)nq * c->n_chain;
-  CHK(compute_fq(c, slot, qbin));
-  if (flags & PYIID_DEVICE) {
-    HIPCHK(hipMemcpyAsync(fq, c->fq32.p, sizeof(float) * cnt, hipMemcpyDeviceToDevice, c->stream));
-  } else {
-    CHK(download(c, fq, c->fq32.p, sizeof(float) * cnt, flags));
-  }
+  if (flags & PYIID_DEVICE) return compute_fq(c, slot, qbin, fq);
+  void* p = nullptr;
+  CHK(arena_result(c, fq, sizeof(float) * cnt, &p));
+  CHK(compute_fq(c, slot, qbin, static_cast<float*>(p)));
+  if (!p) CHK(download(c, fq, c->fq32.p, sizeof(float) * cnt, flags));
   return finish(c, flags);
 }
 
@@ -2560,17 +2689,33 @@ int pyiid_grad_fq(pyiid_ctx* c, int slot, double qbin, void* grad, float* fq, in
   CHK(ensure_norm(c, slot));
   Table& t = c->tab[slot];
   void* gdst = grad;
+  c->grad_spread = use_spread_grad(c, t);
+  if (c->grad_spread) {
+    float* fdst = fq;
+    bool copy = false;
+    if (!(flags & PYIID_DEVICE)) {
+      void *g = nullptr, *f = nullptr;
+      CHK(arena_result(c, grad, gbytes, &g));
+      copy = !g;
+      if (copy) {
+        CHK(c->io_c.reserve(gbytes));
+        g = c->io_c.p;
+      }
+      gdst = g;
+      if (fq) CHK(arena_result(c, fq, sizeof(float) * nq, &f));
+      fdst = static_cast<float*>(f);
+    }
+    CHK(run_spread_grad(c, slot, qbin, gdst, (flags & PYIID_F64) != 0));
+    if (copy) CHK(download(c, grad, gdst, gbytes, flags));
+    if (fq) {
+      CHK(compute_fq(c, slot, qbin, fdst));
+      if (!fdst) CHK(download(c, fq, c->fq32.p, sizeof(float) * nq, flags));
+    }
+    return finish(c, flags);
+  }
   if (!(flags & PYIID_DEVICE)) {
     CHK(c->io_c.reserve(gbytes));
     gdst = c->io_c.p;
-  }
-  c->grad_spread = use_spread_grad(c, t);
-  if (c->grad_spread) {
-    CHK(run_spread_grad(c, slot, qbin, gdst, (flags & PYIID_F64) != 0));
-    if (fq) CHK(compute_fq(c, slot, qbin));
-    if (!(flags & PYIID_DEVICE)) CHK(download(c, grad, gdst, gbytes, flags));
-    if (fq) CHK(download(c, fq, c->fq32.p, sizeof(float) * nq, flags));
-    return finish(c, flags);
   }
   CHK(tune_grad(c, slot, qbin));
   const bool sym = c->sym_k != 0;
@@ -2771,28 +2916,33 @@ int pyiid_pdf_energy_forces(pyiid_ctx* c, int slot, double qbin, const double* g
   CHK(check_pdf_setup(c, slot, potential));
   if (!gobs) return fail(PYIID_E_INVALID, "null target");
   const int B = c->n_chain, nr = c->t_nr;
-  CHK(c->gobs.reserve(sizeof(double) * (size_t)nr * B));
-  CHK(upload(c, c->gobs.p, gobs, sizeof(double) * (size_t)nr * B, flags));
-  double* fdst = nullptr;
-  if (forces) {
-    if (flags & PYIID_DEVICE) {
-      fdst = forces;
-    } else {
-      CHK(c->io_c.reserve(sizeof(double) * 3 * std::max<int64_t>(1, c->n)));
-      fdst = c->io_c.as<double>();
-    }
+  const double* target = gobs;  // a device target is read where it is
+  if (!(flags & PYIID_DEVICE)) {
+    CHK(c->gobs.reserve(sizeof(double) * (size_t)nr * B));
+    CHK(upload(c, c->gobs.p, gobs, sizeof(double) * (size_t)nr * B, flags));
+    target = c->gobs.as<double>();
   }
-  CHK(energy_forces_device(c, slot, qbin, potential, c->gobs.as<double>(), conv, fdst));
+  double* fdst = forces;
+  bool copy = false;
+  if (forces && !(flags & PYIID_DEVICE)) {
+    void* p = nullptr;
+    CHK(arena_result(c, forces, sizeof(double) * 3 * c->n, &p));
+    copy = !p;
+    if (copy) {
+      CHK(c->io_c.reserve(sizeof(double) * 3 * std::max<int64_t>(1, c->n)));
+      p = c->io_c.p;
+    }
+    fdst = static_cast<double*>(p);
+  }
+  CHK(energy_forces_device(c, slot, qbin, potential, target, conv, fdst));
+  if (copy) CHK(download(c, forces, fdst, sizeof(double) * 3 * c->n, flags));
   if (energy) {
     std::vector<double> o5(5 * (size_t)B + 1);
-    HIPCHK(hipMemcpyAsync(o5.data(), c->out5.p, sizeof(double) * o5.size(), hipMemcpyDeviceToHost,
-                          c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    CHK(download(c, o5.data(), c->out5.p, sizeof(double) * o5.size(), 0));
+    CHK(arena_flush(c));
     CHK(note_far(c, o5[5 * (size_t)B]));
     for (int b = 0; b < B; ++b) energy[b] = o5[5 * (size_t)b] * conv;
   }
-  if (forces && !(flags & PYIID_DEVICE))
-    CHK(download(c, forces, fdst, sizeof(double) * 3 * c->n, flags));
   return finish(c, flags);
 }
 
@@ -2896,6 +3046,7 @@ int pyiid_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step, do
   const int B = c->n_chain;
   if (n_proposals == 0) return PYIID_OK;
   c->extent_exact = false;
+  c->reach_set = false;
   CHK(prepare_history(c, n_proposals));
   CHK(refresh_exact(c));
   RunClock clock(c, times_ms != nullptr);
@@ -2910,9 +3061,8 @@ int pyiid_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step, do
     CHK(download(c, accepted, h.acchist.p, sizeof(int32_t) * (size_t)n_proposals * B, flags));
   if (!(flags & PYIID_DEVICE)) {
     double far = 0.0;
-    HIPCHK(hipMemcpyAsync(&far, c->out5.as<double>() + 5 * static_cast<size_t>(B), sizeof(far),
-                          hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    CHK(download(c, &far, c->out5.as<double>() + 5 * static_cast<size_t>(B), sizeof(far), 0));
+    CHK(arena_flush(c));
     CHK(note_far(c, far));
   }
   return finish(c, flags);
@@ -3087,6 +3237,7 @@ int pyiid_sur_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step
   const int B = c->n_chain;
   if (n_proposals == 0) return PYIID_OK;
   c->extent_exact = false;
+  c->reach_set = false;
   CHK(prepare_history(c, n_proposals));
   RunClock clock(c, times_ms != nullptr);
   bool exact_block = false;

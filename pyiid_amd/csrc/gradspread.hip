@@ -88,50 +88,12 @@ __device__ __forceinline__ size_t split_at(int k) {
   return static_cast<size_t>(k >> 5) * 64 + (k & 31);
 }
 
-// ---- extent ----
-
-// Points of a row that the structure's distances reach (a multiple of 32),
-// from its bounding sphere.
-__global__ __launch_bounds__(1024) void extent_kernel(const AtomRec* __restrict__ pos, int n,
-                                                      double inv_h, int full,
-                                                      int* __restrict__ out) {
-  __shared__ double sh[16][6];
-  __shared__ double rad[16];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  double v[6];  // max of x, y, z and of -x, -y, -z
-  for (int k = 0; k < 6; ++k) v[k] = -1e308;
-  bool bad = false;
-  for (int a = threadIdx.x; a < n; a += 1024) {
-    const AtomRec p = pos[a];
-    const double x[3] = {p.x, p.y, p.z};
-    for (int k = 0; k < 3; ++k) {
-      bad = bad || !(fabs(x[k]) < 1e300);
-      v[k] = fmax(v[k], x[k]);
-      v[k + 3] = fmax(v[k + 3], -x[k]);
-    }
-  }
-  for (int off = 32; off > 0; off >>= 1)
-    for (int k = 0; k < 6; ++k) v[k] = fmax(v[k], __shfl_xor(v[k], off, 64));
-  if (lane == 0)
-    for (int k = 0; k < 6; ++k) sh[wave][k] = v[k];
-  const int any_bad = __syncthreads_or(bad ? 1 : 0);
-  for (int w = 0; w < 16; ++w)
-    for (int k = 0; k < 6; ++k) v[k] = fmax(v[k], sh[w][k]);
-  double r2 = 0.0;
-  for (int a = threadIdx.x; a < n; a += 1024) {
-    const AtomRec p = pos[a];
-    const double x = p.x - 0.5 * (v[0] - v[3]), y = p.y - 0.5 * (v[1] - v[4]),
-                 z = p.z - 0.5 * (v[2] - v[5]);
-    r2 = fmax(r2, x * x + y * y + z * z);
-  }
-  for (int off = 32; off > 0; off >>= 1) r2 = fmax(r2, __shfl_xor(r2, off, 64));
-  if (lane == 0) rad[wave] = r2;
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  for (int w = 0; w < 16; ++w) r2 = fmax(r2, rad[w]);
-  const double t = 2.0 * sqrt(r2) * 1.000001 * inv_h;
-  const double want = any_bad || !(t < full) ? full : fmin(static_cast<double>(full), t + kGNodes + 10.0);
-  *out = (static_cast<int>(want) + 31) & ~31;
+// Points of a row in use for distances up to *reach (null: k_fixed).
+__device__ __forceinline__ int points_used(const double* reach, double inv_h, int k_fixed, int nq) {
+  if (!reach) return k_fixed;
+  const int full = row_points(nq);
+  const double t = *reach * inv_h + (kGNodes + 10.0);
+  return ((t < full ? static_cast<int>(t) : full) + 31) & ~31;
 }
 
 // ---- spreading ----
@@ -190,14 +152,14 @@ __device__ void spread_grad_rare(unsigned long long* grid, int plane, int* bad, 
 // that its largest entry lies in [2^14, 2^15).
 __global__ __launch_bounds__(1024, 8) void spread_grad_kernel(
     const AtomRec* __restrict__ pos, int p0, int n_rows, const int* __restrict__ runs, double inv_h, int nf, int plane, int row_len, int k_fixed,
-    const int* __restrict__ k_dev, float scale, double near,
+    const double* __restrict__ reach, int nq, float scale, double near,
     _Float16* __restrict__ rows, float* __restrict__ row_scale) {
   extern __shared__ unsigned long long grid[];
   __shared__ int bad;
   __shared__ unsigned int top[3];
   const int p = p0 + blockIdx.x;
   const int n_thread = blockDim.x;
-  const int k_used = k_dev ? *k_dev : k_fixed;
+  const int k_used = points_used(reach, inv_h, k_fixed, nq);
   const int k_end = min(k_used, plane);  // no distance reaches past k_used
   const int run = blockIdx.y;
   const int jb = runs[run], je = runs[run + 1];
@@ -343,7 +305,7 @@ template <typename OUT, bool MULTI>
 __global__ __launch_bounds__(256, 2) void gemm_split_kernel(
     const _Float16* __restrict__ rows, const float* __restrict__ row_scale, int n_rows, int n_run,
     const _Float16* __restrict__ w, const float* __restrict__ inv_phihat, int row_len, int k_fixed,
-    const int* __restrict__ k_dev, int nq, int n_ct, int n_rt, float unit,
+    const double* __restrict__ reach, double inv_h, int nq, int n_ct, int n_rt, float unit,
     const double* __restrict__ gs, const float* __restrict__ ftab,
     const int* __restrict__ run_elem, const AtomRec* __restrict__ pos,
     const int32_t* __restrict__ perm, int p0, OUT* __restrict__ out) {
@@ -356,7 +318,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(
   const int bm = rt * 128, bn = ct * 128;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave >> 1, wn = wave & 1;
-  const int k_used = k_dev ? *k_dev : k_fixed;
+  const int k_used = points_used(reach, inv_h, k_fixed, nq);
   const int nk = k_used >> 5;
   const int steps = MULTI ? nk * n_run : nk;
 
@@ -485,13 +447,6 @@ size_t grad_lds_bytes(int nq) {
   return sizeof(unsigned long long) * 3 * static_cast<size_t>(row_points(nq) | 1);
 }
 
-hipError_t launch_grad_extent(hipStream_t st, const AtomRec* pos, int64_t n, int nq, double dq,
-                              int* out) {
-  hipLaunchKernelGGL(extent_kernel, dim3(1), dim3(1024), 0, st, pos, static_cast<int>(n),
-                     dq * half_grid(nq) / M_PI, row_points(nq), out);
-  return hipGetLastError();
-}
-
 hipError_t launch_sine_matrix(hipStream_t st, int nq, void* w, float* inv_phihat) {
   const int len = grad_row_len(nq);
   if (nq > 65535) return hipErrorInvalidValue;
@@ -502,7 +457,7 @@ hipError_t launch_sine_matrix(hipStream_t st, int nq, void* w, float* inv_phihat
 
 hipError_t launch_spread_grad(hipStream_t st, const AtomRec* pos, int p0, int n_atoms, int64_t n,
                               const int* runs, int n_run, int nq, double dq, double r_max,
-                              int k_fixed, const int* k_dev, void* rows, float* row_scale) {
+                              int k_fixed, const double* reach, void* rows, float* row_scale) {
   const int nf = 2 * half_grid(nq);
   const double inv_h = dq * half_grid(nq) / M_PI;
   const size_t lds = grad_lds_bytes(nq);
@@ -516,14 +471,14 @@ hipError_t launch_spread_grad(hipStream_t st, const AtomRec* pos, int p0, int n_
   const unsigned threads = n <= 256 ? 256 : n <= 2048 ? 512 : 1024;
   hipLaunchKernelGGL(spread_grad_kernel, dim3(n_atoms, n_run), dim3(threads), lds, st, pos, p0,
                      3 * n_atoms, runs, inv_h, nf, row_points(nq) | 1, grad_row_len(nq), k_fixed,
-                     k_dev, std::ldexp(1.0f, s), 1.2 * std::ldexp(1.0, s - 31),
+                     reach, nq, std::ldexp(1.0f, s), 1.2 * std::ldexp(1.0, s - 31),
                      static_cast<_Float16*>(rows), row_scale);
   return hipGetLastError();
 }
 
 hipError_t launch_gemm_split(hipStream_t st, const void* rows, const float* row_scale, int n_atoms,
                              int n_run, const void* w, const float* inv_phihat, int nq, double dq,
-                             int k_fixed, const int* k_dev, const double* gs, const float* ftab,
+                             int k_fixed, const double* reach, const double* gs, const float* ftab,
                              const int* run_elem, bool weighted, const AtomRec* pos,
                              const int32_t* perm, int p0, void* out, bool out_f64) {
   const int n_rows = 3 * n_atoms;
@@ -535,8 +490,8 @@ hipError_t launch_gemm_split(hipStream_t st, const void* rows, const float* row_
 #define PYIID_GEMM(T, M)                                                                        \
   hipLaunchKernelGGL((gemm_split_kernel<T, M>), grid, dim3(256), 0, st,                         \
                      static_cast<const _Float16*>(rows), row_scale, n_rows, n_run,              \
-                     static_cast<const _Float16*>(w), inv_phihat, len, k_fixed, k_dev, nq, n_ct, \
-                     n_rt, unit, gs, ftab, run_elem, pos, perm, p0, static_cast<T*>(out))
+                     static_cast<const _Float16*>(w), inv_phihat, len, k_fixed, reach, inv_h, nq, \
+                     n_ct, n_rt, unit, gs, ftab, run_elem, pos, perm, p0, static_cast<T*>(out))
   if (weighted) {
     if (out_f64)
       PYIID_GEMM(double, true);

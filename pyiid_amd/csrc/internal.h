@@ -137,6 +137,22 @@ hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_
                                bool weighted, const float* ftab, int nq, double dq, int shift,
                                int scale_bits, const double* scale, double* part, double* out_f64,
                                float* out_f32);
+// F of chains of at most kSmallAtoms atoms (off: n_chain + 1 offsets) in one
+// launch; the grid must fit kSmallFqLds.
+constexpr int kSmallAtoms = 192;
+constexpr size_t kSmallFqLds = 40 * 1024;
+hipError_t launch_small_fq(hipStream_t st, const AtomRec* pos, const int* off, int n_chain,
+                           int n_pair, bool weighted, const float* ftab, int nq, double dq,
+                           int scale_bits, const double* scale, double* out_f64, float* out_f32);
+// Atom records from float positions and elements; keep (nullable) takes a copy
+// of the positions, reach (nullable) a bound of their distances (one block
+// then: for at most kReachAtoms atoms).
+constexpr int64_t kReachAtoms = 4096;
+hipError_t launch_pack(hipStream_t st, const float* p, const int32_t* e, int64_t n, AtomRec* out,
+                       float* keep, double* reach);
+// *reach: a bound of the distances within pos (its bounding sphere's diameter;
+// infinite where a position is not finite)
+hipError_t launch_reach(hipStream_t st, const AtomRec* pos, int64_t n, double* reach);
 // out[p] = pos[perm[p]]
 hipError_t launch_gather(hipStream_t st, const AtomRec* pos, const int32_t* perm, int64_t n,
                          AtomRec* out);
@@ -146,22 +162,20 @@ constexpr size_t kGradLds = 160 * 1024 - 512;   // a block's three grids live in
 int grad_row_len(int nq);                     // points per row (a multiple of 32)
 size_t grad_lds_bytes(int nq);
 double grad_reach(int nq, double dq, double r_max);  // points of a row that r_max reaches
-// *out: points of a row (a multiple of 32) that distances within pos reach
-hipError_t launch_grad_extent(hipStream_t st, const AtomRec* pos, int64_t n, int nq, double dq,
-                              int* out);
 // w: 2 * nq * grad_row_len(nq) halves; inv_phihat: nq floats
 hipError_t launch_sine_matrix(hipStream_t st, int nq, void* w, float* inv_phihat);
 // Grids of positions [p0, p0 + n_atoms) against each of the n_run element
 // runs [runs[e], runs[e + 1]): rows (e * 3 n_atoms + 3 (p - p0) + c), 2 *
-// grad_row_len halves each, and row_scale.  Points used: k_fixed, or *k_dev.
+// grad_row_len halves each, and row_scale.  Points used: k_fixed, or those that
+// distances up to *reach need.
 hipError_t launch_spread_grad(hipStream_t st, const AtomRec* pos, int p0, int n_atoms, int64_t n,
                               const int* runs, int n_run, int nq, double dq, double r_max,
-                              int k_fixed, const int* k_dev, void* rows, float* row_scale);
+                              int k_fixed, const double* reach, void* rows, float* row_scale);
 // out[perm[p]][c][m] = gs[m] f_p(m) sum_e f_e(m) sum_k rows w / phihat
 // (single element: without f).  perm null: identity.
 hipError_t launch_gemm_split(hipStream_t st, const void* rows, const float* row_scale, int n_atoms,
                              int n_run, const void* w, const float* inv_phihat, int nq, double dq,
-                             int k_fixed, const int* k_dev, const double* gs, const float* ftab,
+                             int k_fixed, const double* reach, const double* gs, const float* ftab,
                              const int* run_elem, bool weighted, const AtomRec* pos,
                              const int32_t* perm, int p0, void* out, bool out_f64);
 

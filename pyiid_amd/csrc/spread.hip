@@ -115,6 +115,29 @@ __device__ void spread_rare(unsigned long long* hist, int n_grid, double t, doub
   }
 }
 
+// A pair in the fixed point's fast range.
+__device__ __forceinline__ void spread_pair(unsigned long long* hist, double t, double nf,
+                                            double half_nf, float scale) {
+  float w = scale * __builtin_amdgcn_rcpf(static_cast<float>(t));
+  if (t > half_nf) {
+    bool neg;
+    t = fold(t, nf, neg);
+    if (neg) w = -w;
+  }
+  const double fl = floor(t);
+  const float y = static_cast<float>(t - fl) - 0.5f;
+  const float y2 = y * y;
+  unsigned long long* h = hist + (static_cast<int>(fl) + 1);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const float e = fmaf(fmaf(kFqVal[k][4], y2, kFqVal[k][2]), y2, kFqVal[k][0]);
+    const float o = y * fmaf(fmaf(kFqVal[k][5], y2, kFqVal[k][3]), y2, kFqVal[k][1]);
+    const int a = nearest((e + o) * w), b = nearest((e - o) * w);
+    atomicAdd(&h[k], static_cast<unsigned long long>(static_cast<long long>(a)));
+    atomicAdd(&h[kFqW - 1 - k], static_cast<unsigned long long>(static_cast<long long>(b)));
+  }
+}
+
 // One block (16 waves) per work unit: a run of items of one chain and element
 // pair, whose pairs are spread into the block's grid in LDS, then added to the
 // chain's grid in global memory.  An item is an i tile of at most 64 positions
@@ -158,24 +181,7 @@ __global__ __launch_bounds__(1024, 8) void spread_fq_kernel(
         rare = true;
         continue;
       }
-      float w = scale * __builtin_amdgcn_rcpf(static_cast<float>(t));
-      if (t > half_nf) {
-        bool neg;
-        t = fold(t, static_cast<double>(nf), neg);
-        if (neg) w = -w;
-      }
-      const double fl = floor(t);
-      const float y = static_cast<float>(t - fl) - 0.5f;
-      const float y2 = y * y;
-      unsigned long long* h = hist + (static_cast<int>(fl) + 1);
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const float e = fmaf(fmaf(kFqVal[k][4], y2, kFqVal[k][2]), y2, kFqVal[k][0]);
-        const float o = y * fmaf(fmaf(kFqVal[k][5], y2, kFqVal[k][3]), y2, kFqVal[k][1]);
-        const int a = nearest((e + o) * w), b = nearest((e - o) * w);
-        atomicAdd(&h[k], static_cast<unsigned long long>(static_cast<long long>(a)));
-        atomicAdd(&h[kFqW - 1 - k], static_cast<unsigned long long>(static_cast<long long>(b)));
-      }
+      spread_pair(hist, t, static_cast<double>(nf), half_nf, scale);
     }
   }
   // few pairs of a physical structure, if any, are left for a second look
@@ -210,11 +216,53 @@ __global__ __launch_bounds__(1024, 8) void spread_fq_kernel(
 
 constexpr int kTrChunk = 2048;  // grid points in LDS at a time (16 KiB)
 
+// sum over grid points [lo, hi) of value(k) sin(2 pi (first + k - 3) m / n_f):
+// the sine starts from an exact phase (reduced as an integer below 2^31: n_f <=
+// 12 * 3,400, g + n_f < 1.6 n_f) and follows the FP64 three-term recurrence.
+template <typename F>
+__device__ __forceinline__ double sine_sum(F value, int lo, int hi, int first, int m, int nf) {
+  const double two_over = 2.0 / static_cast<double>(nf);
+  const double c2 = 2.0 * cospi(two_over * m);
+  const unsigned g = static_cast<unsigned>(first + lo - 3 + nf);
+  const unsigned s0 = g * static_cast<unsigned>(m) % static_cast<unsigned>(nf);
+  const unsigned s1 = (g - 1u) * static_cast<unsigned>(m) % static_cast<unsigned>(nf);
+  double y = sinpi(two_over * static_cast<double>(s0));
+  double yp = sinpi(two_over * static_cast<double>(s1));
+  double acc = 0.0;
+#pragma unroll 4
+  for (int k = lo; k < hi; ++k) {
+    acc = fma(value(k), y, acc);
+    const double yn = fma(c2, y, -yp);
+    yp = y;
+    y = yn;
+  }
+  return acc;
+}
+
+// h / phihat(m) and the fixed point's unit
+__device__ __forceinline__ double fq_unit(int m, int nf, double inv_h, int shift, int scale_bits) {
+  const double q = 2.0 * M_PI * m / nf;  // Q h
+  const double a = sqrt(fmax(kFqBeta * kFqBeta - 0.25 * kFqW * kFqW * q * q, 1.0));
+  return ldexp(inv_h, shift - scale_bits) * (sinh(kFqBeta) / kFqBeta) * a / sinh(a);
+}
+
+// The close contacts' part of sum sin(Q r) / r (almost always none)
+__device__ __forceinline__ double fq_nodes(const unsigned long long* nodes, int m, int nf,
+                                           double inv_h, int shift) {
+  const double q = 2.0 * M_PI * m / nf;
+  double t = 0.0;
+  for (int k = 0; k < kFqNodes; ++k) {
+    const long long v = static_cast<long long>(nodes[k]);
+    if (v != 0)
+      t += static_cast<double>(v) * (ldexp(inv_h, shift) / kNodeScale) * sin(q * fq_node(k)) /
+           fq_node(k);
+  }
+  return nodes[kFqNodes] != 0ull ? __builtin_nan("") : t;
+}
+
 // part[b][z][m]: one block takes 64 bins (lanes) of one chain against one of
 // the n_split parts of one element pair's grid; its 16 waves take consecutive
-// slices of every chunk of points.  sin(2 pi g m / n_f) starts from an exact
-// phase and follows the FP64 three-term recurrence along g.  The parts are
-// there to fill the chip: one block per 64 bins took 47 us for 1,250 bins and
+// slices of every chunk of points.  The parts are there to fill the chip: one block per 64 bins took 47 us for 1,250 bins and
 // 155 us for three element pairs at 1,500.
 __global__ __launch_bounds__(1024) void transform_fq_kernel(
     const unsigned long long* __restrict__ grids, int n_pair, int n_split, int nf, int n_grid,
@@ -229,8 +277,6 @@ __global__ __launch_bounds__(1024) void transform_fq_kernel(
   const unsigned long long* h = grids + (static_cast<size_t>(b) * n_pair + pair) * stride;
   const int g_lo = static_cast<int>(static_cast<int64_t>(n_grid) * split / n_split);
   const int g_hi = static_cast<int>(static_cast<int64_t>(n_grid) * (split + 1) / n_split);
-  const double two_over = 2.0 / static_cast<double>(nf);
-  const double c2 = 2.0 * cospi(two_over * m);
   double acc = 0.0;
   for (int g0 = g_lo; g0 < g_hi; g0 += kTrChunk) {
     const int cnt = min(kTrChunk, g_hi - g0);
@@ -238,21 +284,7 @@ __global__ __launch_bounds__(1024) void transform_fq_kernel(
     for (int g = threadIdx.x; g < cnt; g += blockDim.x)
       buf[g] = static_cast<double>(static_cast<long long>(h[g0 + g]));
     __syncthreads();
-    const int lo = cnt * wave / 16, hi = cnt * (wave + 1) / 16;
-    // phases of grid points g0 + lo - 3 and one before, reduced as integers
-    // (below 2^31: n_f <= 12 * 3,400, g + n_f < 1.6 n_f)
-    const unsigned g = static_cast<unsigned>(g0 + lo - 3 + nf);
-    const unsigned s0 = g * static_cast<unsigned>(m) % static_cast<unsigned>(nf);
-    const unsigned s1 = (g - 1u) * static_cast<unsigned>(m) % static_cast<unsigned>(nf);
-    double y = sinpi(two_over * static_cast<double>(s0));
-    double yp = sinpi(two_over * static_cast<double>(s1));
-#pragma unroll 4
-    for (int k = lo; k < hi; ++k) {
-      acc = fma(buf[k], y, acc);
-      const double yn = fma(c2, y, -yp);
-      yp = y;
-      y = yn;
-    }
+    acc += sine_sum([&](int k) { return buf[k]; }, cnt * wave / 16, cnt * (wave + 1) / 16, g0, m, nf);
   }
   sums[wave][lane] = acc;
   __syncthreads();
@@ -260,18 +292,8 @@ __global__ __launch_bounds__(1024) void transform_fq_kernel(
   double total = 0.0;
 #pragma unroll
   for (int k = 0; k < 16; ++k) total += sums[k][lane];
-  const double q = M_PI * two_over * m;  // Q h
-  const double a = sqrt(fmax(kFqBeta * kFqBeta - 0.25 * kFqW * kFqW * q * q, 1.0));
-  total *= ldexp(inv_h, shift - scale_bits) * (sinh(kFqBeta) / kFqBeta) * a / sinh(a);
-  if (split == 0) {  // close contacts (almost always none)
-    for (int k = 0; k < kFqNodes; ++k) {
-      const long long v = static_cast<long long>(h[n_grid + k]);
-      if (v != 0)
-        total += static_cast<double>(v) * (ldexp(inv_h, shift) / kNodeScale) *
-                 sin(q * fq_node(k)) / fq_node(k);
-    }
-    if (h[n_grid + kFqNodes] != 0ull) total = __builtin_nan("");
-  }
+  total *= fq_unit(m, nf, inv_h, shift, scale_bits);
+  if (split == 0) total += fq_nodes(h + n_grid, m, nf, inv_h, shift);
   if (weighted) {
     int ei = 0, ej = pair;
     while (ej > ei) ej -= ++ei;
@@ -304,6 +326,169 @@ __global__ __launch_bounds__(256) void finish_fq_kernel(
   for (int64_t w = static_cast<int64_t>(blockIdx.x - n_out) * 256 + threadIdx.x; w < words2;
        w += static_cast<int64_t>(gridDim.x - n_out) * 256)
     grids[w] = ulonglong2{0ull, 0ull};
+}
+
+// F of chains of at most kSmallAtoms atoms in one launch instead of three: every
+// block of 64 bins spreads all pairs of its chain again (at most 18 for each of
+// its threads) and transforms the grid where it lies, in LDS.  Element pairs
+// follow one another.  55 atoms, 250 bins: 9 us of kernels and two launches less.
+__global__ __launch_bounds__(1024) void small_fq_kernel(
+    const AtomRec* __restrict__ pos, const int* __restrict__ off, int n_pair, int nf, int n_grid,
+    int stride, int scale_bits, float scale, double near, const float* __restrict__ ftab, int nq,
+    double inv_h, int weighted, const double* __restrict__ fscale, double* __restrict__ out64,
+    float* __restrict__ out32) {
+  extern __shared__ unsigned long long hist[];
+  __shared__ double sums[16][65];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m = blockIdx.x * 64 + lane;
+  const int b = blockIdx.y;
+  const int i0 = off[b], n = off[b + 1] - i0;
+  const int pairs = n * (n - 1) / 2;
+  const double half_nf = 0.5 * nf;
+  double total = 0.0;
+  int ei = 0, ej = 0;
+  for (int p = 0; p < n_pair; ++p) {
+    __syncthreads();
+    for (int g = threadIdx.x; g < stride; g += 1024) hist[g] = 0ull;
+    __syncthreads();
+    for (int k = threadIdx.x; k < pairs; k += 1024) {
+      int i = static_cast<int>((1.0f + __builtin_amdgcn_sqrtf(1.0f + 8.0f * k)) * 0.5f);
+      if (i * (i - 1) / 2 > k) --i;
+      if ((i + 1) * i / 2 <= k) ++i;
+      const AtomRec a = pos[i0 + i], c = pos[i0 + k - i * (i - 1) / 2];
+      if (weighted) {
+        const int x = static_cast<int>(a.w), y = static_cast<int>(c.w);
+        if (max(x, y) != ei || min(x, y) != ej) continue;
+      }
+      const double dx = a.x - c.x, dy = a.y - c.y, dz = a.z - c.z;
+      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+      if (!(r2 > 0.0)) continue;
+      const double t = scaled_root(r2, inv_h);
+      if (t >= near && t < kFqFar)
+        spread_pair(hist, t, static_cast<double>(nf), half_nf, scale);
+      else
+        spread_rare(hist, n_grid, sqrt(r2) * inv_h, static_cast<double>(nf),
+                    static_cast<double>(scale));
+    }
+    __syncthreads();
+    double* grid = reinterpret_cast<double*>(hist);  // the points in place, once
+    for (int g = threadIdx.x; g < n_grid; g += 1024)
+      grid[g] = static_cast<double>(static_cast<long long>(hist[g]));
+    __syncthreads();
+    sums[wave][lane] = sine_sum([&](int k) { return grid[k]; }, n_grid * wave / 16,
+                                n_grid * (wave + 1) / 16, 0, m, nf);
+    __syncthreads();
+    if (wave == 0 && m < nq) {
+      double v = 0.0;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) v += sums[k][lane];
+      v = v * fq_unit(m, nf, inv_h, 0, scale_bits) + fq_nodes(hist + n_grid, m, nf, inv_h, 0);
+      if (weighted)
+        v *= static_cast<double>(ftab[static_cast<size_t>(ei) * nq + m]) *
+             static_cast<double>(ftab[static_cast<size_t>(ej) * nq + m]);
+      total += v;
+    }
+    if (++ej > ei) {
+      ++ei;
+      ej = 0;
+    }
+  }
+  if (wave != 0 || m >= nq) return;
+  const size_t o = static_cast<size_t>(b) * nq + m;
+  const double v = total * fscale[o];
+  if (out64) out64[o] = v;
+  if (out32) out32[o] = static_cast<float>(v);
+}
+
+// Bound of the distances between the block's positions x[3] per call of get(a):
+// the diameter of the sphere about the middle of their box.
+template <typename G>
+__device__ double block_reach(G get, int n) {
+  __shared__ double box[16][6];
+  __shared__ double rad[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double v[6];  // max of x, y, z and of -x, -y, -z
+  for (int k = 0; k < 6; ++k) v[k] = -1e308;
+  bool bad = false;
+  for (int a = threadIdx.x; a < n; a += 1024) {
+    double x[3];
+    get(a, x);
+    for (int k = 0; k < 3; ++k) {
+      bad = bad || !(fabs(x[k]) < 1e150);
+      v[k] = fmax(v[k], x[k]);
+      v[k + 3] = fmax(v[k + 3], -x[k]);
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1)
+    for (int k = 0; k < 6; ++k) v[k] = fmax(v[k], __shfl_xor(v[k], off, 64));
+  if (lane == 0)
+    for (int k = 0; k < 6; ++k) box[wave][k] = v[k];
+  const int any_bad = __syncthreads_or(bad ? 1 : 0);
+  for (int w = 0; w < 16; ++w)
+    for (int k = 0; k < 6; ++k) v[k] = fmax(v[k], box[w][k]);
+  double r2 = 0.0;
+  for (int a = threadIdx.x; a < n; a += 1024) {
+    double x[3];
+    get(a, x);
+    double d = 0.0;
+    for (int k = 0; k < 3; ++k) d += (x[k] - 0.5 * (v[k] - v[k + 3])) * (x[k] - 0.5 * (v[k] - v[k + 3]));
+    r2 = fmax(r2, d);
+  }
+  for (int off = 32; off > 0; off >>= 1) r2 = fmax(r2, __shfl_xor(r2, off, 64));
+  if (lane == 0) rad[wave] = r2;
+  __syncthreads();
+  for (int w = 0; w < 16; ++w) r2 = fmax(r2, rad[w]);
+  return any_bad ? __builtin_inf() : 2.0 * sqrt(r2) * 1.000001;
+}
+
+__global__ __launch_bounds__(1024) void reach_kernel(const AtomRec* __restrict__ pos, int n,
+                                                     double* __restrict__ reach) {
+  const double r = block_reach(
+      [&](int a, double* x) {
+        const AtomRec p = pos[a];
+        x[0] = p.x;
+        x[1] = p.y;
+        x[2] = p.z;
+      },
+      n);
+  if (threadIdx.x == 0) *reach = r;
+}
+
+__device__ __forceinline__ void pack_one(const float* __restrict__ p, const int32_t* __restrict__ e,
+                                         int64_t i, AtomRec* __restrict__ out,
+                                         float* __restrict__ keep) {
+  const float x = p[3 * i + 0], y = p[3 * i + 1], z = p[3 * i + 2];
+  AtomRec a;
+  a.x = x;
+  a.y = y;
+  a.z = z;
+  a.w = static_cast<double>(e[i]);
+  out[i] = a;
+  if (keep) {
+    keep[3 * i + 0] = x;
+    keep[3 * i + 1] = y;
+    keep[3 * i + 2] = z;
+  }
+}
+
+__global__ void pack_kernel(const float* __restrict__ p, const int32_t* __restrict__ e, int64_t n,
+                            AtomRec* __restrict__ out, float* __restrict__ keep) {
+  const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (i < n) pack_one(p, e, i, out, keep);
+}
+
+__global__ __launch_bounds__(1024) void pack_reach_kernel(const float* __restrict__ p,
+                                                          const int32_t* __restrict__ e, int n,
+                                                          AtomRec* __restrict__ out,
+                                                          float* __restrict__ keep,
+                                                          double* __restrict__ reach) {
+  for (int i = threadIdx.x; i < n; i += 1024) pack_one(p, e, i, out, keep);
+  const double r = block_reach(
+      [&](int a, double* x) {
+        for (int k = 0; k < 3; ++k) x[k] = p[3 * a + k];
+      },
+      n);
+  if (threadIdx.x == 0) *reach = r;
 }
 
 __global__ void gather_kernel(const AtomRec* __restrict__ pos, const int32_t* __restrict__ perm,
@@ -365,6 +550,40 @@ hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_
   hipLaunchKernelGGL(finish_fq_kernel, dim3(static_cast<unsigned>(n_out + n_clear)), dim3(256), 0,
                      st, part, n_pair * n_split, nq, total, static_cast<int>(n_out), scale, out_f64,
                      out_f32, reinterpret_cast<ulonglong2*>(grids), words2);
+  return hipGetLastError();
+}
+
+hipError_t launch_small_fq(hipStream_t st, const AtomRec* pos, const int* off, int n_chain,
+                           int n_pair, bool weighted, const float* ftab, int nq, double dq,
+                           int scale_bits, const double* scale, double* out_f64, float* out_f32) {
+  const int nf = 12 * nq, stride = fq_grid_stride(nq);
+  const size_t lds = sizeof(unsigned long long) * static_cast<size_t>(stride);
+  if (lds > kSmallFqLds || n_chain > 65535) return hipErrorInvalidValue;
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(small_fq_kernel),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kSmallFqLds));
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL(small_fq_kernel, dim3((nq + 63) / 64, n_chain), dim3(1024), lds, st, pos, off,
+                     n_pair, nf, fq_grid_points(nq), stride, scale_bits,
+                     std::ldexp(1.0f, scale_bits), std::ldexp(1.0, scale_bits - 31), ftab, nq,
+                     dq * nf / (2.0 * M_PI), weighted ? 1 : 0, scale, out_f64, out_f32);
+  return hipGetLastError();
+}
+
+hipError_t launch_pack(hipStream_t st, const float* p, const int32_t* e, int64_t n, AtomRec* out,
+                       float* keep, double* reach) {
+  if (n == 0) return hipSuccess;
+  if (reach && n <= kReachAtoms)
+    hipLaunchKernelGGL(pack_reach_kernel, dim3(1), dim3(1024), 0, st, p, e, static_cast<int>(n), out,
+                       keep, reach);
+  else
+    hipLaunchKernelGGL(pack_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st,
+                       p, e, n, out, keep);
+  return hipGetLastError();
+}
+
+hipError_t launch_reach(hipStream_t st, const AtomRec* pos, int64_t n, double* reach) {
+  hipLaunchKernelGGL(reach_kernel, dim3(1), dim3(1024), 0, st, pos, static_cast<int>(n), reach);
   return hipGetLastError();
 }
 
