@@ -1555,7 +1555,18 @@ bool use_spread_grad(pyiid_ctx* c, const Table& t) {
          c->sym_k_fixed == 0 && grad_lds_bytes(t.nq) <= kGradLds;
 }
 
-int run_spread_grad(pyiid_ctx* c, int slot, double qbin, void* out, bool out_f64) {
+// Whether F of a gradient call rides along with it: few atoms, where launches
+// are what counts; a single element, whose transform needs no further sum.
+constexpr int64_t kBothAtoms = 2048;
+constexpr int kBothBins = 512;
+bool use_spread_both(pyiid_ctx* c, const Table& t) {
+  return use_spread_grad(c, t) && use_spread_fq(c, t) && !use_small_fq(c, t) &&
+         c->n <= kBothAtoms && t.nq <= kBothBins && element_pairs(t) == 1;
+}
+
+// The gradient, and with fq (device floats) F in the same launches
+// (use_spread_both).
+int run_spread_grad(pyiid_ctx* c, int slot, double qbin, void* out, bool out_f64, float* fq) {
   Table& t = c->tab[slot];
   GradSet& s = c->grad;
   const int nq = t.nq;
@@ -1617,18 +1628,31 @@ int run_spread_grad(pyiid_ctx* c, int slot, double qbin, void* out, bool out_f64
     }
     reach = c->reach.as<double>();
   }
+  if (fq) CHK(ensure_spread(c, t));
+  unsigned long long* grids = fq ? c->spread.grids.as<unsigned long long>() : nullptr;
   Timed tm(c, 0);
+  if (fq) {
+    const int bits = fq_scale_bits(nq, dq, c->r_max);
+    c->spread.dirty = true;
+    HIPCHK(launch_spread_both(c->stream, sp, static_cast<int>(c->n), s.runs.as<int>(), s.n_run, nq,
+                              dq, c->r_max, k_fixed, reach, s.rows.p, s.row_scale.as<float>(),
+                              c->spread.units.as<SpreadUnit>(), c->spread.n_units,
+                              c->spread.items.as<SpreadItem>(), bits, grids));
+    HIPCHK(launch_transform_one(c->stream, grids, nq, dq, bits, t.fsu.as<double>(), fq));
+  }
   for (int64_t p0 = 0; p0 < c->n; p0 += chunk) {
     const int m = static_cast<int>(std::min<int64_t>(chunk, c->n - p0));
-    HIPCHK(launch_spread_grad(c->stream, sp, static_cast<int>(p0), m, c->n, s.runs.as<int>(),
-                              s.n_run, nq, dq, c->r_max, k_fixed, reach, s.rows.p,
-                              s.row_scale.as<float>()));
+    if (!fq)
+      HIPCHK(launch_spread_grad(c->stream, sp, static_cast<int>(p0), m, c->n, s.runs.as<int>(),
+                                s.n_run, nq, dq, c->r_max, k_fixed, reach, s.rows.p,
+                                s.row_scale.as<float>()));
     HIPCHK(launch_gemm_split(c->stream, s.rows.p, s.row_scale.as<float>(), m, s.n_run,
                              s.w[slot].p, s.inv_phihat[slot].as<float>(), nq, dq, k_fixed, reach,
                              t.gs.as<double>(), t.tab.as<float>(), s.run_elem.as<int>(), weighted,
                              sp, weighted ? s.perm.as<int32_t>() : nullptr, static_cast<int>(p0),
-                             out, out_f64));
+                             out, out_f64, grids, grids ? fq_grid_stride(nq) : 0));
   }
+  if (fq) c->spread.dirty = false;
   return tm.done();
 }
 
@@ -2705,9 +2729,10 @@ int pyiid_grad_fq(pyiid_ctx* c, int slot, double qbin, void* grad, float* fq, in
       if (fq) CHK(arena_result(c, fq, sizeof(float) * nq, &f));
       fdst = static_cast<float*>(f);
     }
-    CHK(run_spread_grad(c, slot, qbin, gdst, (flags & PYIID_F64) != 0));
+    const bool both = fq && fdst && use_spread_both(c, t);
+    CHK(run_spread_grad(c, slot, qbin, gdst, (flags & PYIID_F64) != 0, both ? fdst : nullptr));
     if (copy) CHK(download(c, grad, gdst, gbytes, flags));
-    if (fq) {
+    if (fq && !both) {
       CHK(compute_fq(c, slot, qbin, fdst));
       if (!fdst) CHK(download(c, fq, c->fq32.p, sizeof(float) * nq, flags));
     }

@@ -1,0 +1,182 @@
+// The F(Q) grid of spread.hip: its window, fixed point and the spreading of one
+// work unit, shared with gradspread.hip (which runs units beside its own blocks).
+#pragma once
+
+#include "pair_math.h"
+
+namespace pyiid {
+namespace {
+
+// ---- window of the F grid ----
+constexpr int kFqW = 6;             // grid points per pair
+constexpr double kFqBeta = 15.160;  // window shape (smallest r.m.s. error at 6 points)
+// phi_j(y), j < 3, y in [-1/2, 1/2] about the middle of the window;
+// phi_{5-j}(y) = phi_j(-y)
+constexpr float kFqVal[3][6] = {
+    {0.000792858506f, -0.00591184293f, 0.0172319146f, -0.0255775783f, 0.0208579919f,
+     -0.00803987611f},
+    {0.0737481676f, -0.206023853f, 0.19830423f, -0.0388040482f, -0.062571443f, 0.0402357172f},
+    {0.425458973f, -0.352369105f, -0.215536146f, 0.244299265f, 0.041713486f, -0.0805066679f},
+};
+// Fixed point of the grid: phi_j 2^s / t, t = r / h.  s is chosen from the
+// structure's extent so that a pair at its largest distance still has 2^24
+// units (at most 2^25), and s >= 36.  From t = 2^(s - 31) on (0.7 A for a
+// particle of 85 A at 25 1/A) the value is below 2^31 and one int32 conversion
+// serves; closer pairs take spread_rare.
+constexpr int kFqBits = 24;
+constexpr int kFqMinScale = 36, kFqMaxScale = 48;
+// Below t = kFqClose the window's error over 1/r would show: there sin(Qr)/r,
+// an even function of r, is interpolated in r^2 from kFqNodes Chebyshev nodes
+// on (0, kFqClose h) (error below 1e-9 for Q h <= pi / 6).  Their weights
+// follow the grid, scaled by 2^30.
+constexpr double kFqClose = 2.0;
+constexpr int kFqNodes = 5;
+constexpr double kNodeScale = 1073741824.0;
+
+__host__ __device__ inline double fq_node(int k) {  // t of node k
+  constexpr double c[kFqNodes] = {0.98768834059513773, 0.89100652418836787, 0.70710678118654752,
+                                  0.45399049973954675, 0.15643446504023087};  // cos((2k+1) pi/20)
+  return kFqClose * c[k];
+}
+
+// ---- spreading ----
+
+// Brings t = r / h into [0, n_f / 2]; neg: the reflected half (sin changes sign).
+__device__ __forceinline__ double fold(double t, double nf, bool& neg) {
+  const double u = t - nf * floor(t / nf);
+  neg = u > 0.5 * nf;
+  return neg ? nf - u : u;
+}
+
+constexpr double kFqFar = 1e15;  // beyond: spread_rare
+
+// A pair closer than the fixed point's fast range, or at an infinite
+// distance: 64-bit conversions.  Few pairs of a physical structure come here.
+__device__ void spread_rare(unsigned long long* hist, int n_grid, double t, double nf,
+                                         double scale) {
+  unsigned long long* nodes = hist + n_grid;
+  if (!(t < 1e300)) {  // infinite: F is not a number
+    atomicAdd(&nodes[kFqNodes], 1ull);
+    return;
+  }
+  if (t < kFqClose) {
+    const double s = t * t;
+    for (int k = 0; k < kFqNodes; ++k) {
+      double l = 1.0;
+      for (int j = 0; j < kFqNodes; ++j)
+        if (j != k) l *= (s - fq_node(j) * fq_node(j)) / (fq_node(k) * fq_node(k) - fq_node(j) * fq_node(j));
+      atomicAdd(&nodes[k], static_cast<unsigned long long>(static_cast<long long>(rint(l * kNodeScale))));
+    }
+    return;
+  }
+  bool neg;
+  const double tf = fold(t, nf, neg);
+  const double fl = floor(tf);
+  const double y = tf - fl - 0.5, w = (neg ? -scale : scale) / t;
+  unsigned long long* h = hist + (static_cast<int>(fl) + 1);
+  for (int j = 0; j < kFqW; ++j) {
+    const float* c = kFqVal[j < 3 ? j : kFqW - 1 - j];
+    const double z = j < 3 ? y : -y;
+    double p = c[5];
+    for (int k = 4; k >= 0; --k) p = p * z + static_cast<double>(c[k]);
+    atomicAdd(&h[j], static_cast<unsigned long long>(static_cast<long long>(rint(p * w))));
+  }
+}
+
+// A pair in the fixed point's fast range.
+__device__ __forceinline__ void spread_pair(unsigned long long* hist, double t, double nf,
+                                            double half_nf, float scale) {
+  float w = scale * __builtin_amdgcn_rcpf(static_cast<float>(t));
+  if (t > half_nf) {
+    bool neg;
+    t = fold(t, nf, neg);
+    if (neg) w = -w;
+  }
+  const double fl = floor(t);
+  const float y = static_cast<float>(t - fl) - 0.5f;
+  const float y2 = y * y;
+  unsigned long long* h = hist + (static_cast<int>(fl) + 1);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const float e = fmaf(fmaf(kFqVal[k][4], y2, kFqVal[k][2]), y2, kFqVal[k][0]);
+    const float o = y * fmaf(fmaf(kFqVal[k][5], y2, kFqVal[k][3]), y2, kFqVal[k][1]);
+    const int a = nearest((e + o) * w), b = nearest((e - o) * w);
+    atomicAdd(&h[k], static_cast<unsigned long long>(static_cast<long long>(a)));
+    atomicAdd(&h[kFqW - 1 - k], static_cast<unsigned long long>(static_cast<long long>(b)));
+  }
+}
+
+// One block (at least 4 waves) per work unit: a run of items of one chain and element
+// pair, whose pairs are spread into the block's grid in LDS, then added to the
+// chain's grid in global memory.  An item is an i tile of at most 64 positions
+// (one lane each) against a j range; the waves take consecutive slices of
+// the range, and a j atom's position is wave-uniform (scalar loads, so the
+// FP64 differences take it from SGPRs).
+//
+// Per 64 pairs about 16 FP64 or conversion instructions (distance to 1e-14:
+// a phase of 1,500 rad to 1e-11), 18 FMAs for the window, 6 conversions to
+// integer and 6 ds_add_u64.  The LDS adds (29 ns per CU) and the VALU (about
+// as long, 4 SIMDs) run side by side, and 2 blocks (32 waves) per CU hide
+// each other's latency.
+__device__ __forceinline__ void spread_fq_unit(
+    const AtomRec* __restrict__ pos, const SpreadUnit& un, const SpreadItem* __restrict__ items,
+    double inv_h, int nf, int n_grid, int stride, int shift, float scale, double near,
+    unsigned long long* hist, unsigned long long* __restrict__ grids) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n_wave = blockDim.x >> 6;
+  for (int g = threadIdx.x; g < stride; g += blockDim.x) hist[g] = 0ull;
+  __syncthreads();
+  const double half_nf = 0.5 * nf;
+  bool rare = false;
+  for (int it = un.begin; it < un.end; ++it) {
+    const SpreadItem item = items[it];
+    const int len = item.j1 - item.j0;
+    const int jb = item.j0 + static_cast<int>(static_cast<int64_t>(len) * wave / n_wave);
+    const int je = item.j0 + static_cast<int>(static_cast<int64_t>(len) * (wave + 1) / n_wave);
+    const int i = item.i0 + lane;
+    const bool have = i < item.i1;
+    const AtomRec pi = pos[have ? i : item.i0];
+    for (int j = jb; j < je; ++j) {
+      const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
+      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+      // j < i; a pair at distance 0 (and one with a NaN) contributes nothing
+      if (!(have && j < i && r2 > 0.0)) continue;
+      double t = scaled_root(r2, inv_h);
+      if (!(t >= near && t < kFqFar)) {
+        rare = true;
+        continue;
+      }
+      spread_pair(hist, t, static_cast<double>(nf), half_nf, scale);
+    }
+  }
+  // few pairs of a physical structure, if any, are left for a second look
+  if (__syncthreads_or(rare ? 1 : 0)) {
+    for (int it = un.begin; it < un.end; ++it) {
+      const SpreadItem item = items[it];
+      const int i = item.i0 + lane;
+      if (i >= item.i1) continue;
+      const AtomRec pi = pos[i];
+      for (int j = item.j0 + wave; j < item.j1; j += n_wave) {
+        const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
+        const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+        if (!(j < i && r2 > 0.0)) continue;
+        const double t = scaled_root(r2, inv_h);
+        if (t >= near && t < kFqFar) continue;
+        spread_rare(hist, n_grid, sqrt(r2) * inv_h, static_cast<double>(nf),
+                    static_cast<double>(scale));
+      }
+    }
+    __syncthreads();
+  }
+  unsigned long long* out = grids + static_cast<size_t>(un.grid) * stride;
+  for (int g = threadIdx.x; g < stride; g += blockDim.x) {
+    const long long v = static_cast<long long>(hist[g]);
+    if (v == 0) continue;
+    const long long s = (shift == 0 || g == n_grid + kFqNodes) ? v : (v + (1ll << (shift - 1))) >> shift;
+    atomicAdd(&out[g], static_cast<unsigned long long>(s));
+  }
+}
+
+}  // namespace
+}  // namespace pyiid

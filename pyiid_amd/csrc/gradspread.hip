@@ -28,7 +28,7 @@
 // flat_multi_cpu_wrap.py:63-102.
 #include <cmath>
 
-#include "pair_math.h"
+#include "fq_grid.h"
 
 namespace pyiid {
 namespace {
@@ -150,11 +150,11 @@ __device__ void spread_grad_rare(unsigned long long* grid, int plane, int* bad, 
 //
 // Afterwards the grids leave as split rows (hi and lo halves), each scaled so
 // that its largest entry lies in [2^14, 2^15).
-__global__ __launch_bounds__(1024, 8) void spread_grad_kernel(
-    const AtomRec* __restrict__ pos, int p0, int n_rows, const int* __restrict__ runs, double inv_h, int nf, int plane, int row_len, int k_fixed,
-    const double* __restrict__ reach, int nq, float scale, double near,
-    _Float16* __restrict__ rows, float* __restrict__ row_scale) {
-  extern __shared__ unsigned long long grid[];
+__device__ __forceinline__ void spread_grad_rows(
+    const AtomRec* __restrict__ pos, int p0, int n_rows, const int* __restrict__ runs, double inv_h,
+    int nf, int plane, int row_len, int k_fixed, const double* __restrict__ reach, int nq,
+    float scale, double near, _Float16* __restrict__ rows, float* __restrict__ row_scale,
+    unsigned long long* grid) {
   __shared__ int bad;
   __shared__ unsigned int top[3];
   const int p = p0 + blockIdx.x;
@@ -257,6 +257,34 @@ __global__ __launch_bounds__(1024, 8) void spread_grad_kernel(
   }
 }
 
+__global__ __launch_bounds__(1024, 8) void spread_grad_kernel(
+    const AtomRec* __restrict__ pos, int p0, int n_rows, const int* __restrict__ runs, double inv_h,
+    int nf, int plane, int row_len, int k_fixed, const double* __restrict__ reach, int nq,
+    float scale, double near, _Float16* __restrict__ rows, float* __restrict__ row_scale) {
+  extern __shared__ unsigned long long grid[];
+  spread_grad_rows(pos, p0, n_rows, runs, inv_h, nf, plane, row_len, k_fixed, reach, nq, scale, near,
+                   rows, row_scale, grid);
+}
+
+// The same with the work units of F(Q) as further blocks behind the atoms': for a
+// structure of a few hundred atoms a launch costs more than either part (505
+// atoms, 164 bins: six launches 22.9 us a call among others, four 18.9).
+__global__ __launch_bounds__(1024, 8) void spread_both_kernel(
+    const AtomRec* __restrict__ pos, int n_atoms, const int* __restrict__ runs, double inv_h, int nf,
+    int plane, int row_len, int k_fixed, const double* __restrict__ reach, int nq, float scale,
+    double near, _Float16* __restrict__ rows, float* __restrict__ row_scale,
+    const SpreadUnit* __restrict__ units, const SpreadItem* __restrict__ items, double fq_inv_h,
+    int fq_nf, int fq_points, int fq_stride, float fq_scale, double fq_near,
+    unsigned long long* __restrict__ grids) {
+  extern __shared__ unsigned long long grid[];
+  if (static_cast<int>(blockIdx.x) < n_atoms)
+    spread_grad_rows(pos, 0, 3 * n_atoms, runs, inv_h, nf, plane, row_len, k_fixed, reach, nq, scale,
+                     near, rows, row_scale, grid);
+  else if (blockIdx.y == 0)
+    spread_fq_unit(pos, units[blockIdx.x - n_atoms], items, fq_inv_h, fq_nf, fq_points, fq_stride, 0,
+                   fq_scale, fq_near, grid, grids);
+}
+
 // ---- the sine matrix ----
 
 // w[m][k], split like the rows, scaled by 2^14: node columns
@@ -308,10 +336,17 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(
     const double* __restrict__ reach, double inv_h, int nq, int n_ct, int n_rt, float unit,
     const double* __restrict__ gs, const float* __restrict__ ftab,
     const int* __restrict__ run_elem, const AtomRec* __restrict__ pos,
-    const int32_t* __restrict__ perm, int p0, OUT* __restrict__ out) {
+    const int32_t* __restrict__ perm, int p0, OUT* __restrict__ out, int n_tile,
+    ulonglong2* __restrict__ clear, int64_t clear2) {
   __shared__ __align__(16) unsigned char tile[2][2][128 * 128];
   __shared__ float rsc[2][128];  // the row scales of this and the next run
   const int bid = blockIdx.x;
+  if (bid >= n_tile) {  // blocks behind the tiles clear the F grids for the next call
+    for (int64_t e = static_cast<int64_t>(bid - n_tile) * 256 + threadIdx.x; e < clear2;
+         e += static_cast<int64_t>(gridDim.x - n_tile) * 256)
+      clear[e] = ulonglong2{0ull, 0ull};
+    return;
+  }
   const int rt = (bid / 8) / n_ct * 8 + bid % 8;
   const int ct = (bid / 8) % n_ct;
   if (rt >= n_rt) return;  // padding block (uniform, before any barrier)
@@ -455,24 +490,63 @@ hipError_t launch_sine_matrix(hipStream_t st, int nq, void* w, float* inv_phihat
   return hipGetLastError();
 }
 
+namespace {
+struct GradLaunch {
+  int nf, plane, row_len;
+  double inv_h, near;
+  float scale;
+  size_t lds;
+  unsigned threads;
+};
+GradLaunch grad_launch(int64_t n, int nq, double dq, double r_max) {
+  GradLaunch g;
+  g.nf = 2 * half_grid(nq);
+  g.inv_h = dq * half_grid(nq) / M_PI;
+  int s = kGMinScale;
+  while (s < kGMaxScale && std::ldexp(1.0, s - kGBits) < r_max * g.inv_h && r_max < 1e30) ++s;
+  g.scale = std::ldexp(1.0f, s);
+  g.near = 1.2 * std::ldexp(1.0, s - 31);
+  g.plane = row_points(nq) | 1;
+  g.row_len = grad_row_len(nq);
+  g.lds = grad_lds_bytes(nq);
+  g.threads = n <= 256 ? 256 : n <= 2048 ? 512 : 1024;
+  return g;
+}
+}  // namespace
+
 hipError_t launch_spread_grad(hipStream_t st, const AtomRec* pos, int p0, int n_atoms, int64_t n,
                               const int* runs, int n_run, int nq, double dq, double r_max,
                               int k_fixed, const double* reach, void* rows, float* row_scale) {
-  const int nf = 2 * half_grid(nq);
-  const double inv_h = dq * half_grid(nq) / M_PI;
-  const size_t lds = grad_lds_bytes(nq);
-  if (lds > kGradLds || n_run > 65535) return hipErrorInvalidValue;
+  const GradLaunch g = grad_launch(n, nq, dq, r_max);
+  if (g.lds > kGradLds || n_run > 65535) return hipErrorInvalidValue;
   static const hipError_t attr =
       hipFuncSetAttribute(reinterpret_cast<const void*>(spread_grad_kernel),
                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kGradLds));
   if (attr != hipSuccess) return attr;
-  int s = kGMinScale;
-  while (s < kGMaxScale && std::ldexp(1.0, s - kGBits) < r_max * inv_h && r_max < 1e30) ++s;
-  const unsigned threads = n <= 256 ? 256 : n <= 2048 ? 512 : 1024;
-  hipLaunchKernelGGL(spread_grad_kernel, dim3(n_atoms, n_run), dim3(threads), lds, st, pos, p0,
-                     3 * n_atoms, runs, inv_h, nf, row_points(nq) | 1, grad_row_len(nq), k_fixed,
-                     reach, nq, std::ldexp(1.0f, s), 1.2 * std::ldexp(1.0, s - 31),
-                     static_cast<_Float16*>(rows), row_scale);
+  hipLaunchKernelGGL(spread_grad_kernel, dim3(n_atoms, n_run), dim3(g.threads), g.lds, st, pos, p0,
+                     3 * n_atoms, runs, g.inv_h, g.nf, g.plane, g.row_len, k_fixed, reach, nq,
+                     g.scale, g.near, static_cast<_Float16*>(rows), row_scale);
+  return hipGetLastError();
+}
+
+hipError_t launch_spread_both(hipStream_t st, const AtomRec* pos, int n_atoms, const int* runs,
+                              int n_run, int nq, double dq, double r_max, int k_fixed,
+                              const double* reach, void* rows, float* row_scale,
+                              const SpreadUnit* units, int n_units, const SpreadItem* items,
+                              int scale_bits, unsigned long long* grids) {
+  const GradLaunch g = grad_launch(n_atoms, nq, dq, r_max);
+  const int fq_nf = 12 * nq, stride = fq_grid_stride(nq);
+  const size_t lds = std::max(g.lds, sizeof(unsigned long long) * static_cast<size_t>(stride));
+  if (lds > kGradLds || n_run > 65535) return hipErrorInvalidValue;
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(spread_both_kernel),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kGradLds));
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL(spread_both_kernel, dim3(n_atoms + n_units, n_run), dim3(g.threads), lds, st,
+                     pos, n_atoms, runs, g.inv_h, g.nf, g.plane, g.row_len, k_fixed, reach, nq,
+                     g.scale, g.near, static_cast<_Float16*>(rows), row_scale, units, items,
+                     dq * fq_nf / (2.0 * M_PI), fq_nf, fq_grid_points(nq), stride,
+                     std::ldexp(1.0f, scale_bits), std::ldexp(1.0, scale_bits - 31), grids);
   return hipGetLastError();
 }
 
@@ -480,18 +554,22 @@ hipError_t launch_gemm_split(hipStream_t st, const void* rows, const float* row_
                              int n_run, const void* w, const float* inv_phihat, int nq, double dq,
                              int k_fixed, const double* reach, const double* gs, const float* ftab,
                              const int* run_elem, bool weighted, const AtomRec* pos,
-                             const int32_t* perm, int p0, void* out, bool out_f64) {
+                             const int32_t* perm, int p0, void* out, bool out_f64,
+                             unsigned long long* clear, int64_t clear_words) {
   const int n_rows = 3 * n_atoms;
   const int n_ct = (nq + 127) / 128, n_rt = (n_rows + 127) / 128;
   const double inv_h = dq * half_grid(nq) / M_PI;
   const float unit = static_cast<float>(inv_h * inv_h);
-  const dim3 grid(8u * static_cast<unsigned>((n_rt + 7) / 8) * n_ct);
+  const int n_tile = 8 * ((n_rt + 7) / 8) * n_ct;
+  const int64_t clear2 = clear ? clear_words / 2 : 0;  // an even number of words
+  const dim3 grid(static_cast<unsigned>(n_tile + std::min<int64_t>((clear2 + 511) / 512, 256)));
   const int len = grad_row_len(nq);
 #define PYIID_GEMM(T, M)                                                                        \
   hipLaunchKernelGGL((gemm_split_kernel<T, M>), grid, dim3(256), 0, st,                         \
                      static_cast<const _Float16*>(rows), row_scale, n_rows, n_run,              \
                      static_cast<const _Float16*>(w), inv_phihat, len, k_fixed, reach, inv_h, nq, \
-                     n_ct, n_rt, unit, gs, ftab, run_elem, pos, perm, p0, static_cast<T*>(out))
+                     n_ct, n_rt, unit, gs, ftab, run_elem, pos, perm, p0, static_cast<T*>(out), \
+                     n_tile, reinterpret_cast<ulonglong2*>(clear), clear2)
   if (weighted) {
     if (out_f64)
       PYIID_GEMM(double, true);

@@ -137,6 +137,9 @@ hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_
                                bool weighted, const float* ftab, int nq, double dq, int shift,
                                int scale_bits, const double* scale, double* part, double* out_f64,
                                float* out_f32);
+// out[q] = scale[q] * transform of one chain's single grid, which stays as it is
+hipError_t launch_transform_one(hipStream_t st, const unsigned long long* grids, int nq, double dq,
+                                int scale_bits, const double* scale, float* out);
 // F of chains of at most kSmallAtoms atoms (off: n_chain + 1 offsets) in one
 // launch; the grid must fit kSmallFqLds.
 constexpr int kSmallAtoms = 192;
@@ -172,12 +175,21 @@ hipError_t launch_spread_grad(hipStream_t st, const AtomRec* pos, int p0, int n_
                               const int* runs, int n_run, int nq, double dq, double r_max,
                               int k_fixed, const double* reach, void* rows, float* row_scale);
 // out[perm[p]][c][m] = gs[m] f_p(m) sum_e f_e(m) sum_k rows w / phihat
-// (single element: without f).  perm null: identity.
+// (single element: without f).  perm null: identity.  clear (nullable): an even
+// number of words that blocks of the launch set to zero.
 hipError_t launch_gemm_split(hipStream_t st, const void* rows, const float* row_scale, int n_atoms,
                              int n_run, const void* w, const float* inv_phihat, int nq, double dq,
                              int k_fixed, const double* reach, const double* gs, const float* ftab,
                              const int* run_elem, bool weighted, const AtomRec* pos,
-                             const int32_t* perm, int p0, void* out, bool out_f64);
+                             const int32_t* perm, int p0, void* out, bool out_f64,
+                             unsigned long long* clear, int64_t clear_words);
+// The rows of all atoms and the F grids of launch_spread_fq's units (shift 0)
+// in one launch.
+hipError_t launch_spread_both(hipStream_t st, const AtomRec* pos, int n_atoms, const int* runs,
+                              int n_run, int nq, double dq, double r_max, int k_fixed,
+                              const double* reach, void* rows, float* row_scale,
+                              const SpreadUnit* units, int n_units, const SpreadItem* items,
+                              int scale_bits, unsigned long long* grids);
 
 // ---- contracted forces from a pair-force table (forcetab.hip) ----
 // Unit: positions [i0, i1) in `tiles` (1, 2, 4, 8 or 16) tiles of 64 against

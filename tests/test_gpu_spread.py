@@ -251,3 +251,22 @@ def test_gradient_of_positions_moved_on_the_device(ctx):
         grad_check(ctx, pos, None, 0.05, 400, per_atom=per_atom)
         ctx.set_positions(pos)
         np.testing.assert_array_equal(got, ctx.grad_fq(_lib.SLOT_FQ, 0.05, 150, 400))
+
+
+@pytest.mark.parametrize("n,nq", [(193, 512), (300, 100), (505, 164), (2048, 65), (2049, 65)])
+def test_gradient_with_f_in_its_launches(ctx, n, nq):
+    """F that rides along with a gradient equals F asked for alone, again on a
+    second call (its grids are cleared by the gradient's last launch), and both
+    match the oracle."""
+    pos = structures.jitter(structures.fcc_nearest(n), 0.05, seed=n).astype(np.float32)
+    per_atom = load(ctx, pos, np.full(n, 79), 0.1, nq)
+    alone = ctx.fq(_lib.SLOT_FQ, 0.1, nq)
+    for _ in range(2):
+        fq = np.empty(nq, np.float32)
+        g = ctx.grad_fq(_lib.SLOT_FQ, 0.1, n, nq, fq_out=fq)
+        # one transform block per 64 bins instead of several parts: FP64 rounding
+        np.testing.assert_allclose(fq, alone, rtol=3e-7, atol=1e-9)
+    rows = np.arange(0, n, 37)
+    want = oracle.grad_fq(pos, per_atom, 0.1, atom_index=rows)
+    assert np.abs(g[rows] - want).max() < 2e-6 * np.abs(want).max()
+    np.testing.assert_array_equal(ctx.fq(_lib.SLOT_FQ, 0.1, nq), alone)
