@@ -175,14 +175,16 @@ __global__ __launch_bounds__(1024, 8) void table_force_kernel(
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n_slice = (blockDim.x >> 6) / un.tiles;
-  const int tile = wave % un.tiles, slice = wave / un.tiles;
+  // (tiles and the block's waves are powers of two)
+  const int tile_bits = __ffs(un.tiles) - 1, slice_bits = __ffs(blockDim.x >> 6) - 1 - tile_bits;
+  const int n_slice = 1 << slice_bits;
+  const int tile = wave & (un.tiles - 1), slice = wave >> tile_bits;
   const int i = un.i0 + tile * 64 + lane;
   const bool have = i < un.i1;
-  const int len = un.j1 - un.j0;
+  const int64_t len = un.j1 - un.j0;
   // (wave-uniform, so that the j atoms come by scalar loads)
-  const int jb = __builtin_amdgcn_readfirstlane(un.j0 + static_cast<int>(static_cast<int64_t>(len) * slice / n_slice));
-  const int je = __builtin_amdgcn_readfirstlane(un.j0 + static_cast<int>(static_cast<int64_t>(len) * (slice + 1) / n_slice));
+  const int jb = __builtin_amdgcn_readfirstlane(un.j0 + static_cast<int>(len * slice >> slice_bits));
+  const int je = __builtin_amdgcn_readfirstlane(un.j0 + static_cast<int>(len * (slice + 1) >> slice_bits));
   const AtomRec pi = pos[have ? i : un.i0];
   const double limit = static_cast<double>(n_cell);
   double gx = 0.0, gy = 0.0, gz = 0.0;
@@ -213,9 +215,8 @@ __global__ __launch_bounds__(1024, 8) void table_force_kernel(
 #pragma unroll
       for (int e = 0; e < kAhead; ++e) {
         in[e] = t[e] < limit;  // else past the table, or r2 outside float's range
-        const double fl = floor(t[e]);
-        y[e] = static_cast<float>(t[e] - fl) - 0.5f;
-        const int cell = in[e] ? static_cast<int>(fl) : 0;
+        y[e] = static_cast<float>(__builtin_amdgcn_fract(t[e])) - 0.5f;
+        const int cell = in[e] ? static_cast<int>(t[e]) : 0;
         a[e] = l4[cell];
         b[e] = l2[cell];
       }

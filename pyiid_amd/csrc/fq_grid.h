@@ -92,10 +92,9 @@ __device__ __forceinline__ void spread_pair(unsigned long long* hist, double t, 
     t = fold(t, nf, neg);
     if (neg) w = -w;
   }
-  const double fl = floor(t);
-  const float y = static_cast<float>(t - fl) - 0.5f;
+  const float y = static_cast<float>(__builtin_amdgcn_fract(t)) - 0.5f;
   const float y2 = y * y;
-  unsigned long long* h = hist + (static_cast<int>(fl) + 1);
+  unsigned long long* h = hist + (static_cast<int>(t) + 1);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const float e = fmaf(fmaf(kFqVal[k][4], y2, kFqVal[k][2]), y2, kFqVal[k][0]);
@@ -124,16 +123,16 @@ __device__ __forceinline__ void spread_fq_unit(
     unsigned long long* hist, unsigned long long* __restrict__ grids) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n_wave = blockDim.x >> 6;
+  const int n_wave = blockDim.x >> 6, wave_bits = __ffs(n_wave) - 1;  // a power of two
   for (int g = threadIdx.x; g < stride; g += blockDim.x) hist[g] = 0ull;
   __syncthreads();
   const double half_nf = 0.5 * nf;
   bool rare = false;
   for (int it = un.begin; it < un.end; ++it) {
     const SpreadItem item = items[it];
-    const int len = item.j1 - item.j0;
-    const int jb = item.j0 + static_cast<int>(static_cast<int64_t>(len) * wave / n_wave);
-    const int je = item.j0 + static_cast<int>(static_cast<int64_t>(len) * (wave + 1) / n_wave);
+    const int64_t len = item.j1 - item.j0;
+    const int jb = item.j0 + static_cast<int>(len * wave >> wave_bits);
+    const int je = item.j0 + static_cast<int>(len * (wave + 1) >> wave_bits);
     const int i = item.i0 + lane;
     const bool have = i < item.i1;
     const AtomRec pi = pos[have ? i : item.i0];

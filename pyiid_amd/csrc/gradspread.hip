@@ -27,6 +27,7 @@
 // Reference semantics (pyIID): cpu_flat.py:117-153, cpu_experimental.py:8-15,
 // flat_multi_cpu_wrap.py:63-102.
 #include <cmath>
+#include <type_traits>
 
 #include "fq_grid.h"
 
@@ -65,6 +66,12 @@ constexpr int kGNodes = 8;
 // the F grid (2^24 units at the largest distance), at least 35; from t = 1.2
 // 2^(s - 31) on one int32 conversion serves (1.2 A at 25 1/A).
 constexpr int kGBits = 24, kGMinScale = 35, kGMaxScale = 48;
+// 32-bit entries: 2^kGNarrow, pairs from t = kGNarrowNear = 1.2 2^(kGNarrow - 31) on, and
+// structures up to kGNarrowReach grid points across (their quanta add 1e-7 / phihat there;
+// denser rows than that outgrow 31 bits in any case).  kGTap bounds |chi_k| + |phi_k| / t.
+constexpr int kGNarrow = 33;
+constexpr double kGNarrowNear = 4.8, kGNarrowReach = 2048.0;
+constexpr float kGTap[4] = {0.0047f, 0.1071f, 0.3521f, 0.3613f};
 constexpr double kGFar = 1e15;  // beyond: the second look
 
 __host__ __device__ inline double g_node(int k) {
@@ -113,8 +120,10 @@ __device__ void spread_grad_rare(unsigned long long* grid, int plane, int* bad, 
   };
   if (t < kGClose) {
     const double s = t * t;
+#pragma unroll 1
     for (int k = 0; k < kGNodes; ++k) {
       double l = scale;
+#pragma unroll 1
       for (int j = 0; j < kGNodes; ++j)
         if (j != k)
           l *= (s - g_node(j) * g_node(j)) / (g_node(k) * g_node(k) - g_node(j) * g_node(j));
@@ -128,6 +137,7 @@ __device__ void spread_grad_rare(unsigned long long* grid, int plane, int* bad, 
   const double fl = floor(u);
   const double y = u - fl - 0.5;
   const int g = kGNodes + static_cast<int>(fl) + 1;
+#pragma unroll 1
   for (int j = 0; j < kGw; ++j) {
     const int jj = j < 4 ? j : kGw - 1 - j;
     const double z = j < 4 ? y : -y;
@@ -140,39 +150,19 @@ __device__ void spread_grad_rare(unsigned long long* grid, int plane, int* bad, 
   }
 }
 
-// One block per atom and element run: the lanes of its waves take the run's
-// atoms in turn and add their 8 points to the block's three grids in LDS.
-// ds_add_u64 bounds it: 24 per 64 pairs, 115 ns per CU at random addresses,
-// against about 90 ns of VALU work on the 4 SIMDs beside it.  64-bit sums are
-// needed: entries reach far above the noise level where distant atoms add up
-// coherently, and 32 bits scaled to a safe bound would leave 1e-6 of the
-// gradient.
-//
-// Afterwards the grids leave as split rows (hi and lo halves), each scaled so
-// that its largest entry lies in [2^14, 2^15).
-__device__ __forceinline__ void spread_grad_rows(
-    const AtomRec* __restrict__ pos, int p0, int n_rows, const int* __restrict__ runs, double inv_h,
-    int nf, int plane, int row_len, int k_fixed, const double* __restrict__ reach, int nq,
-    float scale, double near, _Float16* __restrict__ rows, float* __restrict__ row_scale,
-    unsigned long long* grid) {
-  __shared__ int bad;
-  __shared__ unsigned int top[3];
-  const int p = p0 + blockIdx.x;
-  const int n_thread = blockDim.x;
-  const int k_used = points_used(reach, inv_h, k_fixed, nq);
-  const int k_end = min(k_used, plane);  // no distance reaches past k_used
-  const int run = blockIdx.y;
-  const int jb = runs[run], je = runs[run + 1];
-  for (int c = 0; c < 3; ++c)
-    for (int g = threadIdx.x; g < k_end; g += n_thread) grid[c * plane + g] = 0ull;
-  if (threadIdx.x == 0) bad = 0;
-  if (threadIdx.x < 3) top[threadIdx.x] = 0u;
-  __syncthreads();
-  const AtomRec pi = pos[p];
+// Adds every j of the run to the atom's three grids, WIDE in 64-bit entries, else
+// in 32-bit ones with a count of the pairs per cell as a fourth.  Returns
+// whether a pair is left out (rare).
+template <bool WIDE>
+__device__ __forceinline__ bool spread_grad_pairs(const AtomRec* __restrict__ pos, const AtomRec& pi,
+                                                  int jb, int je, double inv_h, double nf, float scale,
+                                                  double near, unsigned long long* grid, int plane) {
+  typedef typename std::conditional<WIDE, unsigned long long, unsigned int>::type entry_t;
+  typedef typename std::conditional<WIDE, long long, int>::type signed_t;
   const double half_nf = 0.5 * nf;
-  const float fh = static_cast<float>(inv_h);
+  const float fs = scale * static_cast<float>(inv_h);
   bool rare = false;
-  for (int j = jb + static_cast<int>(threadIdx.x); j < je; j += n_thread) {
+  for (int j = jb + static_cast<int>(threadIdx.x); j < je; j += blockDim.x) {
     const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
     if (!(r2 > 0.0)) continue;  // the atom itself, a duplicate, a NaN
@@ -182,7 +172,7 @@ __device__ __forceinline__ void spread_grad_rows(
       continue;
     }
     float it = __builtin_amdgcn_rcpf(static_cast<float>(t));
-    const float w = scale * it * it * fh;
+    const float w = fs * it * it;
     const float wx = w * static_cast<float>(dx), wy = w * static_cast<float>(dy),
                 wz = w * static_cast<float>(dz);
     if (t > half_nf) {
@@ -192,11 +182,11 @@ __device__ __forceinline__ void spread_grad_rows(
         it = -it;
       }
     }
-    const double fl = floor(t);
-    const float y = static_cast<float>(t - fl) - 0.5f;
+    const float y = static_cast<float>(__builtin_amdgcn_fract(t)) - 0.5f;
     const float y2 = y * y;
-    unsigned long long* gx = grid + kGNodes + static_cast<int>(fl) + 1;
-    unsigned long long *gy = gx + plane, *gz = gy + plane;
+    entry_t* gx = reinterpret_cast<entry_t*>(grid) + kGNodes + static_cast<int>(t) + 1;
+    entry_t *gy = gx + plane, *gz = gy + plane;
+    if (!WIDE) atomicAdd(gz + plane, static_cast<entry_t>(1));
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const float ec = fmaf(fmaf(fmaf(kChi[k][6], y2, kChi[k][4]), y2, kChi[k][2]), y2, kChi[k][0]);
@@ -206,8 +196,8 @@ __device__ __forceinline__ void spread_grad_rows(
       // point k: chi - phi / t at y; point 7 - k: -chi - phi / t at -y
       const float a = fmaf(y, fmaf(-it, op, oc), fmaf(-it, ep, ec));
       const float b = fmaf(y, fmaf(it, op, oc), -fmaf(it, ep, ec));
-      auto add = [](unsigned long long* at, float v) {
-        atomicAdd(at, static_cast<unsigned long long>(static_cast<long long>(nearest(v))));
+      auto add = [](entry_t* at, float v) {
+        atomicAdd(at, static_cast<entry_t>(static_cast<signed_t>(nearest(v))));
       };
       add(&gx[k], a * wx);
       add(&gy[k], a * wy);
@@ -217,53 +207,121 @@ __device__ __forceinline__ void spread_grad_rows(
       add(&gz[kGw - 1 - k], b * wz);
     }
   }
-  // few pairs of a physical structure, if any, are left for a second look
-  if (__syncthreads_or(rare ? 1 : 0)) {
-    for (int j = jb + static_cast<int>(threadIdx.x); j < je; j += n_thread) {
-      const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
-      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-      if (!(r2 > 0.0)) continue;
-      const double t = scaled_root(r2, inv_h);
-      if (t >= near && t < kGFar) continue;
-      const double d[3] = {dx * inv_h, dy * inv_h, dz * inv_h};
-      spread_grad_rare(grid, plane, &bad, d, sqrt(r2) * inv_h, static_cast<double>(nf),
-                       static_cast<double>(scale));
-    }
+  return rare;
+}
+
+// One block per atom and element run: the lanes of its waves take the run's
+// atoms in turn and add their 8 points to the block's three grids in LDS.
+// The LDS adds bound it: 24 per 64 pairs, at random addresses, which cost
+// twice as much as adds without bank conflicts.
+//
+// narrow: 32-bit entries of 2^kGNarrow.  A count per cell (a 25th add) bounds every
+// entry by what its cells' pairs can amount to; where that exceeds 31 bits (or a
+// pair is rare) the block starts again with 64-bit entries of `scale`.  With
+// 64-bit entries alone LDS was busy for 86% of the kernel, two thirds of that
+// bank conflicts; 32-bit ones: F and gradient of 6,699 atoms and 1,250 bins
+// 659 -> 538 us, of 20,000 atoms of two elements and 1,500 bins 6.9 -> 5.8 ms
+// (error against 64 bits 1.8e-7 -> 2.0e-7 and 2.0e-7 -> 2.5e-7 of the largest
+// entry; 5e-7 and 7e-7 with the recurrence).
+//
+// Afterwards the grids leave as split rows (hi and lo halves), each scaled so
+// that its largest entry lies in [2^14, 2^15).
+__device__ __forceinline__ void spread_grad_rows(
+    const AtomRec* __restrict__ pos, int p0, int n_rows, const int* __restrict__ runs, double inv_h,
+    int nf, int plane, int row_len, int k_fixed, const double* __restrict__ reach, int nq,
+    float scale, double near, bool narrow, _Float16* __restrict__ rows,
+    float* __restrict__ row_scale, unsigned long long* grid) {
+  __shared__ int bad;
+  __shared__ unsigned int top[3];
+  const int p = p0 + blockIdx.x;
+  const int n_thread = blockDim.x;
+  const int k_used = points_used(reach, inv_h, k_fixed, nq);
+  const int k_end = min(k_used, plane);  // no distance reaches past k_used
+  const int run = blockIdx.y;
+  const int jb = runs[run], je = runs[run + 1];
+  unsigned int* grid32 = reinterpret_cast<unsigned int*>(grid);
+  if (threadIdx.x == 0) bad = 0;
+  if (threadIdx.x < 3) top[threadIdx.x] = 0u;
+  const AtomRec pi = pos[p];
+  bool wide = !narrow;
+  if (narrow) {
+    for (int g = threadIdx.x; g < k_end; g += n_thread)
+      for (int c = 0; c < 4; ++c) grid32[c * plane + g] = 0u;
     __syncthreads();
+    bool over = spread_grad_pairs<false>(pos, pi, jb, je, inv_h, static_cast<double>(nf),
+                                         std::ldexp(1.0f, kGNarrow), kGNarrowNear, grid, plane);
+    __syncthreads();
+    const unsigned int* count = grid32 + 3 * plane;
+    for (int g = kGNodes + 1 + static_cast<int>(threadIdx.x); g < k_end; g += n_thread) {
+      float m = 0.f;
+#pragma unroll
+      for (int k = 0; k < kGw; ++k)  // tap k of the cell at g - k
+        m = fmaf(static_cast<float>(count[max(g - k, 0)]), kGTap[k < 4 ? k : kGw - 1 - k], m);
+      // (the cell at g - 7 is the nearest)
+      const int t = max(g - (kGw - 1) - kGNodes - 1, static_cast<int>(kGNarrowNear));
+      over = over || !(m < 0.2499f * static_cast<float>(t));  // entry < 2^33 m / t
+    }
+    wide = __syncthreads_or(over ? 1 : 0) != 0;
   }
+  if (wide) {
+    for (int c = 0; c < 3; ++c)
+      for (int g = threadIdx.x; g < k_end; g += n_thread) grid[c * plane + g] = 0ull;
+    __syncthreads();
+    const bool rare = spread_grad_pairs<true>(pos, pi, jb, je, inv_h, static_cast<double>(nf), scale,
+                                              near, grid, plane);
+    // few pairs of a physical structure, if any, are left for a second look
+    if (__syncthreads_or(rare ? 1 : 0)) {
+      for (int j = jb + static_cast<int>(threadIdx.x); j < je; j += n_thread) {
+        const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
+        const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+        if (!(r2 > 0.0)) continue;
+        const double t = scaled_root(r2, inv_h);
+        if (t >= near && t < kGFar) continue;
+        const double d[3] = {dx * inv_h, dy * inv_h, dz * inv_h};
+        spread_grad_rare(grid, plane, &bad, d, sqrt(r2) * inv_h, static_cast<double>(nf),
+                         static_cast<double>(scale));
+      }
+      __syncthreads();
+    }
+  }
+  auto entry = [&](int at) {
+    return wide ? static_cast<float>(static_cast<long long>(grid[at]))
+                : static_cast<float>(static_cast<int>(grid32[at]));
+  };
   // the largest entry of each row, as a non-negative float's bits
   for (int c = 0; c < 3; ++c) {
     float m = 0.f;
-    for (int k = threadIdx.x; k < k_end; k += n_thread)
-      m = fmaxf(m, fabsf(static_cast<float>(static_cast<long long>(grid[c * plane + k]))));
+    for (int k = threadIdx.x; k < k_end; k += n_thread) m = fmaxf(m, fabsf(entry(c * plane + k)));
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
     if ((threadIdx.x & 63) == 0) atomicMax(&top[c], __float_as_uint(m));
   }
   __syncthreads();
+  const float unit = wide ? 1.0f / scale : std::ldexp(1.0f, -kGNarrow);
   for (int c = 0; c < 3; ++c) {
     const size_t row = static_cast<size_t>(run) * n_rows + 3 * static_cast<size_t>(blockIdx.x) + c;
     const float m = __uint_as_float(top[c]);
     int e = 0;
     if (m > 0.f) (void)frexpf(m, &e);  // m in [2^(e-1), 2^e)
+    const float up = ldexpf(1.0f, 15 - e);
     _Float16* out = rows + row * 2 * row_len;
     for (int k = threadIdx.x; k < k_used; k += n_thread) {
-      const double v = k < k_end ? static_cast<double>(static_cast<long long>(grid[c * plane + k])) : 0.0;
-      const float x = static_cast<float>(ldexp(v, 15 - e));
+      const float x = k < k_end ? entry(c * plane + k) * up : 0.f;
       const _Float16 hi = static_cast<_Float16>(x);
       out[split_at(k)] = hi;
       out[split_at(k) + 32] = static_cast<_Float16>(x - static_cast<float>(hi));
     }
-    if (threadIdx.x == 0) row_scale[row] = bad ? __builtin_nanf("") : ldexpf(1.0f / scale, e - 15);
+    if (threadIdx.x == 0) row_scale[row] = bad ? __builtin_nanf("") : ldexpf(unit, e - 15);
   }
 }
 
 __global__ __launch_bounds__(1024, 8) void spread_grad_kernel(
     const AtomRec* __restrict__ pos, int p0, int n_rows, const int* __restrict__ runs, double inv_h,
     int nf, int plane, int row_len, int k_fixed, const double* __restrict__ reach, int nq,
-    float scale, double near, _Float16* __restrict__ rows, float* __restrict__ row_scale) {
+    float scale, double near, bool narrow, _Float16* __restrict__ rows,
+    float* __restrict__ row_scale) {
   extern __shared__ unsigned long long grid[];
   spread_grad_rows(pos, p0, n_rows, runs, inv_h, nf, plane, row_len, k_fixed, reach, nq, scale, near,
-                   rows, row_scale, grid);
+                   narrow, rows, row_scale, grid);
 }
 
 // The same with the work units of F(Q) as further blocks behind the atoms': for a
@@ -272,14 +330,14 @@ __global__ __launch_bounds__(1024, 8) void spread_grad_kernel(
 __global__ __launch_bounds__(1024, 8) void spread_both_kernel(
     const AtomRec* __restrict__ pos, int n_atoms, const int* __restrict__ runs, double inv_h, int nf,
     int plane, int row_len, int k_fixed, const double* __restrict__ reach, int nq, float scale,
-    double near, _Float16* __restrict__ rows, float* __restrict__ row_scale,
+    double near, bool narrow, _Float16* __restrict__ rows, float* __restrict__ row_scale,
     const SpreadUnit* __restrict__ units, const SpreadItem* __restrict__ items, double fq_inv_h,
     int fq_nf, int fq_points, int fq_stride, float fq_scale, double fq_near,
     unsigned long long* __restrict__ grids) {
   extern __shared__ unsigned long long grid[];
   if (static_cast<int>(blockIdx.x) < n_atoms)
     spread_grad_rows(pos, 0, 3 * n_atoms, runs, inv_h, nf, plane, row_len, k_fixed, reach, nq, scale,
-                     near, rows, row_scale, grid);
+                     near, narrow, rows, row_scale, grid);
   else if (blockIdx.y == 0)
     spread_fq_unit(pos, units[blockIdx.x - n_atoms], items, fq_inv_h, fq_nf, fq_points, fq_stride, 0,
                    fq_scale, fq_near, grid, grids);
@@ -497,6 +555,7 @@ struct GradLaunch {
   float scale;
   size_t lds;
   unsigned threads;
+  bool narrow;
 };
 GradLaunch grad_launch(int64_t n, int nq, double dq, double r_max) {
   GradLaunch g;
@@ -506,6 +565,7 @@ GradLaunch grad_launch(int64_t n, int nq, double dq, double r_max) {
   while (s < kGMaxScale && std::ldexp(1.0, s - kGBits) < r_max * g.inv_h && r_max < 1e30) ++s;
   g.scale = std::ldexp(1.0f, s);
   g.near = 1.2 * std::ldexp(1.0, s - 31);
+  g.narrow = r_max * g.inv_h <= kGNarrowReach;
   g.plane = row_points(nq) | 1;
   g.row_len = grad_row_len(nq);
   g.lds = grad_lds_bytes(nq);
@@ -525,7 +585,7 @@ hipError_t launch_spread_grad(hipStream_t st, const AtomRec* pos, int p0, int n_
   if (attr != hipSuccess) return attr;
   hipLaunchKernelGGL(spread_grad_kernel, dim3(n_atoms, n_run), dim3(g.threads), g.lds, st, pos, p0,
                      3 * n_atoms, runs, g.inv_h, g.nf, g.plane, g.row_len, k_fixed, reach, nq,
-                     g.scale, g.near, static_cast<_Float16*>(rows), row_scale);
+                     g.scale, g.near, g.narrow, static_cast<_Float16*>(rows), row_scale);
   return hipGetLastError();
 }
 
@@ -544,7 +604,7 @@ hipError_t launch_spread_both(hipStream_t st, const AtomRec* pos, int n_atoms, c
   if (attr != hipSuccess) return attr;
   hipLaunchKernelGGL(spread_both_kernel, dim3(n_atoms + n_units, n_run), dim3(g.threads), lds, st,
                      pos, n_atoms, runs, g.inv_h, g.nf, g.plane, g.row_len, k_fixed, reach, nq,
-                     g.scale, g.near, static_cast<_Float16*>(rows), row_scale, units, items,
+                     g.scale, g.near, g.narrow, static_cast<_Float16*>(rows), row_scale, units, items,
                      dq * fq_nf / (2.0 * M_PI), fq_nf, fq_grid_points(nq), stride,
                      std::ldexp(1.0f, scale_bits), std::ldexp(1.0, scale_bits - 31), grids);
   return hipGetLastError();

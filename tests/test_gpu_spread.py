@@ -270,3 +270,27 @@ def test_gradient_with_f_in_its_launches(ctx, n, nq):
     want = oracle.grad_fq(pos, per_atom, 0.1, atom_index=rows)
     assert np.abs(g[rows] - want).max() < 2e-6 * np.abs(want).max()
     np.testing.assert_array_equal(ctx.fq(_lib.SLOT_FQ, 0.1, nq), alone)
+
+
+@pytest.mark.parametrize("m", [60, 118, 119, 120, 400])
+@pytest.mark.parametrize("cap", [np.pi, 0.35])
+def test_gradient_of_a_shell(ctx, m, cap):
+    """Atoms at one distance from atom 0, all around it or on one side, where
+    their entries add up to more than 31 bits: 32-bit grids of up to about 118
+    atoms at 10 A, 64-bit ones beyond."""
+    z = 1.0 - (1.0 - np.cos(cap)) * (np.arange(m) + 0.5) / m
+    phi = np.arange(m) * np.pi * (3.0 - np.sqrt(5.0))
+    s = np.sqrt(1.0 - z * z)
+    shell = 10.0 * np.stack([s * np.cos(phi), s * np.sin(phi), z], 1)
+    pos = np.concatenate([np.zeros((1, 3)), shell]).astype(np.float32)
+    grad_check(ctx, pos, np.full(m + 1, 79), 0.1, 250)
+
+
+@pytest.mark.parametrize("r", [0.2675, 0.268, 0.2685])
+@pytest.mark.parametrize("far", [40.0, 114.2, 114.4])
+def test_gradient_choice_of_grid(ctx, r, far):
+    """A pair at the least distance of the 32-bit grids, and a structure at
+    their largest extent (4.8 and 2,048 spacings of 0.0558 A)."""
+    pos = structures.jitter(structures.fcc_nearest(50), 0.05, seed=5).astype(np.float32)
+    pos[7], pos[20], pos[30] = 0.0, (r, 0, 0), (0, 0, far)
+    grad_check(ctx, pos, np.full(50, 79), 0.1, 250)
