@@ -232,8 +232,10 @@ struct pyiid_ctx {
 
   // transform
   Buf tmat;  // float [n_r][nq]
+  Buf tsplit, tsplit_scale;  // its split operand (from kSplitBins bins on)
+  Buf gsplit, gsplit_scale;  // split gradient rows of one chunk
   int t_nr = 0, t_nq = 0;
-  bool t_set = false;
+  bool t_set = false, t_split = false;
 
   ItemSet fq_items;     // unordered pairs, ranges per chain
   SpreadSet spread;     // unordered pairs of the F(Q) spreading kernel
@@ -1597,7 +1599,7 @@ int run_spread_grad(pyiid_ctx* c, int slot, double qbin, void* out, bool out_f64
   }
   const int len = grad_row_len(nq);
   if (s.w_nq[slot] != nq) {
-    CHK(s.w[slot].reserve(sizeof(uint16_t) * 2 * static_cast<size_t>(len) * nq));
+    CHK(s.w[slot].reserve(split_bytes(nq, len)));
     CHK(s.inv_phihat[slot].reserve(sizeof(float) * nq));
     HIPCHK(launch_sine_matrix(c->stream, nq, s.w[slot].p, s.inv_phihat[slot].as<float>()));
     s.w_nq[slot] = nq;
@@ -1605,7 +1607,7 @@ int run_spread_grad(pyiid_ctx* c, int slot, double qbin, void* out, bool out_f64
   const size_t per_atom = sizeof(uint16_t) * 6 * static_cast<size_t>(len) * s.n_run;
   const int64_t chunk = std::min<int64_t>(
       c->n, std::max<int64_t>(128, static_cast<int64_t>(kGradRowBudget / per_atom) / 128 * 128));
-  CHK(s.rows.reserve(per_atom * chunk));
+  CHK(s.rows.reserve(s.n_run * split_bytes(3 * chunk, len)));
   CHK(s.row_scale.reserve(sizeof(float) * 3 * static_cast<size_t>(chunk) * s.n_run));
   const AtomRec* sp = c->pos.as<AtomRec>();
   if (weighted) {
@@ -1833,6 +1835,44 @@ int gemm_t(pyiid_ctx* c, const void* a, bool a64, int64_t rows, double* out) {
   Timed tm(c, 2);
   HIPCHK(launch_gemm_nt(c->stream, a, a64, rows, c->t_nq, c->tmat.as<float>(), c->t_nr, out,
                         nullptr));
+  return tm.done();
+}
+
+bool caller_captures(pyiid_ctx* c) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(c->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
+// Whether b can be made `want` bytes now: not in a capture of the caller's, and
+// there has to be the memory.
+bool scratch(pyiid_ctx* c, Buf& b, size_t want) {
+  if (want <= b.bytes) return true;
+  if (caller_captures(c)) return false;
+  if (b.reserve(want) == PYIID_OK) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
+// out = rows of the gradient times T^T: on split operands where they pay, in
+// chunks of 64 MB of split rows.
+constexpr size_t kSplitBudget = static_cast<size_t>(64) << 20;
+int gemm_grad(pyiid_ctx* c, const void* a, bool a64, int64_t rows, double* out) {
+  const int k = c->t_nq, n = c->t_nr, len = split_row_len(k);
+  const int64_t chunk = std::min<int64_t>(
+      (rows + 127) / 128 * 128,
+      std::max<int64_t>(1, static_cast<int64_t>(kSplitBudget / split_bytes(128, len))) * 128);
+  if (!c->t_split || rows * k < kSplitWork || !scratch(c, c->gsplit, split_bytes(chunk, len)) ||
+      !scratch(c, c->gsplit_scale, sizeof(float) * chunk))
+    return gemm_t(c, a, a64, rows, out);
+  Timed tm(c, 2);
+  for (int64_t r0 = 0; r0 < rows; r0 += chunk) {
+    const int m = static_cast<int>(std::min(chunk, rows - r0));
+    const char* part = static_cast<const char*>(a) + (a64 ? 8 : 4) * r0 * k;
+    HIPCHK(launch_split_rows(c->stream, part, a64, m, k, c->gsplit.p, c->gsplit_scale.as<float>()));
+    HIPCHK(launch_gemm_grad(c->stream, c->gsplit.p, c->gsplit_scale.as<float>(), part, a64, m, k,
+                            c->tsplit.p, c->tsplit_scale.as<float>(), c->tmat.as<float>(), n,
+                            out + r0 * n));
+  }
   return tm.done();
 }
 
@@ -2415,7 +2455,7 @@ int pyiid_destroy(pyiid_ctx* c) {
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
   destroy_graph(c->hmc);
-  for (Buf* b : {&c->posf, &c->elem, &c->pos, &c->counts_d, &c->natoms_d, &c->off_d, &c->tmat, &c->gpart,
+  for (Buf* b : {&c->posf, &c->elem, &c->pos, &c->counts_d, &c->natoms_d, &c->off_d, &c->tmat, &c->tsplit, &c->tsplit_scale, &c->gsplit, &c->gsplit_scale, &c->gpart,
                  &c->fpart, &c->fq64, &c->fq32, &c->g64, &c->io_a, &c->io_b,
                  &c->io_c, &c->w, &c->out5, &c->u, &c->ucoef, &c->upart, &c->gobs, &c->fq_items.items,
                  &c->fq_items.ranges, &c->fq_items.perm, &c->spread.units, &c->spread.items,
@@ -2841,6 +2881,14 @@ int pyiid_set_transform(pyiid_ctx* c, double rstep, double qstep, const double* 
   }
   CHK(c->tmat.reserve(sizeof(float) * tm.size()));
   HIPCHK(hipMemcpy(c->tmat.p, tm.data(), sizeof(float) * tm.size(), hipMemcpyHostToDevice));
+  c->t_split = n_q >= kSplitBins && !caller_captures(c) &&
+               scratch(c, c->tsplit, split_bytes(n_r, split_row_len(n_q))) &&
+               scratch(c, c->tsplit_scale, sizeof(float) * n_r);
+  if (c->t_split) {
+    HIPCHK(launch_split_rows(c->stream, c->tmat.p, false, n_r, n_q, c->tsplit.p,
+                             c->tsplit_scale.as<float>()));
+    HIPCHK(hipStreamSynchronize(c->stream));
+  }
   c->t_nr = n_r;
   c->t_nq = n_q;
   c->t_set = true;
@@ -2886,7 +2934,7 @@ int pyiid_grad_pdf(pyiid_ctx* c, const void* grad_fq, int64_t rows, double* grad
     CHK(c->io_c.reserve(out_bytes));
     dst = c->io_c.as<double>();
   }
-  CHK(gemm_t(c, src, a64, rows, dst));
+  CHK(gemm_grad(c, src, a64, rows, dst));
   if (!(flags & PYIID_DEVICE)) CHK(download(c, grad_gr, dst, out_bytes, flags));
   return finish(c, flags);
 }

@@ -19,10 +19,7 @@
 // of Q_max) r.m.s. over the band.  A grid of n_f = 4 n_q has 1.3e-7 for chi
 // and left the gradient 3.8e-7 off at 6,699 atoms.
 //
-// The product's operands are split into two halves, x = hi + lo, each 11
-// bits, rows scaled by a power of two of their own: hi hi + hi lo + lo hi in
-// FP32 leaves 2^-22 of an entry, at three FP16 products for one in FP32, whose
-// matrix rate is 16 times lower.
+// The product runs on split operands (split_gemm.h).
 //
 // Reference semantics (pyIID): cpu_flat.py:117-153, cpu_experimental.py:8-15,
 // flat_multi_cpu_wrap.py:63-102.
@@ -30,6 +27,7 @@
 #include <type_traits>
 
 #include "fq_grid.h"
+#include "split_gemm.h"
 
 namespace pyiid {
 namespace {
@@ -85,15 +83,6 @@ __host__ __device__ inline double g_node(int k) {
 __host__ __device__ inline int half_grid(int nq) { return (9 * nq + 3) / 4; }
 // Row length of the grids: nodes, then grid points -4 .. n_f / 2 + 4.
 __host__ __device__ inline int row_points(int nq) { return kGNodes + half_grid(nq) + 9; }
-
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-
-// Element k of a split row: 32 hi, then 32 lo, for every 32 points.
-__device__ __forceinline__ size_t split_at(int k) {
-  return static_cast<size_t>(k >> 5) * 64 + (k & 31);
-}
 
 // Points of a row in use for distances up to *reach (null: k_fixed).
 __device__ __forceinline__ int points_used(const double* reach, double inv_h, int k_fixed, int nq) {
@@ -299,16 +288,18 @@ __device__ __forceinline__ void spread_grad_rows(
   const float unit = wide ? 1.0f / scale : std::ldexp(1.0f, -kGNarrow);
   for (int c = 0; c < 3; ++c) {
     const size_t row = static_cast<size_t>(run) * n_rows + 3 * static_cast<size_t>(blockIdx.x) + c;
+    const size_t split_row = static_cast<size_t>(run) * ((n_rows + 127) / 128 * 128) +
+                             3 * static_cast<size_t>(blockIdx.x) + c;
     const float m = __uint_as_float(top[c]);
     int e = 0;
     if (m > 0.f) (void)frexpf(m, &e);  // m in [2^(e-1), 2^e)
     const float up = ldexpf(1.0f, 15 - e);
-    _Float16* out = rows + row * 2 * row_len;
     for (int k = threadIdx.x; k < k_used; k += n_thread) {
       const float x = k < k_end ? entry(c * plane + k) * up : 0.f;
       const _Float16 hi = static_cast<_Float16>(x);
-      out[split_at(k)] = hi;
-      out[split_at(k) + 32] = static_cast<_Float16>(x - static_cast<float>(hi));
+      const size_t at = split_at(split_row, k, row_len);
+      rows[at] = hi;
+      rows[at + 32] = static_cast<_Float16>(x - static_cast<float>(hi));
     }
     if (threadIdx.x == 0) row_scale[row] = bad ? __builtin_nanf("") : ldexpf(unit, e - 15);
   }
@@ -365,30 +356,19 @@ __global__ void sine_matrix_kernel(int nq, int nf, int row_len, _Float16* __rest
   }
   const float x = static_cast<float>(v * 16384.0);
   const _Float16 hi = static_cast<_Float16>(x);
-  _Float16* out = w + static_cast<size_t>(m) * 2 * row_len;
-  out[split_at(k)] = hi;
-  out[split_at(k) + 32] = static_cast<_Float16>(static_cast<float>(v * 16384.0 - static_cast<double>(hi)));
+  const size_t at = split_at(m, k, row_len);
+  w[at] = hi;
+  w[at + 32] = static_cast<_Float16>(static_cast<float>(v * 16384.0 - static_cast<double>(hi)));
   if (k == 0) inv_phihat[m] = static_cast<float>(1.0 / phihat / 16384.0);
 }
 
 // ---- rows times sine matrix ----
 
 // out[atom][c][m] = gs[m] f_i(m) / phihat(m) sum_run f_run(m) sum_k rows w.
-// Block tile 128 rows x 128 bins, 4 waves of 64 x 64 (2 x 2 MFMA 32x32x16 in
-// FP16, three products each), K in steps of 32 through double-buffered LDS.  A
-// row's 32 hi and 32 lo values of a step are one 128-byte line in memory and in
-// LDS, where its eight 16-byte chunks are permuted by the row (chunk ^ row mod
-// 8), so the eight rows read together meet different banks.  Consecutive
-// blocks of an XCD (block id mod 8) share a row tile, which stays in its L2.
-// Sums leave the MFMA accumulators every 128 points: a single FP32 chain over
-// the row rounds at the size of its running sum, and left the gradient 3.9e-7
-// off at 6,699 atoms.
-// Operand layout (lane l): A[l % 32][8 (l / 32) + i], B likewise; result
-// register v: row v % 4 + 8 (v / 4) + 4 (l / 32), column l % 32.
-constexpr int kFold = 4;  // steps of 32 points
-
-template <typename OUT, bool MULTI>
-__global__ __launch_bounds__(256, 2) void gemm_split_kernel(
+// Consecutive blocks of an XCD (block id mod 8) share a row tile, which stays in
+// its L2.
+template <int WM, int WN, int MX, int NY, typename OUT, bool MULTI>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(
     const _Float16* __restrict__ rows, const float* __restrict__ row_scale, int n_rows, int n_run,
     const _Float16* __restrict__ w, const float* __restrict__ inv_phihat, int row_len, int k_fixed,
     const double* __restrict__ reach, double inv_h, int nq, int n_ct, int n_rt, float unit,
@@ -396,140 +376,63 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(
     const int* __restrict__ run_elem, const AtomRec* __restrict__ pos,
     const int32_t* __restrict__ perm, int p0, OUT* __restrict__ out, int n_tile,
     ulonglong2* __restrict__ clear, int64_t clear2) {
-  __shared__ __align__(16) unsigned char tile[2][2][128 * 128];
-  __shared__ float rsc[2][128];  // the row scales of this and the next run
+  __shared__ __align__(16) unsigned char tile[split_lds<WM, WN, MX, NY>()];
+  __shared__ float rsc[2][32 * WM * MX];  // the row scales of this and the next run
   const int bid = blockIdx.x;
   if (bid >= n_tile) {  // blocks behind the tiles clear the F grids for the next call
-    for (int64_t e = static_cast<int64_t>(bid - n_tile) * 256 + threadIdx.x; e < clear2;
-         e += static_cast<int64_t>(gridDim.x - n_tile) * 256)
+    for (int64_t e = static_cast<int64_t>(bid - n_tile) * blockDim.x + threadIdx.x; e < clear2;
+         e += static_cast<int64_t>(gridDim.x - n_tile) * blockDim.x)
       clear[e] = ulonglong2{0ull, 0ull};
     return;
   }
   const int rt = (bid / 8) / n_ct * 8 + bid % 8;
   const int ct = (bid / 8) % n_ct;
   if (rt >= n_rt) return;  // padding block (uniform, before any barrier)
-  const int bm = rt * 128, bn = ct * 128;
+  const int bm = rt * 32 * WM * MX, bn = ct * 32 * WN * NY;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int k_used = points_used(reach, inv_h, k_fixed, nq);
-  const int nk = k_used >> 5;
-  const int steps = MULTI ? nk * n_run : nk;
-
-  // a thread moves chunk c = threadIdx.x % 8 of rows threadIdx.x / 8 + 32 s
-  const int chunk = threadIdx.x & 7, trow = threadIdx.x >> 3;
-  v4u ra[4], rb[4];
-  auto load = [&](int step) {
-    const int run = MULTI ? step / nk : 0, kk = MULTI ? step % nk : step;
-    const size_t at = static_cast<size_t>(kk) * 64 + chunk * 8;
+  const int nk = points_used(reach, inv_h, k_fixed, nq) >> 5;
+  v16f tot[MX][NY];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int r = min(bm + trow + 32 * s, n_rows - 1), q = min(bn + trow + 32 * s, nq - 1);
-      ra[s] = *reinterpret_cast<const v4u*>(
-          rows + (static_cast<size_t>(run) * n_rows + r) * 2 * row_len + at);
-      rb[s] = *reinterpret_cast<const v4u*>(w + static_cast<size_t>(q) * 2 * row_len + at);
-    }
-  };
-  auto store = [&](int buf) {
+  for (int x = 0; x < MX; ++x)
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int r = trow + 32 * s;
-      const int at = r * 128 + ((chunk ^ (r & 7)) * 16);
-      *reinterpret_cast<v4u*>(&tile[buf][0][at]) = ra[s];
-      *reinterpret_cast<v4u*>(&tile[buf][1][at]) = rb[s];
-    }
-  };
-  v16f acc[2][2], tot[2][2];
+    for (int y = 0; y < NY; ++y)
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[x][y][v] = 0.f, tot[x][y][v] = 0.f;
-  auto fragment = [&](const unsigned char* base, int r, int c) {
-    return *reinterpret_cast<const v8h*>(base + r * 128 + ((c ^ (r & 7)) * 16));
-  };
-  auto stage = [&](int run) {
-    if (threadIdx.x < 128)
+      for (int v = 0; v < 16; ++v) tot[x][y][v] = 0.f;
+  auto at_run = [&](int run) {
+    if (threadIdx.x < 32 * WM * MX)
       rsc[run & 1][threadIdx.x] = row_scale[static_cast<size_t>(run) * n_rows +
                                             min(bm + static_cast<int>(threadIdx.x), n_rows - 1)];
   };
-  auto fold = [&](int run) {  // with several elements weighted by f_run and the row scale
+  auto fold = [&](int run, const v16f (&acc)[MX][NY]) {
 #pragma unroll
-    for (int y = 0; y < 2; ++y) {
-      const int m = min(bn + wn * 64 + y * 32 + (lane & 31), nq - 1);
+    for (int y = 0; y < NY; ++y) {
+      // with several elements weighted by f_run and the row scale
+      const int m = min(bn + ((wave % WN) * NY + y) * 32 + (lane & 31), nq - 1);
       const float f = MULTI ? ftab[static_cast<size_t>(run_elem[run]) * nq + m] : 1.f;
 #pragma unroll
-      for (int x = 0; x < 2; ++x)
+      for (int x = 0; x < MX; ++x)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const int r = wm * 64 + x * 32 + (v & 3) + 8 * (v >> 2) + 4 * (lane >> 5);
+          const int r = ((wave / WN) * MX + x) * 32 + (v & 3) + 8 * (v >> 2) + 4 * (lane >> 5);
           tot[x][y][v] = MULTI ? fmaf(acc[x][y][v] * f, rsc[run & 1][r], tot[x][y][v])
                                : tot[x][y][v] + acc[x][y][v];
-          acc[x][y][v] = 0.f;
         }
     }
   };
-  load(0);
-  store(0);
-  stage(0);
-  __syncthreads();
-  for (int step = 0; step < steps; ++step) {
-    const int cur = step & 1;
-    if (step + 1 < steps) load(step + 1);
-    const unsigned char* a_s = tile[cur][0];
-    const unsigned char* b_s = tile[cur][1];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {  // 16 of the step's 32 points
-      const int c = h * 2 + (lane >> 5);
-      v8h ah[2], al[2], bh[2], bl[2];
-#pragma unroll
-      for (int x = 0; x < 2; ++x) {
-        const int r = wm * 64 + x * 32 + (lane & 31);
-        ah[x] = fragment(a_s, r, c);
-        al[x] = fragment(a_s, r, c + 4);
-        const int q = wn * 64 + x * 32 + (lane & 31);
-        bh[x] = fragment(b_s, q, c);
-        bl[x] = fragment(b_s, q, c + 4);
-      }
-#pragma unroll
-      for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y) {
-          acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[x], bh[y], acc[x][y], 0, 0, 0);
-          acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[x], bl[y], acc[x][y], 0, 0, 0);
-          acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[x], bh[y], acc[x][y], 0, 0, 0);
-        }
-    }
-    if (step + 1 < steps) store(cur ^ 1);
-    const int kk = MULTI ? step % nk : step;
-    if (kk + 1 == nk || kk % kFold == kFold - 1) {
-      const int run = MULTI ? step / nk : 0;
-      fold(run);
-      if (MULTI && kk + 1 == nk && run + 1 < n_run) stage(run + 1);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int y = 0; y < 2; ++y) {
-    const int m = bn + wn * 64 + y * 32 + (lane & 31);
-    if (m >= nq) continue;
+  split_product<WM, WN, MX, NY>(rows, n_rows, w, row_len, nk, MULTI ? n_run : 1, bm, bn, tile,
+                                        fold, at_run);
+  split_results<WM, WN, MX, NY>(tot, [&](int i, int j, float t) {
+    const int r = bm + i, m = bn + j;
+    if (r >= n_rows || m >= nq) return;
+    const int p = p0 + r / 3;
+    float g;
+    if constexpr (MULTI)
+      g = t * ftab[static_cast<size_t>(static_cast<int>(pos[p].w)) * nq + m];
+    else
+      g = t * rsc[0][i];
     const float col = static_cast<float>(gs[m] * static_cast<double>(unit)) * inv_phihat[m];
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int r = bm + wm * 64 + x * 32 + (v & 3) + 8 * (v >> 2) + 4 * (lane >> 5);
-        if (r >= n_rows) continue;
-        const int p = p0 + r / 3;
-        float g;
-        if constexpr (MULTI)
-          g = tot[x][y][v] * ftab[static_cast<size_t>(static_cast<int>(pos[p].w)) * nq + m];
-        else
-          g = tot[x][y][v] * rsc[0][r - bm];
-        const size_t o = (3 * static_cast<size_t>(perm ? perm[p] : p) + r % 3) * nq + m;
-        out[o] = static_cast<OUT>(g * col);
-      }
-  }
+    out[(3 * static_cast<size_t>(perm ? perm[p] : p) + r % 3) * nq + m] = static_cast<OUT>(g * col);
+  });
 }
 
 }  // namespace
@@ -617,19 +520,27 @@ hipError_t launch_gemm_split(hipStream_t st, const void* rows, const float* row_
                              const int32_t* perm, int p0, void* out, bool out_f64,
                              unsigned long long* clear, int64_t clear_words) {
   const int n_rows = 3 * n_atoms;
-  const int n_ct = (nq + 127) / 128, n_rt = (n_rows + 127) / 128;
   const double inv_h = dq * half_grid(nq) / M_PI;
   const float unit = static_cast<float>(inv_h * inv_h);
+  const bool large = split_large(n_rows, nq);
+  const int n_ct = large ? (nq + 127) / 128 : (nq + 63) / 64, n_rt = (n_rows + 127) / 128;
   const int n_tile = 8 * ((n_rt + 7) / 8) * n_ct;
   const int64_t clear2 = clear ? clear_words / 2 : 0;  // an even number of words
   const dim3 grid(static_cast<unsigned>(n_tile + std::min<int64_t>((clear2 + 511) / 512, 256)));
   const int len = grad_row_len(nq);
-#define PYIID_GEMM(T, M)                                                                        \
-  hipLaunchKernelGGL((gemm_split_kernel<T, M>), grid, dim3(256), 0, st,                         \
+#define PYIID_TILES(T, M, WM, WN, MX, NY)                                                       \
+  hipLaunchKernelGGL((gemm_split_kernel<WM, WN, MX, NY, T, M>), grid, dim3(64 * WM * WN), 0, st, \
                      static_cast<const _Float16*>(rows), row_scale, n_rows, n_run,              \
                      static_cast<const _Float16*>(w), inv_phihat, len, k_fixed, reach, inv_h, nq, \
                      n_ct, n_rt, unit, gs, ftab, run_elem, pos, perm, p0, static_cast<T*>(out), \
                      n_tile, reinterpret_cast<ulonglong2*>(clear), clear2)
+#define PYIID_GEMM(T, M)                 \
+  do {                                   \
+    if (large)                           \
+      PYIID_TILES(T, M, 2, 2, 2, 2);     \
+    else                                 \
+      PYIID_TILES(T, M, 4, 2, 1, 1);     \
+  } while (0)
   if (weighted) {
     if (out_f64)
       PYIID_GEMM(double, true);
@@ -642,6 +553,7 @@ hipError_t launch_gemm_split(hipStream_t st, const void* rows, const float* row_
       PYIID_GEMM(float, false);
   }
 #undef PYIID_GEMM
+#undef PYIID_TILES
   return hipGetLastError();
 }
 

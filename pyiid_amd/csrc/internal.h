@@ -165,11 +165,15 @@ constexpr size_t kGradLds = 160 * 1024 - 512;   // a block's three grids live in
 int grad_row_len(int nq);                     // points per row (a multiple of 32)
 size_t grad_lds_bytes(int nq);
 double grad_reach(int nq, double dq, double r_max);  // points of a row that r_max reaches
-// w: 2 * nq * grad_row_len(nq) halves; inv_phihat: nq floats
+// bytes of a split operand: tiles of 128 rows, two halves for every point
+inline size_t split_bytes(int64_t rows, int row_len) {
+  return static_cast<size_t>((rows + 127) / 128) * 128 * row_len * 4;
+}
+// w: split_bytes(nq, grad_row_len(nq)); inv_phihat: nq floats
 hipError_t launch_sine_matrix(hipStream_t st, int nq, void* w, float* inv_phihat);
 // Grids of positions [p0, p0 + n_atoms) against each of the n_run element
-// runs [runs[e], runs[e + 1]): rows (e * 3 n_atoms + 3 (p - p0) + c), 2 *
-// grad_row_len halves each, and row_scale.  Points used: k_fixed, or those that
+// runs [runs[e], runs[e + 1]): rows 3 (p - p0) + c of a split operand for each e,
+// and row_scale (e * 3 n_atoms + 3 (p - p0) + c).  Points used: k_fixed, or those that
 // distances up to *reach need.
 hipError_t launch_spread_grad(hipStream_t st, const AtomRec* pos, int p0, int n_atoms, int64_t n,
                               const int* runs, int n_run, int nq, double dq, double r_max,
@@ -223,6 +227,20 @@ hipError_t launch_reduce_force(hipStream_t st, const double* part, int64_t n,
 // C[m][ldc] = A[m][K] . B[n][K]^T in FP32 MFMA; A float or double.
 hipError_t launch_gemm_nt(hipStream_t st, const void* a, bool a_f64, int64_t m, int k,
                           const float* b, int n, double* c_f64, float* c_f32);
+// The same for rows of the gradient, on split operands (split_bytes(rows,
+// split_row_len(k)) and a scale per row) of both factors; a: the rows themselves,
+// t: T.  From kSplitBins bins and kSplitWork entries on, where the split's
+// launch is worth it (us, 4,000 points, against launch_gemm_nt: 96 rows of 330 bins
+// 25 and 29, 129 of 330 22 and 29, 192 of 128 14 and 12, 258 of 128 14 and 14, 960 of
+// 330 24 and 66).
+constexpr int kSplitBins = 128;
+constexpr int64_t kSplitWork = 32768;
+inline int split_row_len(int k) { return (k + 31) / 32 * 32; }
+hipError_t launch_split_rows(hipStream_t st, const void* a, bool a_f64, int64_t m, int k, void* rows,
+                             float* scale);
+hipError_t launch_gemm_grad(hipStream_t st, const void* rows, const float* row_scale, const void* a,
+                            bool a_f64, int m, int k, const void* ts, const float* t_scale,
+                            const float* t, int n, double* out);
 // Per chain b (one block each): potential value/scale and the adjoint
 // w[b][t] (FP64).  out5[b] = {value, scale, a_opt, res.res, g.res}.
 hipError_t launch_potential(hipStream_t st, int potential, const double* gobs,

@@ -4,9 +4,11 @@
 // The reference transform (kernels/master_kernel.py:39-203) is an odd-extended
 // zero-padded inverse FFT followed by linear interpolation onto the r grid;
 // it is exactly G = T . F with a dense R x Q matrix T (built on the host in
-// FP64, stored here as FP32).  grad G = grad F . T^T is the only dense
-// contraction of the path and runs on v_mfma_f32_16x16x4_f32.
-#include "internal.h"
+// FP64, stored here as FP32).  grad G = grad F . T^T runs on split operands
+// (split_gemm.h), smaller products on v_mfma_f32_16x16x4_f32.
+#include <cmath>
+
+#include "split_gemm.h"
 
 namespace pyiid {
 namespace {
@@ -71,7 +73,78 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const void* __restrict__
   }
 }
 
-// The same product for tall A (the gradient rows): block tile 128 x 128,
+// The same product for more rows: block tile 64 x 64, 4 waves of 32 x 32,
+// each wave 2 x 2 MFMA 16x16x4 tiles; K staged through LDS 16 at a time.
+// MFMA f32 16x16x4 operand layout (lane l): A[l%16][l/16], B[l/16][l%16];
+// result register v holds C[4*(l/16)+v][l%16].
+template <bool A64>
+__global__ __launch_bounds__(256) void gemm_nt_kernel(const void* __restrict__ a_raw, int64_t m,
+                                                      int k, const float* __restrict__ b, int n,
+                                                      double* __restrict__ c64,
+                                                      float* __restrict__ c32) {
+  constexpr int KS = 16;
+  __shared__ float as[64][KS + 1];
+  __shared__ float bs[64][KS + 1];
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int64_t bm = static_cast<int64_t>(blockIdx.y) * 64;
+  const int bn = blockIdx.x * 64;
+  v4f acc[2][2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) acc[x][y] = v4f{0.f, 0.f, 0.f, 0.f};
+
+  for (int k0 = 0; k0 < k; k0 += KS) {
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int idx = threadIdx.x + e * 256;
+      const int row = idx / KS, kk = idx % KS;
+      const int64_t ar = bm + row;
+      float av = 0.0f;
+      if (ar < m && k0 + kk < k) {
+        if constexpr (A64)
+          av = static_cast<float>(static_cast<const double*>(a_raw)[ar * k + k0 + kk]);
+        else
+          av = static_cast<const float*>(a_raw)[ar * k + k0 + kk];
+      }
+      as[row][kk] = av;
+      const int br = bn + row;
+      bs[row][kk] = (br < n && k0 + kk < k) ? b[(int64_t)br * k + k0 + kk] : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < KS; kk += 4) {
+      float af[2], bf[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) af[x] = as[wm * 32 + x * 16 + (lane & 15)][kk + (lane >> 4)];
+#pragma unroll
+      for (int y = 0; y < 2; ++y) bf[y] = bs[wn * 32 + y * 16 + (lane & 15)][kk + (lane >> 4)];
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+          acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[x], bf[y], acc[x][y], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int64_t row = bm + wm * 32 + x * 16 + 4 * (lane >> 4) + v;
+        const int col = bn + wn * 32 + y * 16 + (lane & 15);
+        if (row < m && col < n) {
+          if (c64) c64[row * n + col] = static_cast<double>(acc[x][y][v]);
+          if (c32) c32[row * n + col] = acc[x][y][v];
+        }
+      }
+}
+
+// The same product for tall A: block tile 128 x 128,
 // 4 waves of 64 x 64 (4 x 4 MFMA 16x16x4 tiles), K in chunks of 16 through
 // double-buffered LDS; the next chunk's global loads are in flight during the
 // current chunk's MFMAs, one barrier per chunk.  Blocks are dispatched round
@@ -175,6 +248,104 @@ __global__ __launch_bounds__(256) void gemm_nt128_kernel(const void* __restrict_
           if (c32) c32[row * n + col] = acc[x][y][v];
         }
       }
+}
+
+// ---- the gradient's transform on split operands ----
+
+// Rows of a (m x k) as a split operand, each scaled so that its largest entry
+// lies in [2^14, 2^15); scale gives the way back, or NaN for a row with an entry
+// that is not finite or a largest one outside [1e-20, 1e20].  A wave per row.
+template <bool A64>
+__global__ __launch_bounds__(256) void split_rows_kernel(const void* __restrict__ a_raw, int64_t m,
+                                                         int k, int row_len,
+                                                         _Float16* __restrict__ rows,
+                                                         float* __restrict__ scale) {
+  const int lane = threadIdx.x & 63;
+  const int64_t r = blockIdx.x * 4ll + (threadIdx.x >> 6);
+  if (r >= m) return;
+  auto at = [&](int i) {
+    if constexpr (A64)
+      return static_cast<float>(static_cast<const double*>(a_raw)[r * k + i]);
+    else
+      return static_cast<const float*>(a_raw)[r * k + i];
+  };
+  float top = 0.f;
+  bool bad = false;
+  for (int i = lane; i < k; i += 64) {
+    const float v = fabsf(at(i));
+    bad = bad || !(v <= 1e20f);
+    top = fmaxf(top, v);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off, 64));
+  bad = __any(bad || (top > 0.f && top < 1e-20f));
+  int e = 0;
+  if (top > 0.f && !bad) (void)frexpf(top, &e);  // top in [2^(e-1), 2^e)
+  const float up = ldexpf(1.0f, 15 - e);
+  for (int i = lane; i < row_len; i += 64) {
+    const float x = i < k && !bad ? at(i) * up : 0.f;
+    const _Float16 hi = static_cast<_Float16>(x);
+    const size_t o = split_at(r, i, row_len);
+    rows[o] = hi;
+    rows[o + 32] = static_cast<_Float16>(x - static_cast<float>(hi));
+  }
+  if (lane == 0) scale[r] = bad ? __builtin_nanf("") : ldexpf(1.0f, e - 15);
+}
+
+// c[r][t] = sum_q a[r][q] T[t][q] for the rows [r0, r0 + m) that split_rows_kernel
+// made, against T split alike.  Rows it could not scale are summed as they are.
+// 3,867 rows of 330 bins to 4,000 points (31 GFLOP in FP16, 124 MB of results):
+// 65 us with the rows' split, against 136 us on the FP32 matrix cores, which
+// reached 75 TFLOP/s of their 157.
+template <int WM, int WN, int MX, int NY, bool A64>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_grad_kernel(
+    const _Float16* __restrict__ rows, const float* __restrict__ row_scale, int m,
+    const _Float16* __restrict__ ts, const float* __restrict__ t_scale, int n, int row_len,
+    const void* __restrict__ a_raw, const float* __restrict__ t, int k, int n_ct, int n_rt,
+    double* __restrict__ c64) {
+  __shared__ __align__(16) unsigned char tile[split_lds<WM, WN, MX, NY>()];
+  __shared__ float rs[32 * WM * MX], cs[32 * WN * NY];
+  // consecutive blocks of an XCD (block id mod 8) share a row tile
+  const int rt = static_cast<int>(blockIdx.x / 8) / n_ct * 8 + static_cast<int>(blockIdx.x % 8);
+  const int ct = static_cast<int>(blockIdx.x / 8) % n_ct;
+  if (rt >= n_rt) return;  // padding block (uniform, before any barrier)
+  const int bm = rt * 32 * WM * MX, bn = ct * 32 * WN * NY;
+  v16f tot[MX][NY];
+#pragma unroll
+  for (int x = 0; x < MX; ++x)
+#pragma unroll
+    for (int y = 0; y < NY; ++y)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) tot[x][y][v] = 0.f;
+  auto at_run = [&](int) {
+    const int i = threadIdx.x;
+    if (i < 32 * WM * MX) rs[i] = row_scale[min(bm + i, m - 1)];
+    if (i < 32 * WN * NY) cs[i] = t_scale[min(bn + i, n - 1)];
+  };
+  auto fold = [&](int, const v16f (&acc)[MX][NY]) {
+#pragma unroll
+    for (int x = 0; x < MX; ++x)
+#pragma unroll
+      for (int y = 0; y < NY; ++y)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) tot[x][y][v] += acc[x][y][v];
+  };
+  split_product<WM, WN, MX, NY>(rows, m, ts, row_len, row_len >> 5, 1, bm, bn, tile, fold, at_run);
+  split_results<WM, WN, MX, NY>(tot, [&](int i, int j, float v) {
+    const int r = bm + i, col = bn + j;
+    if (r >= m || col >= n) return;
+    float g = v * rs[i] * cs[j];
+    if (rs[i] != rs[i] || cs[j] != cs[j]) {
+      g = 0.f;
+      for (int q = 0; q < k; ++q) {
+        const size_t at = static_cast<size_t>(r) * k + q;
+        const float av = A64 ? static_cast<float>(static_cast<const double*>(a_raw)[at])
+                             : static_cast<const float*>(a_raw)[at];
+        g = fmaf(av, t[static_cast<size_t>(col) * k + q], g);
+      }
+    }
+    c64[static_cast<size_t>(r) * n + col] = static_cast<double>(g);
+  });
 }
 
 // The block's sums of three values, in every thread (one pass through LDS).
@@ -428,11 +599,61 @@ hipError_t launch_gemm_nt(hipStream_t st, const void* a, bool a_f64, int64_t m, 
     return hipGetLastError();
   }
   if (m < 1) return hipSuccess;
-  dim3 grid((n + 15) / 16, static_cast<unsigned>((m + 15) / 16));
+  // few rows: many short blocks (66 rows of 330 bins to 4,000 points: 20 us, 29 in
+  // 64 x 64 tiles); from 81 on the tiles read less (96 rows of 128 bins: 12 us, 14
+  // in 16 x 16 tiles; 960 rows: 26, 110)
+  if (m <= 80) {
+    const dim3 grid((n + 15) / 16, static_cast<unsigned>((m + 15) / 16));
+    if (a_f64)
+      hipLaunchKernelGGL(gemm_rows_kernel<true>, grid, dim3(256), 0, st, a, m, k, b, n, c_f64, c_f32);
+    else
+      hipLaunchKernelGGL(gemm_rows_kernel<false>, grid, dim3(256), 0, st, a, m, k, b, n, c_f64, c_f32);
+    return hipGetLastError();
+  }
+  const dim3 grid((n + 63) / 64, static_cast<unsigned>((m + 63) / 64));
   if (a_f64)
-    hipLaunchKernelGGL(gemm_rows_kernel<true>, grid, dim3(256), 0, st, a, m, k, b, n, c_f64, c_f32);
+    hipLaunchKernelGGL(gemm_nt_kernel<true>, grid, dim3(256), 0, st, a, m, k, b, n, c_f64, c_f32);
   else
-    hipLaunchKernelGGL(gemm_rows_kernel<false>, grid, dim3(256), 0, st, a, m, k, b, n, c_f64, c_f32);
+    hipLaunchKernelGGL(gemm_nt_kernel<false>, grid, dim3(256), 0, st, a, m, k, b, n, c_f64, c_f32);
+  return hipGetLastError();
+}
+
+hipError_t launch_split_rows(hipStream_t st, const void* a, bool a_f64, int64_t m, int k, void* rows,
+                             float* scale) {
+  if (m < 1) return hipSuccess;
+  const dim3 grid(static_cast<unsigned>((m + 3) / 4));
+  const int len = split_row_len(k);
+  if (a_f64)
+    hipLaunchKernelGGL(split_rows_kernel<true>, grid, dim3(256), 0, st, a, m, k, len,
+                       static_cast<_Float16*>(rows), scale);
+  else
+    hipLaunchKernelGGL(split_rows_kernel<false>, grid, dim3(256), 0, st, a, m, k, len,
+                       static_cast<_Float16*>(rows), scale);
+  return hipGetLastError();
+}
+
+hipError_t launch_gemm_grad(hipStream_t st, const void* rows, const float* row_scale, const void* a,
+                            bool a_f64, int m, int k, const void* ts, const float* t_scale,
+                            const float* t, int n, double* out) {
+  const bool large = split_large(m, n);
+  const int n_ct = large ? (n + 127) / 128 : (n + 63) / 64, n_rt = (m + 127) / 128;
+  const int64_t blocks = 8ll * ((n_rt + 7) / 8) * n_ct;
+  if (blocks > 2147483647LL) return hipErrorInvalidValue;
+  const dim3 grid(static_cast<unsigned>(blocks));
+#define PYIID_TILES(A64, WM, WN, MX, NY)                                                          \
+  hipLaunchKernelGGL((gemm_grad_kernel<WM, WN, MX, NY, A64>), grid, dim3(64 * WM * WN), 0, st,    \
+                     static_cast<const _Float16*>(rows), row_scale, m,                            \
+                     static_cast<const _Float16*>(ts), t_scale, n, split_row_len(k), a, t, k,     \
+                     n_ct, n_rt, out)
+  if (large && a_f64)
+    PYIID_TILES(true, 2, 2, 2, 2);
+  else if (large)
+    PYIID_TILES(false, 2, 2, 2, 2);
+  else if (a_f64)
+    PYIID_TILES(true, 4, 2, 1, 1);
+  else
+    PYIID_TILES(false, 4, 2, 1, 1);
+#undef PYIID_TILES
   return hipGetLastError();
 }
 

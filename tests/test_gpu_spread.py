@@ -294,3 +294,44 @@ def test_gradient_choice_of_grid(ctx, r, far):
     pos = structures.jitter(structures.fcc_nearest(50), 0.05, seed=5).astype(np.float32)
     pos[7], pos[20], pos[30] = 0.0, (r, 0, 0), (0, 0, far)
     grad_check(ctx, pos, np.full(50, 79), 0.1, 250)
+
+
+@pytest.mark.parametrize("n,nq,n_r", [(86, 128, 4000), (86, 129, 63), (100, 330, 1001), (343, 160, 2001),
+                                      (700, 200, 3969), (701, 130, 4001)])
+@pytest.mark.parametrize("f64", [False, True])
+def test_gradient_transform_on_split_operands(ctx, n, nq, n_r, f64):
+    """Tiles of 128 x 64 and (from 700 atoms here) 128 x 128 against the FP64
+    product, with rows of zeros, of far magnitudes and with an infinity or a
+    NaN.  Each operand is left 2^-22 of itself off by its split and by the
+    product of the low halves; 2^-20 of the sum of magnitudes covers the three
+    and the FP32 sums."""
+    dq = 0.05
+    r = 0.01 * np.arange(n_r)
+    ctx.set_transform(0.01, dq, r, 0.0, nq)
+    eye = np.zeros((66, 3, nq), np.float32)  # too few entries for the split
+    t = np.empty((n_r, nq))
+    for m0 in range(0, nq, 66):
+        m1 = min(m0 + 66, nq)
+        eye[:] = 0.0
+        eye[np.arange(m1 - m0), 0, np.arange(m0, m1)] = 1.0
+        for m in range(m0, m1, 22):
+            k = min(22, m1 - m)
+            t[:, m:m + k] = ctx.grad_pdf(eye[m - m0:m - m0 + k], n_r)[:, 0].T
+    rs = np.random.RandomState(n + nq)
+    a = rs.standard_normal((n, 3, nq)).astype(np.float32)
+    a *= np.exp(rs.uniform(-8, 8, (n, 3, 1))).astype(np.float32)
+    a[0, 0], a[1, 1], a[2, 2] = 0.0, a[1, 1] * np.float32(1e25), a[2, 2] * np.float32(1e-25)
+    a[3, 0, 5], a[4, 1, nq - 1] = np.inf, np.nan
+    got = ctx.grad_pdf(a.astype(np.float64) if f64 else a, n_r)
+    x = a.astype(np.float64).reshape(-1, nq)
+    ok = np.isfinite(x).all(1)
+    want = x[ok] @ t.T
+    allowed = 2.0 ** -20 * (np.abs(x[ok]) @ np.abs(t).T) + 2.0 ** -30 * (
+        np.abs(x[ok]).max(1, keepdims=True) * np.abs(t).sum(1)) + 1e-38
+    off = np.abs(got.reshape(-1, n_r)[ok] - want) / allowed
+    assert off.max() < 1.0, off.max()
+    with np.errstate(invalid="ignore"):
+        bad = x[~ok] @ t.T
+    assert np.isnan(got[4, 1]).all()
+    np.testing.assert_array_equal(np.isnan(got[3, 0]), np.isnan(bad[0]))
+    np.testing.assert_array_equal(np.isposinf(got[3, 0]), np.isposinf(bad[0]))
