@@ -13,10 +13,11 @@
 //     its cell's six coefficients from LDS and adds P (q_i - q_j) to atom i.
 //
 // A recurrence per pair and bin took 5.8 VALU instructions for each; the table
-// takes about 30 instructions per ordered pair, whatever the number of bins.
+// takes 34 instructions per ordered pair, whatever the number of bins.
 //
 // Reference semantics (pyIID): calc_1d.py:78-95 through cpu_flat.py:117-153.
 #include <cmath>
+#include <type_traits>
 
 #include "pair_math.h"
 
@@ -51,23 +52,25 @@ NodeFit node_fit() {
 constexpr int kTabSplit = 2;     // halves of a chunk of bins, side by side in a block
 constexpr int kTabChunk = 1024;  // bins staged in LDS at a time
 
-// Block: 64 / PARTS cells x 6 nodes x 2 halves of every chunk of bins of one
-// table (chain, element pair); a wave holds PARTS parts of its half side by
-// side.  sin and cos of Q r follow the FP64 three-term recurrence along Q from
-// the part's first bin.  Tables of 64 chains are bound by their FP64 operations
-// (PARTS = 1: the two starting phases of a chain of 165 bins are a few percent);
-// a single table of 400 cells by the chain's length (PARTS = 4).
-template <int PARTS>
-__global__ __launch_bounds__(64 * kNodes * kTabSplit) void force_table_kernel(
+// Block: CELLS cells x 6 nodes x 2 halves of every chunk of bins of one table
+// (chain, element pair); a wave holds the cells of 64 / CELLS nodes, or PARTS parts
+// of its half side by side.  sin and cos of Q r follow the FP64 three-term
+// recurrence along Q from the part's first bin.  Tables of 64 chains are bound by
+// their FP64 operations (PARTS = 1: the two starting phases of a chain of 165 bins
+// are a few percent); a single table of 400 cells by the chain's length (PARTS = 4).
+template <int CELLS, int PARTS>
+__global__ __launch_bounds__(64 * kNodes * kTabSplit * CELLS * PARTS / 64) void force_table_kernel(
     const double2* __restrict__ coef, int nq, double dq, int n_cell, double h, NodeFit fit,
     float4* __restrict__ t4, float2* __restrict__ t2) {
-  constexpr int kCells = 64 / PARTS;
+  constexpr int kNodesPer = 64 / (CELLS * PARTS);  // of a wave
+  constexpr int kWaves = kNodes / kNodesPer;       // of a half
   __shared__ double2 cf[kTabChunk];
-  __shared__ double val[kTabSplit][2][kNodes][64];
+  __shared__ double val[kTabSplit][2][kNodes][CELLS * PARTS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int node = wave % kNodes, half = wave / kNodes;
-  const int cell = blockIdx.x * kCells + lane % kCells;
-  const int sub = half * PARTS + lane / kCells;
+  const int in_cell = lane % CELLS, part = lane / CELLS % PARTS;
+  const int node = wave % kWaves * kNodesPer + lane / (CELLS * PARTS), half = wave / kWaves;
+  const int cell = blockIdx.x * CELLS + in_cell;
+  const int sub = half * PARTS + part;
   const size_t table = blockIdx.y;
   const double x = dq * ((cell + 0.5 + fit.y[node]) * h) / M_PI;  // phase per bin / pi
   double s1, c1;
@@ -79,8 +82,8 @@ __global__ __launch_bounds__(64 * kNodes * kTabSplit) void force_table_kernel(
     if (m0 > 0) __syncthreads();
     for (int m = threadIdx.x; m < cnt; m += blockDim.x) cf[m] = coef[table * nq + m0 + m];
     const int lo = cnt * sub / (kTabSplit * PARTS), hi = cnt * (sub + 1) / (kTabSplit * PARTS);
-    double s, c;
-    sincospi(x * (m0 + lo), &s, &c);
+    double s = 0.0, c = 1.0;
+    if (m0 + lo > 0) sincospi(x * (m0 + lo), &s, &c);
     double sp = s * c1 - c * s1, cp = c * c1 + s * s1;  // one bin before
     __syncthreads();
 #pragma unroll 8
@@ -95,10 +98,10 @@ __global__ __launch_bounds__(64 * kNodes * kTabSplit) void force_table_kernel(
       c = cn;
     }
   }
-  val[half][0][node][lane] = a;
-  val[half][1][node][lane] = b;
+  val[half][0][node][part * CELLS + in_cell] = a;
+  val[half][1][node][part * CELLS + in_cell] = b;
   __syncthreads();
-  if (cell >= n_cell || half != 0 || lane >= kCells) return;
+  if (cell >= n_cell || half != 0 || part != 0) return;
   double p = 0.0;
 #pragma unroll
   for (int n = 0; n < kNodes; ++n) {
@@ -106,13 +109,13 @@ __global__ __launch_bounds__(64 * kNodes * kTabSplit) void force_table_kernel(
     double an = 0.0, bn = 0.0;
 #pragma unroll
     for (int k = 0; k < PARTS; ++k) {
-      an += val[0][0][n][k * kCells + lane] + val[1][0][n][k * kCells + lane];
-      bn += val[0][1][n][k * kCells + lane] + val[1][1][n][k * kCells + lane];
+      an += val[0][0][n][k * CELLS + in_cell] + val[1][0][n][k * CELLS + in_cell];
+      bn += val[0][1][n][k * CELLS + in_cell] + val[1][1][n][k * CELLS + in_cell];
     }
     p = fma(fit.c[node][n], (an - bn * inv) * (inv * inv), p);
   }
   const size_t at = table * n_cell + cell;
-  // wave k holds coefficient k: 0..3 in t4, 4 and 5 in t2
+  // node k holds coefficient k: 0..3 in t4, 4 and 5 in t2
   if (node < 4)
     reinterpret_cast<float*>(t4 + at)[node] = static_cast<float>(p);
   else
@@ -141,7 +144,8 @@ __device__ double pair_force_far(double r, const float* u, const float* fi,
   return (a - b / r) / (r * r);
 }
 
-constexpr int kAhead = 2;
+constexpr int kAhead = 3;
+constexpr double kLeast = 1e-30;  // r^2 of an atom and itself: within float's range
 
 // Block (16 waves): the unit's 64-position i tiles against its j range, its
 // table in LDS.  Wave w takes tile w mod tiles and slice w / tiles of the
@@ -149,8 +153,11 @@ constexpr int kAhead = 2;
 // its atom: FP32 sums over 64 j atoms, FP64 across them, then across slices
 // through LDS and across planes in reduce_force_kernel, in a fixed order.
 //
-// Per 64 ordered pairs: 11 FP64 and 8 conversion or transcendental
-// instructions, 8 FMAs, and one ds_read_b128 + ds_read_b64 gather.  Forming
+// VALU issue bounds it: 34 instructions for 64 ordered pairs, 11 of them FP64 and 8
+// conversions or roots, and one ds_read_b128 + ds_read_b64 gather.  The range check
+// is on r^2, no check singles out the atom itself, and three pairs side by side
+// in one basic block cover each other's latency: 64 chains of 5,000 atoms 1.64 ->
+// 1.44 ms (two pairs 1.49, four, which spill, 1.70).  Forming
 // every pair from both sides keeps the accumulators in registers: the
 // exchange of unordered pairs between lanes would cost about as much as the
 // distance saved.
@@ -186,51 +193,54 @@ __global__ __launch_bounds__(1024, 8) void table_force_kernel(
   const int jb = __builtin_amdgcn_readfirstlane(un.j0 + static_cast<int>(len * slice >> slice_bits));
   const int je = __builtin_amdgcn_readfirstlane(un.j0 + static_cast<int>(len * (slice + 1) >> slice_bits));
   const AtomRec pi = pos[have ? i : un.i0];
-  const double limit = static_cast<double>(n_cell);
+  // r^2 up to which a pair takes the table (half a cell short of its end, so that
+  // rounding cannot lead past it)
+  const double limit = (n_cell - 0.5) / inv_h * ((n_cell - 0.5) / inv_h);
   double gx = 0.0, gy = 0.0, gz = 0.0;
   bool far = false;
+  float fx, fy, fz;
+  auto pairs = [&](int j, auto count) {  // j .. side by side: loads and chains overlap
+    constexpr int kN = decltype(count)::value;
+    double dx[kN], dy[kN], dz[kN], r2[kN], t[kN];
+    float y[kN], p[kN];
+    float4 a[kN];
+    float2 b[kN];
+#pragma unroll
+    for (int e = 0; e < kN; ++e) {
+      dx[e] = pi.x - pos[j + e].x;
+      dy[e] = pi.y - pos[j + e].y;
+      dz[e] = pi.z - pos[j + e].z;
+    }
+#pragma unroll
+    for (int e = 0; e < kN; ++e) {
+      // (the atom itself and duplicates: a finite P times a zero difference)
+      r2[e] = fma(dx[e], dx[e], fma(dy[e], dy[e], fma(dz[e], dz[e], kLeast)));
+      t[e] = scaled_root(r2[e], inv_h);
+    }
+#pragma unroll
+    for (int e = 0; e < kN; ++e) {
+      y[e] = static_cast<float>(__builtin_amdgcn_fract(t[e])) - 0.5f;
+      const int cell = r2[e] < limit ? static_cast<int>(t[e]) : 0;
+      a[e] = l4[cell];
+      b[e] = l2[cell];
+    }
+#pragma unroll
+    for (int e = 0; e < kN; ++e) {
+      p[e] = fmaf(fmaf(fmaf(fmaf(fmaf(b[e].y, y[e], b[e].x), y[e], a[e].w), y[e], a[e].z), y[e],
+                       a[e].y), y[e], a[e].x);
+      far = far || r2[e] >= limit;
+      p[e] = r2[e] < limit ? p[e] : 0.f;
+      fx = fmaf(p[e], static_cast<float>(dx[e]), fx);
+      fy = fmaf(p[e], static_cast<float>(dy[e]), fy);
+      fz = fmaf(p[e], static_cast<float>(dz[e]), fz);
+    }
+  };
   for (int j0 = jb; j0 < je; j0 += 64) {
     const int j1 = min(je, j0 + 64);
-    float fx = 0.f, fy = 0.f, fz = 0.f;
-    for (int j = j0; j < j1; j += kAhead) {
-      // kAhead pairs side by side, so that their loads and chains overlap
-      double dx[kAhead], dy[kAhead], dz[kAhead], t[kAhead];
-      bool keep[kAhead], in[kAhead];
-      float y[kAhead], p[kAhead];
-      float4 a[kAhead];
-      float2 b[kAhead];
-#pragma unroll
-      for (int e = 0; e < kAhead; ++e) {
-        const AtomRec* pj = pos + min(j + e, j1 - 1);
-        dx[e] = pi.x - pj->x;
-        dy[e] = pi.y - pj->y;
-        dz[e] = pi.z - pj->z;
-      }
-#pragma unroll
-      for (int e = 0; e < kAhead; ++e) {
-        const double r2 = fma(dx[e], dx[e], fma(dy[e], dy[e], dz[e] * dz[e]));
-        keep[e] = r2 > 0.0 && j + e < j1;  // not the atom itself, a duplicate, a NaN
-        t[e] = scaled_root(r2, inv_h);
-      }
-#pragma unroll
-      for (int e = 0; e < kAhead; ++e) {
-        in[e] = t[e] < limit;  // else past the table, or r2 outside float's range
-        y[e] = static_cast<float>(__builtin_amdgcn_fract(t[e])) - 0.5f;
-        const int cell = in[e] ? static_cast<int>(t[e]) : 0;
-        a[e] = l4[cell];
-        b[e] = l2[cell];
-      }
-#pragma unroll
-      for (int e = 0; e < kAhead; ++e) {
-        far = far || (keep[e] && !in[e]);
-        p[e] = fmaf(fmaf(fmaf(fmaf(fmaf(b[e].y, y[e], b[e].x), y[e], a[e].w), y[e], a[e].z), y[e],
-                         a[e].y), y[e], a[e].x);
-        p[e] = keep[e] && in[e] ? p[e] : 0.f;
-        fx = fmaf(p[e], static_cast<float>(dx[e]), fx);
-        fy = fmaf(p[e], static_cast<float>(dy[e]), fy);
-        fz = fmaf(p[e], static_cast<float>(dz[e]), fz);
-      }
-    }
+    fx = fy = fz = 0.f;
+    int j = j0;
+    for (; j + kAhead <= j1; j += kAhead) pairs(j, std::integral_constant<int, kAhead>());
+    for (; j < j1; ++j) pairs(j, std::integral_constant<int, 1>());
     gx += static_cast<double>(fx);
     gy += static_cast<double>(fy);
     gz += static_cast<double>(fz);
@@ -241,8 +251,8 @@ __global__ __launch_bounds__(1024, 8) void table_force_kernel(
     const float* fj = un.ei < 0 ? nullptr : ftab + static_cast<size_t>(un.ej) * nq;
     for (int j = jb; j < je; ++j) {
       const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
-      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-      if (!(r2 > 0.0) || scaled_root(r2, inv_h) < limit) continue;
+      const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, kLeast)));
+      if (!(r2 >= limit)) continue;
       const double p = pair_force_far(sqrt(r2), uc, fi, fj, nq, dq, far_seen);
       gx = fma(p, dx, gx);
       gy = fma(p, dy, gy);
@@ -305,15 +315,19 @@ hipError_t launch_force_table(hipStream_t st, const double2* coef, int nq, doubl
   // four parts while their blocks fit the chip at once (two per CU): 10 us
   // instead of 16 for one table of 1,600 cells; beyond, the starting phases of
   // the parts cost more than the shorter chains save (16 tables of 1,080 cells:
-  // 20 us against 15)
+  // 20 us against 15).  Up to about four blocks of 64 cells per CU half blocks
+  // leave the CUs more even (14.0 us against 15.4)
+#define PYIID_TABLE(CELLS, PARTS)                                                            \
+  hipLaunchKernelGGL((force_table_kernel<CELLS, PARTS>), dim3((n_cell + CELLS - 1) / CELLS, n_table), \
+                     dim3(kNodes * kTabSplit * CELLS * PARTS), 0, st, coef, nq, dq, n_cell,  \
+                     force_cell(nq, dq), fit, t4, t2)
   if (static_cast<int64_t>((n_cell + 15) / 16) * n_table <= 512)
-    hipLaunchKernelGGL(force_table_kernel<4>, dim3((n_cell + 15) / 16, n_table),
-                       dim3(64 * kNodes * kTabSplit), 0, st, coef, nq, dq, n_cell,
-                       force_cell(nq, dq), fit, t4, t2);
+    PYIID_TABLE(16, 4);
+  else if (static_cast<int64_t>((n_cell + 63) / 64) * n_table <= 1024)
+    PYIID_TABLE(32, 1);
   else
-    hipLaunchKernelGGL(force_table_kernel<1>, dim3((n_cell + 63) / 64, n_table),
-                       dim3(64 * kNodes * kTabSplit), 0, st, coef, nq, dq, n_cell,
-                       force_cell(nq, dq), fit, t4, t2);
+    PYIID_TABLE(64, 1);
+#undef PYIID_TABLE
   return hipGetLastError();
 }
 

@@ -7,14 +7,13 @@
 namespace pyiid {
 namespace {
 
-// t = r / h from r^2, the root refined from FP32 by one Newton step in FP64
-// (relative error 1e-14; not a number where r^2 leaves float's range).
+// t = r / h from r^2: r^2 z with z the FP32 inverse root, refined by one step in FP64
+// with the scale in it (relative error 4e-14).  Where r^2 leaves float's range the
+// result is not a number or below every positive t.
 __device__ __forceinline__ double scaled_root(double r2, double inv_h) {
-  const float r2f = static_cast<float>(r2);
-  const float y0 = __builtin_amdgcn_rsqf(r2f);
-  const float rf = r2f * y0;
-  const double rd = static_cast<double>(rf);
-  return fma(fma(-rd, rd, r2), static_cast<double>(0.5f * y0), rd) * inv_h;
+  const double z = static_cast<double>(__builtin_amdgcn_rsqf(static_cast<float>(r2)));
+  const double a = r2 * z;
+  return a * fma(fma(-a, z, 1.0), 0.5 * inv_h, inv_h);
 }
 
 // Nearest integer of a float below 2^31 (one instruction; ties upwards).
