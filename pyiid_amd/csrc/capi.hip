@@ -226,6 +226,8 @@ struct pyiid_ctx {
   bool extent_exact = false;        // r_max bounds the current positions' distances
   Buf reach;                        // double: such a bound on the device
   bool reach_set = false;           // of the current positions
+  bool share_order = false;         // within one call (SharedOrder)
+  const AtomRec* in_order = nullptr;
 
   Table tab[2];
   uint64_t tab_stamp[2] = {1, 1};
@@ -265,7 +267,7 @@ struct pyiid_ctx {
   std::map<std::vector<int64_t>, std::vector<int64_t>> tuned;
 
   // workspaces
-  Buf upart;  // slices of the adjoint
+  Buf upart, mix;  // slices of the adjoint, its combination per chain
   Buf ucoef;  // double2 [chain][element pair][nq]: the force table's coefficients
   Buf gpart, fpart, fq64, fq32, g64, io_a, io_b, io_c, w, out5, u, uq, gobs, pfpart;
   Buf formcnt;  // uint64 [2]: F-only steps in the three-term / Reinsch form (while timing)
@@ -930,20 +932,22 @@ bool use_spread_fq(pyiid_ctx* c, const Table& t) {
 }
 
 // Whether F(Q) runs in one launch: small chains, whose pairs each block of 64
-// bins spreads for itself.  A block takes 0.6 us for 1,024 pairs (11 us at 192
-// atoms) and the chip about 5 us for two million; past these sizes the repeated
-// spreading takes longer than two more launches (5 us of the host each), and
-// past 512 bins the transform by one block per 64 bins does (60 atoms at 1,400
-// bins: 60 us against 31).
+// bins spreads for itself, where that takes about as long as the three launches
+// for one call alone and less among others (us, 500 bins, alone and among others:
+// 55 atoms 25 and 8 against 32 and 13, 128 atoms 34 and 8 against 34 and 13, 150
+// atoms 39 and 9 against 34 and 13; two elements, 100 atoms 37 and 9 against 37
+// and 15, 128 atoms 41 and 10 against 37 and 15).  The chip takes about 5 us for
+// two million pairs times blocks.
 bool use_small_fq(pyiid_ctx* c, const Table& t) {
-  if (t.nq > 512 || element_pairs(t) > 3) return false;
+  if (element_pairs(t) > 3 || small_fq_lds(t.nq, static_cast<int>(element_pairs(t))) > kSmallFqLds)
+    return false;
   int64_t pairs = 0;
   for (int b = 0; b < c->n_chain; ++b) {
     const int64_t n = c->off[b + 1] - c->off[b];
-    if (n > kSmallAtoms) return false;
+    if (n > (element_pairs(t) == 1 ? kSmallAtoms : kSmallAtoms2)) return false;
     pairs += n * (n - 1) / 2;
   }
-  return pairs * ((t.nq + 63) / 64) * element_pairs(t) <= 2000000;
+  return pairs * ((t.nq + 63) / 64) <= 2000000;
 }
 
 int ensure_offsets(pyiid_ctx* c) {
@@ -1106,9 +1110,36 @@ hipError_t launch_fq_items(pyiid_ctx* c, const Table& t, double qbin, bool count
                    c->fpart.as<double>(), forms);
 }
 
+// Lets the kernels of one call, between which the atoms stay where they are, use
+// one copy of the positions in element order (each set's perm is the same order).
+struct SharedOrder {
+  pyiid_ctx* c;
+  explicit SharedOrder(pyiid_ctx* ctx) : c(ctx) { c->share_order = true; }
+  ~SharedOrder() {
+    c->share_order = false;
+    c->in_order = nullptr;
+  }
+};
+
+int in_element_order(pyiid_ctx* c, const Buf& perm, const Buf& sorted, const AtomRec** sp) {
+  if (c->in_order) {
+    *sp = c->in_order;
+    return PYIID_OK;
+  }
+  HIPCHK(launch_gather(c->stream, c->pos.as<AtomRec>(), perm.as<int32_t>(), c->n, sorted.as<AtomRec>()));
+  *sp = sorted.as<AtomRec>();
+  if (c->share_order) c->in_order = *sp;
+  return PYIID_OK;
+}
+
 // F(Q) of every chain (full grid) into c->fq64 [B][nq] (double) and c->fq32, or
-// into `direct` only (device floats).
-int compute_fq(pyiid_ctx* c, int slot, double qbin, float* direct = nullptr) {
+// into `direct` only (device floats).  clear (nullable): what the caller's next
+// launch has to clear of the grids, in words; then single grids of up to
+// kOnePartBins bins are transformed by one launch instead of two (16 chains of 100
+// to 400 atoms, 330 bins: 8.5 us instead of 13).
+constexpr int kOnePartBins = 1024;
+int compute_fq(pyiid_ctx* c, int slot, double qbin, float* direct = nullptr,
+               int64_t* clear = nullptr) {
   Table& t = c->tab[slot];
   const int nq = t.nq, B = c->n_chain;
   CHK(c->fq64.reserve(sizeof(double) * (size_t)std::max(1, nq) * B));
@@ -1132,10 +1163,7 @@ int compute_fq(pyiid_ctx* c, int slot, double qbin, float* direct = nullptr) {
     }
     CHK(ensure_spread(c, t));
     const AtomRec* sp = c->pos.as<AtomRec>();
-    if (weighted) {
-      HIPCHK(launch_gather(c->stream, sp, s.perm.as<int32_t>(), c->n, s.sorted.as<AtomRec>()));
-      sp = s.sorted.as<AtomRec>();
-    }
+    if (weighted) CHK(in_element_order(c, s.perm, s.sorted, &sp));
     const int bits = fq_scale_bits(nq, dq, c->r_max);
     s.dirty = true;
     Timed tm(c, 1);
@@ -1143,10 +1171,15 @@ int compute_fq(pyiid_ctx* c, int slot, double qbin, float* direct = nullptr) {
                             s.items.as<SpreadItem>(), nq, dq, s.shift, bits,
                             s.grids.as<unsigned long long>()));
     CHK(tm.done());
+    const bool later = clear && element_pairs(t) == 1 && nq <= kOnePartBins;
     HIPCHK(launch_transform_fq(c->stream, s.grids.as<unsigned long long>(), B,
                                static_cast<int>(element_pairs(t)), weighted, t.tab.as<float>(), nq,
-                               dq, s.shift, bits, t.fsu.as<double>(), s.part.as<double>(), out64, out32));
-    s.dirty = false;
+                               dq, s.shift, bits, t.fsu.as<double>(), s.part.as<double>(), out64, out32,
+                               later));
+    if (later)
+      *clear = static_cast<int64_t>(B) * fq_grid_stride(nq);
+    else
+      s.dirty = false;
     return PYIID_OK;
   }
   CHK(ensure_fq_items(c, weighted_table(t)));
@@ -1610,10 +1643,7 @@ int run_spread_grad(pyiid_ctx* c, int slot, double qbin, void* out, bool out_f64
   CHK(s.rows.reserve(s.n_run * split_bytes(3 * chunk, len)));
   CHK(s.row_scale.reserve(sizeof(float) * 3 * static_cast<size_t>(chunk) * s.n_run));
   const AtomRec* sp = c->pos.as<AtomRec>();
-  if (weighted) {
-    HIPCHK(launch_gather(c->stream, sp, s.perm.as<int32_t>(), c->n, s.sorted.as<AtomRec>()));
-    sp = s.sorted.as<AtomRec>();
-  }
+  if (weighted) CHK(in_element_order(c, s.perm, s.sorted, &sp));
   // points of a row in use: from the host's extent when it bounds the current
   // positions, else from the positions on the device (no wait either way)
   int k_fixed = 0;
@@ -1640,7 +1670,8 @@ int run_spread_grad(pyiid_ctx* c, int slot, double qbin, void* out, bool out_f64
                               dq, c->r_max, k_fixed, reach, s.rows.p, s.row_scale.as<float>(),
                               c->spread.units.as<SpreadUnit>(), c->spread.n_units,
                               c->spread.items.as<SpreadItem>(), bits, grids));
-    HIPCHK(launch_transform_one(c->stream, grids, nq, dq, bits, t.fsu.as<double>(), fq));
+    HIPCHK(launch_transform_fq(c->stream, grids, 1, 1, false, nullptr, nq, dq, 0, bits,
+                               t.fsu.as<double>(), nullptr, nullptr, fq, true));
   }
   for (int64_t p0 = 0; p0 < c->n; p0 += chunk) {
     const int m = static_cast<int>(std::min<int64_t>(chunk, c->n - p0));
@@ -1798,10 +1829,7 @@ int contract_forces(pyiid_ctx* c, int slot, double qbin, double scale, double* o
     CHK(s.part.reserve(sizeof(double) * 3 * static_cast<size_t>(std::max<int64_t>(1, c->n)) *
                        s.n_planes));
     const AtomRec* sp = c->pos.as<AtomRec>();
-    if (weighted) {
-      HIPCHK(launch_gather(c->stream, sp, s.perm.as<int32_t>(), c->n, s.sorted.as<AtomRec>()));
-      sp = s.sorted.as<AtomRec>();
-    }
+    if (weighted) CHK(in_element_order(c, s.perm, s.sorted, &sp));
     Timed tm(c, 4);
     HIPCHK(launch_force_table(c->stream, c->ucoef.as<double2>(), nq, dq,
                               static_cast<int>(element_pairs(t)) * B, n_cell, s.t4.as<float4>(),
@@ -1883,23 +1911,28 @@ int gemm_grad(pyiid_ctx* c, const void* a, bool a64, int64_t rows, double* out) 
 int energy_forces_device(pyiid_ctx* c, int slot, double qbin, int potential,
                          const double* gobs_dev, double force_scale, double* forces_dev) {
   const int nq = c->t_nq, nr = c->t_nr, B = c->n_chain;
-  CHK(compute_fq(c, slot, qbin));
+  const SharedOrder shared(c);
+  Table& t = c->tab[slot];
+  int64_t clear = 0;
+  CHK(compute_fq(c, slot, qbin, nullptr, &clear));
   CHK(c->g64.reserve(sizeof(double) * (size_t)nr * B));
   CHK(gemm_t(c, c->fq32.p, false, B, c->g64.as<double>()));
   CHK(reserve_out5(c, B));
-  CHK(c->w.reserve(sizeof(double) * (size_t)nr * B));
-  HIPCHK(launch_potential(c->stream, potential, gobs_dev, c->g64.as<double>(), nr, B,
-                          c->out5.as<double>(), c->w.as<double>()));
+  CHK(c->mix.reserve(sizeof(double2) * B));
+  if (forces_dev) CHK(c->upart.reserve(sizeof(double) * 2 * kAdjointSlices * (size_t)nq * B));
+  HIPCHK(launch_score(c->stream, potential, gobs_dev, c->g64.as<double>(), nr, B, c->out5.as<double>(),
+                      c->mix.as<double2>(), c->tmat.as<float>(), nq,
+                      forces_dev ? c->upart.as<double>() : nullptr,
+                      clear ? c->spread.grids.as<unsigned long long>() : nullptr, clear));
+  if (clear) c->spread.dirty = false;
   if (!forces_dev) return PYIID_OK;
   CHK(c->u.reserve(sizeof(float) * (size_t)nq * B));
   double2* coef = nullptr;
   CHK(reserve_coef(c, slot, qbin, &coef));
-  CHK(c->upart.reserve(sizeof(double) * kAdjointSlices * (size_t)nq * B));
-  HIPCHK(launch_adjoint(c->stream, c->tmat.as<float>(), nr, nq, c->w.as<double>(),
-                        c->tab[slot].gs.as<double>(), B,
-                        static_cast<double>(static_cast<float>(qbin)), c->tab[slot].tab.as<float>(),
-                        weighted_table(c->tab[slot]), static_cast<int>(element_pairs(c->tab[slot])),
-                        c->upart.as<double>(), c->u.as<float>(), coef));
+  HIPCHK(launch_adjoint_sum(c->stream, c->upart.as<double>(), c->mix.as<double2>(), B, nq,
+                            t.gs.as<double>(), static_cast<double>(static_cast<float>(qbin)),
+                            t.tab.as<float>(), weighted_table(t), static_cast<int>(element_pairs(t)),
+                            c->u.as<float>(), coef));
   return contract_forces(c, slot, qbin, force_scale, forces_dev);
 }
 
@@ -2457,7 +2490,7 @@ int pyiid_destroy(pyiid_ctx* c) {
   destroy_graph(c->hmc);
   for (Buf* b : {&c->posf, &c->elem, &c->pos, &c->counts_d, &c->natoms_d, &c->off_d, &c->tmat, &c->tsplit, &c->tsplit_scale, &c->gsplit, &c->gsplit_scale, &c->gpart,
                  &c->fpart, &c->fq64, &c->fq32, &c->g64, &c->io_a, &c->io_b,
-                 &c->io_c, &c->w, &c->out5, &c->u, &c->ucoef, &c->upart, &c->gobs, &c->fq_items.items,
+                 &c->io_c, &c->w, &c->out5, &c->u, &c->ucoef, &c->upart, &c->mix, &c->gobs, &c->fq_items.items,
                  &c->fq_items.ranges, &c->fq_items.perm, &c->spread.units, &c->spread.items,
                  &c->spread.perm, &c->spread.sorted, &c->spread.grids, &c->spread.part,
                  &c->force.units, &c->force.planes, &c->force.perm, &c->force.sorted,
@@ -2770,6 +2803,7 @@ int pyiid_grad_fq(pyiid_ctx* c, int slot, double qbin, void* grad, float* fq, in
       fdst = static_cast<float*>(f);
     }
     const bool both = fq && fdst && use_spread_both(c, t);
+    const SharedOrder shared(c);
     CHK(run_spread_grad(c, slot, qbin, gdst, (flags & PYIID_F64) != 0, both ? fdst : nullptr));
     if (copy) CHK(download(c, grad, gdst, gbytes, flags));
     if (fq && !both) {
@@ -2951,7 +2985,7 @@ int pyiid_potential(pyiid_ctx* c, int potential, const double* gobs, const doubl
   CHK(reserve_out5(c, c->n_chain));
   CHK(upload(c, c->io_a.p, gcalc, sizeof(double) * n, flags));
   CHK(upload(c, c->io_b.p, gobs, sizeof(double) * n, flags));
-  HIPCHK(launch_potential(c->stream, potential, c->io_b.as<double>(), c->io_a.as<double>(), n, 1,
+  HIPCHK(launch_potential(c->stream, potential, c->io_b.as<double>(), c->io_a.as<double>(), n,
                           c->out5.as<double>(), c->w.as<double>()));
   double out5[5];
   HIPCHK(hipMemcpyAsync(out5, c->out5.p, sizeof(out5), hipMemcpyDeviceToHost, c->stream));
@@ -3038,7 +3072,7 @@ int pyiid_fq_energy_forces(pyiid_ctx* c, int slot, double qbin, int32_t q_first,
   CHK(reserve_out5(c, c->n_chain));
   CHK(c->w.reserve(sizeof(double) * ng));
   HIPCHK(launch_potential(c->stream, potential, c->gobs.as<double>(),
-                          c->fq64.as<double>() + q_first, ng, 1, c->out5.as<double>(),
+                          c->fq64.as<double>() + q_first, ng, c->out5.as<double>(),
                           c->w.as<double>()));
   double out5[6];
   HIPCHK(hipMemcpyAsync(out5, c->out5.p, sizeof(out5), hipMemcpyDeviceToHost, c->stream));

@@ -131,19 +131,18 @@ hipError_t launch_spread_fq(hipStream_t st, const AtomRec* pos, const SpreadUnit
 // out[b][q] = scale[b][q] * sum over the chain's element pairs (grid index
 // b * n_pair + e_i (e_i + 1) / 2 + e_j, e_j <= e_i) of f_i f_j times the pair's
 // sum of sin(Q r) / r; clears the grids.  part: n_chain * n_pair *
-// fq_transform_parts * nq doubles.
+// fq_transform_parts * nq doubles.  one_part (single grids only): in one launch,
+// without part, and the grids stay as they are.
 int fq_transform_parts(int nq, int n_chain, int n_pair);
 hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_chain, int n_pair,
                                bool weighted, const float* ftab, int nq, double dq, int shift,
                                int scale_bits, const double* scale, double* part, double* out_f64,
-                               float* out_f32);
-// out[q] = scale[q] * transform of one chain's single grid, which stays as it is
-hipError_t launch_transform_one(hipStream_t st, const unsigned long long* grids, int nq, double dq,
-                                int scale_bits, const double* scale, float* out);
+                               float* out_f32, bool one_part);
 // F of chains of at most kSmallAtoms atoms (off: n_chain + 1 offsets) in one
-// launch; the grid must fit kSmallFqLds.
-constexpr int kSmallAtoms = 192;
-constexpr size_t kSmallFqLds = 40 * 1024;
+// launch; the grids must fit kSmallFqLds.
+constexpr int kSmallAtoms = 128, kSmallAtoms2 = 100;  // one element; two
+constexpr size_t kSmallFqLds = 80 * 1024;
+size_t small_fq_lds(int nq, int n_pair);
 hipError_t launch_small_fq(hipStream_t st, const AtomRec* pos, const int* off, int n_chain,
                            int n_pair, bool weighted, const float* ftab, int nq, double dq,
                            int scale_bits, const double* scale, double* out_f64, float* out_f32);
@@ -208,7 +207,7 @@ constexpr size_t kForceLds = 160 * 1024;
 double force_cell(int nq, double dq);       // cell width of the table
 size_t force_lds_bytes(int64_t n_cell);     // LDS of a block
 // t4 / t2 [table][n_cell]: coefficients 0..3 / 4, 5; coef[table][q] (table =
-// chain * n_pair + pair) as launch_adjoint writes it
+// chain * n_pair + pair) as launch_adjoint_sum writes it
 hipError_t launch_force_table(hipStream_t st, const double2* coef, int nq, double dq, int n_table,
                               int n_cell, float4* t4, float2* t2);
 // part[plane][position][3], or with out the forces themselves (a single plane):
@@ -241,20 +240,26 @@ hipError_t launch_split_rows(hipStream_t st, const void* a, bool a_f64, int64_t 
 hipError_t launch_gemm_grad(hipStream_t st, const void* rows, const float* row_scale, const void* a,
                             bool a_f64, int m, int k, const void* ts, const float* t_scale,
                             const float* t, int n, double* out);
-// Per chain b (one block each): potential value/scale and the adjoint
-// w[b][t] (FP64).  out5[b] = {value, scale, a_opt, res.res, g.res}.
+// Potential value/scale and the adjoint w[t] (FP64) of one array.
+// out5 = {value, scale, a_opt, res.res, g.res}.
 hipError_t launch_potential(hipStream_t st, int potential, const double* gobs,
-                            const double* gcalc, int n, int n_chain, double* out5, double* w);
+                            const double* gcalc, int n, double* out5, double* w);
 // y[row] = sum_t X[row][t] * w[t]  (FP64), one wave per row
 hipError_t launch_gemv_rows(hipStream_t st, const double* x, int64_t rows, int n,
                             const double* w, double* y);
-// u[b][q] = gscale[b][q] * sum_t T[t][q] w[b][t]   (FP64 accumulation) and,
-// unless null, coef[b][pair][q] = (u f_I f_J q dq, u f_I f_J) for the force table;
-// part: kAdjointSlices * n_chain * nq doubles
+// The potential of every chain (out5[b]) and what the adjoint of all needs: mix[b]
+// and, unless part is null, the products of o and g with T (kAdjointSlices * 2 *
+// n_chain * nq doubles).  clear (nullable): an even number of words that blocks of
+// the launch set to zero.
 constexpr int kAdjointSlices = 4;
-hipError_t launch_adjoint(hipStream_t st, const float* t, int n_r, int nq, const double* w,
-                          const double* gscale, int n_chain, double dq, const float* ftab,
-                          bool weighted, int n_pair, double* part, float* u, double2* coef);
+hipError_t launch_score(hipStream_t st, int potential, const double* gobs, const double* gcalc,
+                        int n_r, int n_chain, double* out5, double2* mix, const float* t, int nq,
+                        double* part, unsigned long long* clear, int64_t clear_words);
+// u[b][q] = gscale[b][q] * sum_t T[t][q] w[b][t] (FP64) from these and, unless null,
+// coef[b][pair][q] = (u f_I f_J q dq, u f_I f_J) for the force table
+hipError_t launch_adjoint_sum(hipStream_t st, const double* part, const double2* mix, int n_chain,
+                              int nq, const double* gscale, double dq, const float* ftab,
+                              bool weighted, int n_pair, float* u, double2* coef);
 // the same from u[q] = gscale[q] * w[q - q_first] (0 below q_first), one chain
 hipError_t launch_adjoint_fq(hipStream_t st, int nq, int q_first, const double* w,
                              const double* gscale, double dq, const float* ftab, bool weighted,

@@ -52,34 +52,66 @@ __global__ __launch_bounds__(1024, 8) void spread_fq_kernel(
 
 constexpr int kTrChunk = 2048;  // grid points in LDS at a time (16 KiB)
 
-// sum over grid points [lo, hi) of value(k) sin(2 pi (first + k - 3) m / n_f):
-// the sine starts from an exact phase (reduced as an integer below 2^31: n_f <=
-// 12 * 3,400, g + n_f < 1.6 n_f) and follows the FP64 three-term recurrence.
-template <typename F>
-__device__ __forceinline__ double sine_sum(F value, int lo, int hi, int first, int m, int nf) {
-  const double two_over = 2.0 / static_cast<double>(nf);
-  const double c2 = 2.0 * cospi(two_over * m);
+// What the bins of a block share, made by two of its waves while the others
+// spread or load: 1 / phihat, and sine and cosine of 2 pi m / n_f.
+struct BinTerms {
+  double inv[64], sin1[64], cos1[64];
+};
+
+// acc[p] += sum over grid points [lo, hi) of value(p, k) sin(2 pi (first + k - 3) m /
+// n_f): the sine starts from an exact phase (reduced as an integer below 2^31:
+// n_f <= 12 * 3,400, g + n_f < 1.6 n_f) and follows the FP64 three-term recurrence.
+template <int N, typename F>
+__device__ __forceinline__ void sine_sum(F value, int lo, int hi, int first, int m, int nf,
+                                         double sin1, double cos1, double (&acc)[N]) {
   const unsigned g = static_cast<unsigned>(first + lo - 3 + nf);
   const unsigned s0 = g * static_cast<unsigned>(m) % static_cast<unsigned>(nf);
-  const unsigned s1 = (g - 1u) * static_cast<unsigned>(m) % static_cast<unsigned>(nf);
-  double y = sinpi(two_over * static_cast<double>(s0));
-  double yp = sinpi(two_over * static_cast<double>(s1));
-  double acc = 0.0;
+  const double c2 = 2.0 * cos1;
+  double y, c;
+  sincospi(2.0 / static_cast<double>(nf) * static_cast<double>(s0), &y, &c);
+  double yp = fma(y, cos1, -c * sin1);  // one point before
 #pragma unroll 4
   for (int k = lo; k < hi; ++k) {
-    acc = fma(value(k), y, acc);
+#pragma unroll
+    for (int p = 0; p < N; ++p) acc[p] = fma(value(p, k), y, acc[p]);
     const double yn = fma(c2, y, -yp);
     yp = y;
     y = yn;
   }
-  return acc;
 }
 
-// h / phihat(m) and the fixed point's unit
-__device__ __forceinline__ double fq_unit(int m, int nf, double inv_h, int shift, int scale_bits) {
-  const double q = 2.0 * M_PI * m / nf;  // Q h
-  const double a = sqrt(fmax(kFqBeta * kFqBeta - 0.25 * kFqW * kFqW * q * q, 1.0));
-  return ldexp(inv_h, shift - scale_bits) * (sinh(kFqBeta) / kFqBeta) * a / sinh(a);
+// 1 / phihat(m) but for its constant sinh(beta) / beta, which comes with the unit
+// from fq_unit: sinh(a) = (e^a - e^-a) / 2, where a > 15 leaves e^-2a < 1e-13.
+__device__ __forceinline__ double fq_inv_phihat(int m, int nf) {
+  const double q = 2.0 * M_PI * m / nf;  // Q h <= pi / 6
+  const double a = sqrt(kFqBeta * kFqBeta - 0.25 * kFqW * kFqW * q * q);
+  const double e = exp(-a);
+  return 2.0 * a * e / (1.0 - e * e);
+}
+
+__device__ __forceinline__ void bin_terms(BinTerms& t, int m, int nf, double unit) {
+  const int lane = threadIdx.x & 63, from_last = (blockDim.x >> 6) - 1 - (threadIdx.x >> 6);
+  if (from_last == 0) t.inv[lane] = unit * fq_inv_phihat(m, nf);
+  if (from_last == 1) sincospi(2.0 * m / nf, &t.sin1[lane], &t.cos1[lane]);
+}
+
+// h, the fixed point's unit and the window's constant
+double fq_unit(double inv_h, int shift, int scale_bits) {
+  return std::ldexp(inv_h, shift - scale_bits) * std::sinh(kFqBeta) / kFqBeta;
+}
+
+// One more than the last of [0, cnt) at which get(g) is not zero, for the block:
+// distances reach the first few hundred of a grid's points (a third of them at
+// 55 atoms and 250 bins), and the transform ends there.  top: LDS, zero before;
+// a barrier follows.
+template <typename G>
+__device__ __forceinline__ void last_used(G get, int cnt, int* top) {
+  int mine = 0;
+  for (int g = threadIdx.x; g < cnt; g += blockDim.x)
+    if (get(g)) mine = g + 1;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) mine = max(mine, __shfl_xor(mine, off, 64));
+  if ((threadIdx.x & 63) == 0 && mine > 0) atomicMax(top, mine);
 }
 
 // The close contacts' part of sum sin(Q r) / r (almost always none)
@@ -102,11 +134,13 @@ __device__ __forceinline__ double fq_nodes(const unsigned long long* nodes, int 
 // 155 us for three element pairs at 1,500.
 __global__ __launch_bounds__(1024) void transform_fq_kernel(
     const unsigned long long* __restrict__ grids, int n_pair, int n_split, int nf, int n_grid,
-    int stride, int shift, int scale_bits, const float* __restrict__ ftab, int nq, double inv_h,
+    int stride, int shift, double unit, const float* __restrict__ ftab, int nq, double inv_h,
     int weighted, double* __restrict__ part, const double* __restrict__ scale,
-    float* __restrict__ direct) {
+    double* __restrict__ out64, float* __restrict__ out32) {
   __shared__ __align__(16) double buf[kTrChunk];
   __shared__ double sums[16][65];
+  __shared__ BinTerms terms;
+  __shared__ int top;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = blockIdx.x * 64 + lane;
   const int b = blockIdx.y, z = blockIdx.z;
@@ -114,22 +148,33 @@ __global__ __launch_bounds__(1024) void transform_fq_kernel(
   const unsigned long long* h = grids + (static_cast<size_t>(b) * n_pair + pair) * stride;
   const int g_lo = static_cast<int>(static_cast<int64_t>(n_grid) * split / n_split);
   const int g_hi = static_cast<int>(static_cast<int64_t>(n_grid) * (split + 1) / n_split);
-  double acc = 0.0;
+  double acc[1] = {0.0};
   for (int g0 = g_lo; g0 < g_hi; g0 += kTrChunk) {
     const int cnt = min(kTrChunk, g_hi - g0);
     __syncthreads();
-    for (int g = threadIdx.x; g < cnt; g += blockDim.x)
-      buf[g] = static_cast<double>(static_cast<long long>(h[g0 + g]));
+    if (threadIdx.x == 0) top = 0;
     __syncthreads();
-    acc += sine_sum([&](int k) { return buf[k]; }, cnt * wave / 16, cnt * (wave + 1) / 16, g0, m, nf);
+    last_used(
+        [&](int g) {
+          const long long v = static_cast<long long>(h[g0 + g]);
+          buf[g] = static_cast<double>(v);
+          return v != 0;
+        },
+        cnt, &top);
+    if (g0 == g_lo) bin_terms(terms, m, nf, unit);
+    __syncthreads();
+    const int used = top;
+    if (used > 0)
+      sine_sum<1>([&](int, int k) { return buf[k]; }, used * wave / 16, used * (wave + 1) / 16, g0, m, nf,
+                  terms.sin1[lane], terms.cos1[lane], acc);
   }
-  sums[wave][lane] = acc;
+  sums[wave][lane] = acc[0];
   __syncthreads();
   if (wave != 0 || m >= nq) return;
   double total = 0.0;
 #pragma unroll
   for (int k = 0; k < 16; ++k) total += sums[k][lane];
-  total *= fq_unit(m, nf, inv_h, shift, scale_bits);
+  total *= terms.inv[lane];
   if (split == 0) total += fq_nodes(h + n_grid, m, nf, inv_h, shift);
   if (weighted) {
     int ei = 0, ej = pair;
@@ -137,10 +182,15 @@ __global__ __launch_bounds__(1024) void transform_fq_kernel(
     total *= static_cast<double>(ftab[static_cast<size_t>(ei) * nq + m]) *
              static_cast<double>(ftab[static_cast<size_t>(ej) * nq + m]);
   }
-  if (direct)  // one part: F itself
-    direct[static_cast<size_t>(b) * nq + m] = static_cast<float>(total * scale[static_cast<size_t>(b) * nq + m]);
-  else
+  if (part) {
     part[(static_cast<size_t>(b) * n_pair * n_split + z) * nq + m] = total;
+    return;
+  }
+  // one part: F itself
+  const size_t o = static_cast<size_t>(b) * nq + m;
+  const double v = total * scale[o];
+  if (out64) out64[o] = v;
+  if (out32) out32[o] = static_cast<float>(v);
 }
 
 // F from the parts (blocks below n_out, one thread per chain and bin), and the
@@ -168,72 +218,92 @@ __global__ __launch_bounds__(256) void finish_fq_kernel(
     grids[w] = ulonglong2{0ull, 0ull};
 }
 
-// F of chains of at most kSmallAtoms atoms in one launch instead of three: every
-// block of 64 bins spreads all pairs of its chain again (at most 18 for each of
-// its threads) and transforms the grid where it lies, in LDS.  Element pairs
-// follow one another.  55 atoms, 250 bins: 9 us of kernels and two launches less.
-__global__ __launch_bounds__(1024) void small_fq_kernel(
-    const AtomRec* __restrict__ pos, const int* __restrict__ off, int n_pair, int nf, int n_grid,
-    int stride, int scale_bits, float scale, double near, const float* __restrict__ ftab, int nq,
-    double inv_h, int weighted, const double* __restrict__ fscale, double* __restrict__ out64,
-    float* __restrict__ out32) {
+// F of small chains in one launch instead of three: every block of 64 bins spreads
+// all pairs of its chain again and transforms the grids (N: one for each pair of
+// elements) where they lie, in LDS.  A block has a CU of its own and is bound by its
+// VALU work: 8 waves, so that the sums' starting phases are few (16 waves 14 us, 4
+// waves 12 us, 8 waves 11 us at 55 atoms and 250 bins).
+constexpr int kSmallWaves = 8;
+
+template <int N>
+__global__ __launch_bounds__(64 * kSmallWaves) void small_fq_kernel(
+    const AtomRec* __restrict__ pos, const int* __restrict__ off, int nf, int n_grid, int stride,
+    double unit, float scale, double near, const float* __restrict__ ftab, int nq, double inv_h,
+    const double* __restrict__ fscale, double* __restrict__ out64, float* __restrict__ out32) {
   extern __shared__ unsigned long long hist[];
-  __shared__ double sums[16][65];
+  __shared__ double sums[N][kSmallWaves][65];
+  __shared__ BinTerms terms;
+  __shared__ int top;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = blockIdx.x * 64 + lane;
   const int b = blockIdx.y;
   const int i0 = off[b], n = off[b + 1] - i0;
   const int pairs = n * (n - 1) / 2;
   const double half_nf = 0.5 * nf;
+  for (int g = threadIdx.x; g < N * stride; g += 64 * kSmallWaves) hist[g] = 0ull;
+  if (threadIdx.x == 0) top = 0;
+  __syncthreads();
+  for (int k = threadIdx.x; k < pairs; k += 64 * kSmallWaves) {
+    int i = static_cast<int>((1.0f + __builtin_amdgcn_sqrtf(1.0f + 8.0f * k)) * 0.5f);
+    if (i * (i - 1) / 2 > k) --i;
+    if ((i + 1) * i / 2 <= k) ++i;
+    const AtomRec a = pos[i0 + i], c = pos[i0 + k - i * (i - 1) / 2];
+    const double dx = a.x - c.x, dy = a.y - c.y, dz = a.z - c.z;
+    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    if (!(r2 > 0.0)) continue;
+    unsigned long long* grid = hist;
+    if (N > 1) {
+      const int x = static_cast<int>(a.w), y = static_cast<int>(c.w), hi = max(x, y);
+      grid += (hi * (hi + 1) / 2 + min(x, y)) * stride;
+    }
+    const double t = scaled_root(r2, inv_h);
+    if (t >= near && t < kFqFar)
+      spread_pair(grid, t, static_cast<double>(nf), half_nf, scale);
+    else
+      spread_rare(grid, n_grid, sqrt(r2) * inv_h, static_cast<double>(nf), static_cast<double>(scale));
+  }
+  bin_terms(terms, m, nf, unit);
+  __syncthreads();
+  double* points = reinterpret_cast<double*>(hist);  // the points in place
+  last_used(
+      [&](int g) {
+        long long any = 0;
+#pragma unroll
+        for (int p = 0; p < N; ++p) {
+          const long long v = static_cast<long long>(hist[p * stride + g]);
+          points[p * stride + g] = static_cast<double>(v);
+          any |= v;
+        }
+        return any != 0;
+      },
+      n_grid, &top);
+  __syncthreads();
+  const int used = top;
+  double acc[N] = {};
+  if (used > 0)
+    sine_sum<N>([&](int p, int k) { return points[p * stride + k]; }, used * wave / kSmallWaves,
+                used * (wave + 1) / kSmallWaves, 0, m, nf, terms.sin1[lane], terms.cos1[lane], acc);
+#pragma unroll
+  for (int p = 0; p < N; ++p) sums[p][wave][lane] = acc[p];
+  __syncthreads();
+  if (wave != 0 || m >= nq) return;
   double total = 0.0;
   int ei = 0, ej = 0;
-  for (int p = 0; p < n_pair; ++p) {
-    __syncthreads();
-    for (int g = threadIdx.x; g < stride; g += 1024) hist[g] = 0ull;
-    __syncthreads();
-    for (int k = threadIdx.x; k < pairs; k += 1024) {
-      int i = static_cast<int>((1.0f + __builtin_amdgcn_sqrtf(1.0f + 8.0f * k)) * 0.5f);
-      if (i * (i - 1) / 2 > k) --i;
-      if ((i + 1) * i / 2 <= k) ++i;
-      const AtomRec a = pos[i0 + i], c = pos[i0 + k - i * (i - 1) / 2];
-      if (weighted) {
-        const int x = static_cast<int>(a.w), y = static_cast<int>(c.w);
-        if (max(x, y) != ei || min(x, y) != ej) continue;
-      }
-      const double dx = a.x - c.x, dy = a.y - c.y, dz = a.z - c.z;
-      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-      if (!(r2 > 0.0)) continue;
-      const double t = scaled_root(r2, inv_h);
-      if (t >= near && t < kFqFar)
-        spread_pair(hist, t, static_cast<double>(nf), half_nf, scale);
-      else
-        spread_rare(hist, n_grid, sqrt(r2) * inv_h, static_cast<double>(nf),
-                    static_cast<double>(scale));
-    }
-    __syncthreads();
-    double* grid = reinterpret_cast<double*>(hist);  // the points in place, once
-    for (int g = threadIdx.x; g < n_grid; g += 1024)
-      grid[g] = static_cast<double>(static_cast<long long>(hist[g]));
-    __syncthreads();
-    sums[wave][lane] = sine_sum([&](int k) { return grid[k]; }, n_grid * wave / 16,
-                                n_grid * (wave + 1) / 16, 0, m, nf);
-    __syncthreads();
-    if (wave == 0 && m < nq) {
-      double v = 0.0;
 #pragma unroll
-      for (int k = 0; k < 16; ++k) v += sums[k][lane];
-      v = v * fq_unit(m, nf, inv_h, 0, scale_bits) + fq_nodes(hist + n_grid, m, nf, inv_h, 0);
-      if (weighted)
-        v *= static_cast<double>(ftab[static_cast<size_t>(ei) * nq + m]) *
-             static_cast<double>(ftab[static_cast<size_t>(ej) * nq + m]);
-      total += v;
-    }
+  for (int p = 0; p < N; ++p) {
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < kSmallWaves; ++k) v += sums[p][k][lane];
+    v = v * terms.inv[lane] + fq_nodes(hist + p * stride + n_grid, m, nf, inv_h, 0);
+    if (ftab)
+      v *= static_cast<double>(ftab[static_cast<size_t>(ei) * nq + m]) *
+           static_cast<double>(ftab[static_cast<size_t>(ej) * nq + m]);
+    total += v;
     if (++ej > ei) {
       ++ei;
       ej = 0;
     }
   }
-  if (wave != 0 || m >= nq) return;
   const size_t o = static_cast<size_t>(b) * nq + m;
   const double v = total * fscale[o];
   if (out64) out64[o] = v;
@@ -376,14 +446,16 @@ int fq_transform_parts(int nq, int n_chain, int n_pair) {
 hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_chain, int n_pair,
                                bool weighted, const float* ftab, int nq, double dq, int shift,
                                int scale_bits, const double* scale, double* part, double* out_f64,
-                               float* out_f32) {
+                               float* out_f32, bool one_part) {
   const int nf = 12 * nq, stride = fq_grid_stride(nq);
-  const int n_split = fq_transform_parts(nq, n_chain, n_pair);
+  const int n_split = one_part ? 1 : fq_transform_parts(nq, n_chain, n_pair);
+  const double inv_h = dq * nf / (2.0 * M_PI);
   if (n_chain > 65535 || n_pair * n_split > 65535) return hipErrorInvalidValue;
   hipLaunchKernelGGL(transform_fq_kernel, dim3((nq + 63) / 64, n_chain, n_pair * n_split),
                      dim3(1024), 0, st, grids, n_pair, n_split, nf, fq_grid_points(nq), stride,
-                     shift, scale_bits, ftab, nq, dq * nf / (2.0 * M_PI), weighted ? 1 : 0, part,
-                     static_cast<const double*>(nullptr), static_cast<float*>(nullptr));
+                     shift, fq_unit(inv_h, shift, scale_bits), ftab, nq, inv_h, weighted ? 1 : 0,
+                     one_part ? nullptr : part, scale, out_f64, out_f32);
+  if (one_part) return hipGetLastError();
   const int64_t total = static_cast<int64_t>(n_chain) * nq;
   const int64_t words2 = static_cast<int64_t>(n_chain) * n_pair * stride / 2;  // stride is even
   const int64_t n_out = (total + 255) / 256;
@@ -394,30 +466,37 @@ hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_
   return hipGetLastError();
 }
 
-hipError_t launch_transform_one(hipStream_t st, const unsigned long long* grids, int nq, double dq,
-                                int scale_bits, const double* scale, float* out) {
-  const int nf = 12 * nq;
-  hipLaunchKernelGGL(transform_fq_kernel, dim3((nq + 63) / 64, 1, 1), dim3(1024), 0, st, grids, 1, 1,
-                     nf, fq_grid_points(nq), fq_grid_stride(nq), 0, scale_bits,
-                     static_cast<const float*>(nullptr), nq, dq * nf / (2.0 * M_PI), 0,
-                     static_cast<double*>(nullptr), scale, out);
-  return hipGetLastError();
+size_t small_fq_lds(int nq, int n_pair) {
+  return sizeof(unsigned long long) * static_cast<size_t>(fq_grid_stride(nq)) * n_pair;
 }
 
 hipError_t launch_small_fq(hipStream_t st, const AtomRec* pos, const int* off, int n_chain,
                            int n_pair, bool weighted, const float* ftab, int nq, double dq,
                            int scale_bits, const double* scale, double* out_f64, float* out_f32) {
   const int nf = 12 * nq, stride = fq_grid_stride(nq);
-  const size_t lds = sizeof(unsigned long long) * static_cast<size_t>(stride);
-  if (lds > kSmallFqLds || n_chain > 65535) return hipErrorInvalidValue;
-  static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(small_fq_kernel),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kSmallFqLds));
+  const double inv_h = dq * nf / (2.0 * M_PI);
+  const size_t lds = small_fq_lds(nq, n_pair);
+  if (lds > kSmallFqLds || n_chain > 65535 || (n_pair != 1 && n_pair != 3)) return hipErrorInvalidValue;
+  static const hipError_t attr = [] {
+    const hipError_t e =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(small_fq_kernel<1>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kSmallFqLds));
+    return e != hipSuccess ? e
+                           : hipFuncSetAttribute(reinterpret_cast<const void*>(small_fq_kernel<3>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 static_cast<int>(kSmallFqLds));
+  }();
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(small_fq_kernel, dim3((nq + 63) / 64, n_chain), dim3(1024), lds, st, pos, off,
-                     n_pair, nf, fq_grid_points(nq), stride, scale_bits,
-                     std::ldexp(1.0f, scale_bits), std::ldexp(1.0, scale_bits - 31), ftab, nq,
-                     dq * nf / (2.0 * M_PI), weighted ? 1 : 0, scale, out_f64, out_f32);
+  const dim3 grid((nq + 63) / 64, n_chain), block(64 * kSmallWaves);
+  const double unit = fq_unit(inv_h, 0, scale_bits), near = std::ldexp(1.0, scale_bits - 31);
+  const float one = std::ldexp(1.0f, scale_bits);
+  const float* f = weighted ? ftab : nullptr;
+  if (n_pair == 1)
+    hipLaunchKernelGGL(small_fq_kernel<1>, grid, block, lds, st, pos, off, nf, fq_grid_points(nq),
+                       stride, unit, one, near, f, nq, inv_h, scale, out_f64, out_f32);
+  else
+    hipLaunchKernelGGL(small_fq_kernel<3>, grid, block, lds, st, pos, off, nf, fq_grid_points(nq),
+                       stride, unit, one, near, f, nq, inv_h, scale, out_f64, out_f32);
   return hipGetLastError();
 }
 

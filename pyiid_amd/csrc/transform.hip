@@ -6,6 +6,7 @@
 // it is exactly G = T . F with a dense R x Q matrix T (built on the host in
 // FP64, stored here as FP32).  grad G = grad F . T^T runs on split operands
 // (split_gemm.h), smaller products on v_mfma_f32_16x16x4_f32.
+#include <algorithm>
 #include <cmath>
 
 #include "split_gemm.h"
@@ -373,23 +374,17 @@ __device__ void block_sum3(double& x, double& y, double& z, double (*sh)[16]) {
   }
 }
 
-// One block per chain.  Rw: master_kernel.py:206-236; chi^2: :239-266; the adjoint
+// The block's chain.  Rw: master_kernel.py:206-236; chi^2: :239-266; the adjoint
 // w is d(potential)/d(gcalc) as get_grad_rw / get_grad_chi_sq apply it
 // (:293-375): grad = gradG . w with
 //   w = c * (s * res + (g.res)/(g.g) * (o - 2 a g)),
 //   c = -value/|res|^2 (Rw) or -2 (chi^2), res = o - s g, a = optimal scale.
 constexpr int kPotKeep = 6;
-__global__ __launch_bounds__(1024) void potential_kernel(int potential,
-                                                         const double* __restrict__ o_all,
-                                                         const double* __restrict__ g_all, int n,
-                                                         double* __restrict__ out5_all,
-                                                         double* __restrict__ w_all) {
-  __shared__ double sh[3][16];
-  // one block per chain
-  const double* o = o_all + (size_t)blockIdx.x * n;
-  const double* g = g_all + (size_t)blockIdx.x * n;
-  double* out5 = out5_all + (size_t)blockIdx.x * 5;
-  double* w = w_all ? w_all + (size_t)blockIdx.x * n : nullptr;
+// mix (nullable): w as a combination of o and g, w = mix.x o + mix.y g.
+__device__ __forceinline__ void potential_block(int potential, const double* __restrict__ o,
+                                                const double* __restrict__ g, int n,
+                                                double* __restrict__ out5, double* __restrict__ w,
+                                                double2* __restrict__ mix, double (*sh)[16]) {
   // the thread's points stay in registers between the passes (kPotKeep of them;
   // longer arrays are read again)
   double ok[kPotKeep], gk[kPotKeep];
@@ -447,7 +442,20 @@ __global__ __launch_bounds__(1024) void potential_kernel(int potential,
     out5[2] = a;
     out5[3] = rr;
     out5[4] = gr;
+    if (mix) {
+      const double gfac = gr / gg;
+      *mix = double2{coef * (s + gfac), -coef * (s * s + 2.0 * a * gfac)};
+    }
   }
+}
+
+__global__ __launch_bounds__(1024) void potential_kernel(int potential,
+                                                         const double* __restrict__ o,
+                                                         const double* __restrict__ g, int n,
+                                                         double* __restrict__ out5,
+                                                         double* __restrict__ w) {
+  __shared__ double sh[3][16];
+  potential_block(potential, o, g, n, out5, w, nullptr, sh);
 }
 
 __global__ void gemv_rows_kernel(const double* __restrict__ x, int64_t rows, int n,
@@ -484,71 +492,130 @@ __device__ __forceinline__ void put_u(double v, int b, int q, int nq, double dq,
   }
 }
 
-// part[z][b][q] = sum over slice z of t of w[b][t] T[t][q] in FP64 (T float), on
-// the FP64 matrix cores: a block takes 16 chains x 16 bins, its 16 waves
-// consecutive parts of its slice, 4 of t per MFMA, added in wave order through
-// LDS.  All chains of a tile share the read of T.  It is latency and the reach
-// of a few CUs' loads that count (one block per 64 bins and chain, reading T for
-// each, took 25 us for one chain and 52 us for 64; the tiles in one slice 31 us):
-// four slices give 84 blocks at 330 bins, and a wave has 8 steps' loads in flight.
+// part[z][x][b][q] = sum over slice z of t of x[b][t] T[t][q] in FP64 (T float), on
+// the FP64 matrix cores, for x the target o and the computed g: a block takes
+// 16 chains x 16 bins, its 16 waves consecutive parts of its slice, 4 of t per
+// MFMA, added in wave order through LDS.  All chains of a tile share the read of T.
+// It is latency and the reach of a few CUs' loads that count (one block per 64
+// bins and chain, reading T for each, took 25 us for one chain and 52 us for 64;
+// the tiles in one slice 31 us): four slices give 84 blocks at 330 bins, and a
+// wave has a group's loads in flight.
 // Layout of v_mfma_f64_16x16x4 (lane l): A[l % 16][l / 16], B[l / 16][l % 16];
 // result v: row 4 v + l / 16, column l % 16.
 using v4d = double __attribute__((ext_vector_type(4)));
-constexpr int kAdjWaves = 16, kAdjAhead = 8;
+constexpr int kAdjWaves = 16, kAdjAhead = 1;
 
-__global__ __launch_bounds__(64 * kAdjWaves) void adjoint_kernel(const float* __restrict__ t,
-                                                                 int n_r, int nq,
-                                                                 const double* __restrict__ w,
-                                                                 int n_chain,
-                                                                 double* __restrict__ part) {
-  __shared__ double red[kAdjWaves][4][64];
+__device__ __forceinline__ void adjoint_block(const float* __restrict__ t, int n_r, int nq,
+                                              const double* __restrict__ o,
+                                              const double* __restrict__ g, int n_chain, int bx,
+                                              int by, int bz, double* __restrict__ part,
+                                              double (*red)[8][64]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int q = min(static_cast<int>(blockIdx.x) * 16 + (lane & 15), nq - 1);
-  const int b = min(static_cast<int>(blockIdx.y) * 16 + (lane & 15), n_chain - 1);
-  const int steps = (n_r + 3) / 4;
-  const int64_t sub = blockIdx.z * kAdjWaves + wave, n_sub = gridDim.z * kAdjWaves;
-  const int s0 = static_cast<int>(steps * sub / n_sub), s1 = static_cast<int>(steps * (sub + 1) / n_sub);
-  const double* wb = w + static_cast<size_t>(b) * n_r;
-  v4d acc = v4d{0.0, 0.0, 0.0, 0.0};
+  const int q = min(bx * 16 + (lane & 15), nq - 1);
+  const int b = min(by * 16 + (lane & 15), n_chain - 1);
+  // groups of 16 of t: lane l takes 4 (l / 16) .. + 3 of them, one in each of four
+  // MFMAs (any order of t gives the same sum), so that the lanes of a chain read a
+  // line of o and g
+  const int groups = (n_r + 15) / 16;
+  constexpr int kSub = kAdjointSlices * kAdjWaves;
+  const int sub = bz * kAdjWaves + wave;
+  const int s0 = static_cast<int>(static_cast<int64_t>(groups) * sub / kSub);
+  const int s1 = static_cast<int>(static_cast<int64_t>(groups) * (sub + 1) / kSub);
+  const double *ob = o + static_cast<size_t>(b) * n_r, *gb = g + static_cast<size_t>(b) * n_r;
+  v4d acc_o = v4d{0.0, 0.0, 0.0, 0.0}, acc_g = acc_o;
   for (int s = s0; s < s1; s += kAdjAhead) {
-    double x[kAdjAhead];
-    float y[kAdjAhead];
+    double x[kAdjAhead][4], z[kAdjAhead][4];
+    float y[kAdjAhead][4];
 #pragma unroll
-    for (int e = 0; e < kAdjAhead; ++e) {
-      const int at = min((s + e) * 4 + (lane >> 4), n_r - 1);
-      x[e] = wb[at];
-      y[e] = t[static_cast<size_t>(at) * nq + q];
+    for (int a = 0; a < kAdjAhead; ++a) {
+      const int at = min(s + a, s1 - 1) * 16 + 4 * (lane >> 4);
+      if (at + 3 < n_r) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[a][e] = ob[at + e];
+          z[a][e] = gb[at + e];
+          y[a][e] = t[static_cast<size_t>(at + e) * nq + q];
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int i = min(at + e, n_r - 1);
+          x[a][e] = at + e < n_r ? ob[i] : 0.0;
+          z[a][e] = at + e < n_r ? gb[i] : 0.0;
+          y[a][e] = at + e < n_r ? t[static_cast<size_t>(i) * nq + q] : 0.f;
+        }
+      }
     }
 #pragma unroll
-    for (int e = 0; e < kAdjAhead; ++e) {
-      const bool in = s + e < s1 && (s + e) * 4 + (lane >> 4) < n_r;
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(in ? x[e] : 0.0,
-                                                 in ? static_cast<double>(y[e]) : 0.0, acc, 0, 0, 0);
-    }
+    for (int a = 0; a < kAdjAhead; ++a)
+      if (s + a < s1) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const double tv = static_cast<double>(y[a][e]);
+          acc_o = __builtin_amdgcn_mfma_f64_16x16x4f64(x[a][e], tv, acc_o, 0, 0, 0);
+          acc_g = __builtin_amdgcn_mfma_f64_16x16x4f64(z[a][e], tv, acc_g, 0, 0, 0);
+        }
+      }
   }
 #pragma unroll
-  for (int v = 0; v < 4; ++v) red[wave][v][lane] = acc[v];
+  for (int v = 0; v < 4; ++v) {
+    red[wave][v][lane] = acc_o[v];
+    red[wave][4 + v][lane] = acc_g[v];
+  }
   __syncthreads();
-  if (wave >= 4) return;
-  double v = 0.0;  // wave v adds result v
+  if (wave >= 8) return;
+  double v = 0.0;  // wave v adds result v % 4 of factor v / 4
 #pragma unroll
   for (int k = 0; k < kAdjWaves; ++k) v += red[k][wave][lane];
-  const int row = blockIdx.y * 16 + 4 * wave + (lane >> 4), col = blockIdx.x * 16 + (lane & 15);
+  const int row = by * 16 + 4 * (wave & 3) + (lane >> 4), col = bx * 16 + (lane & 15);
   if (row < n_chain && col < nq)
-    part[(static_cast<size_t>(blockIdx.z) * n_chain + row) * nq + col] = v;
+    part[(static_cast<size_t>(bz * 2 + (wave >> 2)) * n_chain + row) * nq + col] = v;
 }
 
-__global__ void adjoint_sum_kernel(const double* __restrict__ part, int n_slice, int n_chain, int nq,
-                                   const double* __restrict__ gscale, double dq,
+// The potential of every chain (the first n_chain blocks) and, beside it, the
+// adjoint product: the adjoint vector w is a combination of o and g (mix), so
+// T^T o and T^T g need not wait for the sums that w takes.  One after the other they
+// took 14 us for one chain and 18 for 16 (4,000 points, 330 bins), together 9
+// and 11.  The blocks behind clear the F grids for the next call.
+__global__ __launch_bounds__(1024) void score_kernel(
+    int potential, const double* __restrict__ o, const double* __restrict__ g, int n_r, int n_chain,
+    double* __restrict__ out5, double2* __restrict__ mix, const float* __restrict__ t, int nq,
+    int n_bx, int n_adj, double* __restrict__ part, ulonglong2* __restrict__ clear, int64_t clear2) {
+  __shared__ union {
+    double sh[3][16];
+    double red[kAdjWaves][8][64];
+  } lds;
+  const int bid = blockIdx.x;
+  if (bid < n_chain) {
+    const size_t at = static_cast<size_t>(bid) * n_r;
+    potential_block(potential, o + at, g + at, n_r, out5 + 5 * static_cast<size_t>(bid), nullptr,
+                    mix + bid, lds.sh);
+  } else if (bid < n_chain + n_adj) {
+    const int a = bid - n_chain;
+    adjoint_block(t, n_r, nq, o, g, n_chain, a % n_bx, a / n_bx / kAdjointSlices,
+                  a / n_bx % kAdjointSlices, part, lds.red);
+  } else {
+    const int64_t first = bid - n_chain - n_adj;
+    for (int64_t w = first * 1024 + threadIdx.x; w < clear2;
+         w += (static_cast<int64_t>(gridDim.x) - n_chain - n_adj) * 1024)
+      clear[w] = ulonglong2{0ull, 0ull};
+  }
+}
+
+__global__ void adjoint_sum_kernel(const double* __restrict__ part, const double2* __restrict__ mix,
+                                   int n_chain, int nq, const double* __restrict__ gscale, double dq,
                                    const float* __restrict__ ftab, int weighted, int n_pair,
                                    float* __restrict__ u, double2* __restrict__ coef) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
   if (q >= nq) return;
   const size_t e = static_cast<size_t>(b) * nq + q, total = static_cast<size_t>(n_chain) * nq;
-  double v = 0.0;
-#pragma unroll 4
-  for (int s = 0; s < n_slice; ++s) v += part[s * total + e];
-  put_u(v * gscale[e], b, q, nq, dq, ftab, weighted, n_pair, u, coef);
+  double vo = 0.0, vg = 0.0;
+#pragma unroll
+  for (int s = 0; s < kAdjointSlices; ++s) {
+    vo += part[2 * s * total + e];
+    vg += part[(2 * s + 1) * total + e];
+  }
+  put_u(fma(mix[b].x, vo, mix[b].y * vg) * gscale[e], b, q, nq, dq, ftab, weighted, n_pair, u, coef);
 }
 
 __global__ void adjoint_fq_kernel(int nq, int q_first, const double* __restrict__ w,
@@ -658,9 +725,8 @@ hipError_t launch_gemm_grad(hipStream_t st, const void* rows, const float* row_s
 }
 
 hipError_t launch_potential(hipStream_t st, int potential, const double* gobs,
-                            const double* gcalc, int n, int n_chain, double* out5, double* w) {
-  hipLaunchKernelGGL(potential_kernel, dim3(n_chain), dim3(1024), 0, st, potential, gobs, gcalc, n,
-                     out5, w);
+                            const double* gcalc, int n, double* out5, double* w) {
+  hipLaunchKernelGGL(potential_kernel, dim3(1), dim3(1024), 0, st, potential, gobs, gcalc, n, out5, w);
   return hipGetLastError();
 }
 
@@ -672,15 +738,26 @@ hipError_t launch_gemv_rows(hipStream_t st, const double* x, int64_t rows, int n
   return hipGetLastError();
 }
 
-hipError_t launch_adjoint(hipStream_t st, const float* t, int n_r, int nq, const double* w,
-                          const double* gscale, int n_chain, double dq, const float* ftab,
-                          bool weighted, int n_pair, double* part, float* u, double2* coef) {
-  const dim3 tiles((nq + 15) / 16, (n_chain + 15) / 16, kAdjointSlices);
-  hipLaunchKernelGGL(adjoint_kernel, tiles, dim3(64 * kAdjWaves), 0, st, t, n_r, nq, w, n_chain,
-                     part);
-  hipLaunchKernelGGL(adjoint_sum_kernel, dim3((nq + 63) / 64, n_chain), dim3(64), 0, st, part,
-                     kAdjointSlices, n_chain, nq, gscale, dq, ftab, weighted ? 1 : 0, n_pair, u,
-                     coef);
+hipError_t launch_score(hipStream_t st, int potential, const double* gobs, const double* gcalc,
+                        int n_r, int n_chain, double* out5, double2* mix, const float* t, int nq,
+                        double* part, unsigned long long* clear, int64_t clear_words) {
+  const int n_bx = (nq + 15) / 16;
+  const int64_t n_adj = part ? static_cast<int64_t>(n_bx) * ((n_chain + 15) / 16) * kAdjointSlices : 0;
+  const int64_t clear2 = clear ? clear_words / 2 : 0;  // an even number of words
+  const int64_t n_clear = std::min<int64_t>((clear2 + 4095) / 4096, 256);
+  const int64_t blocks = n_chain + n_adj + n_clear;
+  if (blocks > 2147483647LL) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(score_kernel, dim3(static_cast<unsigned>(blocks)), dim3(1024), 0, st, potential,
+                     gobs, gcalc, n_r, n_chain, out5, mix, t, nq, n_bx, static_cast<int>(n_adj), part,
+                     reinterpret_cast<ulonglong2*>(clear), clear2);
+  return hipGetLastError();
+}
+
+hipError_t launch_adjoint_sum(hipStream_t st, const double* part, const double2* mix, int n_chain,
+                              int nq, const double* gscale, double dq, const float* ftab,
+                              bool weighted, int n_pair, float* u, double2* coef) {
+  hipLaunchKernelGGL(adjoint_sum_kernel, dim3((nq + 63) / 64, n_chain), dim3(64), 0, st, part, mix,
+                     n_chain, nq, gscale, dq, ftab, weighted ? 1 : 0, n_pair, u, coef);
   return hipGetLastError();
 }
 

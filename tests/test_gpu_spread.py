@@ -335,3 +335,57 @@ def test_gradient_transform_on_split_operands(ctx, n, nq, n_r, f64):
     assert np.isnan(got[4, 1]).all()
     np.testing.assert_array_equal(np.isnan(got[3, 0]), np.isnan(bad[0]))
     np.testing.assert_array_equal(np.isposinf(got[3, 0]), np.isposinf(bad[0]))
+
+
+@pytest.mark.parametrize("n", [2, 55, 99, 100, 101, 128, 129])
+@pytest.mark.parametrize("nq", [64, 65, 400, 830])
+def test_one_launch_with_two_elements(ctx, n, nq):
+    """F of small structures, one and two elements, up to and past the sizes that
+    one launch takes (128 and 100 atoms, 80 KB of grids)."""
+    pos = structures.jitter(structures.fcc_nearest(n), 0.05, seed=n).astype(np.float32)
+    check(ctx, pos, np.full(n, 79), 25.0 / nq, nq)
+    check(ctx, pos, np.array([28, 79])[np.random.RandomState(n).randint(0, 2, n)], 25.0 / nq, nq)
+
+
+@pytest.mark.parametrize("n_r", [15, 16, 17, 63, 1000])
+@pytest.mark.parametrize("zs", [(79,), (28, 79)])
+def test_energy_and_forces_of_g(ctx, n_r, zs):
+    """Energy and forces against G(r) from the gradient of G(r), for one chain,
+    and for each of 17 (a tile of 16 and one more).  Each entry of the gradient
+    may be off by 2^-20 of the largest, which the adjoint's weights add up; the
+    two numbers of tables in a launch round alike to 1e-6."""
+    nq, qbin, sizes = 200, 0.1, 20 + np.arange(17)
+    r = 2.0 + 0.02 * np.arange(n_r)
+    chains = [structures.jitter(structures.fcc_nearest(n), 0.05, seed=n).astype(np.float32) for n in sizes]
+    numbers = [np.array(zs)[np.arange(n) % len(zs)] for n in sizes]
+    table, index, _ = element_table(np.concatenate(numbers), qbin, nq)
+    ctx.set_transform(0.02, qbin, r, 0.0, nq)
+    alone, targets, at = [], [], 0
+    for pos, n in zip(chains, sizes):
+        ctx.set_positions(pos)
+        ctx.set_elements(index[at:at + n])
+        ctx.set_scatter(_lib.SLOT_PDF, table)
+        at += n
+        fq = ctx.fq(_lib.SLOT_PDF, qbin, nq)
+        g = ctx.pdf(fq, n_r)
+        target = g * (1.0 + 0.3 * np.sin(np.arange(n_r))) + 0.1
+        gg = ctx.grad_pdf(ctx.grad_fq(_lib.SLOT_PDF, qbin, n, nq), n_r)
+        e, f = ctx.pdf_energy_forces(_lib.SLOT_PDF, qbin, target, _lib.POT_RW, 10.0, n)
+        rw, a = oracle.get_rw(target, g)
+        want = 10.0 * oracle.wrap_grad_rw(gg, g, target)
+        res = target - a * g
+        w = 10.0 * np.abs(rw / np.sum(res ** 2) * a * res).sum()
+        assert abs(e - 10.0 * rw) < 1e-5
+        assert np.abs(f - want).max() < 2.0 ** -20 * w * np.abs(gg).max() + 1e-6 * np.abs(want).max()
+        alone.append((e, f))
+        targets.append(target)
+    ctx.set_batch(chains)
+    ctx.set_elements(index)
+    ctx.set_scatter(_lib.SLOT_PDF, table)
+    e, f = ctx.pdf_energy_forces(_lib.SLOT_PDF, qbin, np.array(targets), _lib.POT_RW, 10.0, len(index))
+    at = 0
+    for b, n in enumerate(sizes):
+        scale = np.abs(alone[b][1]).max()
+        assert abs(e[b] - alone[b][0]) < 1e-6 * abs(alone[b][0])
+        assert np.abs(f[at:at + n] - alone[b][1]).max() < 1e-6 * scale
+        at += n
