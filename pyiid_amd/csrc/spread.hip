@@ -311,16 +311,20 @@ __global__ __launch_bounds__(64 * kSmallWaves) void small_fq_kernel(
 }
 
 // Bound of the distances between the block's positions x[3] per call of get(a):
-// the diameter of the sphere about the middle of their box.
+// the diameter of the sphere about the middle of their box.  Waves reduce by
+// shuffles, then each reduces the waves' values the same way.  Latency and the
+// shuffles of the waves on one CU bound it, so few waves: with the packing 3.9 us
+// at 55 atoms (1 wave), 4.4 at 300 (4), 6.9 at 1,500 (8), where 16 waves that
+// each read all waves' values took 9 to 10.
 template <typename G>
 __device__ double block_reach(G get, int n) {
   __shared__ double box[16][6];
   __shared__ double rad[16];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_wave = blockDim.x >> 6;
   double v[6];  // max of x, y, z and of -x, -y, -z
   for (int k = 0; k < 6; ++k) v[k] = -1e308;
   bool bad = false;
-  for (int a = threadIdx.x; a < n; a += 1024) {
+  for (int a = threadIdx.x; a < n; a += blockDim.x) {
     double x[3];
     get(a, x);
     for (int k = 0; k < 3; ++k) {
@@ -334,10 +338,14 @@ __device__ double block_reach(G get, int n) {
   if (lane == 0)
     for (int k = 0; k < 6; ++k) box[wave][k] = v[k];
   const int any_bad = __syncthreads_or(bad ? 1 : 0);
-  for (int w = 0; w < 16; ++w)
-    for (int k = 0; k < 6; ++k) v[k] = fmax(v[k], box[w][k]);
+  if (n_wave > 1) {
+    const int w = min(lane & 15, n_wave - 1);
+    for (int k = 0; k < 6; ++k) v[k] = box[w][k];
+    for (int off = 8; off > 0; off >>= 1)
+      for (int k = 0; k < 6; ++k) v[k] = fmax(v[k], __shfl_xor(v[k], off, 64));
+  }
   double r2 = 0.0;
-  for (int a = threadIdx.x; a < n; a += 1024) {
+  for (int a = threadIdx.x; a < n; a += blockDim.x) {
     double x[3];
     get(a, x);
     double d = 0.0;
@@ -347,7 +355,10 @@ __device__ double block_reach(G get, int n) {
   for (int off = 32; off > 0; off >>= 1) r2 = fmax(r2, __shfl_xor(r2, off, 64));
   if (lane == 0) rad[wave] = r2;
   __syncthreads();
-  for (int w = 0; w < 16; ++w) r2 = fmax(r2, rad[w]);
+  if (n_wave > 1) {
+    r2 = rad[min(lane & 15, n_wave - 1)];
+    for (int off = 8; off > 0; off >>= 1) r2 = fmax(r2, __shfl_xor(r2, off, 64));
+  }
   return any_bad ? __builtin_inf() : 2.0 * sqrt(r2) * 1.000001;
 }
 
@@ -392,7 +403,7 @@ __global__ __launch_bounds__(1024) void pack_reach_kernel(const float* __restric
                                                           AtomRec* __restrict__ out,
                                                           float* __restrict__ keep,
                                                           double* __restrict__ reach) {
-  for (int i = threadIdx.x; i < n; i += 1024) pack_one(p, e, i, out, keep);
+  for (int i = threadIdx.x; i < n; i += blockDim.x) pack_one(p, e, i, out, keep);
   const double r = block_reach(
       [&](int a, double* x) {
         for (int k = 0; k < 3; ++k) x[k] = p[3 * a + k];
@@ -504,8 +515,8 @@ hipError_t launch_pack(hipStream_t st, const float* p, const int32_t* e, int64_t
                        float* keep, double* reach) {
   if (n == 0) return hipSuccess;
   if (reach && n <= kReachAtoms)
-    hipLaunchKernelGGL(pack_reach_kernel, dim3(1), dim3(1024), 0, st, p, e, static_cast<int>(n), out,
-                       keep, reach);
+    hipLaunchKernelGGL(pack_reach_kernel, dim3(1), dim3(n <= 256 ? 64 : n <= 1024 ? 256 : 512), 0, st,
+                       p, e, static_cast<int>(n), out, keep, reach);
   else
     hipLaunchKernelGGL(pack_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st,
                        p, e, n, out, keep);
