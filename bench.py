@@ -23,6 +23,7 @@ sys.path.insert(0, ROOT)
 METRIC = ("Debye F(Q)+grad pair·Q evals/s; HMC wall-s to target Rw "
           "(surrogate vs exact)")
 PEAK_FP32_TFLOPS = 157.3   # MI355X FP32 vector peak (published)
+PEAK_FP16_TFLOPS = 2500.0  # MI355X dense FP16 matrix peak
 FLOP_PER_PAIR_Q = 21       # F + grad, sin/cos counted as 1 FLOP, FMA as 2
 QBIN, NQ, RADIUS, LATTICE, SIGMA, SEED = 0.02, 1250, 30.0, 4.08, 0.05, 0
 
@@ -37,8 +38,9 @@ def workload():
 
 
 def read_traffic(label="au6699_q1250", kernel="fused_grad"):
-    """HBM bytes per launch of the F + gradient kernel (`kernel`: fused_grad,
-    the ordered one, or sym_grad) on workload `label` from the committed
+    """HBM bytes per launch of the F + gradient kernel (`kernel`: spread_grad
+    with its matrix product, fused_grad, the ordered recurrence kernel, or
+    sym_grad) on workload `label` from the committed
     rocprof counter summary (FETCH_SIZE + WRITE_SIZE, scaled by the copy-kernel
     calibration), or None when it has not been measured."""
     path = os.path.join(ROOT, "profiles", "%s_%s_traffic.txt" % (kernel, label))
@@ -69,11 +71,46 @@ def grad_kernel_setup(ctx):
 def grad_kernel_name(ctx):
     """(profile name, description) of the kernel the last grad_fq ran."""
     sym, bpw, group = ctx.grad_shape()
+    if bpw == 0:
+        return "spread_grad", ("spread_grad_kernel (pairs onto a grid per atom) and "
+                               "gemm_split_kernel (sine transform, split FP16 MFMA)")
     if sym:
         return "sym_grad", ("sym_grad_kernel (F + grad, unordered pairs), %d bins per wave, "
                             "%d tiles per item" % (bpw, group))
     return "fused_grad", ("fused_grad_kernel (F + grad, ordered pairs), %d bins per wave, "
                           "%d j ranges per tile" % (bpw, group))
+
+
+def grad_roofline(ctx, pos, nq, n_run, avg_s, label):
+    """What the F + gradient kernels' average launch time `avg_s` means.
+
+    The recurrence kernels: FLOP_PER_PAIR_Q per pair and bin against the FP32
+    peak.  The spreading kernels do no work per pair and bin: their floating
+    point work is the product of the atoms' grids (3 rows each, for each of
+    `n_run` elements) with the sine matrix, three FP16 products for one, over
+    the grid points that the structure's extent reaches, against the dense FP16
+    matrix peak; the pairs' adds in LDS (25 per ordered pair) stand beside it."""
+    kname, kdesc = grad_kernel_name(ctx)
+    n = len(pos)
+    if kname != "spread_grad":
+        flop, peak, bound = FLOP_PER_PAIR_Q * (n * (n - 1) // 2) * nq, PEAK_FP32_TFLOPS, "valu"
+    else:
+        x = pos.astype(np.float64)
+        extent = 2.0 * np.linalg.norm(x - 0.5 * (x.max(0) + x.min(0)), axis=1).max()
+        half = (9 * nq + 3) // 4
+        points = min(extent * QBIN * half / np.pi + 18.0, half + 17)
+        flop = 6 * 3 * n * nq * n_run * ((int(points) + 31) // 32 * 32)
+        peak, bound = PEAK_FP16_TFLOPS, "lds, mfma"
+    achieved = flop / avg_s / 1e12
+    out = {"kernel": kdesc, "bound": bound, "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
+           "frac": achieved / peak, "traffic": read_traffic(label, kname),
+           "avg_launch_ms": avg_s * 1e3}
+    if kname == "spread_grad":
+        out["flop"] = flop
+        out["lds_adds_per_s"] = 25.0 * n * (n - 1) / avg_s
+    else:
+        out["flop_per_unit"] = FLOP_PER_PAIR_Q
+    return out
 
 
 def host_cpu():
@@ -312,8 +349,7 @@ def headline_20k(steps=3, warmup=1):
     sphere (r = 43.3 A, 1,250 bins of 0.02) and the 20,000-atom Pt/Ni random
     alloy (50/50 seeded, nearest FCC sites at a = 3.724 A, 1,500 bins of
     0.02), device-resident inputs and outputs.  Per workload: wall time per
-    step, the fused kernel's average launch (HIP events) and its algorithmic
-    fraction of FP32 peak."""
+    step and the F + gradient kernels' roofline (HIP events)."""
     import torch
     from pyiid_amd import _lib, structures
     from pyiid_amd.formfactors import element_table
@@ -351,15 +387,11 @@ def headline_20k(steps=3, warmup=1):
         wall = (time.perf_counter() - t0) / steps
         ms, k = ctx.kernel_time(_lib.KERNEL_FUSED)
         ctx.enable_timing(False)
-        kname, kdesc = grad_kernel_name(ctx)
-        ctx.close()
         pairs = n * (n - 1) // 2
-        avg_s = ms / max(1, k) / 1e3
-        achieved = FLOP_PER_PAIR_Q * pairs * nq / avg_s / 1e12
+        roof = grad_roofline(ctx, pos, nq, len(np.unique(index)), ms / max(1, k) / 1e3, label)
+        ctx.close()
         out[label] = {"atoms": n, "q_bins": nq, "steps": steps, "ms_per_step": wall * 1e3,
-                      "pair_q_per_s": pairs * nq / wall, "kernel": kdesc,
-                      "fused_avg_launch_ms": avg_s * 1e3, "achieved_tflops": achieved,
-                      "frac": achieved / PEAK_FP32_TFLOPS, "traffic": read_traffic(label, kname)}
+                      "pair_q_per_s": pairs * nq / wall, "roofline": roof}
         del g, f
     return out
 
@@ -532,9 +564,8 @@ def kernel_suite(reps=3):
     ms = timed(c20, _lib.KERNEL_FUSED, lambda: _lib.check(c20.lib.pyiid_grad_fq(
         c20.handle, _lib.SLOT_FQ, ctypes.c_double(QBIN), ctypes.c_void_p(g20.data_ptr()),
         ctypes.c_void_p(f20.data_ptr()), dev)))
-    out["fused_grad_kernel_20k"] = {"ms": ms, "atoms": n20, "kernel": grad_kernel_name(c20)[1],
-                                    "pair_q_per_s": p20 * NQ / (ms * 1e-3),
-                                    "tflops_alg": FLOP_PER_PAIR_Q * p20 * NQ / (ms * 1e-3) / 1e12}
+    out["grad_kernel_20k"] = {"ms": ms, "atoms": n20, "pair_q_per_s": p20 * NQ / (ms * 1e-3),
+                              "roofline": grad_roofline(c20, pos20, NQ, 1, ms * 1e-3, "au20113_q1250")}
     del g20, f20
     c20.close()
     # the 20,000-atom Pt/Ni random alloy (50/50, Cromer-Mann per element), 1,500 bins
@@ -555,9 +586,9 @@ def kernel_suite(reps=3):
     ms = timed(ca, _lib.KERNEL_FUSED, lambda: _lib.check(ca.lib.pyiid_grad_fq(
         ca.handle, _lib.SLOT_FQ, ctypes.c_double(QBIN), ctypes.c_void_p(ga.data_ptr()),
         ctypes.c_void_p(fa.data_ptr()), dev)))
-    out["fused_grad_kernel_alloy20k"] = {"ms": ms, "kernel": grad_kernel_name(ca)[1],
-                                         "pair_q_per_s": pa * 1500 / (ms * 1e-3),
-                                         "tflops_alg": FLOP_PER_PAIR_Q * pa * 1500 / (ms * 1e-3) / 1e12}
+    out["grad_kernel_alloy20k"] = {"ms": ms, "pair_q_per_s": pa * 1500 / (ms * 1e-3),
+                                   "roofline": grad_roofline(ca, posa, 1500, 2, ms * 1e-3,
+                                                             "ptni20000_q1500")}
     del ga, fa
     ca.close()
     d = torch.empty((pairs, 3), dtype=torch.float32, device="cuda")
@@ -713,11 +744,10 @@ def main():
     t1 = time.perf_counter()
     fused_ms, fused_n = ctx.kernel_time(_lib.KERNEL_FUSED)
     ctx.enable_timing(False)
-    kname, kdesc = grad_kernel_name(ctx)
     elapsed = t1 - t0
     value = pairs * NQ * args.steps / elapsed
-    avg_s = fused_ms / max(1, fused_n) / 1e3
-    achieved = FLOP_PER_PAIR_Q * pairs * NQ / avg_s / 1e12
+    roof = grad_roofline(ctx, pos, NQ, 1, fused_ms / max(1, fused_n) / 1e3, "au6699_q1250")
+    roof["launches"] = fused_n
 
     out = {
         "metric": METRIC,
@@ -741,18 +771,7 @@ def main():
             "q_bins": NQ,
             "parallelism": "single GPU",
         },
-        "roofline": {
-            "kernel": kdesc,
-            "bound": "valu",
-            "achieved": achieved,
-            "peak": PEAK_FP32_TFLOPS,
-            "unit": "TFLOP/s",
-            "frac": achieved / PEAK_FP32_TFLOPS,
-            "traffic": read_traffic("au6699_q1250", kname),
-            "avg_launch_ms": avg_s * 1e3,
-            "launches": fused_n,
-            "flop_per_unit": FLOP_PER_PAIR_Q,
-        },
+        "roofline": roof,
     }
     ctx.close()
     if not args.skip_20k:

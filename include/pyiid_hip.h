@@ -64,28 +64,33 @@ int pyiid_set_stream(pyiid_ctx *ctx, void *stream);
 int pyiid_synchronize(pyiid_ctx *ctx);
 /* Kernel timing with HIP events on the launch stream: when enabled, every
  * launch of the Debye kernels is bracketed by events and its duration summed.
- * kind: 0 = F+grad kernel (ordered or symmetric, pyiid_grad_shape tells
- *       which), 1 = F-only kernel, 2 = transform GEMM,
- *       3 = pair-geometry kernel, 4 = contracted-force (unordered pair) kernel. */
+ * kind: 0 = F+grad kernels (spreading, ordered or symmetric, pyiid_grad_shape
+ *       tells which; the spreading one with its matrix product), 1 = F-only
+ *       kernel (spreading: without its transform), 2 = transform GEMM,
+ *       3 = pair-geometry kernel, 4 = contracted-force kernels. */
 int pyiid_enable_timing(pyiid_ctx *ctx, int enable);
 int pyiid_kernel_time(pyiid_ctx *ctx, int kind, double *total_ms, int64_t *launches);
-/* While timing is enabled, the F-only kernel counts its (wave, j atom) steps
- * by recurrence form: the three-term form, or the Reinsch form that a wave
+/* While timing is enabled, the F-only recurrence kernel (which runs when its
+ * bins per wave are fixed, with compensated sums, or past the spreading kernel's
+ * limits) counts its (wave, j atom) steps by recurrence form: the three-term form, or the Reinsch form that a wave
  * takes when any of its pairs has a per-bin phase step within 0.2 of a
  * multiple of pi.  Counts since timing was last enabled.  No counterpart in
  * the reference. */
 int pyiid_fq_form_counts(pyiid_ctx *ctx, int64_t *three_term, int64_t *reinsch);
-/* Q bins per wave of the F-only kernel: 64, 72, 80, 88, 96 or 112 fixes the
- * launch shape; 0 (the default) lets the autotuner time the six once per
- * problem shape and keep the fastest.  The shapes differ only in how the bins are
+/* Q bins per wave of the F-only recurrence kernel: 64, 72, 80, 88, 96 or 112 runs
+ * pyiid_fq on that kernel with that launch shape; 0 (the default) runs the
+ * spreading kernel, and past its limits (compensated sums, about 3,400 bins)
+ * the recurrence kernel at the shape that the autotuner found fastest.
+ * The shapes differ only in how the bins are
  * grouped, so F agrees between them to FP32 rounding.  No counterpart in the
  * reference (its kernels have no launch-shape choice). */
 int pyiid_set_fq_bins_per_wave(pyiid_ctx *ctx, int m);
 /* Q bins per wave of the ordered-pair F + gradient kernel: 16 or 32 runs
  * pyiid_grad_fq on that kernel with that launch shape (and the default j
- * split); 0 (the default) lets the autotuner choose between the symmetric
- * (unordered-pair) kernel and the ordered one, and time the ordered one's two
- * shapes with three split sizes each, once per problem shape.  Kernels and
+ * split); 0 (the default) runs the spreading kernel, and past its limits
+ * (compensated sums, about 3,000 bins) lets the autotuner choose between the
+ * symmetric (unordered-pair) kernel and the ordered one, and time the ordered one's
+ * two shapes with three split sizes each, once per problem shape.  Kernels and
  * shapes differ only in how the sums are grouped, so the results agree to
  * FP32 rounding.  No counterpart in the reference (its kernels have no
  * launch-shape choice). */
@@ -93,8 +98,8 @@ int pyiid_set_grad_bins_per_wave(pyiid_ctx *ctx, int m);
 /* Tiles of 64 atoms per I group and per J range of a work item of the
  * symmetric F + gradient kernel: 4, 8, 16 or 32 runs pyiid_grad_fq on that
  * kernel with that grouping (unless compensated sums are on or the ordered
- * kernel's bins per wave are fixed); 0 (the default) leaves the choice to the
- * autotuner.  Larger groups write fewer partial-sum slots (about 3 nq 64 x 4
+ * kernel's bins per wave are fixed); 0 (the default) leaves the choice as
+ * pyiid_set_grad_bins_per_wave says.  Larger groups write fewer partial-sum slots (about 3 nq 64 x 4
  * bytes each, tiles^2 / k of them) and give fewer, longer blocks.  No
  * counterpart in the reference. */
 int pyiid_set_grad_tiles_per_item(pyiid_ctx *ctx, int k);
@@ -103,9 +108,9 @@ int pyiid_set_grad_tiles_per_item(pyiid_ctx *ctx, int k);
  * lets the autotuner time both.  The results agree to FP32 rounding.  No
  * counterpart in the reference. */
 int pyiid_set_grad_sym_bins_per_wave(pyiid_ctx *ctx, int m);
-/* Kernel of pyiid_grad_fq: PYIID_GRAD_AUTO (the default) lets the autotuner
- * choose, PYIID_GRAD_ORDERED and PYIID_GRAD_SYMMETRIC restrict it to one
- * kernel (whose launch shapes are still autotuned unless fixed by the setters
+/* Kernel of pyiid_grad_fq: PYIID_GRAD_AUTO (the default) runs the spreading
+ * kernel within its limits and lets the autotuner choose past them,
+ * PYIID_GRAD_ORDERED and PYIID_GRAD_SYMMETRIC restrict it to one recurrence kernel (whose launch shapes are still autotuned unless fixed by the setters
  * above).  Compensated sums always run the ordered kernel.  No counterpart in
  * the reference. */
 #define PYIID_GRAD_AUTO 0
@@ -119,18 +124,21 @@ int pyiid_set_grad_kernel(pyiid_ctx *ctx, int kernel);
  * for the spreading kernel (whose pair work does not depend on the bins).  No
  * counterpart in the reference. */
 int pyiid_grad_shape(pyiid_ctx *ctx, int *symmetric, int *bins_per_wave, int *group);
-/* Autotuning of the Debye kernels' launch shapes (F + gradient kernel and its
- * grouping, F-only bins per wave, contracted-force Q groups), on by
+/* Autotuning of the recurrence kernels' launch shapes (F + gradient kernel and
+ * its grouping, F-only bins per wave, contracted-force Q groups; the spreading
+ * kernels have none), on by
  * default: the first call for a problem shape times the candidates and keeps
  * the fastest.  Off (enable = 0): every call uses fixed default shapes (the
  * ordered F + gradient kernel unless pyiid_set_grad_tiles_per_item is set), so
  * results are the same bit for bit from run to run and context to context;
  * with it on they agree to FP32 rounding.  No counterpart in the reference. */
 int pyiid_set_autotune(pyiid_ctx *ctx, int enable);
-/* Summation of the Debye kernels' FP32 per-bin sums.
- *  - PYIID_PRECISION_DEFAULT: plain FP32 sums over runs of at most 2,048
- *    j atoms, then FP64 across runs and tiles.
- *  - PYIID_PRECISION_COMPENSATED: compensated FP32 sums.  The terms of each
+/* Summation of the Debye kernels.
+ *  - PYIID_PRECISION_DEFAULT: the spreading kernels (fixed-point sums over
+ *    pairs); in the recurrence kernels plain FP32 per-bin sums over runs of at
+ *    most 2,048 j atoms, then FP64 across runs and tiles.
+ *  - PYIID_PRECISION_COMPENSATED: the recurrence kernels with compensated FP32
+ *    per-bin sums.  The terms of each
  *    256-atom j tile gather in a second register, which an error-free TwoSum
  *    folds into the running sum.  The F + gradient kernel then runs 16 bins
  *    per wave in 8-wave blocks.
@@ -171,8 +179,7 @@ int pyiid_set_scatter(pyiid_ctx *ctx, int slot, const float *table, int32_t n_el
  * (cpu_wrappers/flat_multi_cpu_wrap.py:22-60, gpu_wrappers/gpu_wrap.py:119-156). */
 int pyiid_fq(pyiid_ctx *ctx, int slot, double qbin, float *fq, int flags);
 /* -1/2 dF/dq as the reference returns it: (N, 3, n_q), Q fastest; float32,
- * or double with PYIID_F64.  `fq` (nullable) receives F(Q) from the same
- * fused kernel.  Replaces wrap_fq_grad(atoms, qbin, sum_type)
+ * or double with PYIID_F64.  `fq` (nullable) receives F(Q).  Replaces wrap_fq_grad(atoms, qbin, sum_type)
  * (flat_multi_cpu_wrap.py:63-102, gpu_wrap.py:159-194). */
 int pyiid_grad_fq(pyiid_ctx *ctx, int slot, double qbin, void *grad, float *fq, int flags);
 /* Flat pair geometry for pairs k in [k_offset, k_offset + k_count) with

@@ -159,7 +159,7 @@ class Context:
     """One device context: a HIP stream plus the device-resident structure,
     scatter tables, transform and workspaces (``pyiid_ctx``).
 
-    Launch shapes are autotuned per problem shape; the environment variable
+    The recurrence kernels' launch shapes are autotuned per problem shape; the environment variable
     PYIID_AUTOTUNE=0 starts every context with fixed shapes instead
     (results that repeat bit for bit), as ``set_autotune(False)`` does."""
 
@@ -205,11 +205,13 @@ class Context:
                                            else PRECISION_DEFAULT))
 
     def set_fq_bins_per_wave(self, m):
-        """Fix the F-only kernel's Q bins per wave (64, 72, 80, 88, 96, 112), or 0 to autotune."""
+        """Run F on the recurrence kernel with these Q bins per wave (64, 72, 80, 88, 96, 112); 0:
+        the spreading kernel."""
         check(self.lib.pyiid_set_fq_bins_per_wave(self.handle, int(m)))
 
     def set_grad_bins_per_wave(self, m):
-        """Fix the fused F + gradient kernel's Q bins per wave (16, 32), or 0 to autotune."""
+        """Run F + gradient on the ordered recurrence kernel with these Q bins per wave (16, 32);
+        0: the spreading kernel."""
         check(self.lib.pyiid_set_grad_bins_per_wave(self.handle, int(m)))
 
     def set_grad_tiles_per_item(self, k):
@@ -221,12 +223,14 @@ class Context:
         check(self.lib.pyiid_set_grad_sym_bins_per_wave(self.handle, int(m)))
 
     def set_grad_kernel(self, kernel):
-        """GRAD_AUTO, GRAD_ORDERED or GRAD_SYMMETRIC: the kernel of grad_fq."""
+        """The kernel of grad_fq: GRAD_AUTO (spreading), or the GRAD_ORDERED or GRAD_SYMMETRIC
+        recurrence kernel."""
         check(self.lib.pyiid_set_grad_kernel(self.handle, int(kernel)))
 
     def grad_shape(self):
         """Launch shape of the last grad_fq: (symmetric, bins per wave, group), where group is
-        the symmetric kernel's tiles per item or the ordered kernel's j ranges per tile."""
+        the symmetric kernel's tiles per item or the ordered kernel's j ranges per tile; all
+        zero for the spreading kernel."""
         a, b, g = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
         check(self.lib.pyiid_grad_shape(self.handle, ctypes.byref(a), ctypes.byref(b),
                                         ctypes.byref(g)))

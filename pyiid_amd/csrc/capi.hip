@@ -226,6 +226,9 @@ struct pyiid_ctx {
   bool extent_exact = false;        // r_max bounds the current positions' distances
   Buf reach;                        // double: such a bound on the device
   bool reach_set = false;           // of the current positions
+  Buf place, ordered;               // an atom's place in element order; the positions so
+  uint64_t place_stamp = ~0ull;
+  bool order_set = false;           // ordered holds the current positions
   bool share_order = false;         // within one call (SharedOrder)
   const AtomRec* in_order = nullptr;
 
@@ -454,7 +457,8 @@ int ensure_packed(pyiid_ctx* c) {
   if (!c->pos_set) return fail(PYIID_E_STATE, "positions not set");
   if (!c->pos_dirty || c->n == 0) return PYIID_OK;
   HIPCHK(launch_pack(c->stream, c->posf.as<float>(), c->elem.as<int32_t>(), c->n,
-                     c->pos.as<AtomRec>(), nullptr, nullptr));
+                     c->pos.as<AtomRec>(), nullptr, nullptr, nullptr, nullptr));
+  c->order_set = false;
   c->pos_dirty = false;
   return PYIID_OK;
 }
@@ -935,16 +939,19 @@ bool use_spread_fq(pyiid_ctx* c, const Table& t) {
 // bins spreads for itself, where that takes about as long as the three launches
 // for one call alone and less among others (us, 500 bins, alone and among others:
 // 55 atoms 25 and 8 against 32 and 13, 128 atoms 34 and 8 against 34 and 13, 150
-// atoms 39 and 9 against 34 and 13; two elements, 100 atoms 37 and 9 against 37
-// and 15, 128 atoms 41 and 10 against 37 and 15).  The chip takes about 5 us for
-// two million pairs times blocks.
+// atoms 39 and 9 against 34 and 13; 260 bins, two elements, 85 atoms 30 and 9
+// against 30 and 14, 96 atoms 33 and 9 against 30 and 14; three elements, 55
+// atoms 31 and 9 against 29 and 14, 85 atoms 35 and 9 against 30 and 14).  The chip
+// takes about 5 us for two million pairs times blocks.
 bool use_small_fq(pyiid_ctx* c, const Table& t) {
-  if (element_pairs(t) > 3 || small_fq_lds(t.nq, static_cast<int>(element_pairs(t))) > kSmallFqLds)
+  if (element_pairs(t) > 6 || small_fq_lds(t.nq, static_cast<int>(element_pairs(t))) > kSmallFqLds)
     return false;
+  const int64_t kinds = element_pairs(t);
+  const int most = kinds == 1 ? kSmallAtoms : kinds == 3 ? kSmallAtoms2 : kSmallAtoms3;
   int64_t pairs = 0;
   for (int b = 0; b < c->n_chain; ++b) {
     const int64_t n = c->off[b + 1] - c->off[b];
-    if (n > (element_pairs(t) == 1 ? kSmallAtoms : kSmallAtoms2)) return false;
+    if (n > most) return false;
     pairs += n * (n - 1) / 2;
   }
   return pairs * ((t.nq + 63) / 64) <= 2000000;
@@ -1110,6 +1117,21 @@ hipError_t launch_fq_items(pyiid_ctx* c, const Table& t, double qbin, bool count
                    c->fpart.as<double>(), forms);
 }
 
+bool caller_captures(pyiid_ctx* c) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(c->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
+// Whether b can be made `want` bytes now: not in a capture of the caller's, and
+// there has to be the memory.
+bool scratch(pyiid_ctx* c, Buf& b, size_t want) {
+  if (want <= b.bytes) return true;
+  if (caller_captures(c)) return false;
+  if (b.reserve(want) == PYIID_OK) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 // Lets the kernels of one call, between which the atoms stay where they are, use
 // one copy of the positions in element order (each set's perm is the same order).
 struct SharedOrder {
@@ -1121,14 +1143,28 @@ struct SharedOrder {
   }
 };
 
+// The positions in element order: from the packing, or gathered.  After the first
+// gather of a structure the packing of uploads places the atoms itself (a launch
+// less per call).
 int in_element_order(pyiid_ctx* c, const Buf& perm, const Buf& sorted, const AtomRec** sp) {
-  if (c->in_order) {
-    *sp = c->in_order;
+  if (c->order_set || c->in_order) {
+    *sp = c->order_set ? c->ordered.as<AtomRec>() : c->in_order;
     return PYIID_OK;
   }
   HIPCHK(launch_gather(c->stream, c->pos.as<AtomRec>(), perm.as<int32_t>(), c->n, sorted.as<AtomRec>()));
   *sp = sorted.as<AtomRec>();
   if (c->share_order) c->in_order = *sp;
+  if (c->place_stamp != c->struct_stamp && !c->capturing &&
+      scratch(c, c->ordered, sizeof(AtomRec) * c->n) && scratch(c, c->place, sizeof(int32_t) * c->n) &&
+      !caller_captures(c)) {
+    std::vector<int32_t> order, place(static_cast<size_t>(c->n));
+    std::vector<std::vector<ElemRun>> runs;
+    element_runs(c, true, order, runs);
+    for (int64_t p = 0; p < c->n; ++p) place[order[p]] = static_cast<int32_t>(p);
+    HIPCHK(hipStreamSynchronize(c->stream));  // a packing under way reads the last places
+    CHK(upload_vec(c->place, place));
+    c->place_stamp = c->struct_stamp;
+  }
   return PYIID_OK;
 }
 
@@ -1866,21 +1902,6 @@ int gemm_t(pyiid_ctx* c, const void* a, bool a64, int64_t rows, double* out) {
   return tm.done();
 }
 
-bool caller_captures(pyiid_ctx* c) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(c->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
-}
-
-// Whether b can be made `want` bytes now: not in a capture of the caller's, and
-// there has to be the memory.
-bool scratch(pyiid_ctx* c, Buf& b, size_t want) {
-  if (want <= b.bytes) return true;
-  if (caller_captures(c)) return false;
-  if (b.reserve(want) == PYIID_OK) return true;
-  (void)hipGetLastError();
-  return false;
-}
-
 // out = rows of the gradient times T^T: on split operands where they pay, in
 // chunks of 64 MB of split rows.
 constexpr size_t kSplitBudget = static_cast<size_t>(64) << 20;
@@ -1998,9 +2019,12 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
     // (the gradient of a single structure asks how far its distances reach)
     CHK(c->reach.reserve(sizeof(double)));
     const bool reach = (flags & PYIID_DEVICE) && c->n_chain == 1 && n <= kReachAtoms;
+    const bool order = c->place_stamp == c->struct_stamp;
     HIPCHK(launch_pack(c->stream, src, c->elem.as<int32_t>(), n, c->pos.as<AtomRec>(),
-                       c->posf.as<float>(), reach ? c->reach.as<double>() : nullptr));
+                       c->posf.as<float>(), reach ? c->reach.as<double>() : nullptr,
+                       order ? c->place.as<int32_t>() : nullptr, c->ordered.as<AtomRec>()));
     c->reach_set = reach;
+    c->order_set = order;
     c->pos_dirty = false;
   } else {
     CHK(upload(c, c->posf.p, pos, sizeof(float) * 3 * n, flags));
@@ -2488,7 +2512,7 @@ int pyiid_destroy(pyiid_ctx* c) {
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
   destroy_graph(c->hmc);
-  for (Buf* b : {&c->posf, &c->elem, &c->pos, &c->counts_d, &c->natoms_d, &c->off_d, &c->tmat, &c->tsplit, &c->tsplit_scale, &c->gsplit, &c->gsplit_scale, &c->gpart,
+  for (Buf* b : {&c->posf, &c->elem, &c->pos, &c->counts_d, &c->natoms_d, &c->off_d, &c->tmat, &c->place, &c->ordered, &c->tsplit, &c->tsplit_scale, &c->gsplit, &c->gsplit_scale, &c->gpart,
                  &c->fpart, &c->fq64, &c->fq32, &c->g64, &c->io_a, &c->io_b,
                  &c->io_c, &c->w, &c->out5, &c->u, &c->ucoef, &c->upart, &c->mix, &c->gobs, &c->fq_items.items,
                  &c->fq_items.ranges, &c->fq_items.perm, &c->spread.units, &c->spread.items,
@@ -3154,6 +3178,7 @@ int pyiid_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step, do
   if (n_proposals == 0) return PYIID_OK;
   c->extent_exact = false;
   c->reach_set = false;
+  c->order_set = false;
   CHK(prepare_history(c, n_proposals));
   CHK(refresh_exact(c));
   RunClock clock(c, times_ms != nullptr);
@@ -3345,6 +3370,7 @@ int pyiid_sur_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step
   if (n_proposals == 0) return PYIID_OK;
   c->extent_exact = false;
   c->reach_set = false;
+  c->order_set = false;
   CHK(prepare_history(c, n_proposals));
   RunClock clock(c, times_ms != nullptr);
   bool exact_block = false;

@@ -140,7 +140,7 @@ hipError_t launch_transform_fq(hipStream_t st, unsigned long long* grids, int n_
                                float* out_f32, bool one_part);
 // F of chains of at most kSmallAtoms atoms (off: n_chain + 1 offsets) in one
 // launch; the grids must fit kSmallFqLds.
-constexpr int kSmallAtoms = 128, kSmallAtoms2 = 100;  // one element; two
+constexpr int kSmallAtoms = 128, kSmallAtoms2 = 85, kSmallAtoms3 = 70;  // by elements
 constexpr size_t kSmallFqLds = 80 * 1024;
 size_t small_fq_lds(int nq, int n_pair);
 hipError_t launch_small_fq(hipStream_t st, const AtomRec* pos, const int* off, int n_chain,
@@ -148,10 +148,11 @@ hipError_t launch_small_fq(hipStream_t st, const AtomRec* pos, const int* off, i
                            int scale_bits, const double* scale, double* out_f64, float* out_f32);
 // Atom records from float positions and elements; keep (nullable) takes a copy
 // of the positions, reach (nullable) a bound of their distances (one block
-// then: for at most kReachAtoms atoms).
+// then: for at most kReachAtoms atoms); with place (nullable) ordered[place[i]]
+// takes the record too.
 constexpr int64_t kReachAtoms = 4096;
 hipError_t launch_pack(hipStream_t st, const float* p, const int32_t* e, int64_t n, AtomRec* out,
-                       float* keep, double* reach);
+                       float* keep, double* reach, const int32_t* place, AtomRec* ordered);
 // *reach: a bound of the distances within pos (its bounding sphere's diameter;
 // infinite where a position is not finite)
 hipError_t launch_reach(hipStream_t st, const AtomRec* pos, int64_t n, double* reach);

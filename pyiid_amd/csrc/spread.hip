@@ -377,7 +377,8 @@ __global__ __launch_bounds__(1024) void reach_kernel(const AtomRec* __restrict__
 
 __device__ __forceinline__ void pack_one(const float* __restrict__ p, const int32_t* __restrict__ e,
                                          int64_t i, AtomRec* __restrict__ out,
-                                         float* __restrict__ keep) {
+                                         float* __restrict__ keep, const int32_t* __restrict__ place,
+                                         AtomRec* __restrict__ ordered) {
   const float x = p[3 * i + 0], y = p[3 * i + 1], z = p[3 * i + 2];
   AtomRec a;
   a.x = x;
@@ -385,6 +386,7 @@ __device__ __forceinline__ void pack_one(const float* __restrict__ p, const int3
   a.z = z;
   a.w = static_cast<double>(e[i]);
   out[i] = a;
+  if (place) ordered[place[i]] = a;
   if (keep) {
     keep[3 * i + 0] = x;
     keep[3 * i + 1] = y;
@@ -393,17 +395,21 @@ __device__ __forceinline__ void pack_one(const float* __restrict__ p, const int3
 }
 
 __global__ void pack_kernel(const float* __restrict__ p, const int32_t* __restrict__ e, int64_t n,
-                            AtomRec* __restrict__ out, float* __restrict__ keep) {
+                            AtomRec* __restrict__ out, float* __restrict__ keep,
+                            const int32_t* __restrict__ place, AtomRec* __restrict__ ordered) {
   const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-  if (i < n) pack_one(p, e, i, out, keep);
+  if (i < n) pack_one(p, e, i, out, keep, place, ordered);
 }
 
 __global__ __launch_bounds__(1024) void pack_reach_kernel(const float* __restrict__ p,
                                                           const int32_t* __restrict__ e, int n,
                                                           AtomRec* __restrict__ out,
                                                           float* __restrict__ keep,
-                                                          double* __restrict__ reach) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) pack_one(p, e, i, out, keep);
+                                                          double* __restrict__ reach,
+                                                          const int32_t* __restrict__ place,
+                                                          AtomRec* __restrict__ ordered) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x)
+    pack_one(p, e, i, out, keep, place, ordered);
   const double r = block_reach(
       [&](int a, double* x) {
         for (int k = 0; k < 3; ++k) x[k] = p[3 * a + k];
@@ -487,39 +493,45 @@ hipError_t launch_small_fq(hipStream_t st, const AtomRec* pos, const int* off, i
   const int nf = 12 * nq, stride = fq_grid_stride(nq);
   const double inv_h = dq * nf / (2.0 * M_PI);
   const size_t lds = small_fq_lds(nq, n_pair);
-  if (lds > kSmallFqLds || n_chain > 65535 || (n_pair != 1 && n_pair != 3)) return hipErrorInvalidValue;
+  if (lds > kSmallFqLds || n_chain > 65535 || (n_pair != 1 && n_pair != 3 && n_pair != 6))
+    return hipErrorInvalidValue;
   static const hipError_t attr = [] {
-    const hipError_t e =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(small_fq_kernel<1>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kSmallFqLds));
-    return e != hipSuccess ? e
-                           : hipFuncSetAttribute(reinterpret_cast<const void*>(small_fq_kernel<3>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 static_cast<int>(kSmallFqLds));
+    for (const void* f : {reinterpret_cast<const void*>(small_fq_kernel<1>),
+                          reinterpret_cast<const void*>(small_fq_kernel<3>),
+                          reinterpret_cast<const void*>(small_fq_kernel<6>)}) {
+      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               static_cast<int>(kSmallFqLds));
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
   }();
   if (attr != hipSuccess) return attr;
   const dim3 grid((nq + 63) / 64, n_chain), block(64 * kSmallWaves);
   const double unit = fq_unit(inv_h, 0, scale_bits), near = std::ldexp(1.0, scale_bits - 31);
   const float one = std::ldexp(1.0f, scale_bits);
   const float* f = weighted ? ftab : nullptr;
+#define PYIID_SMALL(N)                                                                            \
+  hipLaunchKernelGGL(small_fq_kernel<N>, grid, block, lds, st, pos, off, nf, fq_grid_points(nq),  \
+                     stride, unit, one, near, f, nq, inv_h, scale, out_f64, out_f32)
   if (n_pair == 1)
-    hipLaunchKernelGGL(small_fq_kernel<1>, grid, block, lds, st, pos, off, nf, fq_grid_points(nq),
-                       stride, unit, one, near, f, nq, inv_h, scale, out_f64, out_f32);
+    PYIID_SMALL(1);
+  else if (n_pair == 3)
+    PYIID_SMALL(3);
   else
-    hipLaunchKernelGGL(small_fq_kernel<3>, grid, block, lds, st, pos, off, nf, fq_grid_points(nq),
-                       stride, unit, one, near, f, nq, inv_h, scale, out_f64, out_f32);
+    PYIID_SMALL(6);
+#undef PYIID_SMALL
   return hipGetLastError();
 }
 
 hipError_t launch_pack(hipStream_t st, const float* p, const int32_t* e, int64_t n, AtomRec* out,
-                       float* keep, double* reach) {
+                       float* keep, double* reach, const int32_t* place, AtomRec* ordered) {
   if (n == 0) return hipSuccess;
   if (reach && n <= kReachAtoms)
     hipLaunchKernelGGL(pack_reach_kernel, dim3(1), dim3(n <= 256 ? 64 : n <= 1024 ? 256 : 512), 0, st,
-                       p, e, static_cast<int>(n), out, keep, reach);
+                       p, e, static_cast<int>(n), out, keep, reach, place, ordered);
   else
     hipLaunchKernelGGL(pack_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st,
-                       p, e, n, out, keep);
+                       p, e, n, out, keep, place, ordered);
   return hipGetLastError();
 }
 

@@ -337,14 +337,15 @@ def test_gradient_transform_on_split_operands(ctx, n, nq, n_r, f64):
     np.testing.assert_array_equal(np.isposinf(got[3, 0]), np.isposinf(bad[0]))
 
 
-@pytest.mark.parametrize("n", [2, 55, 99, 100, 101, 128, 129])
-@pytest.mark.parametrize("nq", [64, 65, 400, 830])
+@pytest.mark.parametrize("n", [2, 55, 70, 71, 85, 86, 128, 129])
+@pytest.mark.parametrize("nq", [64, 65, 270, 400, 830])
 def test_one_launch_with_two_elements(ctx, n, nq):
-    """F of small structures, one and two elements, up to and past the sizes that
-    one launch takes (128 and 100 atoms, 80 KB of grids)."""
+    """F of small structures, one to three elements, up to and past the sizes that
+    one launch takes (128, 85 and 70 atoms, 80 KB of grids)."""
     pos = structures.jitter(structures.fcc_nearest(n), 0.05, seed=n).astype(np.float32)
     check(ctx, pos, np.full(n, 79), 25.0 / nq, nq)
     check(ctx, pos, np.array([28, 79])[np.random.RandomState(n).randint(0, 2, n)], 25.0 / nq, nq)
+    check(ctx, pos, np.array([28, 78, 79])[np.random.RandomState(n).randint(0, 3, n)], 25.0 / nq, nq)
 
 
 @pytest.mark.parametrize("n_r", [15, 16, 17, 63, 1000])
@@ -389,3 +390,52 @@ def test_energy_and_forces_of_g(ctx, n_r, zs):
         assert abs(e[b] - alone[b][0]) < 1e-6 * abs(alone[b][0])
         assert np.abs(f[at:at + n] - alone[b][1]).max() < 1e-6 * scale
         at += n
+
+
+@pytest.mark.parametrize("kinds", [2, 3])
+def test_uploads_in_element_order(ctx, kinds):
+    """From the second upload of a structure on the packing puts the atoms in
+    element order: F, gradient and forces equal a new context's, also after the
+    elements have changed and after a sampler has moved the atoms."""
+    n, nq, qbin, zs = 150, 300, 0.08, np.array([28, 78, 79])[:kinds]
+    rs = np.random.RandomState(kinds)
+    base = structures.fcc_nearest(n)
+    target = 0.5 + 0.1 * np.cos(np.arange(400))
+
+    def elements(c, numbers):
+        table, index, _ = element_table(numbers, qbin, nq)
+        c.set_elements(index)
+        c.set_scatter(_lib.SLOT_FQ, table)
+        c.set_scatter(_lib.SLOT_PDF, table)
+        c.set_transform(0.02, qbin, 2.0 + 0.02 * np.arange(400), 0.0, nq)
+
+    def results(c, pos):
+        c.set_positions(pos)
+        fq = np.empty(nq, np.float32)
+        g = c.grad_fq(_lib.SLOT_FQ, qbin, n, nq, fq_out=fq)
+        e, f = c.pdf_energy_forces(_lib.SLOT_PDF, qbin, target, _lib.POT_RW, 10.0, n)
+        return c.fq(_lib.SLOT_FQ, qbin, nq), fq, g, np.float64(e), f
+
+    def fresh(numbers, pos):
+        c = _lib.Context(0)
+        c.set_positions(pos)
+        elements(c, numbers)
+        out = results(c, pos)
+        c.close()
+        return out
+
+    ctx.set_positions(base.astype(np.float32))
+    for step in range(6):
+        numbers = zs[np.random.RandomState(step // 3).permutation(np.arange(n) % kinds)]
+        pos = (base + rs.normal(0, 0.05, (n, 3))).astype(np.float32)
+        if step % 3 == 0:
+            elements(ctx, numbers)
+        for got, want in zip(results(ctx, pos), fresh(numbers, pos)):
+            np.testing.assert_array_equal(got, want)
+        if step == 4:
+            ctx.hmc_setup(_lib.SLOT_PDF, qbin, target, _lib.POT_RW, 10.0, np.full(n, 100.0))
+            ctx.hmc_run(2, 2, 0.5, 1.0, 1, 1)
+            after, want = ctx.fq(_lib.SLOT_FQ, qbin, nq), fresh(numbers, ctx.get_positions(n))[0]
+            # the sampler's positions are FP64, those handed out float32 (6e-7 A)
+            assert np.abs(after - want).max() < 1e-4 * np.abs(want).max()
+            assert np.abs(ctx.get_positions(n) - pos).max() > 1e-3
