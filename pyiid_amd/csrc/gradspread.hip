@@ -305,7 +305,7 @@ __device__ __forceinline__ void spread_grad_rows(
   }
 }
 
-__global__ __launch_bounds__(1024, 8) void spread_grad_kernel(
+__global__ __launch_bounds__(512, 8) void spread_grad_kernel(
     const AtomRec* __restrict__ pos, int p0, int n_rows, const int* __restrict__ runs, double inv_h,
     int nf, int plane, int row_len, int k_fixed, const double* __restrict__ reach, int nq,
     float scale, double near, bool narrow, _Float16* __restrict__ rows,
@@ -318,7 +318,7 @@ __global__ __launch_bounds__(1024, 8) void spread_grad_kernel(
 // The same with the work units of F(Q) as further blocks behind the atoms': for a
 // structure of a few hundred atoms a launch costs more than either part (505
 // atoms, 164 bins: six launches 22.9 us a call among others, four 18.9).
-__global__ __launch_bounds__(1024, 8) void spread_both_kernel(
+__global__ __launch_bounds__(512, 8) void spread_both_kernel(
     const AtomRec* __restrict__ pos, int n_atoms, const int* __restrict__ runs, double inv_h, int nf,
     int plane, int row_len, int k_fixed, const double* __restrict__ reach, int nq, float scale,
     double near, bool narrow, _Float16* __restrict__ rows, float* __restrict__ row_scale,
@@ -472,7 +472,12 @@ GradLaunch grad_launch(int64_t n, int nq, double dq, double r_max) {
   g.plane = row_points(nq) | 1;
   g.row_len = grad_row_len(nq);
   g.lds = grad_lds_bytes(nq);
-  g.threads = n <= 256 ? 256 : n <= 2048 ? 512 : 1024;
+  // small blocks where six or more fit a CU: their starts and ends overlap better and
+  // fewer lanes idle in the last round of atoms (us, alone and among others, 256, 512
+  // and 1,024 threads: 1,289 atoms, 330 bins 61 32, 61 34, 66 39; 4,000 atoms of two
+  // elements, 600 bins 312 263, 318 268, 343 295; 6,699 atoms, 1,250 bins, whose grids
+  // leave two blocks, 683 607, 615 547, 615 550)
+  g.threads = n <= 256 || g.lds <= 27 * 1024 ? 256 : 512;
   return g;
 }
 }  // namespace
