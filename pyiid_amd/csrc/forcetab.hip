@@ -50,7 +50,7 @@ NodeFit node_fit() {
 }
 
 constexpr int kTabSplit = 2;     // halves of a chunk of bins, side by side in a block
-constexpr int kTabChunk = 1024;  // bins staged in LDS at a time
+constexpr int kTabChunk = 1024;  // bins staged in LDS at a time (PARTS > 1)
 
 // Block: CELLS cells x 6 nodes x 2 halves of every chunk of bins of one table
 // (chain, element pair); a wave holds the cells of 64 / CELLS nodes, or PARTS parts
@@ -58,68 +58,107 @@ constexpr int kTabChunk = 1024;  // bins staged in LDS at a time
 // recurrence along Q from the part's first bin.  Tables of 64 chains are bound by
 // their FP64 operations (PARTS = 1: the two starting phases of a chain of 165 bins
 // are a few percent); a single table of 400 cells by the chain's length (PARTS = 4).
-template <int CELLS, int PARTS>
+// TABLES tables of a block share the sines and cosines, half of the operations of
+// one alone; their coefficients, the same for a whole wave, come by scalar loads,
+// for LDS reads of every bin by every wave bound the kernel (256 tables of 2,100
+// cells: one a block from LDS 208 us, by scalar loads 240, four from LDS 241, by
+// scalar loads 127).
+template <int CELLS, int PARTS, int TABLES>
 __global__ __launch_bounds__(64 * kNodes * kTabSplit * CELLS * PARTS / 64) void force_table_kernel(
-    const double2* __restrict__ coef, int nq, double dq, int n_cell, double h, NodeFit fit,
+    const double2* __restrict__ coef, int nq, double dq, int n_table, int n_cell, double h, NodeFit fit,
     float4* __restrict__ t4, float2* __restrict__ t2) {
   constexpr int kNodesPer = 64 / (CELLS * PARTS);  // of a wave
   constexpr int kWaves = kNodes / kNodesPer;       // of a half
-  __shared__ double2 cf[kTabChunk];
   __shared__ double val[kTabSplit][2][kNodes][CELLS * PARTS];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int in_cell = lane % CELLS, part = lane / CELLS % PARTS;
   const int node = wave % kWaves * kNodesPer + lane / (CELLS * PARTS), half = wave / kWaves;
   const int cell = blockIdx.x * CELLS + in_cell;
   const int sub = half * PARTS + part;
-  const size_t table = blockIdx.y;
+  const int table0 = blockIdx.y * TABLES;
   const double x = dq * ((cell + 0.5 + fit.y[node]) * h) / M_PI;  // phase per bin / pi
   double s1, c1;
   sincospi(x, &s1, &c1);
   const double k2 = 2.0 * c1;
-  double a = 0.0, b = 0.0;
-  for (int m0 = 0; m0 < nq; m0 += kTabChunk) {
-    const int cnt = min(kTabChunk, nq - m0);
-    if (m0 > 0) __syncthreads();
-    for (int m = threadIdx.x; m < cnt; m += blockDim.x) cf[m] = coef[table * nq + m0 + m];
-    const int lo = cnt * sub / (kTabSplit * PARTS), hi = cnt * (sub + 1) / (kTabSplit * PARTS);
-    double s = 0.0, c = 1.0;
-    if (m0 + lo > 0) sincospi(x * (m0 + lo), &s, &c);
-    double sp = s * c1 - c * s1, cp = c * c1 + s * s1;  // one bin before
-    __syncthreads();
-#pragma unroll 8
+  double a[TABLES] = {}, b[TABLES] = {};
+  auto start = [&](int m, double& s, double& c, double& sp, double& cp) {
+    s = 0.0;
+    c = 1.0;
+    if (m > 0) sincospi(x * m, &s, &c);
+    sp = s * c1 - c * s1;  // one bin before
+    cp = c * c1 + s * s1;
+  };
+  double s, c, sp, cp;
+  if constexpr (TABLES > 1) {
+    static_assert(PARTS == 1, "the bins are the wave's");
+    const double2* w[TABLES];
+#pragma unroll
+    for (int k = 0; k < TABLES; ++k) w[k] = coef + static_cast<size_t>(min(table0 + k, n_table - 1)) * nq;
+    const int lo = nq * half / kTabSplit, hi = nq * (half + 1) / kTabSplit;
+    start(lo, s, c, sp, cp);
+#pragma unroll 4
     for (int m = lo; m < hi; ++m) {
-      const double2 w = cf[m];
-      a = fma(w.x, c, a);
-      b = fma(w.y, s, b);
+#pragma unroll
+      for (int k = 0; k < TABLES; ++k) {
+        a[k] = fma(w[k][m].x, c, a[k]);
+        b[k] = fma(w[k][m].y, s, b[k]);
+      }
       const double sn = fma(k2, s, -sp), cn = fma(k2, c, -cp);
       sp = s;
       cp = c;
       s = sn;
       c = cn;
     }
-  }
-  val[half][0][node][part * CELLS + in_cell] = a;
-  val[half][1][node][part * CELLS + in_cell] = b;
-  __syncthreads();
-  if (cell >= n_cell || half != 0 || part != 0) return;
-  double p = 0.0;
-#pragma unroll
-  for (int n = 0; n < kNodes; ++n) {
-    const double inv = 1.0 / ((cell + 0.5 + fit.y[n]) * h);
-    double an = 0.0, bn = 0.0;
-#pragma unroll
-    for (int k = 0; k < PARTS; ++k) {
-      an += val[0][0][n][k * CELLS + in_cell] + val[1][0][n][k * CELLS + in_cell];
-      bn += val[0][1][n][k * CELLS + in_cell] + val[1][1][n][k * CELLS + in_cell];
+  } else {
+    __shared__ double2 cf[kTabChunk];
+    for (int m0 = 0; m0 < nq; m0 += kTabChunk) {
+      const int cnt = min(kTabChunk, nq - m0);
+      if (m0 > 0) __syncthreads();
+      for (int m = threadIdx.x; m < cnt; m += blockDim.x)
+        cf[m] = coef[static_cast<size_t>(table0) * nq + m0 + m];
+      const int lo = cnt * sub / (kTabSplit * PARTS), hi = cnt * (sub + 1) / (kTabSplit * PARTS);
+      start(m0 + lo, s, c, sp, cp);
+      __syncthreads();
+#pragma unroll 8
+      for (int m = lo; m < hi; ++m) {
+        a[0] = fma(cf[m].x, c, a[0]);
+        b[0] = fma(cf[m].y, s, b[0]);
+        const double sn = fma(k2, s, -sp), cn = fma(k2, c, -cp);
+        sp = s;
+        cp = c;
+        s = sn;
+        c = cn;
+      }
     }
-    p = fma(fit.c[node][n], (an - bn * inv) * (inv * inv), p);
   }
-  const size_t at = table * n_cell + cell;
-  // node k holds coefficient k: 0..3 in t4, 4 and 5 in t2
-  if (node < 4)
-    reinterpret_cast<float*>(t4 + at)[node] = static_cast<float>(p);
-  else
-    reinterpret_cast<float*>(t2 + at)[node - 4] = static_cast<float>(p);
+#pragma unroll
+  for (int k = 0; k < TABLES; ++k) {
+    if (k > 0) __syncthreads();  // the table before is done
+    val[half][0][node][part * CELLS + in_cell] = a[k];
+    val[half][1][node][part * CELLS + in_cell] = b[k];
+    __syncthreads();
+    const int table = table0 + k;
+    if (cell >= n_cell || half != 0 || part != 0 || table >= n_table) continue;
+    double p = 0.0;
+#pragma unroll
+    for (int n = 0; n < kNodes; ++n) {
+      const double inv = 1.0 / ((cell + 0.5 + fit.y[n]) * h);
+      double an = 0.0, bn = 0.0;
+#pragma unroll
+      for (int q = 0; q < PARTS; ++q) {
+        an += val[0][0][n][q * CELLS + in_cell] + val[1][0][n][q * CELLS + in_cell];
+        bn += val[0][1][n][q * CELLS + in_cell] + val[1][1][n][q * CELLS + in_cell];
+      }
+      p = fma(fit.c[node][n], (an - bn * inv) * (inv * inv), p);
+    }
+    const size_t at = static_cast<size_t>(table) * n_cell + cell;
+    // node k holds coefficient k: 0..3 in t4, 4 and 5 in t2
+    if (node < 4)
+      reinterpret_cast<float*>(t4 + at)[node] = static_cast<float>(p);
+    else
+      reinterpret_cast<float*>(t2 + at)[node - 4] = static_cast<float>(p);
+  }
 }
 
 // P(r) beyond the table (an atom that has left the extent the table was made
@@ -316,17 +355,22 @@ hipError_t launch_force_table(hipStream_t st, const double2* coef, int nq, doubl
   // instead of 16 for one table of 1,600 cells; beyond, the starting phases of
   // the parts cost more than the shorter chains save (16 tables of 1,080 cells:
   // 20 us against 15).  Up to about four blocks of 64 cells per CU half blocks
-  // leave the CUs more even (14.0 us against 15.4)
-#define PYIID_TABLE(CELLS, PARTS)                                                            \
-  hipLaunchKernelGGL((force_table_kernel<CELLS, PARTS>), dim3((n_cell + CELLS - 1) / CELLS, n_table), \
-                     dim3(kNodes * kTabSplit * CELLS * PARTS), 0, st, coef, nq, dq, n_cell,  \
-                     force_cell(nq, dq), fit, t4, t2)
+  // leave the CUs more even (14.0 us against 15.4).  Many tables go by fours (64 of
+  // 2,400 cells: 50 us against 70)
+  const int64_t blocks = static_cast<int64_t>((n_cell + 63) / 64) * n_table;
+#define PYIID_TABLE(CELLS, PARTS, TABLES)                                                        \
+  hipLaunchKernelGGL((force_table_kernel<CELLS, PARTS, TABLES>),                               \
+                     dim3((n_cell + CELLS - 1) / CELLS, (n_table + TABLES - 1) / TABLES),      \
+                     dim3(kNodes * kTabSplit * CELLS * PARTS), 0, st, coef, nq, dq, n_table,   \
+                     n_cell, force_cell(nq, dq), fit, t4, t2)
   if (static_cast<int64_t>((n_cell + 15) / 16) * n_table <= 512)
-    PYIID_TABLE(16, 4);
-  else if (static_cast<int64_t>((n_cell + 63) / 64) * n_table <= 1024)
-    PYIID_TABLE(32, 1);
+    PYIID_TABLE(16, 4, 1);
+  else if (blocks <= 1024)
+    PYIID_TABLE(32, 1, 1);
+  else if (blocks <= 2048)
+    PYIID_TABLE(64, 1, 1);
   else
-    PYIID_TABLE(64, 1);
+    PYIID_TABLE(64, 1, 4);
 #undef PYIID_TABLE
   return hipGetLastError();
 }

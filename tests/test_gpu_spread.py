@@ -439,3 +439,30 @@ def test_uploads_in_element_order(ctx, kinds):
             # the sampler's positions are FP64, those handed out float32 (6e-7 A)
             assert np.abs(after - want).max() < 1e-4 * np.abs(want).max()
             assert np.abs(ctx.get_positions(n) - pos).max() > 1e-3
+
+
+@pytest.mark.parametrize("chains", [61, 66])
+@pytest.mark.parametrize("nq", [200, 201])
+def test_forces_of_many_chains(ctx, chains, nq):
+    """Tables made four to a block (more than 2,048 blocks of 64 cells; the last
+    four are not whole) against one chain alone, whose table rounds alike to
+    1e-6."""
+    qbin, n, r = 25.0 / nq, 24, 2.0 + 0.02 * np.arange(200)
+    base = structures.fcc_nearest(n)
+    pos = [structures.jitter(base, 0.05, seed=b).astype(np.float32) for b in range(chains)]
+    for p in pos:
+        p[0] += np.float32(55.0)  # a wide extent: about 2,200 cells
+    table, index, _ = element_table(np.full(n * chains, 79), qbin, nq)
+    target = np.tile(0.5 + 0.1 * np.cos(np.arange(200)), (chains, 1))
+    ctx.set_batch(pos)
+    ctx.set_elements(index)
+    ctx.set_scatter(_lib.SLOT_PDF, table)
+    ctx.set_transform(0.02, qbin, r, 0.0, nq)
+    e, f = ctx.pdf_energy_forces(_lib.SLOT_PDF, qbin, target, _lib.POT_RW, 10.0, n * chains)
+    for b in (0, 1, chains // 2, chains - 2, chains - 1):
+        ctx.set_positions(pos[b])
+        ctx.set_elements(index[:n])
+        ctx.set_scatter(_lib.SLOT_PDF, table)
+        want_e, want = ctx.pdf_energy_forces(_lib.SLOT_PDF, qbin, target[b], _lib.POT_RW, 10.0, n)
+        assert abs(e[b] - want_e) < 1e-6 * abs(want_e)
+        assert np.abs(f[b * n:(b + 1) * n] - want).max() < 1e-6 * np.abs(want).max()
