@@ -83,11 +83,12 @@ __device__ void spread_rare(unsigned long long* hist, int n_grid, double t, doub
   }
 }
 
-// A pair in the fixed point's fast range.
-__device__ __forceinline__ void spread_pair(unsigned long long* hist, double t, double nf,
+// A pair in the fixed point's fast range; false past kFqFar.
+__device__ __forceinline__ bool spread_pair(unsigned long long* hist, double t, double nf,
                                             double half_nf, float scale) {
   float w = scale * __builtin_amdgcn_rcpf(static_cast<float>(t));
   if (t > half_nf) {
+    if (!(t < kFqFar)) return false;
     bool neg;
     t = fold(t, nf, neg);
     if (neg) w = -w;
@@ -103,6 +104,7 @@ __device__ __forceinline__ void spread_pair(unsigned long long* hist, double t, 
     atomicAdd(&h[k], static_cast<unsigned long long>(static_cast<long long>(a)));
     atomicAdd(&h[kFqW - 1 - k], static_cast<unsigned long long>(static_cast<long long>(b)));
   }
+  return true;
 }
 
 // One block (at least 4 waves) per work unit: a run of items of one chain and element
@@ -112,11 +114,13 @@ __device__ __forceinline__ void spread_pair(unsigned long long* hist, double t, 
 // the range, and a j atom's position is wave-uniform (scalar loads, so the
 // FP64 differences take it from SGPRs).
 //
-// Per 64 pairs about 16 FP64 or conversion instructions (distance to 1e-14:
-// a phase of 1,500 rad to 1e-11), 18 FMAs for the window, 6 conversions to
-// integer and 6 ds_add_u64.  The LDS adds (29 ns per CU) and the VALU (about
-// as long, 4 SIMDs) run side by side, and 2 blocks (32 waves) per CU hide
-// each other's latency.
+// Per 64 pairs about 14 FP64 or conversion instructions (distance to 4e-14:
+// a phase of 1,500 rad to 6e-11), 18 FMAs for the window, 6 conversions to
+// integer and 6 ds_add_u64.  The LDS adds bound it (busy 93% of the time, two
+// thirds of that bank conflicts of random addresses); the VALU is busy nearly as
+// long beside it, and 2 blocks (32 waves) per CU hide each other's latency.  A
+// tile off the diagonal needs two comparisons a pair (1,988 -> 1,930 us for 64
+// chains of 5,000 atoms, where every pair took five).
 __device__ __forceinline__ void spread_fq_unit(
     const AtomRec* __restrict__ pos, const SpreadUnit& un, const SpreadItem* __restrict__ items,
     double inv_h, int nf, int n_grid, int stride, int shift, float scale, double near,
@@ -134,19 +138,24 @@ __device__ __forceinline__ void spread_fq_unit(
     const int jb = item.j0 + static_cast<int>(len * wave >> wave_bits);
     const int je = item.j0 + static_cast<int>(len * (wave + 1) >> wave_bits);
     const int i = item.i0 + lane;
-    const bool have = i < item.i1;
-    const AtomRec pi = pos[have ? i : item.i0];
-    for (int j = jb; j < je; ++j) {
-      const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
+    if (i >= item.i1) continue;
+    const AtomRec pi = pos[i];
+    // (a pair at distance 0, or with a NaN, contributes nothing)
+    auto pair = [&](const AtomRec& pj) {
+      const double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
       const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-      // j < i; a pair at distance 0 (and one with a NaN) contributes nothing
-      if (!(have && j < i && r2 > 0.0)) continue;
-      double t = scaled_root(r2, inv_h);
-      if (!(t >= near && t < kFqFar)) {
+      const double t = scaled_root(r2, inv_h);
+      if (t >= near) {
+        if (!spread_pair(hist, t, static_cast<double>(nf), half_nf, scale)) rare = true;
+      } else if (r2 > 0.0) {
         rare = true;
-        continue;
       }
-      spread_pair(hist, t, static_cast<double>(nf), half_nf, scale);
+    };
+    if (item.j1 <= item.i0) {
+      for (int j = jb; j < je; ++j) pair(pos[j]);
+    } else {
+      for (int j = jb; j < je; ++j)
+        if (j < i) pair(pos[j]);
     }
   }
   // few pairs of a physical structure, if any, are left for a second look

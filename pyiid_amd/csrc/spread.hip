@@ -257,9 +257,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void small_fq_kernel(
       grid += (hi * (hi + 1) / 2 + min(x, y)) * stride;
     }
     const double t = scaled_root(r2, inv_h);
-    if (t >= near && t < kFqFar)
-      spread_pair(grid, t, static_cast<double>(nf), half_nf, scale);
-    else
+    if (!(t >= near && spread_pair(grid, t, static_cast<double>(nf), half_nf, scale)))
       spread_rare(grid, n_grid, sqrt(r2) * inv_h, static_cast<double>(nf), static_cast<double>(scale));
   }
   bin_terms(terms, m, nf, unit);
