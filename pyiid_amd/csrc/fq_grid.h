@@ -11,12 +11,17 @@ namespace {
 constexpr int kFqW = 6;             // grid points per pair
 constexpr double kFqBeta = 15.160;  // window shape (smallest r.m.s. error at 6 points)
 // phi_j(y), j < 3, y in [-1/2, 1/2] about the middle of the window;
-// phi_{5-j}(y) = phi_j(-y)
+// phi_{5-j}(y) = phi_j(-y).  A least squares fit with every coefficient rounded to
+// its nearest float had its mean over y 1.7e-8 short of phihat, and v_rcp_f32, which
+// makes 1/t, is 6.8e-9 short on average: F was off by one factor, 1 - 2.4e-8, which
+// no number of pairs averages out (6,699 atoms, 1,250 bins: 4.7e-8 of the largest F
+// at worst).  Here the fit and the choice of floats hold the mean, with v_rcp_f32's,
+// within 4e-9 over the band (3.8e-9 r.m.s. of single places).
 constexpr float kFqVal[3][6] = {
-    {0.000792858506f, -0.00591184293f, 0.0172319146f, -0.0255775783f, 0.0208579919f,
-     -0.00803987611f},
-    {0.0737481676f, -0.206023853f, 0.19830423f, -0.0388040482f, -0.062571443f, 0.0402357172f},
-    {0.425458973f, -0.352369105f, -0.215536146f, 0.244299265f, 0.041713486f, -0.0805066679f},
+    {0.000792802835f, -0.00590729201f, 0.0172293913f, -0.0255970359f, 0.0208720788f,
+     -0.00801460911f},
+    {0.0737483203f, -0.206045285f, 0.198311478f, -0.0387120843f, -0.0626117215f, 0.0401164442f},
+    {0.425458878f, -0.352327496f, -0.215540871f, 0.244120404f, 0.0417396985f, -0.0802748948f},
 };
 // Fixed point of the grid: phi_j 2^s / t, t = r / h.  s is chosen from the
 // structure's extent so that a pair at its largest distance still has 2^24

@@ -16,9 +16,9 @@
 // q = 0 (the Kaiser-Bessel window's transform), and the phi_j(y) are the least
 // squares solution of sum_j phi_j(y) exp(i q (g_j - y)) = phihat(q) over the
 // band |q| <= pi / 6, fitted by polynomials of degree 5 in y.  The result is
-// exp(i Q r) to 2.3e-8 at worst and 3.6e-9 r.m.s. over the band and y
-// (coefficients rounded to float: 2.5e-8 r.m.s.; single-precision sin and cos
-// of the phase have 3e-8).
+// exp(i Q r) to 2.6e-8 at worst and 3.8e-9 r.m.s. over the band and y, with the
+// float coefficients too; evaluated in single precision 2.3e-8 r.m.s., which pairs
+// average out (single-precision sin and cos of the phase have 3e-8).
 //
 // The grid is folded: sin(2 pi g m / n_f) is odd about g = 0 and g = n_f / 2
 // and has period n_f, so a distance of any size is brought into [0, n_f / 2]
