@@ -4,6 +4,8 @@
 
 #include "pair_math.h"
 
+#include "fold.h"
+
 namespace pyiid {
 namespace {
 
@@ -46,17 +48,9 @@ __host__ __device__ inline double fq_node(int k) {  // t of node k
 
 // ---- spreading ----
 
-// Brings t = r / h into [0, n_f / 2]; neg: the reflected half (sin changes sign).
-__device__ __forceinline__ double fold(double t, double nf, bool& neg) {
-  const double u = t - nf * floor(t / nf);
-  neg = u > 0.5 * nf;
-  return neg ? nf - u : u;
-}
-
-constexpr double kFqFar = 1e15;  // beyond: spread_rare
-
 // A pair closer than the fixed point's fast range, or at an infinite
-// distance: 64-bit conversions.  Few pairs of a physical structure come here.
+// distance: 64-bit conversions.  Few pairs of a physical structure come here, and
+// those from kFarthest on add nothing.
 __device__ void spread_rare(unsigned long long* hist, int n_grid, double t, double nf,
                                          double scale) {
   unsigned long long* nodes = hist + n_grid;
@@ -75,7 +69,8 @@ __device__ void spread_rare(unsigned long long* hist, int n_grid, double t, doub
     return;
   }
   bool neg;
-  const double tf = fold(t, nf, neg);
+  double tf;
+  if (!fold(t, nf, tf, neg)) return;
   const double fl = floor(tf);
   const double y = tf - fl - 0.5, w = (neg ? -scale : scale) / t;
   unsigned long long* h = hist + (static_cast<int>(fl) + 1);
@@ -88,14 +83,13 @@ __device__ void spread_rare(unsigned long long* hist, int n_grid, double t, doub
   }
 }
 
-// A pair in the fixed point's fast range; false past kFqFar.
+// A pair in the fixed point's fast range; false past kFarthest.
 __device__ __forceinline__ bool spread_pair(unsigned long long* hist, double t, double nf,
                                             double half_nf, float scale) {
   float w = scale * __builtin_amdgcn_rcpf(static_cast<float>(t));
   if (t > half_nf) {
-    if (!(t < kFqFar)) return false;
     bool neg;
-    t = fold(t, nf, neg);
+    if (!fold(t, nf, t, neg)) return false;
     if (neg) w = -w;
   }
   const float y = static_cast<float>(__builtin_amdgcn_fract(t)) - 0.5f;
@@ -175,7 +169,7 @@ __device__ __forceinline__ void spread_fq_unit(
         const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
         if (!(j < i && r2 > 0.0)) continue;
         const double t = scaled_root(r2, inv_h);
-        if (t >= near && t < kFqFar) continue;
+        if (t >= near && t < kFarthest) continue;
         spread_rare(hist, n_grid, sqrt(r2) * inv_h, static_cast<double>(nf),
                     static_cast<double>(scale));
       }

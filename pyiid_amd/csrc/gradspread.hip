@@ -70,7 +70,6 @@ constexpr int kGBits = 24, kGMinScale = 35, kGMaxScale = 48;
 constexpr int kGNarrow = 33;
 constexpr double kGNarrowNear = 4.8, kGNarrowReach = 2048.0;
 constexpr float kGTap[4] = {0.0047f, 0.1071f, 0.3521f, 0.3613f};
-constexpr double kGFar = 1e15;  // beyond: the second look
 
 __host__ __device__ inline double g_node(int k) {
   constexpr double c[kGNodes] = {  // cos((2 k + 1) pi / 32)
@@ -95,7 +94,7 @@ __device__ __forceinline__ int points_used(const double* reach, double inv_h, in
 // ---- spreading ----
 
 // A pair closer than the fixed point's fast range, or at an infinite
-// distance: FP64 and 64-bit conversions.
+// distance: FP64 and 64-bit conversions.  Pairs from kFarthest on add nothing.
 __device__ void spread_grad_rare(unsigned long long* grid, int plane, int* bad, const double* d,
                                  double t, double nf, double scale) {
   if (!(t < 1e300)) {
@@ -120,9 +119,9 @@ __device__ void spread_grad_rare(unsigned long long* grid, int plane, int* bad, 
     }
     return;
   }
-  double u = t - nf * floor(t / nf);
-  const bool neg = u > 0.5 * nf;
-  if (neg) u = nf - u;
+  bool neg;
+  double u;
+  if (!fold(t, nf, u, neg)) return;
   const double fl = floor(u);
   const double y = u - fl - 0.5;
   const int g = kGNodes + static_cast<int>(fl) + 1;
@@ -156,7 +155,7 @@ __device__ __forceinline__ bool spread_grad_pairs(const AtomRec* __restrict__ po
     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
     if (!(r2 > 0.0)) continue;  // the atom itself, a duplicate, a NaN
     double t = scaled_root(r2, inv_h);
-    if (!(t >= near && t < kGFar)) {
+    if (!(t >= near && t < kFarthest)) {
       rare = true;
       continue;
     }
@@ -165,11 +164,9 @@ __device__ __forceinline__ bool spread_grad_pairs(const AtomRec* __restrict__ po
     const float wx = w * static_cast<float>(dx), wy = w * static_cast<float>(dy),
                 wz = w * static_cast<float>(dz);
     if (t > half_nf) {
-      t -= nf * floor(t / nf);
-      if (t > half_nf) {
-        t = nf - t;
-        it = -it;
-      }
+      bool neg;
+      (void)fold(t, nf, t, neg);  // (t < kFarthest)
+      if (neg) it = -it;
     }
     const float y = static_cast<float>(__builtin_amdgcn_fract(t)) - 0.5f;
     const float y2 = y * y;
@@ -265,7 +262,7 @@ __device__ __forceinline__ void spread_grad_rows(
         const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
         if (!(r2 > 0.0)) continue;
         const double t = scaled_root(r2, inv_h);
-        if (t >= near && t < kGFar) continue;
+        if (t >= near && t < kFarthest) continue;
         const double d[3] = {dx * inv_h, dy * inv_h, dz * inv_h};
         spread_grad_rare(grid, plane, &bad, d, sqrt(r2) * inv_h, static_cast<double>(nf),
                          static_cast<double>(scale));

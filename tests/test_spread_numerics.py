@@ -2,6 +2,7 @@
 share with the host."""
 import os
 import re
+import subprocess
 
 import numpy as np
 
@@ -34,3 +35,52 @@ def test_window_has_no_common_factor():
         z = (taps * np.exp(1j * q * (np.arange(6)[:, None] - 2.5 - y[None]))).sum(0) / phihat
         assert abs(z.mean() * (1.0 - 6.755e-9) - 1.0) < 4e-9, q
         assert np.sqrt((np.abs(z - 1.0) ** 2).mean()) < 1.2e-8, q
+
+
+FOLD = r"""
+#define __host__
+#define __device__
+#include "fold.h"
+#include <cstdint>
+#include <initializer_list>
+#include <cstdio>
+using namespace pyiid;
+int main() {
+  uint64_t x = 88172645463325252ull, seen = 0, left_out = 0;
+  for (int nf : {12, 13, 90, 1126, 3000, 13500, 40800})
+    for (int k = 0; k < 400000; ++k) {
+      x ^= x << 13; x ^= x >> 7; x ^= x << 17;
+      // magnitudes 1 to 1e300, every eighth next to a multiple of the period
+      double t = std::pow(10.0, (x >> 11) * 0x1p-53 * (k % 3 ? 300.0 : 20.0));
+      if (k % 8 == 0) t = std::nextafter(std::floor(t / nf) * nf, k % 16 ? 0.0 : 1e301);
+      double u = -1.0;
+      bool neg;
+      if (!fold(t, nf, u, neg)) {
+        if (t < 1e15) return std::printf("left out: %.17g\n", t), 1;
+        ++left_out;
+        continue;
+      }
+      if (!(t < 1e15) || !(u >= 0.0 && u <= 0.5 * nf)) return std::printf("%d %.17g -> %.17g\n", nf, t, u), 1;
+      // the place in the period, against the remainder (which is exact)
+      const double r = std::remainder(t, nf);
+      if (std::fabs(std::fabs(r) - u) > 4e-16 * t) return std::printf("%d %.17g -> %.17g not %.17g\n", nf, t, u, r), 1;
+      if (u > 1e-9 * t && u < 0.5 * nf - 1e-9 * t && neg != (r < 0.0)) return std::printf("sign %d %.17g\n", nf, t), 1;
+      ++seen;
+    }
+  double u;
+  bool neg;
+  if (fold(INFINITY, 90, u, neg) || fold(NAN, 90, u, neg)) return 1;
+  return seen > 100000 && left_out > 100000 ? 0 : 2;
+}
+"""
+
+
+def test_folded_place_lies_in_the_grid(tmp_path):
+    """Distances of any finite size, also just beside a multiple of the period:
+    the folded place lies in [0, n_f / 2], which the grids cover, or the pair is
+    left out (from 1e15 on)."""
+    src, exe = tmp_path / "fold.cpp", tmp_path / "fold"
+    src.write_text(FOLD)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", CSRC, "-o", str(exe), str(src)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout
