@@ -453,12 +453,20 @@ int ensure_extent(pyiid_ctx* c) {
   return PYIID_OK;
 }
 
+// The atoms have moved, or are about to: what was taken from their places is not
+// theirs any more.  Every writer of c->pos calls this.
+void positions_changed(pyiid_ctx* c) {
+  c->extent_exact = false;
+  c->reach_set = false;
+  c->order_set = false;
+}
+
 int ensure_packed(pyiid_ctx* c) {
   if (!c->pos_set) return fail(PYIID_E_STATE, "positions not set");
   if (!c->pos_dirty || c->n == 0) return PYIID_OK;
   HIPCHK(launch_pack(c->stream, c->posf.as<float>(), c->elem.as<int32_t>(), c->n,
                      c->pos.as<AtomRec>(), nullptr, nullptr, nullptr, nullptr));
-  c->order_set = false;
+  positions_changed(c);
   c->pos_dirty = false;
   return PYIID_OK;
 }
@@ -2008,6 +2016,7 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
   CHK(c->pos.reserve(sizeof(AtomRec) * std::max<int64_t>(1, n)));
   // one kernel reads the caller's device positions, or the arena's copy of host
   // ones, and writes the records and the float copy; nothing waits
+  positions_changed(c);
   const float* src = pos;
   if (!(flags & PYIID_DEVICE) && n > 0) {
     void* p = nullptr;
@@ -2028,14 +2037,12 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
     c->pos_dirty = false;
   } else {
     CHK(upload(c, c->posf.p, pos, sizeof(float) * 3 * n, flags));
-    c->reach_set = false;
     c->pos_set = true;
     c->pos_dirty = true;
     CHK(ensure_packed(c));
     HIPCHK(hipStreamSynchronize(c->stream));
   }
   c->pos_set = true;
-  c->extent_exact = false;
   if (!(flags & PYIID_DEVICE) && n <= kExtentAtoms) {
     c->r_max = chain_extent(pos, 3, c->off);
     c->extent_off = c->off;
@@ -3176,9 +3183,7 @@ int pyiid_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step, do
     return fail(PYIID_E_INVALID, "need n_proposals >= 0, n_leapfrog >= 1, beta > 0");
   const int B = c->n_chain;
   if (n_proposals == 0) return PYIID_OK;
-  c->extent_exact = false;
-  c->reach_set = false;
-  c->order_set = false;
+  positions_changed(c);
   CHK(prepare_history(c, n_proposals));
   CHK(refresh_exact(c));
   RunClock clock(c, times_ms != nullptr);
@@ -3368,9 +3373,7 @@ int pyiid_sur_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step
   if (min_chain_atoms(c) < 2) return fail(PYIID_E_INVALID, "every chain needs at least two atoms");
   const int B = c->n_chain;
   if (n_proposals == 0) return PYIID_OK;
-  c->extent_exact = false;
-  c->reach_set = false;
-  c->order_set = false;
+  positions_changed(c);
   CHK(prepare_history(c, n_proposals));
   RunClock clock(c, times_ms != nullptr);
   bool exact_block = false;

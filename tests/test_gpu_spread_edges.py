@@ -61,3 +61,32 @@ def test_very_far_atoms_add_nothing(ctx, far):
     assert np.abs(fq * (n + 1.0) - f0).max() < 2e-7 * np.abs(f0).max()
     assert np.abs(g1[:n] - g0).max() < 1e-6 * np.abs(g0).max()
     assert np.abs(g1[n]).max() < 1e-7 * np.abs(g0).max()
+
+
+def test_gradient_after_a_sampler_and_new_elements(ctx):
+    """A sampler brings the atoms closer together, which the next gradient takes
+    note of; new elements then put the atoms back to where they were uploaded,
+    farther apart, and the gradient has to reach that far again."""
+    n, nq, qbin = 3, 250, 0.1
+    pos = np.array([(0, 0, 0), (10, 0, 0), (0, 10, 0)], np.float32)
+    r = 1.0 + 0.02 * np.arange(100)
+    per_atom = load(ctx, pos, np.full(n, 79), qbin, nq)
+    ctx.set_scatter(_lib.SLOT_PDF, per_atom[:1])
+    ctx.set_transform(0.02, qbin, r, 0.0, nq)
+    want = ctx.grad_fq(_lib.SLOT_FQ, qbin, n, nq)
+
+    def spread():
+        p = ctx.get_positions(n)
+        return max(np.linalg.norm(p[a] - p[b]) for a in range(n) for b in range(a))
+    for seed in range(200):  # nearly free flight: every proposal is accepted
+        ctx.set_positions(pos)
+        ctx.hmc_setup(_lib.SLOT_PDF, qbin, np.cos(r), _lib.POT_RW, 1e-9, np.full(n, 1.0))
+        ctx.hmc_run(1, 1, 3.0, 1.0, seed, 1, use_graph=False)
+        if spread() < 8.0:
+            break
+    assert spread() < 8.0
+    closer = ctx.grad_fq(_lib.SLOT_FQ, qbin, n, nq)
+    assert np.abs(closer - want).max() > 0.1 * np.abs(want).max()
+    ctx.set_elements(np.zeros(n, np.int32))
+    np.testing.assert_array_equal(ctx.get_positions(n), pos)
+    np.testing.assert_array_equal(ctx.grad_fq(_lib.SLOT_FQ, qbin, n, nq), want)
