@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "../../include/pyiid_hip.h"
+#include "extent.h"
 #include "internal.h"
 
 using namespace pyiid;
@@ -410,37 +411,12 @@ __global__ void unpack_kernel(const AtomRec* __restrict__ a, int64_t n, float* _
 // (about 10 us at the limit); larger ones once per layout.
 constexpr int64_t kExtentAtoms = 4096;
 
-template <typename T>
-double chain_extent(const T* p, int stride, const std::vector<int64_t>& off) {
-  double r_max = 0.0;
-  for (size_t b = 0; b + 1 < off.size(); ++b) {
-    if (off[b + 1] - off[b] < 2) continue;
-    double lo[3], hi[3], mid[3];
-    for (int k = 0; k < 3; ++k) lo[k] = hi[k] = p[off[b] * stride + k];
-    for (int64_t a = off[b]; a < off[b + 1]; ++a)
-      for (int k = 0; k < 3; ++k) {
-        lo[k] = std::min<double>(lo[k], p[a * stride + k]);
-        hi[k] = std::max<double>(hi[k], p[a * stride + k]);
-      }
-    double diag = 0.0, rad = 0.0;
-    for (int k = 0; k < 3; ++k) {
-      mid[k] = 0.5 * (lo[k] + hi[k]);
-      diag += (hi[k] - lo[k]) * (hi[k] - lo[k]);
-    }
-    for (int64_t a = off[b]; a < off[b + 1]; ++a) {
-      double d = 0.0;
-      for (int k = 0; k < 3; ++k) d += (p[a * stride + k] - mid[k]) * (p[a * stride + k] - mid[k]);
-      rad = std::max(rad, d);
-    }
-    r_max = std::max(r_max, std::min(std::sqrt(diag), 2.0 * std::sqrt(rad)));
-  }
-  return r_max;
-}
-
 // r_max of the current layout, from the device positions when no host upload
-// gave it (once per layout; waits for the stream).
+// gave it (once per layout, and again while a position is not finite; waits for
+// the stream).
 int ensure_extent(pyiid_ctx* c) {
-  if (c->extent_off == c->off) return PYIID_OK;
+  if (c->extent_off == c->off && (std::isfinite(c->r_max) || c->extent_exact || c->capturing))
+    return PYIID_OK;
   if (c->capturing) return fail(PYIID_E_STATE, "structure changed during graph capture");
   std::vector<double> h(static_cast<size_t>(c->n) * 4);
   if (c->n > 0) {

@@ -90,3 +90,41 @@ def test_gradient_after_a_sampler_and_new_elements(ctx):
     ctx.set_elements(np.zeros(n, np.int32))
     np.testing.assert_array_equal(ctx.get_positions(n), pos)
     np.testing.assert_array_equal(ctx.grad_fq(_lib.SLOT_FQ, qbin, n, nq), want)
+
+
+@pytest.mark.parametrize("where", [0, 7])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_host_and_device_positions_that_are_not_finite(fixed_shapes, where, value):
+    """One atom's x is not finite: from host arrays, where the extent is taken on
+    the host, F, gradient, energy and forces are those of a device upload, where
+    it is taken on the GPU; the pairs of the other atoms are all there."""
+    import torch
+    n, nq, qbin = 60, 250, 0.1
+    pos = structures.jitter(structures.fcc_nearest(n), 0.05, seed=4).astype(np.float32)
+    rest = np.arange(n) != where
+    table, index, _ = element_table(np.full(n, 79), qbin, nq)
+    r = 2.0 + 0.02 * np.arange(300)
+
+    def results(device, p):
+        c = _lib.Context(0)
+        try:
+            c.set_positions(torch.from_numpy(p).cuda() if device else p,
+                            flags=_lib.PYIID_DEVICE if device else 0)
+            c.set_elements(np.zeros(len(p), np.int32))
+            c.set_scatter(_lib.SLOT_FQ, table)
+            c.set_scatter(_lib.SLOT_PDF, table)
+            c.set_transform(0.02, qbin, r, 0.0, nq)
+            g = c.grad_fq(_lib.SLOT_FQ, qbin, len(p), nq)
+            e, f = c.pdf_energy_forces(_lib.SLOT_PDF, qbin, np.cos(r), _lib.POT_RW, 1.0, len(p))
+            return g, c.fq(_lib.SLOT_FQ, qbin, nq), np.float64(e), f
+        finally:
+            c.close()
+    moved = pos.copy()
+    moved[where, 0] = value
+    host, device = results(False, moved), results(True, moved)
+    for a, b in zip(host, device):
+        np.testing.assert_array_equal(a, b)
+    if np.isnan(value):  # y and z: the pairs of the others, none with the atom itself
+        want = results(False, pos[rest])[0] * ((n - 1.0) / n)
+        off = np.abs(host[0][rest][:, 1:] - want[:, 1:])
+        assert off.max() < 1e-6 * np.abs(want).max()

@@ -84,3 +84,44 @@ def test_folded_place_lies_in_the_grid(tmp_path):
     subprocess.run(["g++", "-O2", "-std=c++17", "-I", CSRC, "-o", str(exe), str(src)], check=True)
     out = subprocess.run([str(exe)], capture_output=True, text=True)
     assert out.returncode == 0, out.stdout
+
+
+EXTENT = r"""
+#include "extent.h"
+#include <cstdio>
+#include <limits>
+using namespace pyiid;
+int main() {
+  const double inf = std::numeric_limits<double>::infinity(), nan = std::numeric_limits<double>::quiet_NaN();
+  const std::vector<int64_t> one{0, 4}, two{0, 1, 5};  // two: the first chain has no distance
+  for (double bad : {nan, inf, -inf, 1e200})
+    for (int a = 0; a < 4; ++a)
+      for (int k = 0; k < 3; ++k)
+        for (int both = 0; both < 2; ++both) {
+          double p[5][4] = {{0, 0, 0, 0}, {3, 4, 0, 0}, {1, 2, 2, 0}, {0, 1, 0, 0}, {1, 1, 1, 0}};
+          p[a][k] = bad;
+          if (both) p[(a + 1) % 4][k] = -bad;
+          if (!(chain_extent(&p[0][0], 4, one) == inf)) return std::printf("%g at %d %d\n", bad, a, k), 1;
+          float f[5][3];
+          for (int i = 0; i < 5; ++i)
+            for (int c = 0; c < 3; ++c) f[i][c] = static_cast<float>(p[i][c]);
+          if (bad != 1e200 && !(chain_extent(&f[0][0], 3, one) == inf)) return std::printf("float %g\n", bad), 1;
+          const double e = chain_extent(&p[0][0], 4, two);  // the atom alone counts for nothing
+          if (!both && a == 0 && !(e > 0.0 && e < 10.0)) return std::printf("alone %g\n", e), 1;
+        }
+  const double q[4][3] = {{0, 0, 0}, {3, 4, 0}, {1, 2, 2}, {0, 1, 0}};
+  const double e = chain_extent(&q[0][0], 3, one);
+  return e >= 5.0 && e < 5.4 ? 0 : 1;
+}
+"""
+
+
+def test_extent_of_positions_that_are_not_finite(tmp_path):
+    """The bound of the distances is infinite whichever atom's position is not
+    finite (the first one's, or two of opposite sign, too), so that no pair is left
+    out on account of it; a chain of one atom has no distances."""
+    src, exe = tmp_path / "extent.cpp", tmp_path / "extent"
+    src.write_text(EXTENT)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", CSRC, "-o", str(exe), str(src)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout
