@@ -98,7 +98,7 @@ __device__ __forceinline__ int points_used(const double* reach, double inv_h, in
 __device__ void spread_grad_rare(unsigned long long* grid, int plane, int* bad, const double* d,
                                  double t, double nf, double scale) {
   if (!(t < 1e300)) {
-    *bad = 1;
+    atomicOr(bad, 7);
     return;
   }
   auto add = [&](int at, double v) {
@@ -153,10 +153,9 @@ __device__ __forceinline__ bool spread_grad_pairs(const AtomRec* __restrict__ po
   for (int j = jb + static_cast<int>(threadIdx.x); j < je; j += blockDim.x) {
     const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-    if (!(r2 > 0.0)) continue;  // the atom itself, a duplicate, a NaN
-    double t = scaled_root(r2, inv_h);
+    double t = scaled_root(r2, inv_h);  // (not a number at r = 0)
     if (!(t >= near && t < kFarthest)) {
-      rare = true;
+      rare = rare || r2 != 0.0;  // the atom itself and duplicates add nothing
       continue;
     }
     float it = __builtin_amdgcn_rcpf(static_cast<float>(t));
@@ -217,7 +216,7 @@ __device__ __forceinline__ void spread_grad_rows(
     int nf, int plane, int row_len, int k_fixed, const double* __restrict__ reach, int nq,
     float scale, double near, bool narrow, _Float16* __restrict__ rows,
     float* __restrict__ row_scale, unsigned long long* grid) {
-  __shared__ int bad;
+  __shared__ int bad;  // a bit per component that is not a number
   __shared__ unsigned int top[3];
   const int p = p0 + blockIdx.x;
   const int n_thread = blockDim.x;
@@ -260,7 +259,14 @@ __device__ __forceinline__ void spread_grad_rows(
       for (int j = jb + static_cast<int>(threadIdx.x); j < je; j += n_thread) {
         const double dx = pi.x - pos[j].x, dy = pi.y - pos[j].y, dz = pi.z - pos[j].z;
         const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-        if (!(r2 > 0.0)) continue;
+        if (!(r2 > 0.0)) {
+          // a position that is not a number adds nothing, but shows in the
+          // components where it is not
+          const int not_finite = (fabs(dx) < HUGE_VAL ? 0 : 1) | (fabs(dy) < HUGE_VAL ? 0 : 2) |
+                                 (fabs(dz) < HUGE_VAL ? 0 : 4);
+          if (not_finite) atomicOr(&bad, not_finite);
+          continue;
+        }
         const double t = scaled_root(r2, inv_h);
         if (t >= near && t < kFarthest) continue;
         const double d[3] = {dx * inv_h, dy * inv_h, dz * inv_h};
@@ -298,7 +304,7 @@ __device__ __forceinline__ void spread_grad_rows(
       rows[at] = hi;
       rows[at + 32] = static_cast<_Float16>(x - static_cast<float>(hi));
     }
-    if (threadIdx.x == 0) row_scale[row] = bad ? __builtin_nanf("") : ldexpf(unit, e - 15);
+    if (threadIdx.x == 0) row_scale[row] = bad >> c & 1 ? __builtin_nanf("") : ldexpf(unit, e - 15);
   }
 }
 

@@ -128,3 +128,39 @@ def test_host_and_device_positions_that_are_not_finite(fixed_shapes, where, valu
         want = results(False, pos[rest])[0] * ((n - 1.0) / n)
         off = np.abs(host[0][rest][:, 1:] - want[:, 1:])
         assert off.max() < 1e-6 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("kinds", [1, 3])
+@pytest.mark.parametrize("bad", [(0, (0,)), (3, (1,)), (69, (0, 2)), (5, (0, 1, 2))])
+def test_gradient_shows_positions_that_are_not_numbers(ctx, kinds, bad):
+    """One atom has components that are not numbers: so have the same components of
+    every atom's gradient, on the spreading kernel as on the recurrence kernels,
+    and the other components are those of the remaining pairs.  Duplicated atoms
+    are no such case."""
+    n, nq, qbin = 70, 250, 0.1
+    which, where = bad
+    pos = structures.jitter(structures.fcc_nearest(n), 0.05, seed=6).astype(np.float32)
+    pos[40] = pos[41]
+    numbers = np.array([79, 28, 78])[np.arange(n) % kinds]
+    load(ctx, pos, numbers, qbin, nq)
+    assert np.isfinite(ctx.grad_fq(_lib.SLOT_FQ, qbin, n, nq)).all()
+    pos[which, list(where)] = np.nan
+    got = {}
+    try:
+        for kernel in (_lib.GRAD_AUTO, _lib.GRAD_ORDERED, _lib.GRAD_SYMMETRIC):
+            ctx.set_grad_kernel(kernel)
+            ctx.set_positions(pos)
+            got[kernel] = ctx.grad_fq(_lib.SLOT_FQ, qbin, n, nq)
+            assert (ctx.grad_shape() == (False, 0, 0)) == (kernel == _lib.GRAD_AUTO)
+    finally:
+        ctx.set_grad_kernel(_lib.GRAD_AUTO)
+    new, old = got[_lib.GRAD_AUTO], got[_lib.GRAD_ORDERED]
+    for c in range(3):
+        assert np.isnan(new[:, c]).all() == (c in where)
+        np.testing.assert_array_equal(np.isnan(new[:, c]), np.isnan(old[:, c]))
+        np.testing.assert_array_equal(np.isnan(new[:, c]), np.isnan(got[_lib.GRAD_SYMMETRIC][:, c]))
+        if c not in where:
+            assert np.abs(new[:, c] - old[:, c]).max() < 2e-6 * np.abs(old[:, c]).max()
+    import torch
+    ctx.set_positions(torch.from_numpy(pos).cuda(), flags=_lib.PYIID_DEVICE)
+    np.testing.assert_array_equal(ctx.grad_fq(_lib.SLOT_FQ, qbin, n, nq), new)
