@@ -230,6 +230,9 @@ struct pyiid_ctx {
   Buf place, ordered;               // an atom's place in element order; the positions so
   uint64_t place_stamp = ~0ull;
   bool order_set = false;           // ordered holds the current positions
+  // A graph of the caller's holds an upload: its replays move the atoms without the
+  // host's knowledge, and nothing is kept of their places from call to call.
+  bool replays_move = false;
   bool share_order = false;         // within one call (SharedOrder)
   const AtomRec* in_order = nullptr;
 
@@ -411,11 +414,20 @@ __global__ void unpack_kernel(const AtomRec* __restrict__ a, int64_t n, float* _
 // (about 10 us at the limit); larger ones once per layout.
 constexpr int64_t kExtentAtoms = 4096;
 
+// Whether the caller records this call's launches into a graph of its own.  A
+// replay finds the positions of its time, so such a launch must not depend on what
+// is known of the positions now.
+bool caller_captures(pyiid_ctx* c) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(c->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
 // r_max of the current layout, from the device positions when no host upload
 // gave it (once per layout, and again while a position is not finite; waits for
 // the stream).
 int ensure_extent(pyiid_ctx* c) {
-  if (c->extent_off == c->off && (std::isfinite(c->r_max) || c->extent_exact || c->capturing))
+  if (c->extent_off == c->off &&
+      (std::isfinite(c->r_max) || c->extent_exact || c->capturing || caller_captures(c)))
     return PYIID_OK;
   if (c->capturing) return fail(PYIID_E_STATE, "structure changed during graph capture");
   std::vector<double> h(static_cast<size_t>(c->n) * 4);
@@ -1101,11 +1113,6 @@ hipError_t launch_fq_items(pyiid_ctx* c, const Table& t, double qbin, bool count
                    c->fpart.as<double>(), forms);
 }
 
-bool caller_captures(pyiid_ctx* c) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(c->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
-}
-
 // Whether b can be made `want` bytes now: not in a capture of the caller's, and
 // there has to be the memory.
 bool scratch(pyiid_ctx* c, Buf& b, size_t want) {
@@ -1131,16 +1138,17 @@ struct SharedOrder {
 // gather of a structure the packing of uploads places the atoms itself (a launch
 // less per call).
 int in_element_order(pyiid_ctx* c, const Buf& perm, const Buf& sorted, const AtomRec** sp) {
-  if (c->order_set || c->in_order) {
-    *sp = c->order_set ? c->ordered.as<AtomRec>() : c->in_order;
+  const bool keep = c->order_set && !caller_captures(c);
+  if (keep || c->in_order) {
+    *sp = keep ? c->ordered.as<AtomRec>() : c->in_order;
     return PYIID_OK;
   }
   HIPCHK(launch_gather(c->stream, c->pos.as<AtomRec>(), perm.as<int32_t>(), c->n, sorted.as<AtomRec>()));
   *sp = sorted.as<AtomRec>();
   if (c->share_order) c->in_order = *sp;
   if (c->place_stamp != c->struct_stamp && !c->capturing &&
-      scratch(c, c->ordered, sizeof(AtomRec) * c->n) && scratch(c, c->place, sizeof(int32_t) * c->n) &&
-      !caller_captures(c)) {
+      !caller_captures(c) && scratch(c, c->ordered, sizeof(AtomRec) * c->n) &&
+      scratch(c, c->place, sizeof(int32_t) * c->n)) {
     std::vector<int32_t> order, place(static_cast<size_t>(c->n));
     std::vector<std::vector<ElemRun>> runs;
     element_runs(c, true, order, runs);
@@ -1665,18 +1673,20 @@ int run_spread_grad(pyiid_ctx* c, int slot, double qbin, void* out, bool out_f64
   const AtomRec* sp = c->pos.as<AtomRec>();
   if (weighted) CHK(in_element_order(c, s.perm, s.sorted, &sp));
   // points of a row in use: from the host's extent when it bounds the current
-  // positions, else from the positions on the device (no wait either way)
+  // positions, else from the positions on the device (no wait either way); in a
+  // graph from the positions that a replay finds
   int k_fixed = 0;
   const double* reach = nullptr;
-  if (c->extent_exact) {
+  const bool captured = caller_captures(c);
+  if (c->extent_exact && !captured) {
     const double points = grad_reach(nq, dq, c->r_max * 1.000001);
     k_fixed = points < len ? (static_cast<int>(points) + 31) & ~31 : len;
     k_fixed = std::min(k_fixed, len);
   } else {
-    if (!c->reach_set) {
+    if (!c->reach_set || captured) {
       CHK(c->reach.reserve(sizeof(double)));
       HIPCHK(launch_reach(c->stream, sp, c->n, c->reach.as<double>()));
-      c->reach_set = true;
+      c->reach_set = !captured && !c->replays_move;
     }
     reach = c->reach.as<double>();
   }
@@ -1971,6 +1981,12 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
   if (n < 0 || n > 2000000000LL)
     return fail(PYIID_E_INVALID, "atom count %lld out of range", (long long)n);
   if (n > 0 && !pos) return fail(PYIID_E_INVALID, "null positions");
+  if (caller_captures(c)) {
+    // (what a replay would upload is not in host memory of ours any more)
+    if (!(flags & PYIID_DEVICE))
+      return fail(PYIID_E_STATE, "positions in host memory cannot be captured into a graph");
+    c->replays_move = true;
+  }
   const bool same = (n == c->n) && (off == c->off);
   if (!same) {
     // the composition changes: elements reset to 0
@@ -2003,8 +2019,9 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
   if (src && n > 0) {
     // (the gradient of a single structure asks how far its distances reach)
     CHK(c->reach.reserve(sizeof(double)));
-    const bool reach = (flags & PYIID_DEVICE) && c->n_chain == 1 && n <= kReachAtoms;
-    const bool order = c->place_stamp == c->struct_stamp;
+    const bool reach =
+        (flags & PYIID_DEVICE) && c->n_chain == 1 && n <= kReachAtoms && !c->replays_move;
+    const bool order = c->place_stamp == c->struct_stamp && !c->replays_move;
     HIPCHK(launch_pack(c->stream, src, c->elem.as<int32_t>(), n, c->pos.as<AtomRec>(),
                        c->posf.as<float>(), reach ? c->reach.as<double>() : nullptr,
                        order ? c->place.as<int32_t>() : nullptr, c->ordered.as<AtomRec>()));
@@ -2022,7 +2039,7 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
   if (!(flags & PYIID_DEVICE) && n <= kExtentAtoms) {
     c->r_max = chain_extent(pos, 3, c->off);
     c->extent_off = c->off;
-    c->extent_exact = true;
+    c->extent_exact = !c->replays_move;
   }
   return PYIID_OK;
 }

@@ -164,3 +164,167 @@ def test_gradient_shows_positions_that_are_not_numbers(ctx, kinds, bad):
     import torch
     ctx.set_positions(torch.from_numpy(pos).cuda(), flags=_lib.PYIID_DEVICE)
     np.testing.assert_array_equal(ctx.grad_fq(_lib.SLOT_FQ, qbin, n, nq), new)
+
+
+class Captured:
+    """A context on a stream of torch's, whose gradient (with F) goes to `grad` and
+    `fq`; `capture` records calls into a graph."""
+
+    def __init__(self, n, kinds, qbin, nq):
+        import torch
+        self.torch, self.n, self.qbin, self.nq = torch, n, qbin, nq
+        self.stream = torch.cuda.Stream()
+        self.c = _lib.Context(0)
+        self.c.set_stream(self.stream.cuda_stream)
+        self.numbers = np.array([79, 28, 78])[np.random.RandomState(n).permutation(n) % kinds]
+        self.table, self.index, _ = element_table(self.numbers, qbin, nq)
+        self.grad = torch.zeros((n, 3, nq), device="cuda")
+        self.fq = torch.zeros(nq, device="cuda")
+        self.buf = torch.zeros((n, 3), device="cuda")
+        torch.cuda.synchronize()
+
+    def load(self, pos):
+        self.c.set_positions(pos)
+        self.c.set_elements(self.index)
+        for slot in (_lib.SLOT_FQ, _lib.SLOT_PDF):
+            self.c.set_scatter(slot, self.table)
+
+    def eager(self):
+        self.c.grad_fq(_lib.SLOT_FQ, self.qbin, self.n, self.nq, out=self.grad, fq_out=self.fq,
+                       flags=_lib.PYIID_DEVICE)
+
+    def upload(self):
+        self.c.set_positions(self.buf, flags=_lib.PYIID_DEVICE)
+
+    def capture(self, calls):
+        g = self.torch.cuda.CUDAGraph()
+        self.torch.cuda.synchronize()
+        with self.torch.cuda.graph(g, stream=self.stream):
+            for f in calls:
+                f()
+        return g
+
+    def replay(self, g):
+        with self.torch.cuda.stream(self.stream):
+            g.replay()
+
+    def result(self):
+        self.torch.cuda.synchronize()
+        out = self.grad.cpu().numpy(), self.fq.cpu().numpy()
+        with self.torch.cuda.stream(self.stream):
+            self.grad.zero_()
+            self.fq.zero_()
+        return out
+
+    def fill(self, pos):
+        self.buf.copy_(self.torch.from_numpy(pos))
+        self.torch.cuda.synchronize()
+
+    def fresh(self, pos):
+        other = Captured(self.n, 1, self.qbin, self.nq)
+        other.table, other.index = self.table, self.index
+        other.load(pos)
+        other.eager()
+        out = other.result()
+        other.c.close()
+        return out
+
+
+def same(got, want):
+    for a, b in zip(got, want):
+        assert np.any(b)
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("n,kinds,qbin,nq", [(60, 1, 0.1, 250), (300, 1, 0.1, 250), (300, 3, 0.1, 250),
+                                             (5000, 1, 0.02, 300)])
+def test_captured_gradient_follows_the_positions(n, kinds, qbin, nq):
+    """A gradient in a graph, captured when the extent, the reach and the element
+    order of the positions were known, replayed after uploads of larger and smaller
+    structures from the host and the device: each time a new context's result."""
+    base = structures.jitter(structures.fcc_nearest(n), 0.05, seed=n).astype(np.float32)
+    s = Captured(n, kinds, qbin, nq)
+    s.load(base)
+    for _ in range(2):
+        s.fill(base)
+        s.upload() if n > 4096 else s.c.set_positions(base)
+        s.eager()
+        s.eager()
+    g = s.capture([s.eager])
+    s.result()
+    for scale, device in ((1.0, True), (2.0, False), (0.8, True), (1.7, True), (1.3, False)):
+        pos = (base * np.float32(scale)).astype(np.float32)
+        s.fill(pos)
+        s.upload() if device else s.c.set_positions(pos)
+        s.replay(g)
+        want = s.fresh(pos)
+        same(s.result(), want)
+        s.eager()
+        same(s.result(), want)
+    del g
+    s.c.close()
+
+
+@pytest.mark.parametrize("n,kinds", [(60, 1), (300, 3)])
+def test_captured_upload_and_gradient(n, kinds):
+    """An upload and a gradient in a graph, replayed with other positions in the
+    buffer; an eager gradient between the replays finds the atoms where the replay
+    has put them.  Positions in host memory cannot be captured."""
+    nq = 250
+    base = structures.jitter(structures.fcc_nearest(n), 0.05, seed=n).astype(np.float32)
+    s = Captured(n, kinds, 0.1, nq)
+    s.load(base)
+    s.fill(base)
+    for _ in range(2):
+        s.upload()
+        s.eager()
+
+    def refused():
+        with pytest.raises(Exception, match="captured"):
+            s.c.set_positions(base)
+    g = s.capture([s.upload, s.eager, refused])
+    s.result()
+    for scale in (1.0, 1.9, 0.8, 1.6):
+        pos = (base * np.float32(scale)).astype(np.float32)
+        s.fill(pos)
+        s.replay(g)
+        want = s.fresh(pos)
+        same(s.result(), want)
+        s.eager()
+        same(s.result(), want)
+        s.fill((base * np.float32(0.9)).astype(np.float32))
+        s.upload()
+        s.eager()
+        same(s.result(), s.fresh((base * np.float32(0.9)).astype(np.float32)))
+    del g
+    s.c.close()
+
+
+def test_captured_gradient_after_a_sampler():
+    """Atoms of three elements that a sampler has moved since the capture, by up to
+    a hundred A: the replay finds them there.  The extent has grown past 114 A, up
+    to which the gradient's grids are of 32 bits; the graph keeps its choice, the
+    eager call does not, so the two agree to rounding (2^-20 of the largest entry,
+    as the product's two halves allow), not bit for bit."""
+    n, nq, qbin = 300, 250, 0.1
+    base = structures.jitter(structures.fcc_nearest(n), 0.05, seed=n).astype(np.float32)
+    s = Captured(n, 3, qbin, nq)
+    s.load(base)
+    r = 2.0 + 0.02 * np.arange(300)
+    s.c.set_transform(0.02, qbin, r, 0.0, nq)
+    for _ in range(3):
+        s.c.set_positions(base)
+        s.eager()
+    g = s.capture([s.eager])
+    s.replay(g)
+    same(s.result(), s.fresh(base))
+    s.c.hmc_setup(_lib.SLOT_PDF, qbin, np.cos(r), _lib.POT_RW, 1.0, np.full(n, 100.0))
+    s.c.hmc_run(3, 3, 1.0, 1e-3, 1, 1)
+    assert np.abs(s.c.get_positions(n) - base).max() > 0.01
+    s.replay(g)
+    got = s.result()
+    s.eager()
+    for a, b in zip(got, s.result()):
+        assert np.abs(a - b).max() < 2.0 ** -20 * np.abs(b).max()
+    del g
+    s.c.close()
