@@ -227,6 +227,9 @@ struct pyiid_ctx {
   bool extent_exact = false;        // r_max bounds the current positions' distances
   Buf reach;                        // double: such a bound on the device
   bool reach_set = false;           // of the current positions
+  // page-locked, written by the forces' kernel: a pair lay past the force table
+  double* far_seen = nullptr;
+  bool extent_old = false;          // it did: take the extent anew
   Buf place, ordered;               // an atom's place in element order; the positions so
   uint64_t place_stamp = ~0ull;
   bool order_set = false;           // ordered holds the current positions
@@ -315,6 +318,20 @@ int ensure_device(pyiid_ctx* c) {
 constexpr size_t kArenaBytes = static_cast<size_t>(4) << 20;
 constexpr size_t kArenaMost = static_cast<size_t>(1) << 20;  // of one array
 
+void destroy_graph(Hmc& h);
+bool caller_captures(pyiid_ctx* c);
+
+// A force table was too short: the next one is made for the extent of its time,
+// and so are captured proposals.
+int note_far(pyiid_ctx* c) {
+  if (caller_captures(c)) return PYIID_OK;
+  HIPCHK(hipStreamSynchronize(c->stream));  // a proposal's graph may be running
+  *c->far_seen = 0.0;
+  c->extent_old = true;
+  destroy_graph(c->hmc);
+  return PYIID_OK;
+}
+
 int check_ctx(pyiid_ctx* c) {
   if (!c) return fail(PYIID_E_INVALID, "null context");
   CHK(ensure_device(c));
@@ -323,6 +340,7 @@ int check_ctx(pyiid_ctx* c) {
     HIPCHK(hipStreamSynchronize(c->stream));
     c->arena_used = 0;
   }
+  if (c->far_seen && *static_cast<volatile double*>(c->far_seen) != 0.0) return note_far(c);
   return PYIID_OK;
 }
 
@@ -423,11 +441,11 @@ bool caller_captures(pyiid_ctx* c) {
 }
 
 // r_max of the current layout, from the device positions when no host upload
-// gave it (once per layout, and again while a position is not finite; waits for
-// the stream).
+// gave it (once per layout, and again while a position is not finite or after a
+// force table has proved too short; waits for the stream).
 int ensure_extent(pyiid_ctx* c) {
-  if (c->extent_off == c->off &&
-      (std::isfinite(c->r_max) || c->extent_exact || c->capturing || caller_captures(c)))
+  if (c->extent_off == c->off && ((std::isfinite(c->r_max) && !c->extent_old) || c->extent_exact ||
+                                  c->capturing || caller_captures(c)))
     return PYIID_OK;
   if (c->capturing) return fail(PYIID_E_STATE, "structure changed during graph capture");
   std::vector<double> h(static_cast<size_t>(c->n) * 4);
@@ -438,6 +456,7 @@ int ensure_extent(pyiid_ctx* c) {
   }
   c->r_max = chain_extent(h.data(), 4, c->off);
   c->extent_off = c->off;
+  c->extent_old = false;
   return PYIID_OK;
 }
 
@@ -1721,8 +1740,6 @@ int run_spread_grad(pyiid_ctx* c, int slot, double qbin, void* out, bool out_f64
 
 // ---- contracted forces from a pair-force table ----
 
-void destroy_graph(Hmc& h);
-
 constexpr size_t kForceTableBudget = static_cast<size_t>(512) << 20;
 
 // Cells of the force table: the structure's extent and a tenth more (atoms
@@ -1819,25 +1836,19 @@ int reserve_coef(pyiid_ctx* c, int slot, double qbin, double2** coef) {
   return PYIID_OK;
 }
 
-// out5 (5 values per chain) and, behind them, the flag of a pair past the
-// force table.
-int reserve_out5(pyiid_ctx* c, int n_chain) {
-  const size_t want = sizeof(double) * (5 * static_cast<size_t>(n_chain) + 1);
-  if (want > c->out5.bytes) {
-    CHK(c->out5.reserve(want));
-    HIPCHK(hipMemsetAsync(c->out5.p, 0, c->out5.bytes, c->stream));
+// Where the forces' kernel notes a pair past its table (null if there is no
+// page-locked memory: then the table keeps its length).
+double* far_flag(pyiid_ctx* c) {
+  if (!c->far_seen && !caller_captures(c)) {
+    void* m = nullptr;
+    if (hipHostMalloc(&m, sizeof(double), hipHostMallocDefault) == hipSuccess) {
+      c->far_seen = static_cast<double*>(m);
+      *c->far_seen = 0.0;
+    } else {
+      (void)hipGetLastError();
+    }
   }
-  return PYIID_OK;
-}
-
-// A pair lay past the force table: take the extent anew for the next call.
-int note_far(pyiid_ctx* c, double flag) {
-  if (flag == 0.0) return PYIID_OK;
-  c->extent_off.clear();
-  destroy_graph(c->hmc);
-  HIPCHK(hipMemsetAsync(c->out5.as<double>() + 5 * static_cast<size_t>(c->n_chain), 0,
-                        sizeof(double), c->stream));
-  return PYIID_OK;
+  return c->far_seen;
 }
 
 // forces (n x 3 doubles) = scale * sum_q u[chain][q] grad(i, c, q).
@@ -1868,8 +1879,7 @@ int contract_forces(pyiid_ctx* c, int slot, double qbin, double scale, double* o
     HIPCHK(launch_table_force(c->stream, sp, s.units.as<ForceUnit>(), s.n_units, n_cell,
                               s.t4.as<float4>(), s.t2.as<float2>(), c->u.as<float>(),
                               t.tab.as<float>(), nq, dq, c->n, s.part.as<double>(), perm, scale,
-                              s.direct ? out : nullptr,
-                              c->out5.as<double>() + 5 * static_cast<size_t>(B)));
+                              s.direct ? out : nullptr, far_flag(c)));
     CHK(tm.done());
     if (!s.direct)
       HIPCHK(launch_reduce_force(c->stream, s.part.as<double>(), c->n, s.planes.as<int32_t>(), perm,
@@ -1932,7 +1942,7 @@ int energy_forces_device(pyiid_ctx* c, int slot, double qbin, int potential,
   CHK(compute_fq(c, slot, qbin, nullptr, &clear));
   CHK(c->g64.reserve(sizeof(double) * (size_t)nr * B));
   CHK(gemm_t(c, c->fq32.p, false, B, c->g64.as<double>()));
-  CHK(reserve_out5(c, B));
+  CHK(c->out5.reserve(sizeof(double) * 5 * static_cast<size_t>(B)));
   CHK(c->mix.reserve(sizeof(double2) * B));
   if (forces_dev) CHK(c->upart.reserve(sizeof(double) * 2 * kAdjointSlices * (size_t)nq * B));
   HIPCHK(launch_score(c->stream, potential, gobs_dev, c->g64.as<double>(), nr, B, c->out5.as<double>(),
@@ -2039,6 +2049,7 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
   if (!(flags & PYIID_DEVICE) && n <= kExtentAtoms) {
     c->r_max = chain_extent(pos, 3, c->off);
     c->extent_off = c->off;
+    c->extent_old = false;
     c->extent_exact = !c->replays_move;
   }
   return PYIID_OK;
@@ -2546,6 +2557,7 @@ int pyiid_destroy(pyiid_ctx* c) {
   }
   for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
   if (c->arena) (void)hipHostFree(c->arena);
+  if (c->far_seen) (void)hipHostFree(c->far_seen);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
   delete c;
   return PYIID_OK;
@@ -3006,7 +3018,7 @@ int pyiid_potential(pyiid_ctx* c, int potential, const double* gobs, const doubl
   CHK(c->io_a.reserve(sizeof(double) * n));
   CHK(c->io_b.reserve(sizeof(double) * n));
   CHK(c->w.reserve(sizeof(double) * n));
-  CHK(reserve_out5(c, c->n_chain));
+  CHK(c->out5.reserve(sizeof(double) * 5));
   CHK(upload(c, c->io_a.p, gcalc, sizeof(double) * n, flags));
   CHK(upload(c, c->io_b.p, gobs, sizeof(double) * n, flags));
   HIPCHK(launch_potential(c->stream, potential, c->io_b.as<double>(), c->io_a.as<double>(), n,
@@ -3068,10 +3080,9 @@ int pyiid_pdf_energy_forces(pyiid_ctx* c, int slot, double qbin, const double* g
   CHK(energy_forces_device(c, slot, qbin, potential, target, conv, fdst));
   if (copy) CHK(download(c, forces, fdst, sizeof(double) * 3 * c->n, flags));
   if (energy) {
-    std::vector<double> o5(5 * (size_t)B + 1);
+    std::vector<double> o5(5 * (size_t)B);
     CHK(download(c, o5.data(), c->out5.p, sizeof(double) * o5.size(), 0));
     CHK(arena_flush(c));
-    CHK(note_far(c, o5[5 * (size_t)B]));
     for (int b = 0; b < B; ++b) energy[b] = o5[5 * (size_t)b] * conv;
   }
   return finish(c, flags);
@@ -3093,15 +3104,14 @@ int pyiid_fq_energy_forces(pyiid_ctx* c, int slot, double qbin, int32_t q_first,
   CHK(compute_fq(c, slot, qbin));
   CHK(c->gobs.reserve(sizeof(double) * ng));
   CHK(upload(c, c->gobs.p, gobs, sizeof(double) * ng, flags));
-  CHK(reserve_out5(c, c->n_chain));
+  CHK(c->out5.reserve(sizeof(double) * 5));
   CHK(c->w.reserve(sizeof(double) * ng));
   HIPCHK(launch_potential(c->stream, potential, c->gobs.as<double>(),
                           c->fq64.as<double>() + q_first, ng, c->out5.as<double>(),
                           c->w.as<double>()));
-  double out5[6];
+  double out5[5];
   HIPCHK(hipMemcpyAsync(out5, c->out5.p, sizeof(out5), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
-  CHK(note_far(c, out5[5]));  // of the call before
   if (energy) *energy = out5[0] * conv;
   if (!forces) return PYIID_OK;
   if (c->n < 2) {
@@ -3189,12 +3199,6 @@ int pyiid_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step, do
     CHK(download(c, energies, h.ehist.p, sizeof(double) * (size_t)n_proposals * B, flags));
   if (accepted)
     CHK(download(c, accepted, h.acchist.p, sizeof(int32_t) * (size_t)n_proposals * B, flags));
-  if (!(flags & PYIID_DEVICE)) {
-    double far = 0.0;
-    CHK(download(c, &far, c->out5.as<double>() + 5 * static_cast<size_t>(B), sizeof(far), 0));
-    CHK(arena_flush(c));
-    CHK(note_far(c, far));
-  }
   return finish(c, flags);
 }
 

@@ -165,7 +165,7 @@ __global__ __launch_bounds__(64 * kNodes * kTabSplit * CELLS * PARTS / 64) void 
 // for): the sums themselves.
 __device__ double pair_force_far(double r, const float* u, const float* fi,
                                              const float* fj, int nq, double dq, double* far_seen) {
-  *far_seen = 1.0;
+  if (far_seen) *far_seen = 1.0;
   double s1, c1;
   sincos(dq * r, &s1, &c1);
   const double k2 = 2.0 * c1;

@@ -212,7 +212,8 @@ size_t force_lds_bytes(int64_t n_cell);     // LDS of a block
 hipError_t launch_force_table(hipStream_t st, const double2* coef, int nq, double dq, int n_table,
                               int n_cell, float4* t4, float2* t2);
 // part[plane][position][3], or with out the forces themselves (a single plane):
-// out[perm[p]][c] = conv * sum; *far_seen becomes 1 when a pair lies past the table
+// out[perm[p]][c] = conv * sum; *far_seen (nullable, host
+// memory) becomes 1 when a pair lies past the table
 hipError_t launch_table_force(hipStream_t st, const AtomRec* pos, const ForceUnit* units,
                               int n_units, int n_cell, const float4* t4, const float2* t2,
                               const float* u, const float* ftab, int nq, double dq, int64_t n,

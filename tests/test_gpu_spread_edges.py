@@ -328,3 +328,91 @@ def test_captured_gradient_after_a_sampler():
         assert np.abs(a - b).max() < 2.0 ** -20 * np.abs(b).max()
     del g
     s.c.close()
+
+
+def device_forces(c, n, target, chains=1):
+    """Forces alone, all arrays on the GPU: no energy that the host would wait for."""
+    import torch
+    out = torch.zeros((n, 3), dtype=torch.float64, device="cuda")
+    _lib.check(c.lib.pyiid_pdf_energy_forces(c.handle, _lib.SLOT_PDF, 0.1, target.data_ptr(),
+                                             _lib.POT_RW, 1.0, None, out.data_ptr(),
+                                             _lib.PYIID_DEVICE))
+    return out
+
+
+def test_force_table_grows_after_calls_without_energy():
+    """Atoms moved past the force table's end on the device: their pairs are summed
+    directly, and the next call has a table for their extent, whether or not the
+    host asks for energies: the same bits as a new context's."""
+    import torch
+    n, nq, qbin = 90, 250, 0.1
+    base = structures.jitter(structures.fcc_nearest(n), 0.05, seed=2).astype(np.float32)
+    pos = base.copy()
+    pos[40:] += np.float32(17.3)
+    table, _, _ = element_table(np.full(n, 79), qbin, nq)
+    r = 2.0 + 0.02 * np.arange(300)
+    target = torch.from_numpy(np.cos(r)).cuda()
+
+    def context(p):
+        c = _lib.Context(0)
+        c.set_positions(torch.from_numpy(p).cuda(), flags=_lib.PYIID_DEVICE)
+        c.set_elements(np.zeros(n, np.int32))
+        c.set_scatter(_lib.SLOT_PDF, table)
+        c.set_transform(0.02, qbin, r, 0.0, nq)
+        c.set_autotune(True)
+        out = device_forces(c, n, target)
+        c.synchronize()
+        return c, out.cpu().numpy()
+    c, _ = context(base)
+    moved = torch.from_numpy(pos).cuda()
+    got = []
+    for _ in range(2):
+        c.set_positions(moved, flags=_lib.PYIID_DEVICE)
+        out = device_forces(c, n, target)
+        c.synchronize()
+        got.append(out.cpu().numpy())
+    fresh, want = context(pos)
+    assert np.abs(got[0] - want).max() < 1e-6 * np.abs(want).max()
+    np.testing.assert_array_equal(got[1], want)
+    c.close()
+    fresh.close()
+
+
+def test_batch_after_a_larger_one_keeps_its_extent():
+    """Energies of eight chains, then of four: nothing of the first batch's results
+    is taken for a pair past the force table, which would make the next call wait
+    for the extent, and so fail in a capture."""
+    import torch
+    nq, qbin, r = 250, 0.1, 2.0 + 0.02 * np.arange(300)
+    chains = [structures.jitter(structures.fcc_nearest(40), 0.05, seed=b).astype(np.float32)
+              for b in range(8)]
+    stream = torch.cuda.Stream()
+    c = _lib.Context(0)
+    c.set_stream(stream.cuda_stream)
+    table, _, _ = element_table(np.full(40, 79), qbin, nq)
+    target = np.tile(np.cos(r) + 0.5, (8, 1))
+    c.set_transform(0.02, qbin, r, 0.0, nq)
+    for b in (8, 4):
+        c.set_batch(chains[:b])
+        c.set_elements(np.zeros(40 * b, np.int32))
+        c.set_scatter(_lib.SLOT_PDF, table)
+        e, f = c.pdf_energy_forces(_lib.SLOT_PDF, qbin, target[:b], _lib.POT_RW, 1.0, 40 * b)
+        assert np.all(e > 0.0)
+    dev = torch.from_numpy(target).cuda()
+    out = torch.zeros((160, 3), dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream):
+        _lib.check(c.lib.pyiid_pdf_energy_forces(c.handle, _lib.SLOT_PDF, qbin, dev.data_ptr(),
+                                                 _lib.POT_RW, 1.0, None, out.data_ptr(),
+                                                 _lib.PYIID_DEVICE))
+    for _ in range(3):
+        with torch.cuda.stream(stream):
+            out.zero_()
+            g.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.cpu().numpy(), f)
+        np.testing.assert_array_equal(
+            c.pdf_energy_forces(_lib.SLOT_PDF, qbin, target[:4], _lib.POT_RW, 1.0, 160)[1], f)
+    del g
+    c.close()
