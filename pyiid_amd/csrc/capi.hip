@@ -942,12 +942,14 @@ size_t spread_grid_bytes(pyiid_ctx* c, const Table& t) {
 }
 
 // Whether F(Q) runs on the spreading kernel: its grid fits LDS, the grids fit
-// their budget, and neither compensated sums nor a fixed shape of the
-// recurrence kernel is asked for.
+// their budget and their transform a launch, and neither compensated sums nor a
+// fixed shape of the recurrence kernel is asked for.
 bool use_spread_fq(pyiid_ctx* c, const Table& t) {
   return !c->compensated && c->fq_m_fixed == 0 &&
          sizeof(uint64_t) * static_cast<size_t>(fq_grid_stride(t.nq)) <= kSpreadLds &&
-         spread_grid_bytes(c, t) <= kSpreadGridBudget && c->n_chain <= 65535;
+         spread_grid_bytes(c, t) <= kSpreadGridBudget && c->n_chain <= 65535 &&
+         element_pairs(t) * fq_transform_parts(t.nq, c->n_chain, static_cast<int>(element_pairs(t))) <=
+             65535;
 }
 
 // Whether F(Q) runs in one launch: small chains, whose pairs each block of 64

@@ -416,3 +416,31 @@ def test_batch_after_a_larger_one_keeps_its_extent():
             c.pdf_energy_forces(_lib.SLOT_PDF, qbin, target[:4], _lib.POT_RW, 1.0, 160)[1], f)
     del g
     c.close()
+
+
+@pytest.mark.parametrize("rows", [361, 362, 400, 1000])
+def test_tables_of_many_rows(ctx, rows):
+    """A table with a row for every atom and more (element pairs up to and past what
+    one launch of the transform takes): F, gradient and forces against the oracle."""
+    n, nq, qbin = 80, 60, 0.25
+    rs = np.random.RandomState(rows)
+    pos = structures.jitter(structures.fcc_nearest(n), 0.05, seed=rows).astype(np.float32)
+    q = np.arange(nq) * qbin
+    table = (rs.uniform(20, 80, (rows, 1)) * np.exp(-rs.uniform(0.5, 3.0, (rows, 1)) * (q / 12.6) ** 2)
+             ).astype(np.float32)
+    index = rs.permutation(rows)[:n].astype(np.int32)
+    ctx.set_positions(pos)
+    ctx.set_elements(index)
+    ctx.set_scatter(_lib.SLOT_FQ, table)
+    per_atom = table[index]
+    want, gwant = oracle.fq(pos, per_atom, qbin), oracle.grad_fq(pos, per_atom, qbin)
+    for _ in range(2):
+        fq = np.empty(nq, np.float32)
+        g = ctx.grad_fq(_lib.SLOT_FQ, qbin, n, nq, fq_out=fq)
+        assert np.abs(ctx.fq(_lib.SLOT_FQ, qbin, nq) - want).max() < 1e-6 * np.abs(want).max()
+        assert np.abs(fq - want).max() < 1e-6 * np.abs(want).max()
+        assert np.abs(g - gwant).max() < 2e-6 * np.abs(gwant).max()
+        target = want * 0.9 + 0.1
+        e, f = ctx.fq_energy_forces(_lib.SLOT_FQ, qbin, 0, target, _lib.POT_RW, 10.0, n)
+        fwant = 10.0 * oracle.wrap_grad_rw(gwant, want, target)
+        assert np.abs(f - fwant).max() < 5e-6 * np.abs(fwant).max()
