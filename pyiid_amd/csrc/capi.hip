@@ -941,11 +941,16 @@ size_t spread_grid_bytes(pyiid_ctx* c, const Table& t) {
          static_cast<size_t>(element_pairs(t)) * c->n_chain;
 }
 
+// Bins that grids and tables can be made for.  The entry points which take energies
+// accept any bin width: with one that is not positive the recurrence kernels give
+// what the formulas give (F(-Q) = -F(Q)).
+bool gridded(double dq) { return dq > 0.0 && dq < HUGE_VAL; }
+
 // Whether F(Q) runs on the spreading kernel: its grid fits LDS, the grids fit
 // their budget and their transform a launch, and neither compensated sums nor a
 // fixed shape of the recurrence kernel is asked for.
-bool use_spread_fq(pyiid_ctx* c, const Table& t) {
-  return !c->compensated && c->fq_m_fixed == 0 &&
+bool use_spread_fq(pyiid_ctx* c, const Table& t, double dq) {
+  return gridded(dq) && !c->compensated && c->fq_m_fixed == 0 &&
          sizeof(uint64_t) * static_cast<size_t>(fq_grid_stride(t.nq)) <= kSpreadLds &&
          spread_grid_bytes(c, t) <= kSpreadGridBudget && c->n_chain <= 65535 &&
          element_pairs(t) * fq_transform_parts(t.nq, c->n_chain, static_cast<int>(element_pairs(t))) <=
@@ -1197,10 +1202,10 @@ int compute_fq(pyiid_ctx* c, int slot, double qbin, float* direct = nullptr,
   CHK(ensure_norm(c, slot));
   double* out64 = direct ? nullptr : c->fq64.as<double>();
   float* out32 = direct ? direct : c->fq32.as<float>();
-  if (use_spread_fq(c, t)) {
+  const double dq = static_cast<double>(static_cast<float>(qbin));
+  if (use_spread_fq(c, t, dq)) {
     SpreadSet& s = c->spread;
     const bool weighted = weighted_table(t);
-    const double dq = static_cast<double>(static_cast<float>(qbin));
     if (use_small_fq(c, t)) {
       CHK(ensure_extent(c));
       CHK(ensure_offsets(c));
@@ -1634,8 +1639,8 @@ constexpr size_t kGradRowBudget = static_cast<size_t>(1) << 30;
 
 // Whether the gradient runs on the spreading kernel: its grids fit LDS, and
 // neither compensated sums nor a recurrence kernel or its shape is asked for.
-bool use_spread_grad(pyiid_ctx* c, const Table& t) {
-  return !c->compensated && c->grad_kernel == PYIID_GRAD_AUTO && c->grad_m_fixed == 0 &&
+bool use_spread_grad(pyiid_ctx* c, const Table& t, double dq) {
+  return gridded(dq) && !c->compensated && c->grad_kernel == PYIID_GRAD_AUTO && c->grad_m_fixed == 0 &&
          c->sym_k_fixed == 0 && grad_lds_bytes(t.nq) <= kGradLds;
 }
 
@@ -1643,8 +1648,8 @@ bool use_spread_grad(pyiid_ctx* c, const Table& t) {
 // are what counts; a single element, whose transform needs no further sum.
 constexpr int64_t kBothAtoms = 2048;
 constexpr int kBothBins = 512;
-bool use_spread_both(pyiid_ctx* c, const Table& t) {
-  return use_spread_grad(c, t) && use_spread_fq(c, t) && !use_small_fq(c, t) &&
+bool use_spread_both(pyiid_ctx* c, const Table& t, double dq) {
+  return use_spread_grad(c, t, dq) && use_spread_fq(c, t, dq) && !use_small_fq(c, t) &&
          c->n <= kBothAtoms && t.nq <= kBothBins && element_pairs(t) == 1;
 }
 
@@ -1753,6 +1758,7 @@ int64_t force_cells(pyiid_ctx* c, const Table& t, double dq) {
 
 // Whether the tables fit LDS and their budget (else the recurrence kernel runs).
 bool use_force_table(pyiid_ctx* c, const Table& t, double dq) {
+  if (!gridded(dq)) return false;
   const int64_t cells = force_cells(c, t, dq);
   const int64_t pairs = element_pairs(t);
   return force_lds_bytes(cells) <= kForceLds && pairs * c->n_chain <= 65535 &&
@@ -2824,7 +2830,8 @@ int pyiid_grad_fq(pyiid_ctx* c, int slot, double qbin, void* grad, float* fq, in
   CHK(ensure_norm(c, slot));
   Table& t = c->tab[slot];
   void* gdst = grad;
-  c->grad_spread = use_spread_grad(c, t);
+  const double dq = static_cast<double>(static_cast<float>(qbin));
+  c->grad_spread = use_spread_grad(c, t, dq);
   if (c->grad_spread) {
     float* fdst = fq;
     bool copy = false;
@@ -2840,7 +2847,7 @@ int pyiid_grad_fq(pyiid_ctx* c, int slot, double qbin, void* grad, float* fq, in
       if (fq) CHK(arena_result(c, fq, sizeof(float) * nq, &f));
       fdst = static_cast<float*>(f);
     }
-    const bool both = fq && fdst && use_spread_both(c, t);
+    const bool both = fq && fdst && use_spread_both(c, t, dq);
     const SharedOrder shared(c);
     CHK(run_spread_grad(c, slot, qbin, gdst, (flags & PYIID_F64) != 0, both ? fdst : nullptr));
     if (copy) CHK(download(c, grad, gdst, gbytes, flags));

@@ -444,3 +444,36 @@ def test_tables_of_many_rows(ctx, rows):
         e, f = ctx.fq_energy_forces(_lib.SLOT_FQ, qbin, 0, target, _lib.POT_RW, 10.0, n)
         fwant = 10.0 * oracle.wrap_grad_rw(gwant, want, target)
         assert np.abs(f - fwant).max() < 5e-6 * np.abs(fwant).max()
+
+
+@pytest.mark.parametrize("n,kinds", [(40, 1), (40, 2), (300, 1)])
+def test_energies_of_negative_bins(ctx, n, kinds):
+    """Energies and forces take a bin width of either sign: F(-Q) = -F(Q), so that
+    the energy against a target is that of the positive bins against its negative
+    (to the 1e-6 that two kernels differ by; the target is that of a structure 2%
+    smaller, Rw 0.7: near a fit the residual would magnify F's rounding).  F and the
+    gradient refuse it."""
+    nq, qbin, r = 250, 0.1, 2.0 + 0.02 * np.arange(300)
+    pos = structures.jitter(structures.fcc_nearest(n), 0.05, seed=n).astype(np.float32)
+    numbers = np.array([79, 28])[np.arange(n) % kinds]
+    table, index, _ = element_table(numbers, qbin, nq)
+    load(ctx, (pos * np.float32(0.98)).astype(np.float32), numbers, qbin, nq)
+    ctx.set_scatter(_lib.SLOT_PDF, table)
+    ctx.set_transform(0.02, qbin, r, 0.0, nq)
+    fq = ctx.fq(_lib.SLOT_FQ, qbin, nq)
+    ctx.set_positions(pos)
+    for target, call in (
+            (ctx.pdf(fq, 300),
+             lambda q, t: ctx.pdf_energy_forces(_lib.SLOT_PDF, q, t, _lib.POT_RW, 10.0, n)),
+            (fq.astype(np.float64),
+             lambda q, t: ctx.fq_energy_forces(_lib.SLOT_FQ, q, 0, t, _lib.POT_RW, 10.0, n))):
+        e, f = call(qbin, target)
+        en, fn = call(-qbin, -target)
+        assert abs(en - e) < 1e-5 * abs(e)
+        assert np.abs(fn - f).max() < 1e-5 * np.abs(f).max()
+        assert call(-qbin, target)[0] > 1.01 * e
+    for width in (-qbin, 0.0, np.nan):
+        with pytest.raises(ValueError):
+            ctx.fq(_lib.SLOT_FQ, width, nq)
+        with pytest.raises(ValueError):
+            ctx.grad_fq(_lib.SLOT_FQ, width, n, nq)
