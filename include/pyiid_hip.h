@@ -71,15 +71,16 @@ int pyiid_synchronize(pyiid_ctx *ctx);
 int pyiid_enable_timing(pyiid_ctx *ctx, int enable);
 int pyiid_kernel_time(pyiid_ctx *ctx, int kind, double *total_ms, int64_t *launches);
 /* While timing is enabled, the F-only recurrence kernel (which runs when its
- * bins per wave are fixed, with compensated sums, or past the spreading kernel's
- * limits) counts its (wave, j atom) steps by recurrence form: the three-term form, or the Reinsch form that a wave
+ * bins per wave are fixed, with compensated sums, past the spreading kernel's
+ * limits, or where it is the faster of the two) counts its (wave, j atom) steps by recurrence form: the three-term form, or the Reinsch form that a wave
  * takes when any of its pairs has a per-bin phase step within 0.2 of a
  * multiple of pi.  Counts since timing was last enabled.  No counterpart in
  * the reference. */
 int pyiid_fq_form_counts(pyiid_ctx *ctx, int64_t *three_term, int64_t *reinsch);
 /* Q bins per wave of the F-only recurrence kernel: 64, 72, 80, 88, 96 or 112 runs
  * pyiid_fq on that kernel with that launch shape; 0 (the default) runs the
- * spreading kernel, and past its limits (compensated sums, about 3,400 bins)
+ * spreading kernel, and past its limits (compensated sums, about 3,400 bins) or
+ * where it is slower (many elements, batches of many small chains of several)
  * the recurrence kernel at the shape that the autotuner found fastest.
  * The shapes differ only in how the bins are
  * grouped, so F agrees between them to FP32 rounding.  No counterpart in the
@@ -88,7 +89,8 @@ int pyiid_set_fq_bins_per_wave(pyiid_ctx *ctx, int m);
 /* Q bins per wave of the ordered-pair F + gradient kernel: 16 or 32 runs
  * pyiid_grad_fq on that kernel with that launch shape (and the default j
  * split); 0 (the default) runs the spreading kernel, and past its limits
- * (compensated sums, about 3,000 bins) lets the autotuner choose between the
+ * (compensated sums, about 3,000 bins) or where it is slower (few bins, a low
+ * largest Q, many elements) lets the autotuner choose between the
  * symmetric (unordered-pair) kernel and the ordered one, and time the ordered one's
  * two shapes with three split sizes each, once per problem shape.  Kernels and
  * shapes differ only in how the sums are grouped, so the results agree to
@@ -109,7 +111,7 @@ int pyiid_set_grad_tiles_per_item(pyiid_ctx *ctx, int k);
  * counterpart in the reference. */
 int pyiid_set_grad_sym_bins_per_wave(pyiid_ctx *ctx, int m);
 /* Kernel of pyiid_grad_fq: PYIID_GRAD_AUTO (the default) runs the spreading
- * kernel within its limits and lets the autotuner choose past them,
+ * kernel as pyiid_set_grad_bins_per_wave says, else lets the autotuner choose,
  * PYIID_GRAD_ORDERED and PYIID_GRAD_SYMMETRIC restrict it to one recurrence kernel (whose launch shapes are still autotuned unless fixed by the setters
  * above).  Compensated sums always run the ordered kernel.  No counterpart in
  * the reference. */

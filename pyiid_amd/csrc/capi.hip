@@ -20,6 +20,7 @@
 #include "../../include/pyiid_hip.h"
 #include "extent.h"
 #include "internal.h"
+#include "route.h"
 
 using namespace pyiid;
 
@@ -214,7 +215,8 @@ struct pyiid_ctx {
   Buf pos;   // AtomRec [n]
   bool pos_dirty = true;
   std::vector<int32_t> elem_h;
-  int max_elem = 0;
+  int max_elem = 0, kinds = 1;  // largest element index, elements present
+  BatchSize size;
   Buf counts_d, natoms_d;
   Buf off_d;  // int32 chain offsets
   std::vector<int64_t> off_d_of;  // the layout in off_d
@@ -946,17 +948,6 @@ size_t spread_grid_bytes(pyiid_ctx* c, const Table& t) {
 // what the formulas give (F(-Q) = -F(Q)).
 bool gridded(double dq) { return dq > 0.0 && dq < HUGE_VAL; }
 
-// Whether F(Q) runs on the spreading kernel: its grid fits LDS, the grids fit
-// their budget and their transform a launch, and neither compensated sums nor a
-// fixed shape of the recurrence kernel is asked for.
-bool use_spread_fq(pyiid_ctx* c, const Table& t, double dq) {
-  return gridded(dq) && !c->compensated && c->fq_m_fixed == 0 &&
-         sizeof(uint64_t) * static_cast<size_t>(fq_grid_stride(t.nq)) <= kSpreadLds &&
-         spread_grid_bytes(c, t) <= kSpreadGridBudget && c->n_chain <= 65535 &&
-         element_pairs(t) * fq_transform_parts(t.nq, c->n_chain, static_cast<int>(element_pairs(t))) <=
-             65535;
-}
-
 // Whether F(Q) runs in one launch: small chains, whose pairs each block of 64
 // bins spreads for itself, where that takes about as long as the three launches
 // for one call alone and less among others (us, 500 bins, alone and among others:
@@ -970,13 +961,20 @@ bool use_small_fq(pyiid_ctx* c, const Table& t) {
     return false;
   const int64_t kinds = element_pairs(t);
   const int most = kinds == 1 ? kSmallAtoms : kinds == 3 ? kSmallAtoms2 : kSmallAtoms3;
-  int64_t pairs = 0;
-  for (int b = 0; b < c->n_chain; ++b) {
-    const int64_t n = c->off[b + 1] - c->off[b];
-    if (n > most) return false;
-    pairs += n * (n - 1) / 2;
-  }
-  return pairs * ((t.nq + 63) / 64) <= 2000000;
+  return c->size.longest <= most &&
+         c->size.pairs() * static_cast<double>(blocks_of_bins(t.nq)) <= 2e6;
+}
+
+// Whether F(Q) runs on the spreading kernel: its grid fits LDS, the grids fit
+// their budget and their transform a launch, and neither compensated sums nor a
+// fixed shape of the recurrence kernel is asked for; and it is the faster one.
+bool use_spread_fq(pyiid_ctx* c, const Table& t, double dq) {
+  return gridded(dq) && !c->compensated && c->fq_m_fixed == 0 &&
+         sizeof(uint64_t) * static_cast<size_t>(fq_grid_stride(t.nq)) <= kSpreadLds &&
+         spread_grid_bytes(c, t) <= kSpreadGridBudget && c->n_chain <= 65535 &&
+         element_pairs(t) * fq_transform_parts(t.nq, c->n_chain, static_cast<int>(element_pairs(t))) <=
+             65535 &&
+         spread_fq_pays(c->size, t.n_elem, element_pairs(t), t.nq, dq, use_small_fq(c, t));
 }
 
 int ensure_offsets(pyiid_ctx* c) {
@@ -1637,11 +1635,13 @@ int tune_grad(pyiid_ctx* c, int slot, double qbin) {
 // Bytes of the rows of one chunk of atoms; a large structure runs in several.
 constexpr size_t kGradRowBudget = static_cast<size_t>(1) << 30;
 
-// Whether the gradient runs on the spreading kernel: its grids fit LDS, and
-// neither compensated sums nor a recurrence kernel or its shape is asked for.
+// Whether the gradient runs on the spreading kernel: its grids fit LDS, neither
+// compensated sums nor a recurrence kernel or its shape is asked for, and it is the
+// faster one.
 bool use_spread_grad(pyiid_ctx* c, const Table& t, double dq) {
   return gridded(dq) && !c->compensated && c->grad_kernel == PYIID_GRAD_AUTO && c->grad_m_fixed == 0 &&
-         c->sym_k_fixed == 0 && grad_lds_bytes(t.nq) <= kGradLds;
+         c->sym_k_fixed == 0 && grad_lds_bytes(t.nq) <= kGradLds &&
+         spread_grad_pays(c->n, weighted_table(t) ? c->kinds : 1, t.nq, dq);
 }
 
 // Whether F of a gradient call rides along with it: few atoms, where launches
@@ -1756,14 +1756,16 @@ int64_t force_cells(pyiid_ctx* c, const Table& t, double dq) {
   return cells < 1e9 ? static_cast<int64_t>(cells) : static_cast<int64_t>(1e9);
 }
 
-// Whether the tables fit LDS and their budget (else the recurrence kernel runs).
+// Whether the tables fit LDS and their budget, and are the faster way (else the
+// recurrence kernel runs).
 bool use_force_table(pyiid_ctx* c, const Table& t, double dq) {
   if (!gridded(dq)) return false;
   const int64_t cells = force_cells(c, t, dq);
   const int64_t pairs = element_pairs(t);
   return force_lds_bytes(cells) <= kForceLds && pairs * c->n_chain <= 65535 &&
          24.0 * static_cast<double>(cells) * pairs * c->n_chain <=
-             static_cast<double>(kForceTableBudget);
+             static_cast<double>(kForceTableBudget) &&
+         force_table_pays(c->size, t.n_elem, pairs, t.nq, static_cast<double>(cells));
 }
 
 // Units: per chain the i tiles of each element against each element's j run.
@@ -2015,9 +2017,13 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
                             hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->max_elem = 0;
+    c->kinds = 1;
     c->n = n;
     c->off = off;
     c->n_chain = static_cast<int>(off.size()) - 1;
+    c->size = BatchSize();
+    c->size.chains = c->n_chain;
+    for (int b = 0; b < c->n_chain; ++b) c->size.add(off[b + 1] - off[b]);
     c->struct_stamp++;
     c->hmc.set = false;
     destroy_graph(c->hmc);
@@ -2751,12 +2757,15 @@ int pyiid_set_elements(pyiid_ctx* c, const int32_t* elem, int64_t n, int flags) 
     }
   }
   int mx = 0;
+  std::vector<bool> present(1024, false);
   for (int32_t e : h) {
     if (e < 0 || e >= 1024) return fail(PYIID_E_INVALID, "element index %d out of range [0, 1024)", e);
     mx = std::max(mx, static_cast<int>(e));
+    present[e] = true;
   }
   c->elem_h = h;
   c->max_elem = mx;
+  c->kinds = static_cast<int>(std::count(present.begin(), present.end(), true));
   if (n > 0)
     HIPCHK(hipMemcpyAsync(c->elem.p, h.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice,
                           c->stream));

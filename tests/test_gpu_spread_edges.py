@@ -434,13 +434,14 @@ def test_tables_of_many_rows(ctx, rows):
     ctx.set_scatter(_lib.SLOT_FQ, table)
     per_atom = table[index]
     want, gwant = oracle.fq(pos, per_atom, qbin), oracle.grad_fq(pos, per_atom, qbin)
+    # (a structure 2% smaller: near a fit the residual would magnify F's rounding)
+    target = oracle.fq((pos * np.float32(0.98)).astype(np.float32), per_atom, qbin)
     for _ in range(2):
         fq = np.empty(nq, np.float32)
         g = ctx.grad_fq(_lib.SLOT_FQ, qbin, n, nq, fq_out=fq)
         assert np.abs(ctx.fq(_lib.SLOT_FQ, qbin, nq) - want).max() < 1e-6 * np.abs(want).max()
         assert np.abs(fq - want).max() < 1e-6 * np.abs(want).max()
         assert np.abs(g - gwant).max() < 2e-6 * np.abs(gwant).max()
-        target = want * 0.9 + 0.1
         e, f = ctx.fq_energy_forces(_lib.SLOT_FQ, qbin, 0, target, _lib.POT_RW, 10.0, n)
         fwant = 10.0 * oracle.wrap_grad_rw(gwant, want, target)
         assert np.abs(f - fwant).max() < 5e-6 * np.abs(fwant).max()
@@ -477,3 +478,68 @@ def test_energies_of_negative_bins(ctx, n, kinds):
             ctx.fq(_lib.SLOT_FQ, width, nq)
         with pytest.raises(ValueError):
             ctx.grad_fq(_lib.SLOT_FQ, width, n, nq)
+
+
+@pytest.mark.parametrize("n,kinds,nq,q_max,spread", [
+    (400, 1, 40, 1.01, True), (401, 1, 40, 1.01, False), (400, 1, 40, 0.9, False),
+    (650, 1, 129, 1.01, False), (650, 1, 130, 1.01, True), (650, 1, 16, 12.0, True),
+    (650, 1, 16, 11.0, False), (900, 1, 90, 9.9, False), (900, 1, 90, 10.1, True),
+    (900, 1, 257, 1.01, True), (1300, 1, 105, 3.9, False), (1300, 1, 105, 4.1, True),
+    (100, 3, 100, 25.0, True), (100, 4, 100, 25.0, False), (210, 4, 250, 25.0, True),
+    (210, 6, 250, 25.0, False)])
+def test_gradient_beside_the_lines_between_kernels(ctx, n, kinds, nq, q_max, spread):
+    """Both sides of the rule's lines (atoms, bins, largest Q, elements): the kernel
+    it names runs, and F and the gradient are the oracle's (1e-6 and 2e-6 of the
+    largest, as everywhere)."""
+    qbin = q_max / nq
+    pos = structures.jitter(structures.fcc_nearest(n), 0.05, seed=n).astype(np.float32)
+    q = np.arange(nq) * qbin
+    table = np.stack([(20 + 10 * e) * np.exp(-(1 + 0.2 * e) * (q / 12.6) ** 2)
+                      for e in range(kinds)]).astype(np.float32)
+    index = (np.arange(n) % kinds).astype(np.int32)
+    ctx.set_positions(pos)
+    ctx.set_elements(index)
+    ctx.set_scatter(_lib.SLOT_FQ, table)
+    fq = np.empty(nq, np.float32)
+    g = ctx.grad_fq(_lib.SLOT_FQ, qbin, n, nq, fq_out=fq)
+    assert (ctx.grad_shape() == (False, 0, 0)) == spread
+    want = oracle.fq(pos, table[index], qbin)
+    rows = np.arange(0, n, 29)
+    gwant = oracle.grad_fq(pos, table[index], qbin, atom_index=rows)
+    assert np.abs(fq - want).max() < 1e-6 * np.abs(want).max()
+    assert np.abs(ctx.fq(_lib.SLOT_FQ, qbin, nq) - want).max() < 1e-6 * np.abs(want).max()
+    assert np.abs(g[rows] - gwant).max() < 2e-6 * np.abs(gwant).max()
+
+
+@pytest.mark.parametrize("chains,n,kinds", [(1, 90, 12), (1, 90, 40), (40, 45, 3), (40, 130, 3), (20, 100, 6)])
+def test_batches_beside_the_lines_between_kernels(ctx, chains, n, kinds):
+    """F, energies and forces of batches on either side of the rules, against each
+    chain alone in float64."""
+    nq, qbin, r = 100, 0.2, 2.0 + 0.02 * np.arange(120)
+    pos = [structures.jitter(structures.fcc_nearest(n), 0.05, seed=b).astype(np.float32)
+           for b in range(chains)]
+    q = np.arange(nq) * qbin
+    table = np.stack([(20 + 3 * e) * np.exp(-(1 + 0.05 * e) * (q / 12.6) ** 2)
+                      for e in range(kinds)]).astype(np.float32)
+    index = (np.arange(n) % kinds).astype(np.int32)
+    target = np.tile(np.cos(r) + 0.2, (chains, 1))
+    ctx.set_batch(pos)
+    ctx.set_elements(np.tile(index, chains))
+    for slot in (_lib.SLOT_FQ, _lib.SLOT_PDF):
+        ctx.set_scatter(slot, table)
+    ctx.set_transform(0.02, qbin, r, 0.0, nq)
+    for _ in range(2):
+        fq = ctx.fq(_lib.SLOT_FQ, qbin, nq, n_chain=chains).reshape(chains, nq)
+        e, f = ctx.pdf_energy_forces(_lib.SLOT_PDF, qbin, target, _lib.POT_RW, 10.0, n * chains)
+    want_fq = [oracle.fq(p, table[index], qbin) for p in pos]
+    for b in (0, chains // 2, chains - 1):
+        assert np.abs(fq[b] - want_fq[b]).max() < 1e-6 * np.abs(want_fq[b]).max()
+    for b in (0, chains - 1):
+        ctx.set_positions(pos[b])
+        ctx.set_elements(index)
+        ctx.set_transform(0.02, qbin, r, 0.0, nq)
+        g = ctx.pdf(want_fq[b].astype(np.float32), len(r))
+        gg = ctx.grad_pdf(oracle.grad_fq(pos[b], table[index], qbin), len(r))
+        want = 10.0 * oracle.wrap_grad_rw(gg, g, target[0])
+        assert abs(np.atleast_1d(e)[b] - 10.0 * oracle.get_rw(target[0], g)[0]) < 1e-5
+        assert np.abs(f[b * n:(b + 1) * n] - want).max() < 1e-5 * np.abs(want).max()

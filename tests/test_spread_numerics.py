@@ -125,3 +125,64 @@ def test_extent_of_positions_that_are_not_finite(tmp_path):
     subprocess.run(["g++", "-O2", "-std=c++17", "-I", CSRC, "-o", str(exe), str(src)], check=True)
     out = subprocess.run([str(exe)], capture_output=True, text=True)
     assert out.returncode == 0, out.stdout
+
+
+ROUTE = r"""
+#include "route.h"
+#include <cstdio>
+using namespace pyiid;
+int main() {
+  char kind;
+  double chains, n, elements, nq, dq, cells;
+  while (std::scanf(" %c %lf %lf %lf %lf %lf %lf", &kind, &chains, &n, &elements, &nq, &dq, &cells) == 7) {
+    BatchSize s;
+    s.chains = static_cast<int64_t>(chains);
+    for (int b = 0; b < s.chains; ++b) s.add(static_cast<int64_t>(n));
+    const int e = static_cast<int>(elements), q = static_cast<int>(nq);
+    const int64_t pairs = e * (e + 1) / 2;
+    std::printf("%d\n", kind == 'f'   ? spread_fq_pays(s, e, pairs, q, dq, false)
+                        : kind == 'g' ? spread_grad_pays(static_cast<int64_t>(n), e, q, dq)
+                                      : force_table_pays(s, e, pairs, q, cells));
+  }
+}
+"""
+
+# kind (F, gradient, forces), chains, atoms, elements, bins, largest Q, cells, and the
+# time of the recurrence and of the spreading kernel or table (us, MI355X; for the
+# forces without F)
+MEASURED = [
+    ("f", 1, 55, 1, 250, 25.0, 0, 45, 10), ("f", 1, 7000, 1, 3400, 25.0, 0, 5126, 88),
+    ("f", 1, 7000, 1, 100, 1.0, 0, 484, 214), ("f", 1, 7000, 1, 1, 0.1, 0, 450, 600),
+    ("f", 1, 4000, 3, 600, 25.0, 0, 403, 66), ("f", 1, 600, 8, 250, 25.0, 0, 62, 30),
+    ("f", 1, 600, 32, 250, 25.0, 0, 45, 102), ("f", 1, 60, 16, 250, 25.0, 0, 19, 33),
+    ("f", 1, 4000, 16, 250, 25.0, 0, 332, 72), ("f", 1, 300, 128, 250, 25.0, 0, 240, 1127),
+    ("f", 1, 7000, 64, 250, 25.0, 0, 627, 394), ("f", 1, 7000, 128, 250, 25.0, 0, 764, 1344),
+    ("f", 64, 300, 3, 330, 25.0, 0, 393, 117), ("f", 64, 40, 3, 330, 25.0, 0, 32, 69),
+    ("f", 256, 80, 3, 330, 25.0, 0, 93, 223), ("f", 1024, 150, 1, 330, 25.0, 0, 509, 202),
+    ("f", 1024, 40, 1, 330, 25.0, 0, 91, 150), ("f", 256, 600, 6, 330, 25.0, 0, 1292, 970),
+    ("g", 1, 300, 1, 64, 1.0, 0, 45, 39), ("g", 1, 300, 1, 4, 0.4, 0, 44, 83),
+    ("g", 1, 600, 1, 64, 1.0, 0, 45, 56), ("g", 1, 600, 1, 16, 25.0, 0, 42, 33),
+    ("g", 1, 1000, 1, 32, 8.0, 0, 47, 66), ("g", 1, 1000, 1, 100, 25.0, 0, 56, 46),
+    ("g", 1, 2000, 1, 100, 4.0, 0, 170, 205), ("g", 1, 2000, 1, 100, 12.0, 0, 169, 111),
+    ("g", 1, 7000, 1, 16, 2.0, 0, 1311, 1573), ("g", 1, 7000, 1, 64, 8.0, 0, 1373, 1015),
+    ("g", 1, 7000, 1, 200, 1.0, 0, 2168, 1740), ("g", 1, 15000, 1, 8, 25.0, 0, 4975, 5878),
+    ("g", 1, 300, 16, 250, 25.0, 0, 42, 143), ("g", 1, 2000, 8, 250, 25.0, 0, 297, 163),
+    ("g", 1, 2000, 32, 250, 25.0, 0, 397, 643), ("g", 1, 7000, 32, 250, 25.0, 0, 2794, 1816),
+    ("t", 1, 2000, 3, 330, 25.0, 1900, 600, 90), ("t", 1, 600, 16, 250, 25.0, 1230, 190, 109),
+    ("t", 1, 300, 128, 250, 25.0, 970, 1844, 3472), ("t", 1, 4000, 64, 250, 25.0, 2330, 593, 1305),
+    ("t", 256, 300, 6, 330, 25.0, 970, 1013, 1767), ("t", 256, 600, 6, 330, 25.0, 1230, 3102, 2444),
+    ("t", 256, 20, 6, 330, 25.0, 360, 1067, 761), ("t", 64, 300, 3, 330, 25.0, 970, 846, 196),
+]
+
+
+def test_rules_of_the_dispatch_take_the_faster_kernel(tmp_path):
+    src, exe = tmp_path / "route.cpp", tmp_path / "route"
+    src.write_text(ROUTE)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", CSRC, "-o", str(exe), str(src)], check=True)
+    lines = ["%s %d %d %d %d %.9g %d" % (k, b, n, e, nq, q / nq, cells)
+             for k, b, n, e, nq, q, cells, _, _ in MEASURED]
+    out = subprocess.run([str(exe)], input="\n".join(lines), capture_output=True, text=True, check=True)
+    got = [int(x) for x in out.stdout.split()]
+    assert len(got) == len(MEASURED)
+    for row, new in zip(MEASURED, got):
+        assert bool(new) == (row[-1] < row[-2]), row
