@@ -229,6 +229,7 @@ struct pyiid_ctx {
   bool extent_exact = false;        // r_max bounds the current positions' distances
   Buf reach;                        // double: such a bound on the device
   bool reach_set = false;           // of the current positions
+  bool reach_wanted = true;         // the last gradient, if any, asked for it
   // page-locked, written by the forces' kernel: a pair lay past the force table
   double* far_seen = nullptr;
   bool extent_old = false;          // it did: take the extent anew
@@ -2044,7 +2045,8 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
     // (the gradient of a single structure asks how far its distances reach)
     CHK(c->reach.reserve(sizeof(double)));
     const bool reach =
-        (flags & PYIID_DEVICE) && c->n_chain == 1 && n <= kReachAtoms && !c->replays_move;
+        (flags & PYIID_DEVICE) && c->n_chain == 1 && n <= kReachAtoms && c->reach_wanted &&
+        !c->replays_move;
     const bool order = c->place_stamp == c->struct_stamp && !c->replays_move;
     HIPCHK(launch_pack(c->stream, src, c->elem.as<int32_t>(), n, c->pos.as<AtomRec>(),
                        c->posf.as<float>(), reach ? c->reach.as<double>() : nullptr,
@@ -2841,6 +2843,7 @@ int pyiid_grad_fq(pyiid_ctx* c, int slot, double qbin, void* grad, float* fq, in
   void* gdst = grad;
   const double dq = static_cast<double>(static_cast<float>(qbin));
   c->grad_spread = use_spread_grad(c, t, dq);
+  c->reach_wanted = c->grad_spread;
   if (c->grad_spread) {
     float* fdst = fq;
     bool copy = false;

@@ -67,8 +67,8 @@ inline bool spread_grad_pays(int64_t n, int kinds, int nq, double dq) {
   const double atoms = static_cast<double>(n), q_max = nq * dq;
   const double most = std::max(3.2 + 0.0035 * atoms * (1.0 + nq / 450.0), atoms / 125.0);
   if (kinds > 3 && kinds > most) return false;
-  if (q_max >= 1.0) {
-    // from this many bins on whatever the largest Q
+  if (q_max >= 0.95) {
+    // from this many bins on whatever the largest Q (from about 1 1/A on)
     const int bins = n <= 400                                ? 1
                      : n < 700                               ? 130
                      : n < 1250 || (n < 2500 && q_max < 2.0) ? 257
