@@ -319,6 +319,7 @@ class Context:
         rgrid = np.ascontiguousarray(rgrid, dtype=np.float64)
         check(self.lib.pyiid_set_transform(self.handle, float(rstep), float(qstep), _ptr(rgrid),
                                            len(rgrid), float(qmin), int(nq)))
+        self._transform_sizes = (int(nq), len(rgrid))
 
     def pdf(self, fq, n_r, out=None, flags=0):
         if not flags & PYIID_DEVICE:
@@ -329,6 +330,18 @@ class Context:
         return out
 
     def grad_pdf(self, grad_fq, n_r, out=None, flags=0):
+        """grad G(r) (n, 3, n_r) from grad F(Q) (n, 3, n_q); the C call trusts the sizes, so they
+        are compared with the transform's here."""
+        sizes = getattr(self, "_transform_sizes", None)  # none: the call says that it is not set
+        shape = tuple(grad_fq.shape)
+        if len(shape) != 3 or (sizes and (shape[2], n_r) != sizes):
+            raise ValueError("grad_pdf takes (n, 3, n_q) and n_r of the transform %s, got %s and %d"
+                             % (sizes, shape, n_r))
+        if out is not None:
+            size = out.numel() if hasattr(out, "numel") else out.size
+            if size != shape[0] * shape[1] * n_r:
+                raise ValueError("grad_pdf writes %d x %d x %d values, the output holds %d"
+                                 % (shape[0], shape[1], n_r, size))
         if not flags & PYIID_DEVICE:
             if grad_fq.dtype == np.float64:
                 flags |= PYIID_F64
