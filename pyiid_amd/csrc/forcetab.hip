@@ -19,6 +19,7 @@
 #include <cmath>
 #include <type_traits>
 
+#include "lds_limit.h"
 #include "pair_math.h"
 
 namespace pyiid {
@@ -383,9 +384,8 @@ hipError_t launch_table_force(hipStream_t st, const AtomRec* pos, const ForceUni
   if (n_units == 0) return hipSuccess;
   const size_t lds = force_lds_bytes(n_cell);
   if (lds > kForceLds) return hipErrorInvalidValue;
-  static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(table_force_kernel),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kForceLds));
+  static LdsLimit lds_limit;
+  const hipError_t attr = lds_limit.allow({reinterpret_cast<const void*>(table_force_kernel)}, kForceLds);
   if (attr != hipSuccess) return attr;
   hipLaunchKernelGGL(table_force_kernel, dim3(n_units), dim3(1024), lds, st, pos, units, n_cell,
                      1.0 / force_cell(nq, dq), t4, t2, u, ftab, nq, dq, n, part, perm, conv, out,

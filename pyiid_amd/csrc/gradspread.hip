@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "fq_grid.h"
+#include "lds_limit.h"
 #include "split_gemm.h"
 
 namespace pyiid {
@@ -490,9 +491,8 @@ hipError_t launch_spread_grad(hipStream_t st, const AtomRec* pos, int p0, int n_
                               int k_fixed, const double* reach, void* rows, float* row_scale) {
   const GradLaunch g = grad_launch(n, nq, dq, r_max);
   if (g.lds > kGradLds || n_run > 65535) return hipErrorInvalidValue;
-  static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(spread_grad_kernel),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kGradLds));
+  static LdsLimit lds_limit;
+  const hipError_t attr = lds_limit.allow({reinterpret_cast<const void*>(spread_grad_kernel)}, kGradLds);
   if (attr != hipSuccess) return attr;
   hipLaunchKernelGGL(spread_grad_kernel, dim3(n_atoms, n_run), dim3(g.threads), g.lds, st, pos, p0,
                      3 * n_atoms, runs, g.inv_h, g.nf, g.plane, g.row_len, k_fixed, reach, nq,
@@ -509,9 +509,8 @@ hipError_t launch_spread_both(hipStream_t st, const AtomRec* pos, int n_atoms, c
   const int fq_nf = 12 * nq, stride = fq_grid_stride(nq);
   const size_t lds = std::max(g.lds, sizeof(unsigned long long) * static_cast<size_t>(stride));
   if (lds > kGradLds || n_run > 65535) return hipErrorInvalidValue;
-  static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(spread_both_kernel),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kGradLds));
+  static LdsLimit lds_limit;
+  const hipError_t attr = lds_limit.allow({reinterpret_cast<const void*>(spread_both_kernel)}, kGradLds);
   if (attr != hipSuccess) return attr;
   hipLaunchKernelGGL(spread_both_kernel, dim3(n_atoms + n_units, n_run), dim3(g.threads), lds, st,
                      pos, n_atoms, runs, g.inv_h, g.nf, g.plane, g.row_len, k_fixed, reach, nq,

@@ -35,6 +35,7 @@
 #include <cmath>
 
 #include "fq_grid.h"
+#include "lds_limit.h"
 
 namespace pyiid {
 namespace {
@@ -441,9 +442,8 @@ hipError_t launch_spread_fq(hipStream_t st, const AtomRec* pos, const SpreadUnit
   const int nf = 12 * nq, stride = fq_grid_stride(nq);
   const size_t lds = sizeof(unsigned long long) * static_cast<size_t>(stride);
   if (lds > kSpreadLds) return hipErrorInvalidValue;
-  static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(spread_fq_kernel),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kSpreadLds));
+  static LdsLimit lds_limit;
+  const hipError_t attr = lds_limit.allow({reinterpret_cast<const void*>(spread_fq_kernel)}, kSpreadLds);
   if (attr != hipSuccess) return attr;
   hipLaunchKernelGGL(spread_fq_kernel, dim3(n_units), dim3(1024), lds, st, pos, units, items,
                      dq * nf / (2.0 * M_PI), nf, fq_grid_points(nq), stride, shift,
@@ -493,16 +493,11 @@ hipError_t launch_small_fq(hipStream_t st, const AtomRec* pos, const int* off, i
   const size_t lds = small_fq_lds(nq, n_pair);
   if (lds > kSmallFqLds || n_chain > 65535 || (n_pair != 1 && n_pair != 3 && n_pair != 6))
     return hipErrorInvalidValue;
-  static const hipError_t attr = [] {
-    for (const void* f : {reinterpret_cast<const void*>(small_fq_kernel<1>),
-                          reinterpret_cast<const void*>(small_fq_kernel<3>),
-                          reinterpret_cast<const void*>(small_fq_kernel<6>)}) {
-      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               static_cast<int>(kSmallFqLds));
-      if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
-  }();
+  static LdsLimit lds_limit;
+  const hipError_t attr = lds_limit.allow({reinterpret_cast<const void*>(small_fq_kernel<1>),
+                                           reinterpret_cast<const void*>(small_fq_kernel<3>),
+                                           reinterpret_cast<const void*>(small_fq_kernel<6>)},
+                                          kSmallFqLds);
   if (attr != hipSuccess) return attr;
   const dim3 grid((nq + 63) / 64, n_chain), block(64 * kSmallWaves);
   const double unit = fq_unit(inv_h, 0, scale_bits), near = std::ldexp(1.0, scale_bits - 31);

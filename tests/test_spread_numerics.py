@@ -186,3 +186,54 @@ def test_rules_of_the_dispatch_take_the_faster_kernel(tmp_path):
     assert len(got) == len(MEASURED)
     for row, new in zip(MEASURED, got):
         assert bool(new) == (row[-1] < row[-2]), row
+
+
+HIP_STUB = r"""
+#pragma once
+typedef int hipError_t;
+constexpr hipError_t hipSuccess = 0;
+constexpr int hipFuncAttributeMaxDynamicSharedMemorySize = 8;
+inline int stub_device = 0, stub_calls = 0, stub_fail = 0;
+inline hipError_t hipGetDevice(int* d) { return *d = stub_device, hipSuccess; }
+inline hipError_t hipFuncSetAttribute(const void*, int, int bytes) {
+  ++stub_calls;
+  return stub_fail || bytes != 163840 ? 1 : hipSuccess;
+}
+"""
+
+LDS = r"""
+#include "lds_limit.h"
+int main() {
+  static pyiid::LdsLimit one, two;
+  int a, b;
+  stub_fail = 1;  // an error is passed on, and asked for again
+  if (one.allow({&a, &b}, 163840) == hipSuccess) return 1;
+  stub_fail = 0;
+  stub_calls = 0;
+  for (int round = 0; round < 3; ++round)
+    for (stub_device = 0; stub_device < 8; ++stub_device)
+      if (one.allow({&a, &b}, 163840) != hipSuccess) return 2;
+  if (stub_calls != 16) return 3;  // two kernels on eight devices, once each
+  if (two.allow({&a}, 163840) != hipSuccess || stub_calls != 17) return 4;
+  stub_device = 200;
+  for (int round = 0; round < 2; ++round)
+    if (one.allow({&a, &b}, 163840) != hipSuccess) return 5;
+  return stub_calls == 21 ? 0 : 6;
+}
+"""
+
+
+def test_large_lds_is_asked_for_on_every_device(tmp_path):
+    """Each kernel with more than 64 KB of dynamic LDS, once on each device that a
+    context runs on; no launcher keeps the answer of one device for all."""
+    (tmp_path / "hip").mkdir()
+    (tmp_path / "hip" / "hip_runtime.h").write_text(HIP_STUB)
+    src, exe = tmp_path / "lds.cpp", tmp_path / "lds"
+    src.write_text(LDS)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", str(tmp_path), "-I", CSRC, "-o", str(exe), str(src)],
+                   check=True)
+    assert subprocess.run([str(exe)]).returncode == 0
+    for name in os.listdir(CSRC):
+        if name.endswith(".hip"):
+            text = open(os.path.join(CSRC, name)).read()
+            assert "hipFuncSetAttribute" not in text, name
