@@ -133,7 +133,13 @@ int pyiid_grad_shape(pyiid_ctx *ctx, int *symmetric, int *bins_per_wave, int *gr
  * the fastest.  Off (enable = 0): every call uses fixed default shapes (the
  * ordered F + gradient kernel unless pyiid_set_grad_tiles_per_item is set), so
  * results are the same bit for bit from run to run and context to context;
- * with it on they agree to FP32 rounding.  No counterpart in the reference. */
+ * with it on they agree to FP32 rounding.  The spreading kernels' scales and the
+ * force tables' lengths follow how far a structure's distances reach.  With the
+ * autotuner on, positions in device memory and more than 4,096 atoms are asked
+ * for that once per layout; off, every upload is, so that nothing depends on
+ * positions before it, and the first call after an upload from device memory waits
+ * for the stream (not in a graph capture, which keeps what is known).  No
+ * counterpart in the reference. */
 int pyiid_set_autotune(pyiid_ctx *ctx, int enable);
 /* Summation of the Debye kernels.
  *  - PYIID_PRECISION_DEFAULT: the spreading kernels (fixed-point sums over

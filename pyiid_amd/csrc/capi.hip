@@ -232,7 +232,9 @@ struct pyiid_ctx {
   bool reach_wanted = true;         // the last gradient, if any, asked for it
   // page-locked, written by the forces' kernel: a pair lay past the force table
   double* far_seen = nullptr;
+  bool far_unsure = false;          // since the last wait such a kernel has been launched
   bool extent_old = false;          // it did: take the extent anew
+  bool extent_fresh = false;        // r_max was taken after the last upload, or from it
   Buf place, ordered;               // an atom's place in element order; the positions so
   uint64_t place_stamp = ~0ull;
   bool order_set = false;           // ordered holds the current positions
@@ -343,8 +345,13 @@ int check_ctx(pyiid_ctx* c) {
     HIPCHK(hipStreamSynchronize(c->stream));
     c->arena_used = 0;
   }
-  if (c->far_seen && *static_cast<volatile double*>(c->far_seen) != 0.0) return note_far(c);
-  return PYIID_OK;
+  if (!c->far_seen) return PYIID_OK;
+  // (results that repeat bit for bit cannot depend on when the note arrives)
+  if (!c->autotune && c->far_unsure && !caller_captures(c)) {
+    HIPCHK(hipStreamSynchronize(c->stream));
+    c->far_unsure = false;
+  }
+  return *static_cast<volatile double*>(c->far_seen) != 0.0 ? note_far(c) : PYIID_OK;
 }
 
 // Waits for the stream, hands pending results over and empties the arena.
@@ -353,6 +360,7 @@ int arena_flush(pyiid_ctx* c) {
   for (const auto& o : c->arena_out) std::memcpy(o.dst, o.src, o.bytes);
   c->arena_out.clear();
   c->arena_used = 0;
+  c->far_unsure = false;
   return PYIID_OK;
 }
 
@@ -443,13 +451,31 @@ bool caller_captures(pyiid_ctx* c) {
   return hipStreamIsCapturing(c->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
 
+// Takes r_max of the current layout.
+int set_extent(pyiid_ctx* c, double r_max) {
+  const Hmc& h = c->hmc;
+  if (!c->autotune && r_max != c->r_max && (h.exact_g.exec || h.sur_g.exec)) {
+    // captured proposals have the tables and scales of the old one
+    HIPCHK(hipStreamSynchronize(c->stream));
+    destroy_graph(c->hmc);
+  }
+  c->r_max = r_max;
+  c->extent_off = c->off;
+  c->extent_old = false;
+  c->extent_fresh = true;
+  return PYIID_OK;
+}
+
 // r_max of the current layout, from the device positions when no host upload
-// gave it (once per layout, and again while a position is not finite or after a
-// force table has proved too short; waits for the stream).
+// gave it (waits for the stream).  Once per layout, and again while a position is
+// not finite or after a force table has proved too short; without the autotuner
+// after every upload: then results repeat bit for bit, so that scales and tables
+// must not depend on positions before.
 int ensure_extent(pyiid_ctx* c) {
-  if (c->extent_off == c->off && ((std::isfinite(c->r_max) && !c->extent_old) || c->extent_exact ||
-                                  c->capturing || caller_captures(c)))
-    return PYIID_OK;
+  if (c->extent_off == c->off) {
+    const bool stands = std::isfinite(c->r_max) && !c->extent_old && (c->autotune || c->extent_fresh);
+    if (stands || c->extent_exact || c->capturing || caller_captures(c)) return PYIID_OK;
+  }
   if (c->capturing) return fail(PYIID_E_STATE, "structure changed during graph capture");
   std::vector<double> h(static_cast<size_t>(c->n) * 4);
   if (c->n > 0) {
@@ -457,10 +483,7 @@ int ensure_extent(pyiid_ctx* c) {
                           c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
   }
-  c->r_max = chain_extent(h.data(), 4, c->off);
-  c->extent_off = c->off;
-  c->extent_old = false;
-  return PYIID_OK;
+  return set_extent(c, chain_extent(h.data(), 4, c->off));
 }
 
 // The atoms have moved, or are about to: what was taken from their places is not
@@ -477,6 +500,7 @@ int ensure_packed(pyiid_ctx* c) {
   HIPCHK(launch_pack(c->stream, c->posf.as<float>(), c->elem.as<int32_t>(), c->n,
                      c->pos.as<AtomRec>(), nullptr, nullptr, nullptr, nullptr));
   positions_changed(c);
+  c->extent_fresh = false;
   c->pos_dirty = false;
   return PYIID_OK;
 }
@@ -1891,6 +1915,7 @@ int contract_forces(pyiid_ctx* c, int slot, double qbin, double scale, double* o
                               s.t4.as<float4>(), s.t2.as<float2>(), c->u.as<float>(),
                               t.tab.as<float>(), nq, dq, c->n, s.part.as<double>(), perm, scale,
                               s.direct ? out : nullptr, far_flag(c)));
+    c->far_unsure = true;
     CHK(tm.done());
     if (!s.direct)
       HIPCHK(launch_reduce_force(c->stream, s.part.as<double>(), c->n, s.planes.as<int32_t>(), perm,
@@ -2034,6 +2059,7 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
   // one kernel reads the caller's device positions, or the arena's copy of host
   // ones, and writes the records and the float copy; nothing waits
   positions_changed(c);
+  c->extent_fresh = false;
   const float* src = pos;
   if (!(flags & PYIID_DEVICE) && n > 0) {
     void* p = nullptr;
@@ -2062,10 +2088,8 @@ int set_structure(pyiid_ctx* c, const float* pos, int64_t n, const std::vector<i
     HIPCHK(hipStreamSynchronize(c->stream));
   }
   c->pos_set = true;
-  if (!(flags & PYIID_DEVICE) && n <= kExtentAtoms) {
-    c->r_max = chain_extent(pos, 3, c->off);
-    c->extent_off = c->off;
-    c->extent_old = false;
+  if (!(flags & PYIID_DEVICE) && (n <= kExtentAtoms || !c->autotune)) {
+    CHK(set_extent(c, chain_extent(pos, 3, c->off)));
     c->extent_exact = !c->replays_move;
   }
   return PYIID_OK;
@@ -2398,6 +2422,7 @@ int run_proposal(pyiid_ctx* c, bool surrogate, bool use_graph, int n_leapfrog, d
                     g.epoch == g_alloc_epoch.load();
   if (same) {
     HIPCHK(hipGraphLaunch(g.exec, c->stream));
+    c->far_unsure = true;
     if (surrogate) h.fcur_stale = true;
     return PYIID_OK;
   }
@@ -2848,7 +2873,11 @@ int pyiid_grad_fq(pyiid_ctx* c, int slot, double qbin, void* grad, float* fq, in
     float* fdst = fq;
     bool copy = false;
     if (!(flags & PYIID_DEVICE)) {
+      // (F's place first: whether there is one, and so how F is made, does not
+      // depend on what else is in the arena)
       void *g = nullptr, *f = nullptr;
+      if (fq) CHK(arena_result(c, fq, sizeof(float) * nq, &f));
+      fdst = static_cast<float*>(f);
       CHK(arena_result(c, grad, gbytes, &g));
       copy = !g;
       if (copy) {
@@ -2856,8 +2885,6 @@ int pyiid_grad_fq(pyiid_ctx* c, int slot, double qbin, void* grad, float* fq, in
         g = c->io_c.p;
       }
       gdst = g;
-      if (fq) CHK(arena_result(c, fq, sizeof(float) * nq, &f));
-      fdst = static_cast<float*>(f);
     }
     const bool both = fq && fdst && use_spread_both(c, t, dq);
     const SharedOrder shared(c);
@@ -3207,6 +3234,7 @@ int pyiid_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step, do
     return fail(PYIID_E_INVALID, "need n_proposals >= 0, n_leapfrog >= 1, beta > 0");
   const int B = c->n_chain;
   if (n_proposals == 0) return PYIID_OK;
+  if (!c->autotune) CHK(ensure_extent(c));
   positions_changed(c);
   CHK(prepare_history(c, n_proposals));
   CHK(refresh_exact(c));
@@ -3391,6 +3419,7 @@ int pyiid_sur_hmc_run(pyiid_ctx* c, int n_proposals, int n_leapfrog, double step
   if (min_chain_atoms(c) < 2) return fail(PYIID_E_INVALID, "every chain needs at least two atoms");
   const int B = c->n_chain;
   if (n_proposals == 0) return PYIID_OK;
+  if (!c->autotune) CHK(ensure_extent(c));
   positions_changed(c);
   CHK(prepare_history(c, n_proposals));
   RunClock clock(c, times_ms != nullptr);

@@ -543,3 +543,82 @@ def test_batches_beside_the_lines_between_kernels(ctx, chains, n, kinds):
         want = 10.0 * oracle.wrap_grad_rw(gg, g, target[0])
         assert abs(np.atleast_1d(e)[b] - 10.0 * oracle.get_rw(target[0], g)[0]) < 1e-5
         assert np.abs(f[b * n:(b + 1) * n] - want).max() < 1e-5 * np.abs(want).max()
+
+
+def upload_device(c, pos):
+    import torch
+    c.set_positions(torch.from_numpy(pos).cuda(), flags=_lib.PYIID_DEVICE)
+
+
+@pytest.mark.parametrize("n,device", [(300, True), (4097, False), (4097, True)])
+def test_fixed_shapes_forget_earlier_positions(fixed_shapes, n, device):
+    """Without the autotuner, F and gradient have the same bits in a context that has
+    seen the same atoms sixty times farther apart (whose scale sums most pairs in
+    another way) as in a new one."""
+    nq, qbin = 130, 0.2
+    pos = structures.jitter(structures.fcc_nearest(n), 0.05, seed=1).astype(np.float32)
+    table, index, _ = element_table(np.full(n, 79), qbin, nq)
+    got = []
+    for earlier in (True, False):
+        c = _lib.Context(0)
+        for p in ([60 * pos] if earlier else []) + [pos]:
+            if device:
+                upload_device(c, p)
+            else:
+                c.set_positions(p)
+            if p is not pos or not earlier:  # the layout stays
+                c.set_elements(index)
+                c.set_scatter(_lib.SLOT_FQ, table)
+            fq = np.empty(nq, np.float32)
+            out = [c.fq(_lib.SLOT_FQ, qbin, nq),
+                   c.grad_fq(_lib.SLOT_FQ, qbin, n, nq, fq_out=fq), fq]
+        got.append(out)
+        c.close()
+    same(*got)
+
+
+@pytest.mark.parametrize("earlier,device,graph", [(0.4, True, False), (3, True, True), (1, False, True)])
+def test_fixed_shapes_forget_earlier_forces(fixed_shapes, earlier, device, graph):
+    """The same of forces and of the sampler, 16 chains: the tables' length, past
+    which pairs are summed directly, must not be that of earlier positions (0.4 times
+    as far apart, or 3 times, which makes the tables in another way), nor that of
+    a proposal's graph."""
+    n, chains, nq, qbin, r = 40, 16, 250, 0.1, 2.0 + 0.02 * np.arange(300)
+    base = np.concatenate([structures.jitter(structures.fcc_nearest(n), 0.05, seed=b)
+                           for b in range(chains)]).astype(np.float32)
+    table, _, _ = element_table(np.full(n, 79), qbin, nq)
+    target = np.tile(np.cos(r) + 0.2, (chains, 1))
+
+    def results(earlier, device, graph):
+        import torch
+        c = _lib.Context(0)
+        off = np.arange(chains + 1, dtype=np.int64) * n
+
+        def upload(p):
+            dev = torch.from_numpy(p).cuda()
+            _lib.check(c.lib.pyiid_set_batch(c.handle, dev.data_ptr() if device else p.ctypes.data,
+                                             n * chains, off.ctypes.data, chains,
+                                             _lib.PYIID_DEVICE if device else 0))
+            c.synchronize()
+
+        def forces():
+            return c.pdf_energy_forces(_lib.SLOT_PDF, qbin, target, _lib.POT_RW, 1.0, n * chains)
+        upload(np.float32(earlier) * base)
+        c.set_elements(np.zeros(n * chains, np.int32))
+        c.set_scatter(_lib.SLOT_PDF, table)
+        c.set_transform(0.02, qbin, r, 0.0, nq)
+        out = []
+        forces()
+        for scale in (1, 2):
+            upload(np.float32(scale) * base)
+            out += forces()
+            if scale == 1:
+                c.hmc_setup(_lib.SLOT_PDF, qbin, target, _lib.POT_RW, 10.0, np.full(n * chains, 1.0))
+            # (from the forces of the setup or of the run before)
+            for _ in range(2):
+                out.append(c.hmc_run(4, 5, 0.1, 1.0, 1, chains, use_graph=graph)[0])
+            out += [c.get_positions(n * chains), *forces()]
+        c.close()
+        return out
+    want = results(1, False, False)
+    same(results(earlier, device, graph), want)
