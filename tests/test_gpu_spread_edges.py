@@ -8,6 +8,7 @@ import pytest
 from oracle import scatter as oracle
 from pyiid_amd import _lib, structures
 from pyiid_amd.formfactors import element_table
+from test_gpu_spread import force_check
 
 pytestmark = pytest.mark.gpu
 
@@ -622,3 +623,32 @@ def test_fixed_shapes_forget_earlier_forces(fixed_shapes, earlier, device, graph
         return out
     want = results(1, False, False)
     same(results(earlier, device, graph), want)
+
+
+@pytest.mark.parametrize("cells", [6825, 6826, 6827])
+def test_longest_force_table(ctx, cells):
+    """Force tables that fill the 160 KB of LDS but for 40 and 16 bytes, and a
+    structure that would need a cell more than fits (the recurrence kernel).  The
+    outermost pair then moves on the device to where it reads the table's last
+    cell, a tenth beyond the extent that the table was made for."""
+    nq, qbin = 600, 0.05
+    h = np.pi / (5 * nq * np.float64(np.float32(qbin)))
+    inner = structures.jitter(structures.fcc_nearest(68), 0.05, seed=4)
+    inner -= 0.5 * (inner.min(0) + inner.max(0))
+
+    def structure(length):
+        ends = np.array([(0.5 * length, 0, 0), (-0.5 * length, 0, 0)])
+        return np.concatenate([inner, ends]).astype(np.float32)
+
+    def table_cells(pos):
+        x = pos.astype(np.float64)
+        mid = 0.5 * (x.min(0) + x.max(0))
+        reach = min(np.linalg.norm(x.max(0) - x.min(0)), 2 * np.linalg.norm(x - mid, axis=1).max())
+        return int(1.1 * reach / h + 8)
+    base = structure((cells - 7.5) * h / 1.1)
+    assert table_cells(base) == cells
+    assert (24 * cells <= 160 * 1024) == (cells <= 6826)
+    force_check(ctx, base, base, np.full(70, 79), qbin, nq)
+    pos = structure((cells - 0.6) * h)
+    assert int(np.linalg.norm(pos[-1].astype(np.float64) - pos[-2]) / h) == cells - 1
+    force_check(ctx, pos, base, np.full(70, 79), qbin, nq, lambda p: upload_device(ctx, p))
