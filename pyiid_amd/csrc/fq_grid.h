@@ -50,8 +50,14 @@ __host__ __device__ inline double fq_node(int k) {  // t of node k
 
 // A pair closer than the fixed point's fast range, or at an infinite
 // distance: 64-bit conversions.  Few pairs of a physical structure come here, and
-// those from kFarthest on add nothing.
-__device__ void spread_rare(unsigned long long* hist, int n_grid, double t, double nf,
+// those from kFarthest on add nothing.  A call of its own: within the kernels its
+// constants took 50 of their registers for scalars that did not fit, and a block of
+// spread_fq_kernel with 58 vector registers leaves no room for one of
+// transform_fq_kernel beside it, where several streams share the chip (F of 6,699
+// atoms on three streams in turn 57 us, with up to 56 registers 50; of 20,000 atoms
+// of two elements 421 and 406; on one stream alike, also where all pairs are close:
+// 7,000 atoms, 64 bins to 2 1/A 200 -> 185 us).
+__device__ __noinline__ void spread_rare(unsigned long long* hist, int n_grid, double t, double nf,
                                          double scale) {
   unsigned long long* nodes = hist + n_grid;
   if (!(t < 1e300)) {  // infinite: F is not a number

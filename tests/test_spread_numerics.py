@@ -2,9 +2,11 @@
 share with the host."""
 import os
 import re
+import shutil
 import subprocess
 
 import numpy as np
+import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "pyiid_amd", "csrc")
 
@@ -237,3 +239,33 @@ def test_large_lds_is_asked_for_on_every_device(tmp_path):
         if name.endswith(".hip"):
             text = open(os.path.join(CSRC, name)).read()
             assert "hipFuncSetAttribute" not in text, name
+
+
+def vector_registers(source):
+    """Vector registers of each kernel of a source, as the compiler reports them."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    flags = re.search(r"^HIPFLAGS := (.*?[^\\])$", open(os.path.join(CSRC, "Makefile")).read(), re.S | re.M)
+    flags = flags.group(1).replace("\\\n", " ").replace("$(ARCH)", "gfx950").split()
+    out = subprocess.run([hipcc, *flags, "--cuda-device-only", "-Rpass-analysis=kernel-resource-usage", "-c",
+                          os.path.join(CSRC, source), "-o", os.devnull], capture_output=True, text=True)
+    assert out.returncode == 0, out.stderr
+    found, name = {}, None
+    for line in out.stderr.splitlines():
+        m = re.search(r"Function Name: (\S+)", line)
+        name = m.group(1) if m else name
+        m = re.search(r" VGPRs: (\d+)", line)
+        if m:
+            found[name] = int(m.group(1))
+    return found
+
+
+def test_f_kernels_share_a_cu():
+    """A block of the F spreading kernel and one of its transform (16 waves each,
+    four a SIMD) fit the 512 registers of a SIMD together, by eights: calls on
+    several streams overlap there."""
+    regs = vector_registers("spread.hip")
+    spread, = [v for k, v in regs.items() if "16spread_fq_kernel" in k]
+    transform, = [v for k, v in regs.items() if "transform_fq_kernel" in k]
+    assert 4 * 8 * ((spread + 7) // 8 + (transform + 7) // 8) <= 512, (spread, transform)
