@@ -230,7 +230,7 @@ struct pyiid_ctx {
   Buf reach;                        // double: such a bound on the device
   bool reach_set = false;           // of the current positions
   bool reach_wanted = true;         // the last gradient, if any, asked for it
-  // page-locked, written by the forces' kernel: a pair lay past the force table
+  // at the arena's start, written by the forces' kernel: a pair lay past the force table
   double* far_seen = nullptr;
   bool far_unsure = false;          // since the last wait such a kernel has been launched
   bool extent_old = false;          // it did: take the extent anew
@@ -297,7 +297,7 @@ struct pyiid_ctx {
   // caller's arrays once the call has waited for the stream.
   unsigned char* arena = nullptr;
   bool arena_failed = false;
-  size_t arena_used = 0;
+  size_t arena_used = 0;  // kArenaHead with no array in it
   struct HostCopy {
     void* dst;
     const void* src;
@@ -322,6 +322,7 @@ int ensure_device(pyiid_ctx* c) {
 
 constexpr size_t kArenaBytes = static_cast<size_t>(4) << 20;
 constexpr size_t kArenaMost = static_cast<size_t>(1) << 20;  // of one array
+constexpr size_t kArenaHead = 256;                           // far_seen, before the arrays
 
 void destroy_graph(Hmc& h);
 bool caller_captures(pyiid_ctx* c);
@@ -343,7 +344,7 @@ int check_ctx(pyiid_ctx* c) {
   if (!c->arena_out.empty()) {  // left by a call that failed half way
     c->arena_out.clear();
     HIPCHK(hipStreamSynchronize(c->stream));
-    c->arena_used = 0;
+    c->arena_used = kArenaHead;
   }
   if (!c->far_seen) return PYIID_OK;
   // (results that repeat bit for bit cannot depend on when the note arrives)
@@ -359,24 +360,31 @@ int arena_flush(pyiid_ctx* c) {
   HIPCHK(hipStreamSynchronize(c->stream));
   for (const auto& o : c->arena_out) std::memcpy(o.dst, o.src, o.bytes);
   c->arena_out.clear();
-  c->arena_used = 0;
+  c->arena_used = kArenaHead;
   c->far_unsure = false;
   return PYIID_OK;
+}
+
+// Whether there is an arena; makes it.
+bool have_arena(pyiid_ctx* c) {
+  if (c->arena || c->arena_failed) return c->arena;
+  void* m = nullptr;
+  if (hipHostMalloc(&m, kArenaBytes, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    c->arena_failed = true;
+    return false;
+  }
+  c->arena = static_cast<unsigned char*>(m);
+  c->arena_used = kArenaHead;
+  c->far_seen = static_cast<double*>(m);
+  *c->far_seen = 0.0;
+  return true;
 }
 
 // Arena memory for one array, or null (too large, or none to be had).
 int arena_take(pyiid_ctx* c, size_t bytes, void** p) {
   *p = nullptr;
-  if (bytes == 0 || bytes > kArenaMost || c->arena_failed) return PYIID_OK;
-  if (!c->arena) {
-    void* m = nullptr;
-    if (hipHostMalloc(&m, kArenaBytes, hipHostMallocDefault) != hipSuccess) {
-      (void)hipGetLastError();
-      c->arena_failed = true;
-      return PYIID_OK;
-    }
-    c->arena = static_cast<unsigned char*>(m);
-  }
+  if (bytes == 0 || bytes > kArenaMost || !have_arena(c)) return PYIID_OK;
   if (c->arena_used + bytes > kArenaBytes) {
     if (!c->arena_out.empty()) return PYIID_OK;
     CHK(arena_flush(c));
@@ -1874,15 +1882,7 @@ int reserve_coef(pyiid_ctx* c, int slot, double qbin, double2** coef) {
 // Where the forces' kernel notes a pair past its table (null if there is no
 // page-locked memory: then the table keeps its length).
 double* far_flag(pyiid_ctx* c) {
-  if (!c->far_seen && !caller_captures(c)) {
-    void* m = nullptr;
-    if (hipHostMalloc(&m, sizeof(double), hipHostMallocDefault) == hipSuccess) {
-      c->far_seen = static_cast<double*>(m);
-      *c->far_seen = 0.0;
-    } else {
-      (void)hipGetLastError();
-    }
-  }
+  if (!c->far_seen && !caller_captures(c)) (void)have_arena(c);
   return c->far_seen;
 }
 
@@ -2598,7 +2598,6 @@ int pyiid_destroy(pyiid_ctx* c) {
   }
   for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
   if (c->arena) (void)hipHostFree(c->arena);
-  if (c->far_seen) (void)hipHostFree(c->far_seen);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
   delete c;
   return PYIID_OK;
@@ -2606,7 +2605,7 @@ int pyiid_destroy(pyiid_ctx* c) {
 
 int pyiid_set_stream(pyiid_ctx* c, void* stream) {
   CHK(check_ctx(c));
-  if (c->arena_used > 0) CHK(arena_flush(c));  // inputs the old stream may still read
+  if (c->arena_used > kArenaHead) CHK(arena_flush(c));  // inputs the old stream may still read
   c->stream = stream ? static_cast<hipStream_t>(stream) : c->own_stream;
   destroy_graph(c->hmc);
   return PYIID_OK;
