@@ -503,7 +503,7 @@ __device__ __forceinline__ void put_u(double v, int b, int q, int nq, double dq,
 // Layout of v_mfma_f64_16x16x4 (lane l): A[l % 16][l / 16], B[l / 16][l % 16];
 // result v: row 4 v + l / 16, column l % 16.
 using v4d = double __attribute__((ext_vector_type(4)));
-constexpr int kAdjWaves = 16, kAdjAhead = 1;
+constexpr int kAdjWaves = 16;
 
 __device__ __forceinline__ void adjoint_block(const float* __restrict__ t, int n_r, int nq,
                                               const double* __restrict__ o,
@@ -523,39 +523,32 @@ __device__ __forceinline__ void adjoint_block(const float* __restrict__ t, int n
   const int s1 = static_cast<int>(static_cast<int64_t>(groups) * (sub + 1) / kSub);
   const double *ob = o + static_cast<size_t>(b) * n_r, *gb = g + static_cast<size_t>(b) * n_r;
   v4d acc_o = v4d{0.0, 0.0, 0.0, 0.0}, acc_g = acc_o;
-  for (int s = s0; s < s1; s += kAdjAhead) {
-    double x[kAdjAhead][4], z[kAdjAhead][4];
-    float y[kAdjAhead][4];
+  for (int s = s0; s < s1; ++s) {
+    double x[4], z[4];
+    float y[4];
+    const int at = s * 16 + 4 * (lane >> 4);
+    if (at + 3 < n_r) {
 #pragma unroll
-    for (int a = 0; a < kAdjAhead; ++a) {
-      const int at = min(s + a, s1 - 1) * 16 + 4 * (lane >> 4);
-      if (at + 3 < n_r) {
+      for (int e = 0; e < 4; ++e) {
+        x[e] = ob[at + e];
+        z[e] = gb[at + e];
+        y[e] = t[static_cast<size_t>(at + e) * nq + q];
+      }
+    } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          x[a][e] = ob[at + e];
-          z[a][e] = gb[at + e];
-          y[a][e] = t[static_cast<size_t>(at + e) * nq + q];
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int i = min(at + e, n_r - 1);
-          x[a][e] = at + e < n_r ? ob[i] : 0.0;
-          z[a][e] = at + e < n_r ? gb[i] : 0.0;
-          y[a][e] = at + e < n_r ? t[static_cast<size_t>(i) * nq + q] : 0.f;
-        }
+      for (int e = 0; e < 4; ++e) {
+        const int i = min(at + e, n_r - 1);
+        x[e] = at + e < n_r ? ob[i] : 0.0;
+        z[e] = at + e < n_r ? gb[i] : 0.0;
+        y[e] = at + e < n_r ? t[static_cast<size_t>(i) * nq + q] : 0.f;
       }
     }
 #pragma unroll
-    for (int a = 0; a < kAdjAhead; ++a)
-      if (s + a < s1) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const double tv = static_cast<double>(y[a][e]);
-          acc_o = __builtin_amdgcn_mfma_f64_16x16x4f64(x[a][e], tv, acc_o, 0, 0, 0);
-          acc_g = __builtin_amdgcn_mfma_f64_16x16x4f64(z[a][e], tv, acc_g, 0, 0, 0);
-        }
-      }
+    for (int e = 0; e < 4; ++e) {
+      const double tv = static_cast<double>(y[e]);
+      acc_o = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e], tv, acc_o, 0, 0, 0);
+      acc_g = __builtin_amdgcn_mfma_f64_16x16x4f64(z[e], tv, acc_g, 0, 0, 0);
+    }
   }
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
