@@ -748,6 +748,7 @@ def main():
     value = pairs * NQ * args.steps / elapsed
     roof = grad_roofline(ctx, pos, NQ, 1, fused_ms / max(1, fused_n) / 1e3, "au6699_q1250")
     roof["launches"] = fused_n
+    spreading = grad_kernel_name(ctx)[0] == "spread_grad"
 
     out = {
         "metric": METRIC,
@@ -761,6 +762,12 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f32",
+        # what `value` and `dtype` stand for with the kernels that ran
+        "rate": ("pairs x bins delivered per second; every pair is handled once, whatever the bins"
+                 if spreading else "pairs x bins, each computed, per second"),
+        "arithmetic": ("float32 in and out; FP64 distances, fixed-point sums over pairs; the gradient's "
+                       "product on float32 operands split into two FP16 halves (22 bits), FP32 sums"
+                       if spreading else "float32 in and out; FP64 distances, FP32 recurrences and sums"),
         "data": "synthetic",
         "config": {
             "workload": "Au FCC sphere r=30 A (a=4.08 A, 6699 atoms), sigma=0.05 A seeded "
