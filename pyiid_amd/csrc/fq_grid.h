@@ -121,11 +121,11 @@ __device__ __forceinline__ bool spread_pair(unsigned long long* hist, double t, 
 //
 // Per 64 pairs about 14 FP64 or conversion instructions (distance to 4e-14:
 // a phase of 1,500 rad to 6e-11), 18 FMAs for the window, 6 conversions to
-// integer and 6 ds_add_u64.  The LDS adds bound it (busy 93% of the time, two
-// thirds of that bank conflicts of random addresses); the VALU is busy nearly as
-// long beside it, and 2 blocks (32 waves) per CU hide each other's latency.  A
-// tile off the diagonal needs two comparisons a pair (1,988 -> 1,930 us for 64
-// chains of 5,000 atoms, where every pair took five).
+// integer and 6 ds_add_u64.  The LDS adds bound it (64 chains of 5,000 atoms: busy
+// 89% of the time, two thirds of that bank conflicts of random addresses) and the
+// VALU, busy 95% beside them; 2 blocks (32 waves) per CU hide each other's latency.
+// A tile off the diagonal needs two comparisons a pair (1,988 -> 1,930 us for that
+// batch, where every pair took five; 1,775 us with settled clocks).
 __device__ __forceinline__ void spread_fq_unit(
     const AtomRec* __restrict__ pos, const SpreadUnit& un, const SpreadItem* __restrict__ items,
     double inv_h, int nf, int n_grid, int stride, int shift, float scale, double near,
